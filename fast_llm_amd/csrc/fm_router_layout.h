@@ -1,11 +1,12 @@
 // What the router's forward kernel leaves in its workspace, shared with the sparse-map kernels that consume it.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace fm {
 
-// Per workgroup of the router's forward kernel: 2 * experts + 1 floats.
+// Sums over all tokens, per routed expert and in total.
 struct RouterStats {
     static __host__ __device__ int probability_sum(int e) { return e; }
     static __host__ __device__ int count(int experts, int e) { return experts + e; }
@@ -13,7 +14,9 @@ struct RouterStats {
     static __host__ __device__ int size(int experts) { return 2 * experts + 1; }
 };
 
-constexpr int kMaxRouterBlocks = 1024;
+// One workgroup per CU at most: what a workgroup counts is read by every workgroup of the sparse map, so a finer cut
+// costs there what it gains here.
+constexpr int kMaxRouterBlocks = 256;
 constexpr int kRouterTokensPerBlock = 16;
 
 // Workgroups of the router's forward kernel; workgroup b handles the tokens
@@ -25,6 +28,10 @@ inline int router_blocks(int64_t tokens) {
 inline int64_t router_tokens_per_block(int64_t tokens) {
     const int blocks = router_blocks(tokens);
     return blocks > 0 ? (tokens + blocks - 1) / blocks : 0;
+}
+// The workspace starts with int32 counts [workgroup][expert, the shared ones after the routed ones].
+inline size_t router_counts_bytes(int64_t tokens, int64_t experts) {
+    return sizeof(int32_t) * static_cast<size_t>(router_blocks(tokens)) * static_cast<size_t>(experts);
 }
 
 }  // namespace fm

@@ -1,11 +1,9 @@
 // Top-k routing: for every token the k largest router logits, in descending order, their expert indices, and the
 // softmax over just those k logits in fp32 (reference: MixtureOfExpertMLP._topk_routing,
 // fast_llm/layers/decoder/mlp/mixture_of_experts.py:243-244, i.e. torch.topk followed by torch.softmax(dtype=fp32));
-// and the backward of that pair with respect to the logits.
-//
-// One wavefront per token: lane l keeps the logits of experts l, l + 64, ... in registers (at most kMaxPerLane), and
-// k rounds of a wave-wide arg-max (ties go to the lower expert index) pick the experts. Latency-bound: the whole
-// input is tokens * experts values.
+// the rest of the router's front end around it; and the backward of both with respect to the logits.
+#include <type_traits>
+
 #include "fm_common.h"
 #include "fm_router_layout.h"
 
@@ -14,93 +12,7 @@ namespace fm {
 constexpr int kRoutingThreads = 256;  // 4 tokens per workgroup
 constexpr int kMaxPerLane = 16;       // experts <= 1024
 constexpr int kMaxTopK = 64;
-
-struct Candidate {
-    float value;
-    int index;
-};
-
-// The larger value wins; equal values: the lower index. NaN counts as larger than every number, as in torch.topk
-// (the reference's routing, fast_llm/layers/decoder/mlp/mixture_of_experts.py:243): a token with a NaN logit selects
-// that expert and gets NaN scores, so a broken router shows in the loss instead of silently losing a slot.
-__device__ __forceinline__ Candidate better(Candidate a, Candidate b) {
-    const bool a_nan = a.value != a.value, b_nan = b.value != b.value;
-    const bool same = a_nan == b_nan && (a_nan || a.value == b.value);
-    const bool take_b = (b_nan && !a_nan) || (!a_nan && !b_nan && b.value > a.value) || (same && b.index < a.index);
-    return take_b ? b : a;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kRoutingThreads) void topk_routing_kernel(const T *__restrict__ logits,
-                                                                      int64_t *__restrict__ top_experts,
-                                                                      float *__restrict__ scores, int64_t tokens,
-                                                                      int experts, int k) {
-    const int lane = threadIdx.x & 63;
-    const int64_t token = static_cast<int64_t>(blockIdx.x) * (kRoutingThreads / 64) + (threadIdx.x >> 6);
-    if (token >= tokens) return;
-    const T *row = logits + token * experts;
-    float values[kMaxPerLane];
-#pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-        const int e = q * 64 + lane;
-        values[q] = e < experts ? to_float(row[e]) : -INFINITY;
-    }
-    float top_value = 0.f, sum = 0.f, my_value = 0.f;
-    for (int j = 0; j < k; ++j) {
-        Candidate best{-INFINITY, 0x7fffffff};
-#pragma unroll
-        for (int q = 0; q < kMaxPerLane; ++q) {
-            const int e = q * 64 + lane;
-            if (e < experts) best = better(best, Candidate{values[q], e});
-        }
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) {
-            Candidate other{__shfl_xor(best.value, offset, 64), __shfl_xor(best.index, offset, 64)};
-            best = better(best, other);
-        }
-        // Every lane now holds the winner; its owner retires it.
-#pragma unroll
-        for (int q = 0; q < kMaxPerLane; ++q)
-            if (q * 64 + lane == best.index) values[q] = -INFINITY;
-        if (j == 0) top_value = best.value;
-        const float shifted = __expf(best.value - top_value);
-        sum += shifted;
-        if (lane == j) {  // lane j keeps slot j (k <= 64)
-            my_value = shifted;
-            top_experts[token * k + j] = best.index;
-        }
-    }
-    if (lane < k) scores[token * k + lane] = my_value / sum;
-}
-
-// grad_logits[t, e] = scores[t, j] * (grad_scores[t, j] - sum_i scores[t, i] * grad_scores[t, i]) where e is the j-th
-// selected expert of token t, and 0 for every expert that was not selected.
-template <typename T>
-__global__ __launch_bounds__(kRoutingThreads) void topk_routing_backward_kernel(
-    const float *__restrict__ grad_scores, const float *__restrict__ scores, const int64_t *__restrict__ top_experts,
-    T *__restrict__ grad_logits, int64_t tokens, int experts, int k) {
-    const int lane = threadIdx.x & 63;
-    const int64_t token = static_cast<int64_t>(blockIdx.x) * (kRoutingThreads / 64) + (threadIdx.x >> 6);
-    if (token >= tokens) return;
-    const float score = lane < k ? scores[token * k + lane] : 0.f;
-    const float grad = lane < k ? grad_scores[token * k + lane] : 0.f;
-    const float dot = wave_sum(score * grad);
-    const float grad_logit = score * (grad - dot);
-    const int expert = lane < k ? static_cast<int>(top_experts[token * k + lane]) : -1;
-    T *row = grad_logits + token * experts;
-    // Every element of the row is written once, by the lane that owns it: the value of the slot that selected it, or 0.
-    for (int base = 0; base < experts; base += 64) {
-        const int e = base + lane;
-        float value = 0.f;
-        for (int j = 0; j < k; ++j) {
-            const int selected = __shfl(expert, j, 64);
-            const float selected_grad = __shfl(grad_logit, j, 64);
-            if (selected == e) value = selected_grad;
-        }
-        if (e < experts) row[e] = from_float<T>(value);
-    }
-}
-
+constexpr int kRouterMaxThreads = 1024;
 
 // ---- the router front end: routing, auxiliary losses and shared experts in one pass ---------------------------
 // Everything MixtureOfExpertMLP does between the router's logits and the sparse map (reference:
@@ -110,40 +22,76 @@ __global__ __launch_bounds__(kRoutingThreads) void topk_routing_backward_kernel(
 //   * top-k experts and the fp32 softmax over their logits (:243-244);
 //   * the load-balancing loss sum_e mean_t(softmax(logits)[t, e]) * mean_t(selected[t, e]) (:245-254);
 //   * shared experts, prepended to every token's slots with score 1 (:264-278).
-// A workgroup walks a fixed range of tokens, one wavefront per token, and keeps the per-expert sums of its tokens in
-// registers; the sums of all workgroups are then added in a fixed order by a second kernel, so results do not depend
-// on scheduling.
-constexpr int kRouterWaves = kRoutingThreads / 64;
+// A workgroup walks a fixed range of tokens and keeps the per-expert sums of its tokens in registers; the sums of all
+// workgroups are then added in a fixed order by a second kernel, so results do not depend on scheduling.
+//
+// What bounds it is the chain of dependent steps of a token: load a row, then k rounds of an arg-max. A token is
+// therefore shared by no more lanes than it has experts (kGroup = 8 .. 64 lanes, 8 tokens per wavefront at 8
+// experts), a lane holds no more logits than there are (kPerLane), and a round is a maximum of integer keys over the
+// group in DPP and lane-swap instructions followed by one ballot. (A wavefront per token with 16 logits per lane at any
+// number of experts and a butterfly of (value, index) pairs through LDS: 66 us forward, 100 us backward at 16384 tokens
+// and 8 of 128 experts; now 17 and 11. 96 tokens: 42 us, now 5.)
+template <int kGroup, int kPerLane>
+struct RouterShape {
+    static constexpr int kTokens = 64 / kGroup;  // tokens of a wavefront at a time
+    static_assert(kGroup == 64 || kPerLane == 1, "more than one logit per lane: the whole wavefront shares a token");
+};
 
-__device__ __forceinline__ float wave_max(float value) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) value = fmaxf(value, __shfl_xor(value, offset, 64));
+// A float as an integer that orders like it (and -0 like +0); 0 is below -infinity. NaN is above every number, as in
+// torch.topk: a token with a NaN logit selects that expert and gets NaN scores, so a broken router shows in the loss
+// instead of silently losing a slot.
+__device__ __forceinline__ uint32_t order_key(float value) {
+    if (value != value) return 0xffffffffu;
+    const uint32_t bits = __float_as_uint(value + 0.f);
+    return bits & 0x80000000u ? ~bits : bits | 0x80000000u;
+}
+__device__ __forceinline__ float value_of_key(uint32_t key) {
+    if (key == 0xffffffffu) return __uint_as_float(0x7fc00000u);
+    return __uint_as_float(key & 0x80000000u ? key & 0x7fffffffu : ~key);
+}
+constexpr uint32_t kKeyOfMinusInfinity = 0x007fffffu;
+
+// Reduction over the `kGroup` lanes that share a token; every lane gets the result.
+template <int kGroup, typename V, typename Op>
+__device__ __forceinline__ V group_reduce(V value, Op op) {
+    static_assert(sizeof(V) == 4 && kGroup >= 8 && kGroup <= 64, "32-bit values, groups of 8 to 64 lanes");
+    const auto dpp = [&](auto control) {
+        return __builtin_bit_cast(V, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, value), decltype(control)::value, 0xf, 0xf, true));
+    };
+    value = op(value, dpp(std::integral_constant<int, 0xB1>{}));   // lane ^ 1
+    value = op(value, dpp(std::integral_constant<int, 0x4E>{}));   // lane ^ 2
+    value = op(value, dpp(std::integral_constant<int, 0x141>{}));  // the other four of eight (mirrored)
+    if constexpr (kGroup >= 16) value = op(value, dpp(std::integral_constant<int, 0x140>{}));  // the other eight of sixteen
+    if constexpr (kGroup >= 32) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, value);
+        const auto rows = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+        value = op(__builtin_bit_cast(V, static_cast<uint32_t>(rows[0])), __builtin_bit_cast(V, static_cast<uint32_t>(rows[1])));
+    }
+    if constexpr (kGroup >= 64) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, value);
+        const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+        value = op(__builtin_bit_cast(V, static_cast<uint32_t>(halves[0])), __builtin_bit_cast(V, static_cast<uint32_t>(halves[1])));
+    }
     return value;
 }
-
-// log(sum_e exp(values[e])) over the experts of a token (values of absent experts are -inf).
-__device__ __forceinline__ float wave_logsumexp(const float (&values)[kMaxPerLane], int experts) {
-    float maximum = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q)
-        if (q * 64 < experts) maximum = fmaxf(maximum, values[q]);
-    maximum = wave_max(maximum);
-    float sum = 0.f;
-#pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q)
-        if (q * 64 < experts) sum += __expf(values[q] - maximum);
-    return maximum + logf(wave_sum(sum));
+template <int kGroup>
+__device__ __forceinline__ float group_sum(float value) {
+    return group_reduce<kGroup>(value, [](float a, float b) { return a + b; });
+}
+template <int kGroup>
+__device__ __forceinline__ uint32_t group_max(uint32_t value) {
+    return group_reduce<kGroup>(value, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 
 // The logits of a token as the router sees them: raw, and after the jitter (rounded to T like the reference's
-// `logits * noise`).
-template <typename T>
+// `logits * noise`). Lane l of the group holds experts l, l + kGroup, ...; absent ones are -infinity.
+template <typename T, int kGroup, int kPerLane>
 __device__ __forceinline__ void load_router_row(const T *logits, const T *noise, int64_t token, int experts, int lane,
-                                                float (&raw)[kMaxPerLane], float (&routed)[kMaxPerLane],
-                                                float (&factor)[kMaxPerLane]) {
+                                                float (&raw)[kPerLane], float (&routed)[kPerLane],
+                                                float (&factor)[kPerLane]) {
 #pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-        const int e = q * 64 + lane;
+    for (int q = 0; q < kPerLane; ++q) {
+        const int e = q * kGroup + lane;
         raw[q] = routed[q] = -INFINITY;
         factor[q] = 1.f;
         if (e < experts) {
@@ -156,142 +104,241 @@ __device__ __forceinline__ void load_router_row(const T *logits, const T *noise,
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kRoutingThreads) void router_forward_kernel(
+// log(sum_e exp(values[e])) over the experts of a token, given the largest of them.
+template <int kGroup, int kPerLane>
+__device__ __forceinline__ float group_logsumexp(const float (&values)[kPerLane], float maximum) {
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < kPerLane; ++q) sum += __expf(values[q] - maximum);
+    return maximum + logf(group_sum<kGroup>(sum));
+}
+
+// `block_counts`: [workgroup][expert], may be null.
+// kStatistics: also logsumexp, softmax sums and z-loss sums, which only the auxiliary losses and their gradients need.
+template <typename T, int kGroup, int kPerLane, bool kStatistics>
+__global__ __launch_bounds__(kRouterMaxThreads) void router_forward_kernel(
     const T *__restrict__ logits, const T *__restrict__ noise, int64_t *__restrict__ top_experts,
-    float *__restrict__ scores, float *__restrict__ lse, float *__restrict__ partials, int64_t tokens,
-    int64_t per_block, int experts, int k, int shared) {
-    extern __shared__ float block_sums[];  // [waves][stats]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *__restrict__ scores, float *__restrict__ lse, int32_t *__restrict__ block_counts,
+    float *__restrict__ block_sums, int64_t tokens, int64_t per_block, int experts, int k, int shared) {
+    constexpr int kTokens = RouterShape<kGroup, kPerLane>::kTokens;
+    extern __shared__ float lds_sums[];  // [waves][stats]
+    const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int lane = threadIdx.x & (kGroup - 1), group = (threadIdx.x & 63) / kGroup;
     const int64_t begin = blockIdx.x * per_block, end = min(begin + per_block, tokens);
     const int slots = shared + k;
-    float probability_sum[kMaxPerLane], count[kMaxPerLane], z_sum = 0.f;
+    float probability_sum[kPerLane], z_sum = 0.f;
+    int32_t count[kPerLane];
 #pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) probability_sum[q] = count[q] = 0.f;
+    for (int q = 0; q < kPerLane; ++q) probability_sum[q] = 0.f, count[q] = 0;
 
-    for (int64_t token = begin + wave; token < end; token += kRouterWaves) {
-        float raw[kMaxPerLane], values[kMaxPerLane], factor[kMaxPerLane];
-        load_router_row(logits, noise, token, experts, lane, raw, values, factor);
-        const float lse_routed = wave_logsumexp(values, experts);
-        const float lse_raw = noise != nullptr ? wave_logsumexp(raw, experts) : lse_routed;
-        if (lane == 0) {
-            lse[2 * token] = lse_routed;
-            lse[2 * token + 1] = lse_raw;
+    for (int64_t first = begin + wave * kTokens; first < end; first += waves * kTokens) {
+        // Lanes of groups past the last token work on the last one and keep nothing of it.
+        const bool valid = first + group < end;
+        const int64_t token = valid ? first + group : end - 1;
+        float raw[kPerLane], values[kPerLane], factor[kPerLane];
+        load_router_row<T, kGroup, kPerLane>(logits, noise, token, experts, lane, raw, values, factor);
+        uint32_t key[kPerLane], best = 0;
+#pragma unroll
+        for (int q = 0; q < kPerLane; ++q) {
+            key[q] = q * kGroup + lane < experts ? order_key(values[q]) : 0u;
+            best = max(best, key[q]);
         }
-        z_sum += lse_raw * lse_raw;
+        best = group_max<kGroup>(best);
+        const float top_value = value_of_key(best);
+        if constexpr (kStatistics) {
+            const float lse_routed = group_logsumexp<kGroup, kPerLane>(values, top_value);
+            float lse_raw = lse_routed;
+            if (noise != nullptr) {
+                uint32_t raw_best = 0;
 #pragma unroll
-        for (int q = 0; q < kMaxPerLane; ++q)
-            if (q * 64 + lane < experts) probability_sum[q] += __expf(values[q] - lse_routed);
-
-        float top_value = 0.f, sum = 0.f, my_value = 0.f;
-        for (int j = 0; j < k; ++j) {
-            Candidate best{-INFINITY, 0x7fffffff};
-#pragma unroll
-            for (int q = 0; q < kMaxPerLane; ++q) {
-                const int e = q * 64 + lane;
-                if (e < experts) best = better(best, Candidate{values[q], e});
+                for (int q = 0; q < kPerLane; ++q)
+                    raw_best = max(raw_best, q * kGroup + lane < experts ? order_key(raw[q]) : 0u);
+                lse_raw = group_logsumexp<kGroup, kPerLane>(raw, value_of_key(group_max<kGroup>(raw_best)));
             }
-#pragma unroll
-            for (int offset = 32; offset > 0; offset >>= 1) {
-                Candidate other{__shfl_xor(best.value, offset, 64), __shfl_xor(best.index, offset, 64)};
-                best = better(best, other);
-            }
-#pragma unroll
-            for (int q = 0; q < kMaxPerLane; ++q)
-                if (q * 64 + lane == best.index) {
-                    values[q] = -INFINITY;
-                    count[q] += 1.f;
+            if (valid) {
+                if (lane == 0) {
+                    lse[2 * token] = lse_routed;
+                    lse[2 * token + 1] = lse_raw;
+                    z_sum += lse_raw * lse_raw;
                 }
-            if (j == 0) top_value = best.value;
-            const float shifted = __expf(best.value - top_value);
-            sum += shifted;
-            if (lane == j) {
-                my_value = shifted;
-                top_experts[token * slots + shared + j] = best.index;
+#pragma unroll
+                for (int q = 0; q < kPerLane; ++q)
+                    if (q * kGroup + lane < experts) probability_sum[q] += __expf(values[q] - lse_routed);
             }
         }
-        if (lane < k) scores[token * slots + shared + lane] = my_value / sum;
-        if (lane < shared) {
-            top_experts[token * slots + lane] = experts + lane;
-            scores[token * slots + lane] = 1.f;
-        }
-    }
 
-    // Sums of the workgroup's tokens: the four wavefronts' registers, added in wavefront order.
-    const int stats = RouterStats::size(experts);
-    float *mine = block_sums + wave * stats;
+        float sum = 0.f, my_value = 0.f;
+        int my_expert = 0;
+        for (int j = 0; j < k; ++j) {
+            if (j > 0) {
+                best = 0;
 #pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-        const int e = q * 64 + lane;
-        if (e < experts) {
-            mine[RouterStats::probability_sum(e)] = probability_sum[q];
-            mine[RouterStats::count(experts, e)] = count[q];
+                for (int q = 0; q < kPerLane; ++q) best = max(best, key[q]);
+                best = group_max<kGroup>(best);
+            }
+            // The lowest expert with the largest key. A selected expert is then worth -infinity.
+            int winner = -1;
+#pragma unroll
+            for (int q = 0; q < kPerLane; ++q) {
+                uint64_t owners = __ballot(key[q] == best);
+                if constexpr (kGroup < 64) owners = (owners >> (group * kGroup)) & ((1ull << kGroup) - 1);
+                if (winner < 0 && owners != 0) winner = q * kGroup + __ffsll(static_cast<unsigned long long>(owners)) - 1;
+            }
+#pragma unroll
+            for (int q = 0; q < kPerLane; ++q)
+                if (q * kGroup + lane == winner) {
+                    key[q] = kKeyOfMinusInfinity;
+                    count[q] += valid ? 1 : 0;
+                }
+            const float shifted = __expf(value_of_key(best) - top_value);
+            sum += shifted;
+            if (lane == j) {  // lane j keeps slot j
+                my_value = shifted;
+                my_expert = winner;
+            }
+        }
+        if (valid) {
+            if (lane < k) {
+                top_experts[token * slots + shared + lane] = my_expert;
+                scores[token * slots + shared + lane] = my_value / sum;
+            }
+            for (int j = lane; j < shared; j += kGroup) {
+                top_experts[token * slots + j] = experts + j;
+                scores[token * slots + j] = 1.f;
+            }
         }
     }
-    if (lane == 0) mine[RouterStats::z_sum(experts)] = z_sum;
+
+    // Sums of the workgroup's tokens: over the groups of a wavefront, then over the wavefronts in their order.
+#pragma unroll
+    for (int offset = kGroup; offset < 64; offset <<= 1) {
+#pragma unroll
+        for (int q = 0; q < kPerLane; ++q) {
+            count[q] += __shfl_xor(count[q], offset, 64);
+            if constexpr (kStatistics) probability_sum[q] += __shfl_xor(probability_sum[q], offset, 64);
+        }
+        if constexpr (kStatistics) z_sum += __shfl_xor(z_sum, offset, 64);
+    }
+    const int columns = kStatistics ? RouterStats::size(experts) : experts;
+    int32_t *wave_counts = reinterpret_cast<int32_t *>(lds_sums) + wave * columns;
+    float *wave_sums = lds_sums + wave * columns + experts;
+    if (group == 0) {
+#pragma unroll
+        for (int q = 0; q < kPerLane; ++q) {
+            const int e = q * kGroup + lane;
+            if (e < experts) {
+                wave_counts[e] = count[q];
+                if constexpr (kStatistics) wave_sums[e] = probability_sum[q];
+            }
+        }
+        if (kStatistics && lane == 0) wave_sums[experts] = z_sum;
+    }
     __syncthreads();
-    for (int c = threadIdx.x; c < stats; c += kRoutingThreads) {
-        float total = 0.f;
-        for (int w = 0; w < kRouterWaves; ++w) total += block_sums[w * stats + c];
-        partials[static_cast<int64_t>(blockIdx.x) * stats + c] = total;
+    if (block_counts == nullptr) return;
+    for (int c = threadIdx.x; c < columns; c += blockDim.x) {
+        if (c < experts) {
+            int32_t total = 0;
+            for (int w = 0; w < waves; ++w) total += reinterpret_cast<const int32_t *>(lds_sums)[w * columns + c];
+            block_counts[static_cast<int64_t>(blockIdx.x) * (experts + shared) + c] = total;
+        } else {
+            float total = 0.f;
+            for (int w = 0; w < waves; ++w) total += lds_sums[w * columns + c];
+            block_sums[static_cast<int64_t>(blockIdx.x) * (experts + 1) + c - experts] = total;
+        }
+    }
+    // Every token of the range visits the shared experts.
+    for (int j = threadIdx.x; j < shared; j += blockDim.x)
+        block_counts[static_cast<int64_t>(blockIdx.x) * (experts + shared) + experts + j] = static_cast<int32_t>(max(end - begin, int64_t(0)));
+}
+
+// statistics = the sums over the workgroups of the forward kernel (softmax sums and z-loss sum as doubles: up to 256
+// terms of similar size), losses[0] = load-balancing loss, losses[1] = z-loss. One workgroup: 16 threads share a
+// column, each adds up to 16 of its terms, all requested at once (18 us at 128 experts and 256 workgroups; one thread per
+// column that walked down 1024 workgroups took 261).
+__global__ __launch_bounds__(1024) void router_finish_kernel(const int32_t *__restrict__ block_counts,
+                                                            const float *__restrict__ block_sums,
+                                                            float *__restrict__ statistics, float *__restrict__ losses,
+                                                            int blocks, int64_t tokens, int experts, int shared) {
+    static_assert(kMaxRouterBlocks == 256, "16 x 16 terms per column");
+    __shared__ double lds_sums[16][64];
+    __shared__ int32_t lds_counts[16][64];
+    const int column = threadIdx.x & 63, part = threadIdx.x >> 6;
+    double balance = 0.0;
+    for (int base = 0; base < experts + 1; base += 64) {
+        const int c = base + column;
+        float sums[16];
+        int32_t counts[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int b = part * 16 + i;
+            sums[i] = b < blocks && c < experts + 1 ? block_sums[static_cast<int64_t>(b) * (experts + 1) + c] : 0.f;
+            counts[i] = b < blocks && c < experts ? block_counts[static_cast<int64_t>(b) * (experts + shared) + c] : 0;
+        }
+        double sum = 0.0;
+        int32_t count = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum += sums[i], count += counts[i];
+        lds_sums[part][column] = sum;
+        lds_counts[part][column] = count;
+        __syncthreads();
+        if (part == 0 && c < experts + 1) {
+            sum = 0.0, count = 0;
+            for (int p = 0; p < 16; ++p) sum += lds_sums[p][column], count += lds_counts[p][column];
+            if (c < experts) {
+                statistics[RouterStats::probability_sum(c)] = static_cast<float>(sum);
+                statistics[RouterStats::count(experts, c)] = static_cast<float>(count);
+                balance += sum * count;
+            } else {
+                statistics[RouterStats::z_sum(experts)] = static_cast<float>(sum);
+                losses[1] = static_cast<float>(sum / static_cast<double>(tokens));
+            }
+        }
+        __syncthreads();
+    }
+    if (part == 0) {
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) balance += __shfl_xor(balance, offset, 64);
+        if (column == 0) losses[0] = static_cast<float>(balance / static_cast<double>(tokens) / static_cast<double>(tokens));
     }
 }
 
-// statistics[c] = sum over the workgroups of the forward kernel, in workgroup order.
-__global__ __launch_bounds__(kRoutingThreads) void router_reduce_kernel(const float *__restrict__ partials,
-                                                                       float *__restrict__ statistics, int blocks,
-                                                                       int stats) {
-    const int c = blockIdx.x * kRoutingThreads + threadIdx.x;
-    if (c >= stats) return;
-    double total = 0.0;  // up to 1024 terms of similar size: fp32 would lose about 1e-5 of the sum
-    for (int b = 0; b < blocks; ++b) total += partials[static_cast<int64_t>(b) * stats + c];
-    statistics[c] = static_cast<float>(total);
-}
-
-// losses[0] = load-balancing loss, losses[1] = z-loss. One workgroup.
-__global__ __launch_bounds__(kRoutingThreads) void router_losses_kernel(const float *__restrict__ statistics,
-                                                                       float *__restrict__ losses, int64_t tokens,
-                                                                       int experts) {
-    __shared__ float wave_totals[kRouterWaves];
-    float total = 0.f;
-    for (int e = threadIdx.x; e < experts; e += kRoutingThreads)
-        total += statistics[RouterStats::probability_sum(e)] * statistics[RouterStats::count(experts, e)];
-    total = wave_sum(total);
-    if ((threadIdx.x & 63) == 0) wave_totals[threadIdx.x >> 6] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float sum = 0.f;
-        for (int w = 0; w < kRouterWaves; ++w) sum += wave_totals[w];
-        const float count = static_cast<float>(tokens);
-        losses[0] = sum / count / count;
-        losses[1] = statistics[RouterStats::z_sum(experts)] / count;
-    }
-}
-
-// Gradient of the raw logits: through the top-k softmax (as topk_routing_backward_kernel), plus, scaled by the constant
-// gradients the reference attaches to its auxiliary losses (functional/utils.py:63-71),
+// Gradient of the raw logits: through the top-k softmax,
+//   scores[t, j] * (grad_scores[t, j] - sum_i scores[t, i] * grad_scores[t, i]) for the j-th selected expert of token t
+// and 0 for an expert that was not selected; plus, scaled by the constant gradients the reference attaches to its auxiliary losses (functional/utils.py:63-71),
 //   load balancing:  aux_scale * p[t, e] * (count[e] - sum_i p[t, i] * count[i]),  p = softmax of the routed logits
 //   z-loss:          z_scale * lse_raw[t] * softmax(raw logits)[t, e]
 // with aux_scale = aux_grad / tokens^2 and z_scale = 2 * z_grad / tokens; the routed part is multiplied by the jitter.
-template <typename T>
+template <typename T, int kGroup, int kPerLane>
 __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
     const float *__restrict__ grad_scores, const float *__restrict__ scores, const int64_t *__restrict__ top_experts,
     const T *__restrict__ logits, const T *__restrict__ noise, const float *__restrict__ lse,
     const float *__restrict__ statistics, T *__restrict__ grad_logits, float aux_scale, float z_scale, int64_t tokens,
     int experts, int k, int shared) {
-    const int lane = threadIdx.x & 63;
-    const int64_t token = static_cast<int64_t>(blockIdx.x) * kRouterWaves + (threadIdx.x >> 6);
-    if (token >= tokens) return;
+    constexpr int kTokens = RouterShape<kGroup, kPerLane>::kTokens;
+    const int lane = threadIdx.x & (kGroup - 1), group = (threadIdx.x & 63) / kGroup;
+    const int64_t mine = (static_cast<int64_t>(blockIdx.x) * (kRoutingThreads / 64) + (threadIdx.x >> 6)) * kTokens + group;
+    const bool valid = mine < tokens;
+    const int64_t token = valid ? mine : tokens - 1;
     const int slots = shared + k;
-    float raw[kMaxPerLane], routed[kMaxPerLane], factor[kMaxPerLane], grad[kMaxPerLane];
-    load_router_row(logits, noise, token, experts, lane, raw, routed, factor);
-    const float lse_routed = lse[2 * token], lse_raw = lse[2 * token + 1];
+    float raw[kPerLane], routed[kPerLane], factor[kPerLane], grad[kPerLane];
+    // The logits are only needed for the losses and the jitter.
+    const bool with_losses = aux_scale != 0.f || z_scale != 0.f;
+    if (with_losses || noise != nullptr) {
+        load_router_row<T, kGroup, kPerLane>(logits, noise, token, experts, lane, raw, routed, factor);
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPerLane; ++q) factor[q] = 1.f;
+    }
+    const float lse_routed = with_losses ? lse[2 * token] : 0.f, lse_raw = with_losses ? lse[2 * token + 1] : 0.f;
+    const float score = lane < k ? scores[token * slots + shared + lane] : 0.f;
+    const float grad_score = lane < k ? grad_scores[token * slots + shared + lane] : 0.f;
+    const int expert = lane < k ? static_cast<int>(top_experts[token * slots + shared + lane]) : -1;
 
     // Load balancing.
     float weighted = 0.f;
 #pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-        const int e = q * 64 + lane;
+    for (int q = 0; q < kPerLane; ++q) {
+        const int e = q * kGroup + lane;
         grad[q] = 0.f;
         if (e < experts && aux_scale != 0.f) {
             const float probability = __expf(routed[q] - lse_routed);
@@ -301,31 +348,28 @@ __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
         }
     }
     if (aux_scale != 0.f) {
-        weighted = wave_sum(weighted);
+        weighted = group_sum<kGroup>(weighted);
 #pragma unroll
-        for (int q = 0; q < kMaxPerLane; ++q) {
-            const int e = q * 64 + lane;
+        for (int q = 0; q < kPerLane; ++q) {
+            const int e = q * kGroup + lane;
             if (e < experts) grad[q] = aux_scale * (grad[q] - __expf(routed[q] - lse_routed) * weighted);
         }
     }
     // Top-k softmax.
-    const float score = lane < k ? scores[token * slots + shared + lane] : 0.f;
-    const float grad_score = lane < k ? grad_scores[token * slots + shared + lane] : 0.f;
-    const float dot = wave_sum(score * grad_score);
+    const float dot = group_sum<kGroup>(score * grad_score);
     const float grad_selected = score * (grad_score - dot);
-    const int expert = lane < k ? static_cast<int>(top_experts[token * slots + shared + lane]) : -1;
     for (int j = 0; j < k; ++j) {
-        const int selected = __shfl(expert, j, 64);
-        const float value = __shfl(grad_selected, j, 64);
+        const int selected = __shfl(expert, j, kGroup);
+        const float value = __shfl(grad_selected, j, kGroup);
 #pragma unroll
-        for (int q = 0; q < kMaxPerLane; ++q)
-            if (q * 64 + lane == selected) grad[q] += value;
+        for (int q = 0; q < kPerLane; ++q)
+            if (q * kGroup + lane == selected) grad[q] += value;
     }
     // Back through the jitter; z-loss.
 #pragma unroll
-    for (int q = 0; q < kMaxPerLane; ++q) {
-        const int e = q * 64 + lane;
-        if (e < experts) {
+    for (int q = 0; q < kPerLane; ++q) {
+        const int e = q * kGroup + lane;
+        if (valid && e < experts) {
             float value = grad[q] * factor[q];
             if (z_scale != 0.f) value += z_scale * lse_raw * __expf(raw[q] - lse_raw);
             grad_logits[token * experts + e] = from_float<T>(value);
@@ -333,56 +377,25 @@ __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
     }
 }
 
+// Runs the statement with kGroup and kPerLane: the fewest lanes per token that hold its logits, one each as long as a
+// wavefront suffices.
+#define FM_DISPATCH_ROUTER_SHAPE(experts, kGroup, kPerLane, ...)                                        \
+    if (experts <= 8) { constexpr int kGroup = 8, kPerLane = 1; __VA_ARGS__; }                          \
+    else if (experts <= 16) { constexpr int kGroup = 16, kPerLane = 1; __VA_ARGS__; }                   \
+    else if (experts <= 32) { constexpr int kGroup = 32, kPerLane = 1; __VA_ARGS__; }                   \
+    else if (experts <= 64) { constexpr int kGroup = 64, kPerLane = 1; __VA_ARGS__; }                   \
+    else if (experts <= 128) { constexpr int kGroup = 64, kPerLane = 2; __VA_ARGS__; }                  \
+    else if (experts <= 256) { constexpr int kGroup = 64, kPerLane = 4; __VA_ARGS__; }                  \
+    else { constexpr int kGroup = 64, kPerLane = kMaxPerLane; __VA_ARGS__; }
+
 }  // namespace fm
 
 using namespace fm;
 
-extern "C" int fm_topk_routing(const void *logits, void *top_experts, void *scores, int64_t num_tokens,
-                               int64_t num_experts, int64_t experts_per_token, int dtype, void *stream_) {
-    const char *name = "fm_topk_routing";
-    FM_REQUIRE(valid_dtype(dtype), "%s: bad dtype %d", name, dtype);
-    FM_REQUIRE(num_tokens >= 0 && num_experts > 0 && num_experts <= 64 * kMaxPerLane, "%s: %lld experts (1..%d)", name,
-               static_cast<long long>(num_experts), 64 * kMaxPerLane);
-    FM_REQUIRE(experts_per_token > 0 && experts_per_token <= num_experts && experts_per_token <= kMaxTopK,
-               "%s: experts_per_token %lld", name, static_cast<long long>(experts_per_token));
-    if (num_tokens == 0) return FM_OK;
-    FM_REQUIRE(logits && top_experts && scores, "%s: null tensor", name);
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    const int64_t blocks = (num_tokens + kRoutingThreads / 64 - 1) / (kRoutingThreads / 64);
-    FM_REQUIRE(blocks < (int64_t(1) << 31), "%s: too many tokens", name);
-    FM_DISPATCH_DTYPE(dtype, T, {
-        topk_routing_kernel<T><<<blocks, kRoutingThreads, 0, stream>>>(
-            static_cast<const T *>(logits), static_cast<int64_t *>(top_experts), static_cast<float *>(scores),
-            num_tokens, static_cast<int>(num_experts), static_cast<int>(experts_per_token));
-    });
-    return check_launch(name);
-}
-
-extern "C" int fm_topk_routing_backward(const void *grad_scores, const void *scores, const void *top_experts,
-                                        void *grad_logits, int64_t num_tokens, int64_t num_experts,
-                                        int64_t experts_per_token, int dtype, void *stream_) {
-    const char *name = "fm_topk_routing_backward";
-    FM_REQUIRE(valid_dtype(dtype), "%s: bad dtype %d", name, dtype);
-    FM_REQUIRE(num_tokens >= 0 && num_experts > 0, "%s: bad shape", name);
-    FM_REQUIRE(experts_per_token > 0 && experts_per_token <= num_experts && experts_per_token <= kMaxTopK,
-               "%s: experts_per_token %lld", name, static_cast<long long>(experts_per_token));
-    if (num_tokens == 0) return FM_OK;
-    FM_REQUIRE(grad_scores && scores && top_experts && grad_logits, "%s: null tensor", name);
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    const int64_t blocks = (num_tokens + kRoutingThreads / 64 - 1) / (kRoutingThreads / 64);
-    FM_REQUIRE(blocks < (int64_t(1) << 31), "%s: too many tokens", name);
-    FM_DISPATCH_DTYPE(dtype, T, {
-        topk_routing_backward_kernel<T><<<blocks, kRoutingThreads, 0, stream>>>(
-            static_cast<const float *>(grad_scores), static_cast<const float *>(scores),
-            static_cast<const int64_t *>(top_experts), static_cast<T *>(grad_logits), num_tokens,
-            static_cast<int>(num_experts), static_cast<int>(experts_per_token));
-    });
-    return check_launch(name);
-}
-
 extern "C" size_t fm_router_workspace_size(int64_t num_tokens, int64_t num_experts) {
     if (num_tokens <= 0 || num_experts <= 0) return 0;
-    return sizeof(float) * static_cast<size_t>(router_blocks(num_tokens)) * RouterStats::size(static_cast<int>(num_experts));
+    return router_counts_bytes(num_tokens, num_experts + kMaxTopK) +
+           sizeof(float) * static_cast<size_t>(router_blocks(num_tokens)) * (num_experts + 1);
 }
 
 static int check_router_shape(const char *name, int64_t num_tokens, int64_t num_experts, int64_t experts_per_token,
@@ -394,8 +407,72 @@ static int check_router_shape(const char *name, int64_t num_tokens, int64_t num_
                    experts_per_token + shared_experts <= kMaxTopK,
                "%s: experts_per_token %lld, shared_experts %lld", name, static_cast<long long>(experts_per_token),
                static_cast<long long>(shared_experts));
-    FM_REQUIRE((num_tokens + kRouterWaves - 1) / kRouterWaves < (int64_t(1) << 31), "%s: too many tokens", name);
+    FM_REQUIRE(num_tokens < (int64_t(1) << 31), "%s: too many tokens", name);
     return FM_OK;
+}
+
+namespace fm {
+
+template <typename T, int kGroup, int kPerLane, bool kStatistics>
+static void launch_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
+                                  int32_t *block_counts, float *block_sums, int64_t tokens, int experts, int k,
+                                  int shared, hipStream_t stream) {
+    // 16 wavefronts per workgroup (there is one workgroup per CU at most), 4 where their sums would fill LDS.
+    const int threads = experts <= 256 ? kRouterMaxThreads : kRouterMaxThreads / 4;
+    const int columns = kStatistics ? RouterStats::size(experts) : experts;
+    router_forward_kernel<T, kGroup, kPerLane, kStatistics>
+        <<<router_blocks(tokens), threads, sizeof(float) * (threads / 64) * columns, stream>>>(
+            static_cast<const T *>(logits), static_cast<const T *>(noise), static_cast<int64_t *>(top_experts),
+            static_cast<float *>(scores), static_cast<float *>(lse), block_counts, block_sums, tokens,
+            router_tokens_per_block(tokens), experts, k, shared);
+}
+
+static int run_router_backward(const char *name, const void *grad_scores, const void *scores, const void *top_experts,
+                               const void *logits, const void *noise, const void *lse, const void *statistics,
+                               void *grad_logits, float aux_scale, float z_scale, int64_t tokens, int experts, int k,
+                               int shared, int dtype, hipStream_t stream) {
+    FM_DISPATCH_DTYPE(dtype, T, {
+        FM_DISPATCH_ROUTER_SHAPE(experts, kGroup, kPerLane, {
+            constexpr int64_t kTokens = RouterShape<kGroup, kPerLane>::kTokens * (kRoutingThreads / 64);
+            router_backward_kernel<T, kGroup, kPerLane><<<(tokens + kTokens - 1) / kTokens, kRoutingThreads, 0, stream>>>(
+                static_cast<const float *>(grad_scores), static_cast<const float *>(scores),
+                static_cast<const int64_t *>(top_experts), static_cast<const T *>(logits), static_cast<const T *>(noise),
+                static_cast<const float *>(lse), static_cast<const float *>(statistics), static_cast<T *>(grad_logits),
+                aux_scale, z_scale, tokens, experts, k, shared);
+        })
+    });
+    return check_launch(name);
+}
+
+}  // namespace fm
+
+extern "C" int fm_topk_routing(const void *logits, void *top_experts, void *scores, int64_t num_tokens,
+                               int64_t num_experts, int64_t experts_per_token, int dtype, void *stream) {
+    const char *name = "fm_topk_routing";
+    if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, 0, dtype)) return status;
+    if (num_tokens == 0) return FM_OK;
+    FM_REQUIRE(logits && top_experts && scores, "%s: null tensor", name);
+    FM_DISPATCH_DTYPE(dtype, T, {
+        FM_DISPATCH_ROUTER_SHAPE(num_experts, kGroup, kPerLane, {
+            launch_router_forward<T, kGroup, kPerLane, false>(logits, nullptr, top_experts, scores, nullptr, nullptr, nullptr,
+                                                              num_tokens, static_cast<int>(num_experts),
+                                                              static_cast<int>(experts_per_token), 0,
+                                                              static_cast<hipStream_t>(stream));
+        })
+    });
+    return check_launch(name);
+}
+
+extern "C" int fm_topk_routing_backward(const void *grad_scores, const void *scores, const void *top_experts,
+                                        void *grad_logits, int64_t num_tokens, int64_t num_experts,
+                                        int64_t experts_per_token, int dtype, void *stream) {
+    const char *name = "fm_topk_routing_backward";
+    if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, 0, dtype)) return status;
+    if (num_tokens == 0) return FM_OK;
+    FM_REQUIRE(grad_scores && scores && top_experts && grad_logits, "%s: null tensor", name);
+    return run_router_backward(name, grad_scores, scores, top_experts, nullptr, nullptr, nullptr, nullptr, grad_logits,
+                               0.f, 0.f, num_tokens, static_cast<int>(num_experts),
+                               static_cast<int>(experts_per_token), 0, dtype, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int fm_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
@@ -406,23 +483,28 @@ extern "C" int fm_router_forward(const void *logits, const void *noise, void *to
     if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, shared_experts, dtype))
         return status;
     FM_REQUIRE(num_tokens > 0, "%s: no tokens", name);
-    FM_REQUIRE(logits && top_experts && scores && lse && statistics && losses && workspace, "%s: null tensor", name);
+    // The statistics may be left out together: then only the routing and the counts for the sparse map are computed.
+    const bool with_statistics = lse != nullptr || statistics != nullptr || losses != nullptr;
+    FM_REQUIRE(logits && top_experts && scores && workspace && (!with_statistics || (lse && statistics && losses)),
+               "%s: null tensor", name);
     FM_REQUIRE(workspace_size >= fm_router_workspace_size(num_tokens, num_experts), "%s: workspace of %zu bytes, need %zu",
                name, workspace_size, fm_router_workspace_size(num_tokens, num_experts));
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    const int experts = static_cast<int>(num_experts), stats = RouterStats::size(experts);
-    const int blocks = router_blocks(num_tokens);
+    const int experts = static_cast<int>(num_experts), shared = static_cast<int>(shared_experts);
+    int32_t *block_counts = static_cast<int32_t *>(workspace);
+    float *block_sums = reinterpret_cast<float *>(static_cast<char *>(workspace) + router_counts_bytes(num_tokens, num_experts + kMaxTopK));
     FM_DISPATCH_DTYPE(dtype, T, {
-        router_forward_kernel<T><<<blocks, kRoutingThreads, sizeof(float) * kRouterWaves * stats, stream>>>(
-            static_cast<const T *>(logits), static_cast<const T *>(noise), static_cast<int64_t *>(top_experts),
-            static_cast<float *>(scores), static_cast<float *>(lse), static_cast<float *>(workspace), num_tokens,
-            router_tokens_per_block(num_tokens), experts, static_cast<int>(experts_per_token),
-            static_cast<int>(shared_experts));
+        FM_DISPATCH_ROUTER_SHAPE(experts, kGroup, kPerLane, {
+            auto launch = with_statistics ? launch_router_forward<T, kGroup, kPerLane, true>
+                                          : launch_router_forward<T, kGroup, kPerLane, false>;
+            launch(logits, noise, top_experts, scores, lse, block_counts, block_sums, num_tokens, experts,
+                   static_cast<int>(experts_per_token), shared, stream);
+        })
     });
-    router_reduce_kernel<<<(stats + kRoutingThreads - 1) / kRoutingThreads, kRoutingThreads, 0, stream>>>(
-        static_cast<const float *>(workspace), static_cast<float *>(statistics), blocks, stats);
-    router_losses_kernel<<<1, kRoutingThreads, 0, stream>>>(static_cast<const float *>(statistics),
-                                                           static_cast<float *>(losses), num_tokens, experts);
+    if (with_statistics)
+        router_finish_kernel<<<1, 1024, 0, stream>>>(block_counts, block_sums, static_cast<float *>(statistics),
+                                                    static_cast<float *>(losses), router_blocks(num_tokens), num_tokens,
+                                                    experts, shared);
     return check_launch(name);
 }
 
@@ -435,20 +517,14 @@ extern "C" int fm_router_backward(const void *grad_scores, const void *scores, c
     if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, shared_experts, dtype))
         return status;
     if (num_tokens == 0) return FM_OK;
-    FM_REQUIRE(grad_scores && scores && top_experts && logits && lse && statistics && grad_logits, "%s: null tensor",
-               name);
+    const bool with_losses = auxiliary_loss_grad != 0.0 || z_loss_grad != 0.0;
+    FM_REQUIRE(grad_scores && scores && top_experts && logits && grad_logits && (!with_losses || (lse && statistics)),
+               "%s: null tensor", name);
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const double count = static_cast<double>(num_tokens);
     const float aux_scale = static_cast<float>(auxiliary_loss_grad / count / count);
     const float z_scale = static_cast<float>(2.0 * z_loss_grad / count);
-    const int64_t blocks = (num_tokens + kRouterWaves - 1) / kRouterWaves;
-    FM_DISPATCH_DTYPE(dtype, T, {
-        router_backward_kernel<T><<<blocks, kRoutingThreads, 0, stream>>>(
-            static_cast<const float *>(grad_scores), static_cast<const float *>(scores),
-            static_cast<const int64_t *>(top_experts), static_cast<const T *>(logits), static_cast<const T *>(noise),
-            static_cast<const float *>(lse), static_cast<const float *>(statistics), static_cast<T *>(grad_logits),
-            aux_scale, z_scale, num_tokens, static_cast<int>(num_experts), static_cast<int>(experts_per_token),
-            static_cast<int>(shared_experts));
-    });
-    return check_launch(name);
+    return run_router_backward(name, grad_scores, scores, top_experts, logits, noise, lse, statistics, grad_logits,
+                               aux_scale, z_scale, num_tokens, static_cast<int>(num_experts),
+                               static_cast<int>(experts_per_token), static_cast<int>(shared_experts), dtype, stream);
 }

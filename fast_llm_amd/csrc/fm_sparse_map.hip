@@ -1,16 +1,14 @@
 // Routing: build the sparse map (expert histogram -> padded expert offsets -> stable row of every
 // (token, slot) pair) with integer arithmetic only, so the result is bit-exact and run-to-run identical.
 //
-// Three small launches over the flattened `top_experts` (M = tokens * experts_per_token entries):
-//   1. sparse_map_histogram_kernel: one workgroup per 1024 entries. Each wavefront finds, with
-//      ceil(log2 E) ballots, the set of lanes that hold the same expert ("match-any"); the lowest lane of each
+// Two small launches over the flattened `top_experts` (M = tokens * experts_per_token entries):
+//   1. sparse_map_histogram_kernel: one workgroup per 1024 entries (at most 256 workgroups). Each wavefront finds,
+//      with ceil(log2 E) ballots, the set of lanes that hold the same expert ("match-any"); the lowest lane of each
 //      set adds the set size to an LDS histogram. The workgroup writes its E counts to the workspace.
-//   2. sparse_map_layout_kernel: one workgroup. Thread e turns column e of the per-workgroup counts into an
-//      exclusive prefix (in place) and gets count[e]; an LDS scan of the padded counts gives expert_ends,
-//      expert_pad_begins and the first row of every expert.
-//   3. sparse_map_rows_kernel: same partition as (1). rank inside the wavefront = popcount of the match set
-//      below the lane; rank inside the workgroup adds an LDS prefix over the 16 wavefronts; the global stable
-//      rank adds the exclusive prefix from (2). row = begin[e] + rank.
+//   2. sparse_map_rows_kernel: same partition. Every workgroup adds up all counts and those before its own, and an LDS
+//      scan of the padded totals gives expert_ends, expert_pad_begins and the first row of every expert. Rank inside
+//      the wavefront = popcount of the match set below the lane; rank inside the workgroup adds an LDS prefix over the
+//      16 wavefronts; the global stable rank adds the counts before. row = begin[e] + rank.
 // Ranks follow the flattened index order, i.e. the order of a stable sort by expert
 // (reference: fast_llm/functional/triton/sparse_copy.py:249-254).
 #include "fm_common.h"
@@ -23,6 +21,8 @@ namespace fm {
 constexpr int kMapBlock = 1024;  // entries (= threads) per workgroup
 constexpr int kMapWaves = kMapBlock / 64;
 constexpr int kMapMaxExperts = 1024;
+constexpr int kMapMaxBlocks = 256;   // workgroups: every one of them reads the counts of all
+constexpr int kMapCountBatch = 16;   // counts a thread requests at a time
 
 __device__ __forceinline__ int log2_ceil(int value) {
     int bits = 0;
@@ -42,34 +42,90 @@ __device__ __forceinline__ uint64_t match_expert(int expert, bool valid, int num
 }
 
 __global__ __launch_bounds__(kMapBlock) void sparse_map_histogram_kernel(const int64_t *__restrict__ top_experts,
-                                                                         int64_t num_entries, int num_experts,
+                                                                         int64_t num_entries, int64_t entries_per_block,
+                                                                         int num_experts,
                                                                          int32_t *__restrict__ block_counts) {
     extern __shared__ int32_t lds_counts[];  // [num_experts]
     for (int e = threadIdx.x; e < num_experts; e += kMapBlock) lds_counts[e] = 0;
     __syncthreads();
 
-    const int64_t entry = static_cast<int64_t>(blockIdx.x) * kMapBlock + threadIdx.x;
-    int64_t expert64 = entry < num_entries ? top_experts[entry] : -1;
-    const bool valid = expert64 >= 0 && expert64 < num_experts;
-    const int expert = valid ? static_cast<int>(expert64) : 0;
-    const uint64_t same = match_expert(expert, valid, log2_ceil(num_experts));
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * entries_per_block;
+    const int64_t last = min(first + entries_per_block, num_entries);
     const int lane = threadIdx.x & 63;
-    if (valid && (same & ((1ull << lane) - 1)) == 0) atomicAdd(&lds_counts[expert], __popcll(same));
+    for (int64_t chunk = first; chunk < last; chunk += kMapBlock) {
+        const int64_t entry = chunk + threadIdx.x;
+        const int64_t expert64 = entry < last ? top_experts[entry] : -1;
+        const bool valid = expert64 >= 0 && expert64 < num_experts;
+        const int expert = valid ? static_cast<int>(expert64) : 0;
+        const uint64_t same = match_expert(expert, valid, log2_ceil(num_experts));
+        if (valid && (same & ((1ull << lane) - 1)) == 0) atomicAdd(&lds_counts[expert], __popcll(same));
+    }
     __syncthreads();
 
     int32_t *out = block_counts + static_cast<int64_t>(blockIdx.x) * num_experts;
     for (int e = threadIdx.x; e < num_experts; e += kMapBlock) out[e] = lds_counts[e];
 }
 
-// Second half of the layout kernels: thread e holds count[e]; writes expert_ends, expert_pad_begins and the first row
-// of every expert (inclusive scan of the padded counts over experts: wavefront scan, then the wavefront totals).
-__device__ __forceinline__ void write_expert_layout(int64_t count, int num_experts, int64_t pad_to_multiple,
-                                                    int index_dtype, void *__restrict__ expert_ends,
-                                                    void *__restrict__ expert_pad_begins,
-                                                    int32_t *__restrict__ expert_begins) {
-    __shared__ int64_t lds_wave_totals[kMapWaves];
-    const int e = threadIdx.x;
+// Workgroup b ranks the entries [b * entries_per_block, (b + 1) * entries_per_block) of the flattened `top_experts`,
+// 1024 at a time, given how many entries of every expert each workgroup's range has (`block_counts[workgroup][expert]`).
+// Every workgroup adds up the counts of all workgroups by itself, all of them and those of the workgroups before it,
+// and scans the padded totals over the experts: 128 KiB from L2 at 256 workgroups and 128 experts, requested 16 loads
+// at a time by all threads. A kernel of one workgroup in between, one thread per expert walking down the workgroups,
+// was a serial chain of memory latencies: with 1024 workgroups, 16384 tokens and 8 of 128 experts it took 221 us, and
+// this kernel 8; both now take 12.
+__global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(
+    const int64_t *__restrict__ top_experts, int64_t num_entries, int64_t entries_per_block, int num_experts,
+    const int32_t *__restrict__ block_counts, int64_t pad_to_multiple, int index_dtype, void *__restrict__ sparse_rows,
+    void *__restrict__ expert_ends, void *__restrict__ expert_pad_begins) {
+    static_assert(kMapMaxExperts <= kMapBlock, "thread e keeps the running count of expert e in a register");
+    // [kMapWaves][num_experts] counts per wavefront: 64 KiB at 1024 experts. Before the first of them, in the same place:
+    // partial sums [2][kMapBlock], sums [2][num_experts] and the scan's wavefront totals.
+    extern __shared__ __attribute__((aligned(16))) int32_t lds_wave_counts[];
+    int32_t *lds_parts = lds_wave_counts, *lds_totals = lds_parts + 2 * kMapBlock;
+    int64_t *lds_wave_totals = reinterpret_cast<int64_t *>(lds_totals + 2 * num_experts);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int num_bits = log2_ceil(num_experts);
+
+    // Counts of all workgroups and of those before this one, 64 experts (or all, if fewer) at a time: the threads of a
+    // column share the workgroups, eight or more each.
+    const int columns = num_experts >= 64 ? 64 : 1 << max(num_bits, 3);
+    const int column = threadIdx.x & (columns - 1), part = threadIdx.x / columns;
+    const int num_blocks = gridDim.x, per_part = max((num_blocks * columns + kMapBlock - 1) / kMapBlock, 8);
+    const int parts = (num_blocks + per_part - 1) / per_part;
+    for (int base = 0; base < num_experts; base += columns) {
+        const int e = base + column;
+        int32_t all = 0, before = 0;
+        for (int i0 = 0; i0 < per_part; i0 += kMapCountBatch) {
+            int32_t here[kMapCountBatch];
+#pragma unroll
+            for (int i = 0; i < kMapCountBatch; ++i) {
+                const int b = part * per_part + i0 + i;
+                here[i] = i0 + i < per_part && b < num_blocks && e < num_experts
+                              ? block_counts[static_cast<int64_t>(b) * num_experts + e] : 0;
+            }
+#pragma unroll
+            for (int i = 0; i < kMapCountBatch; ++i) {
+                all += here[i];
+                if (part * per_part + i0 + i < static_cast<int>(blockIdx.x)) before += here[i];
+            }
+        }
+        lds_parts[threadIdx.x] = all;
+        lds_parts[kMapBlock + threadIdx.x] = before;
+        __syncthreads();
+        // Two threads per column finish it: one sum each.
+        if (threadIdx.x < 2 * columns) {
+            const int which = threadIdx.x / columns;
+            int32_t total = 0;
+            for (int p = 0; p < parts; ++p) total += lds_parts[which * kMapBlock + p * columns + column];
+            if (e < num_experts) lds_totals[which * num_experts + e] = total;
+        }
+        __syncthreads();
+    }
+
+    // Inclusive scan of the padded counts over the experts: wavefront scan, then the wavefront totals.
+    const int own_expert = threadIdx.x;
+    const int64_t count = own_expert < num_experts ? lds_totals[own_expert] : 0;
+    const int32_t earlier = own_expert < num_experts ? lds_totals[num_experts + own_expert] : 0;
     const int64_t padded = (count + pad_to_multiple - 1) / pad_to_multiple * pad_to_multiple;
     int64_t inclusive = padded;
 #pragma unroll
@@ -79,107 +135,21 @@ __device__ __forceinline__ void write_expert_layout(int64_t count, int num_exper
     }
     if (lane == 63) lds_wave_totals[wave] = inclusive;
     __syncthreads();
-    int64_t base = 0;
-    for (int w = 0; w < wave; ++w) base += lds_wave_totals[w];
-    inclusive += base;
-
-    if (e < num_experts) {
-        const int64_t begin = inclusive - padded;
-        store_index(expert_ends, index_dtype, e, inclusive);
-        store_index(expert_pad_begins, index_dtype, e, begin + count);
-        expert_begins[e] = static_cast<int32_t>(begin);
-    }
-}
-
-__global__ __launch_bounds__(kMapBlock) void sparse_map_layout_kernel(int32_t *__restrict__ block_counts,
-                                                                      int num_blocks, int num_experts,
-                                                                      int64_t pad_to_multiple, int index_dtype,
-                                                                      void *__restrict__ expert_ends,
-                                                                      void *__restrict__ expert_pad_begins,
-                                                                      int32_t *__restrict__ expert_begins) {
-    const int e = threadIdx.x;
-    // Exclusive prefix over workgroups of this expert's counts, in place.
-    int64_t count = 0;
-    if (e < num_experts) {
-        // 16 counts are requested before the first is used: one memory latency per 16 workgroups, not per workgroup
-        // (a load after a store to the same array is not moved ahead of it by the compiler).
-        constexpr int kBatch = 16;
-        int32_t running = 0;
-        for (int b0 = 0; b0 < num_blocks; b0 += kBatch) {
-            int32_t *slot = block_counts + static_cast<int64_t>(b0) * num_experts + e;
-            int32_t here[kBatch];
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i)
-                here[i] = b0 + i < num_blocks ? slot[static_cast<int64_t>(i) * num_experts] : 0;
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
-                if (b0 + i < num_blocks) slot[static_cast<int64_t>(i) * num_experts] = running;
-                running += here[i];
-            }
+    for (int w = 0; w < wave; ++w) inclusive += lds_wave_totals[w];
+    __syncthreads();  // the chunks' counts take the place of the sums
+    // Rows handed out so far to expert threadIdx.x (there are at most as many experts as threads).
+    int32_t running = 0;
+    if (own_expert < num_experts) {
+        const int64_t expert_begin = inclusive - padded;
+        running = static_cast<int32_t>(expert_begin) + earlier;
+        if (blockIdx.x == 0) {
+            store_index(expert_ends, index_dtype, own_expert, inclusive);
+            store_index(expert_pad_begins, index_dtype, own_expert, expert_begin + count);
         }
-        count = running;
     }
-    write_expert_layout(count, num_experts, pad_to_multiple, index_dtype, expert_ends, expert_pad_begins, expert_begins);
-}
 
-// The same from what the router's forward kernel left in its workspace: per workgroup of that kernel (a fixed range
-// of `tokens_per_block` tokens) and routed expert, the number of tokens of the range that selected the expert, as a
-// float (exact: at most 2^24). Shared experts follow the routed ones and are selected by every token.
-__global__ __launch_bounds__(kMapBlock) void sparse_map_layout_from_router_kernel(
-    const float *__restrict__ router_partials, int router_stats, int num_blocks, int64_t num_tokens,
-    int64_t tokens_per_block, int routed_experts, int num_experts, int64_t pad_to_multiple, int index_dtype,
-    void *__restrict__ expert_ends, void *__restrict__ expert_pad_begins, int32_t *__restrict__ block_prefix,
-    int32_t *__restrict__ expert_begins) {
-    const int e = threadIdx.x;
-    int64_t count = 0;
-    if (e < num_experts) {
-        constexpr int kBatch = 16;  // counts requested together, as in sparse_map_layout_kernel
-        int32_t running = 0;
-        for (int b0 = 0; b0 < num_blocks; b0 += kBatch) {
-            int32_t here[kBatch];
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
-                const int b = b0 + i;
-                if (b >= num_blocks) {
-                    here[i] = 0;
-                } else if (e < routed_experts) {
-                    here[i] = static_cast<int32_t>(router_partials[static_cast<int64_t>(b) * router_stats + routed_experts + e]);
-                } else {
-                    const int64_t begin = b * tokens_per_block;
-                    here[i] = static_cast<int32_t>(max(int64_t(0), min(begin + tokens_per_block, num_tokens) - begin));
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
-                if (b0 + i < num_blocks) block_prefix[static_cast<int64_t>(b0 + i) * num_experts + e] = running;
-                running += here[i];
-            }
-        }
-        count = running;
-    }
-    write_expert_layout(count, num_experts, pad_to_multiple, index_dtype, expert_ends, expert_pad_begins, expert_begins);
-}
-
-// Workgroup b ranks the entries [b * entries_per_block, (b + 1) * entries_per_block) of the flattened `top_experts`,
-// 1024 at a time, given the number of earlier entries per expert (`block_prefix[b]`).
-__global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(const int64_t *__restrict__ top_experts,
-                                                                    int64_t num_entries, int64_t entries_per_block,
-                                                                    int num_experts,
-                                                                    const int32_t *__restrict__ block_prefix,
-                                                                    const int32_t *__restrict__ expert_begins,
-                                                                    int index_dtype, void *__restrict__ sparse_rows) {
-    static_assert(kMapMaxExperts <= kMapBlock, "thread e keeps the running count of expert e in a register");
-    extern __shared__ int32_t lds_wave_counts[];  // [kMapWaves][num_experts] counts per wavefront: 64 KiB at 1024 experts
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int num_bits = log2_ceil(num_experts);
     const int64_t first = static_cast<int64_t>(blockIdx.x) * entries_per_block;
     const int64_t last = min(first + entries_per_block, num_entries);
-    // Rows handed out so far to expert threadIdx.x (there are at most as many experts as threads).
-    const int own_expert = threadIdx.x;
-    int32_t running = 0;
-    if (own_expert < num_experts)
-        running = expert_begins[own_expert] + block_prefix[static_cast<int64_t>(blockIdx.x) * num_experts + own_expert];
-
     for (int64_t chunk = first; chunk < last; chunk += kMapBlock) {
         for (int i = threadIdx.x; i < kMapWaves * num_experts; i += kMapBlock) lds_wave_counts[i] = 0;
         __syncthreads();
@@ -213,7 +183,22 @@ __global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(const int64_
     }
 }
 
-static inline int64_t map_num_blocks(int64_t num_entries) { return (num_entries + kMapBlock - 1) / kMapBlock; }
+// Dynamic LDS of the kernel above: the per-wavefront counts, and before them the sums.
+static inline size_t map_rows_lds_bytes(int num_experts) {
+    const size_t counts = static_cast<size_t>(kMapWaves) * num_experts;
+    const size_t sums = 2 * kMapBlock + 2 * static_cast<size_t>(num_experts) + 2 * kMapWaves;
+    return sizeof(int32_t) * (counts > sums ? counts : sums);
+}
+
+// Entries per workgroup: whole 1024s, few enough workgroups that each can read all the others' counts.
+static inline int64_t map_entries_per_block(int64_t num_entries) {
+    const int64_t chunks = (num_entries + kMapBlock - 1) / kMapBlock;
+    return (chunks + kMapMaxBlocks - 1) / kMapMaxBlocks * kMapBlock;
+}
+static inline int64_t map_num_blocks(int64_t num_entries) {
+    const int64_t per_block = map_entries_per_block(num_entries);
+    return per_block > 0 ? (num_entries + per_block - 1) / per_block : 0;
+}
 
 }  // namespace fm
 
@@ -227,27 +212,22 @@ extern "C" size_t fm_sparse_map_workspace_size(int64_t num_rows_dense, int64_t n
 
 namespace fm {
 
-// Validation and the three launches; `workspace` holds fm_sparse_map_workspace_size(...) bytes.
+// The two launches; `workspace` holds fm_sparse_map_workspace_size(...) bytes.
 static int run_sparse_map(const char *name, const int64_t *top_experts, int64_t num_rows_dense,
                           int64_t num_experts_per_token, int64_t num_experts, int64_t pad_to_multiple, int index_dtype,
                           void *sparse_rows, void *expert_ends, void *expert_pad_begins, void *workspace,
                           hipStream_t stream) {
     const int64_t num_entries = num_rows_dense * num_experts_per_token;
-    const int blocks = static_cast<int>(map_num_blocks(num_entries));
+    // At least one workgroup: without entries it still lays out the (empty) experts.
+    const int blocks = static_cast<int>(max(map_num_blocks(num_entries), int64_t(1)));
+    const int64_t entries_per_block = map_entries_per_block(num_entries);
     const int experts = static_cast<int>(num_experts);
     int32_t *block_counts = static_cast<int32_t *>(workspace);
-    int32_t *expert_begins = block_counts + static_cast<int64_t>(blocks) * experts;
-
-    if (blocks > 0) {
-        sparse_map_histogram_kernel<<<blocks, kMapBlock, experts * sizeof(int32_t), stream>>>(
-            top_experts, num_entries, experts, block_counts);
-    }
-    sparse_map_layout_kernel<<<1, kMapBlock, 0, stream>>>(block_counts, blocks, experts, pad_to_multiple, index_dtype,
-                                                          expert_ends, expert_pad_begins, expert_begins);
-    if (blocks > 0) {
-        sparse_map_rows_kernel<<<blocks, kMapBlock, kMapWaves * experts * sizeof(int32_t), stream>>>(
-            top_experts, num_entries, kMapBlock, experts, block_counts, expert_begins, index_dtype, sparse_rows);
-    }
+    sparse_map_histogram_kernel<<<blocks, kMapBlock, experts * sizeof(int32_t), stream>>>(
+        top_experts, num_entries, entries_per_block, experts, block_counts);
+    sparse_map_rows_kernel<<<blocks, kMapBlock, map_rows_lds_bytes(experts), stream>>>(
+        top_experts, num_entries, entries_per_block, experts, block_counts, pad_to_multiple, index_dtype, sparse_rows,
+        expert_ends, expert_pad_begins);
     return check_launch(name);
 }
 
@@ -291,9 +271,7 @@ extern "C" int fm_sparse_map(const int64_t *top_experts, int64_t num_rows_dense,
 
 // ---- the map from the router's own counts ------------------------------------------------------------------
 extern "C" size_t fm_sparse_map_from_router_workspace_size(int64_t num_tokens, int64_t num_experts) {
-    if (num_tokens < 0 || num_experts < 0) return 0;
-    const size_t bytes = static_cast<size_t>(fm::router_blocks(num_tokens) + 1) * num_experts * sizeof(int32_t);
-    return (bytes + 255) / 256 * 256 + 256;
+    return num_tokens < 0 || num_experts < 0 ? 0 : 256;  // the counts are the router's
 }
 
 extern "C" int fm_sparse_map_from_router(const int64_t *top_experts, const void *router_workspace,
@@ -307,31 +285,23 @@ extern "C" int fm_sparse_map_from_router(const int64_t *top_experts, const void 
     FM_REQUIRE(shared_experts >= 0 && experts_per_token > 0 && num_experts > shared_experts,
                "%s: %lld experts of which %lld shared, %lld per token", name, (long long)num_experts,
                (long long)shared_experts, (long long)experts_per_token);
-    const int64_t slots = shared_experts + experts_per_token, routed = num_experts - shared_experts;
+    const int64_t slots = shared_experts + experts_per_token;
     if (int status = check_sparse_map_arguments(name, top_experts, num_tokens, slots, num_experts, pad_to_multiple,
                                                 index_dtype, sparse_rows, expert_ends, expert_pad_begins))
         return status;
     FM_REQUIRE(num_tokens > 0, "%s: no tokens (the router does not run on none either)", name);
-    const int blocks = router_blocks(num_tokens);
-    const int stats = RouterStats::size(static_cast<int>(routed));
-    FM_REQUIRE(router_workspace && router_workspace_size >= sizeof(float) * blocks * stats,
-               "%s: the router workspace must be the %zu bytes fm_router_forward filled, got %zu", name,
-               sizeof(float) * blocks * stats, router_workspace_size);
+    FM_REQUIRE(router_workspace && router_workspace_size >= router_counts_bytes(num_tokens, num_experts),
+               "%s: the router workspace must be the buffer fm_router_forward filled, got %zu bytes", name,
+               router_workspace_size);
     FM_REQUIRE(workspace && aligned16(workspace) &&
                    workspace_size >= fm_sparse_map_from_router_workspace_size(num_tokens, num_experts),
                "%s: workspace of %zu bytes is null, misaligned or too small", name, workspace_size);
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
     const int experts = static_cast<int>(num_experts);
-    const int64_t tokens_per_block = router_tokens_per_block(num_tokens);
-    int32_t *block_prefix = static_cast<int32_t *>(workspace);
-    int32_t *expert_begins = block_prefix + static_cast<int64_t>(blocks) * experts;
-    sparse_map_layout_from_router_kernel<<<1, kMapBlock, 0, stream>>>(
-        static_cast<const float *>(router_workspace), stats, blocks, num_tokens, tokens_per_block,
-        static_cast<int>(routed), experts, pad_to_multiple, index_dtype, expert_ends, expert_pad_begins, block_prefix,
-        expert_begins);
-    sparse_map_rows_kernel<<<blocks, kMapBlock, kMapWaves * experts * sizeof(int32_t), stream>>>(
-        top_experts, num_tokens * slots, tokens_per_block * slots, experts, block_prefix, expert_begins, index_dtype,
-        sparse_rows);
+    sparse_map_rows_kernel<<<router_blocks(num_tokens), kMapBlock, map_rows_lds_bytes(experts),
+                             static_cast<hipStream_t>(stream_)>>>(
+        top_experts, num_tokens * slots, router_tokens_per_block(num_tokens) * slots, experts,
+        static_cast<const int32_t *>(router_workspace), pad_to_multiple, index_dtype, sparse_rows, expert_ends,
+        expert_pad_begins);
     return check_launch(name);
 }
 

@@ -85,11 +85,14 @@ class _TopKRouting(torch.autograd.Function):
         ctx.save_for_backward(scores, top_experts)
         ctx.num_experts, ctx.dtype = logits.size(-1), logits.dtype
         ctx.mark_non_differentiable(top_experts)
+        ctx.set_materialize_grads(False)  # no zero gradient for the experts
         return scores, top_experts
 
     @staticmethod
     def backward(ctx, grad_scores: torch.Tensor, _):
         scores, top_experts = ctx.saved_tensors
+        if grad_scores is None:
+            grad_scores = torch.zeros_like(scores)
         return topk_routing_backward(grad_scores, scores, top_experts, ctx.num_experts, ctx.dtype), None
 
 
@@ -102,11 +105,16 @@ def topk_routing(logits: torch.Tensor, experts_per_token: int) -> tuple[torch.Te
 
 
 def router_forward(
-    logits: torch.Tensor, noise: torch.Tensor | None, experts_per_token: int, shared_experts: int
-) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, RouterCounts]:
+    logits: torch.Tensor,
+    noise: torch.Tensor | None,
+    experts_per_token: int,
+    shared_experts: int,
+    with_losses: bool = True,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor | None, torch.Tensor | None, torch.Tensor | None, RouterCounts]:
     """One pass over `logits` [tokens, routed experts]: (scores fp32, top_experts int64, both
     [tokens, shared_experts + k]; losses [2] fp32 = load-balancing loss, z-loss; lse [tokens, 2] and statistics
-    [2 * experts + 1], both kept for the backward; and the per-workgroup counts for the sparse map)."""
+    [2 * experts + 1], both kept for the backward; and the per-workgroup counts for the sparse map). Without
+    `with_losses`, losses, lse and statistics are not computed and None."""
     assert logits.dim() == 2 and logits.is_contiguous()
     assert noise is None or (noise.shape == logits.shape and noise.dtype == logits.dtype and noise.is_contiguous())
     device = _lib.require_device(logits, noise)
@@ -118,7 +126,10 @@ def router_forward(
     slots = shared_experts + experts_per_token
     new = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=logits.device)  # noqa: E731
     scores, top_experts = new((tokens, slots), torch.float32), new((tokens, slots), torch.int64)
-    lse, statistics, losses = new((tokens, 2), torch.float32), new(2 * experts + 1, torch.float32), new(2, torch.float32)
+    lse = statistics = losses = None
+    if with_losses:
+        lse, statistics = new((tokens, 2), torch.float32), new(2 * experts + 1, torch.float32)
+        losses = new(2, torch.float32)
     workspace_size = _lib.lib().fm_router_workspace_size(tokens, experts)
     workspace = new(workspace_size, torch.uint8)
     _lib.call(
@@ -147,16 +158,17 @@ def router_forward(
 
 class _Router(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, logits, noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad):
+    def forward(ctx, logits, noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad, with_losses):
         logits = logits.detach().contiguous()
         noise = None if noise is None else noise.detach().contiguous()
         scores, top_experts, losses, lse, statistics, counts = router_forward(
-            logits, noise, experts_per_token, shared_experts
+            logits, noise, experts_per_token, shared_experts, with_losses
         )
         ctx.save_for_backward(logits, noise, scores, top_experts, lse, statistics)
         ctx.shape = (experts_per_token, shared_experts)
         ctx.loss_grads = (auxiliary_loss_grad or 0.0, z_loss_grad or 0.0)
-        ctx.mark_non_differentiable(top_experts, losses, counts.workspace)
+        ctx.mark_non_differentiable(*(x for x in (top_experts, losses, counts.workspace) if x is not None))
+        ctx.set_materialize_grads(False)  # no zero gradients for the outputs that have none
         return scores, top_experts, losses, counts.workspace
 
     @staticmethod
@@ -164,6 +176,8 @@ class _Router(torch.autograd.Function):
         logits, noise, scores, top_experts, lse, statistics = ctx.saved_tensors
         experts_per_token, shared_experts = ctx.shape
         device = _lib.require_device(logits)
+        if grad_scores is None:
+            grad_scores = torch.zeros_like(scores)
         grad_logits = torch.empty_like(logits)
         _lib.call(
             "fm_router_backward",
@@ -184,7 +198,7 @@ class _Router(torch.autograd.Function):
             shared_experts,
             _lib.dtype_tag(logits.dtype),
         )
-        return grad_logits, None, None, None, None, None
+        return grad_logits, None, None, None, None, None, None
 
 
 def router(
@@ -196,7 +210,8 @@ def router(
     auxiliary_loss_grad: float | None = None,
     z_loss_grad: float | None = None,
     return_counts: bool = False,
-) -> tuple[torch.Tensor, ...]:
+    with_losses: bool = True,
+) -> tuple[torch.Tensor | None, ...]:
     """
     The router front end of `MixtureOfExpertMLP._forward` for top-k routing (reference:
     fast_llm/layers/decoder/mlp/mixture_of_experts.py:146-171, 237-278) in one pass over `logits` [..., routed experts]:
@@ -206,15 +221,19 @@ def router(
     (functional/utils.py:63-71) gives the losses when the scores are back-propagated:
     `unshared_experts * auxiliary_loss_coefficient * grad_scale` and `z_loss_coefficient * grad_scale`; None or 0:
     that loss contributes no gradient. With `return_counts` a fifth value follows: the `RouterCounts` to hand to
-    `get_sparse_map` together with these `top_experts`.
+    `get_sparse_map` together with these `top_experts`. Without `with_losses` the losses are None and not computed;
+    then neither can have a gradient.
     """
+    if not with_losses and (auxiliary_loss_grad or z_loss_grad):
+        raise ValueError("a loss that is not computed has no gradient")
     flat = logits.flatten(0, -2)
     flat_noise = None if noise is None else noise.flatten(0, -2)
     scores, top_experts, losses, workspace = _Router.apply(
-        flat, flat_noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad
+        flat, flat_noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad, with_losses
     )
     shape = logits.shape[:-1] + (shared_experts + experts_per_token,)
-    result = (scores.view(shape), top_experts.view(shape), losses[0], losses[1])
+    load_balancing_loss, z_loss = (losses[0], losses[1]) if with_losses else (None, None)
+    result = (scores.view(shape), top_experts.view(shape), load_balancing_loss, z_loss)
     if return_counts:
         result += (
             RouterCounts(

@@ -131,6 +131,7 @@ class DroplessMoEMLP(torch.nn.Module):
             auxiliary_loss_grad=self.unshared_experts * self.auxiliary_loss_coefficient * grad_scale if trained else None,
             z_loss_grad=self.z_loss_coefficient * grad_scale if trained else None,
             return_counts=True,
+            with_losses=trained or losses is not None,
         )
         if losses is not None:
             losses.setdefault(LOAD_BALANCING_LOSS, []).append(load_balancing_loss)

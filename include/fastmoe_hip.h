@@ -182,7 +182,8 @@ int fm_topk_routing_backward(const void *grad_scores, const void *scores, const 
  * Outputs: top_experts (int64), scores (fp32), lse [num_tokens, 2] fp32 (logsumexp of the routed and of the given
  * logits; kept for the backward), statistics [2 * num_experts + 1] fp32 (per expert: sum_t softmax, number of tokens
  * that selected it; then sum_t logsumexp^2), losses [2] fp32 (load balancing, z). Sums over tokens are added in a
- * fixed order. `workspace`: fm_router_workspace_size(num_tokens, num_experts) bytes of device memory. */
+ * fixed order. `workspace`: fm_router_workspace_size(num_tokens, num_experts) bytes of device memory. lse, statistics
+ * and losses may all three be null: only the routing and the counts for the sparse map are computed then. */
 size_t fm_router_workspace_size(int64_t num_tokens, int64_t num_experts);
 int fm_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
                       void *statistics, void *losses, void *workspace, size_t workspace_size, int64_t num_tokens,
@@ -192,7 +193,8 @@ int fm_router_forward(const void *logits, const void *noise, void *top_experts, 
  * are ignored) and the constant gradients the reference attaches to the two losses through `AuxiliaryLoss`
  * (fast_llm/functional/utils.py:63-71; mixture_of_experts.py:154, 257-261): auxiliary_loss_grad for the load-balancing
  * loss and z_loss_grad for the z-loss, 0 for a loss that is not trained on. logits, noise, scores, top_experts, lse
- * and statistics are the forward's. grad_logits has `dtype`. */
+ * and statistics are the forward's (lse and statistics may be null if neither loss is trained on). grad_logits has
+ * `dtype`. */
 int fm_router_backward(const void *grad_scores, const void *scores, const void *top_experts, const void *logits,
                        const void *noise, const void *lse, const void *statistics, void *grad_logits,
                        double auxiliary_loss_grad, double z_loss_grad, int64_t num_tokens, int64_t num_experts,

@@ -6,6 +6,7 @@ import torch
 
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.routing import router, topk_routing
+from fast_llm_amd.functional.sparse_copy import get_sparse_map
 from oracle import moe_oracle
 
 pytestmark = pytest.mark.gpu
@@ -38,6 +39,27 @@ def test_topk_routing_forward(tokens, experts, k, dtype, device):
     assert torch.equal(top_experts.cpu(), expected_experts)
     assert torch.allclose(scores.cpu(), expected_scores, rtol=2e-6, atol=1e-7)
     assert torch.allclose(scores.sum(-1).cpu(), torch.ones(tokens), atol=1e-5)
+
+
+# Each side of the numbers of experts at which the kernels change how many lanes share a token (8, 16, 32, 64) and how
+# many logits a lane holds (128, 256), and of the token counts at which workgroups take more than 16 tokens (4096).
+@pytest.mark.parametrize("experts", [2, 9, 16, 17, 32, 33, 65, 129, 256, 257])
+@pytest.mark.parametrize("tokens", [1, 17, 4096, 4111])
+def test_router_group_and_block_edges(tokens, experts, device):
+    k, shared = min(experts, 5), 2
+    logits = _distinct_logits(tokens, experts, torch.float32, torch.Generator().manual_seed(experts))
+    expected = moe_oracle.router(logits, k, shared_experts=shared)
+    for with_losses in (True, False):
+        scores, top_experts, auxiliary_loss, z_loss, counts = router(
+            logits.to(device), k, shared_experts=shared, return_counts=True, with_losses=with_losses
+        )
+        assert torch.equal(top_experts.cpu(), expected.top_experts)
+        assert torch.allclose(scores.cpu(), expected.scores, rtol=2e-6, atol=1e-7)
+        sparse_map = get_sparse_map(top_experts, experts + shared, router_counts=counts)
+        oracle_map = moe_oracle.sparse_map(expected.top_experts, experts + shared)
+        for name in ("sparse_rows", "expert_ends", "expert_pad_begins"):
+            assert torch.equal(getattr(sparse_map, name).cpu().long(), getattr(oracle_map, name)), name
+    assert auxiliary_loss is None and z_loss is None
 
 
 def test_topk_routing_ties_go_to_the_lower_expert(device):
