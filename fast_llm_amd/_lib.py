@@ -104,7 +104,7 @@ def check(status: int) -> None:
     if status == FM_NOTE_GENERIC_KERNEL:
         warnings.warn(
             "a grouped product with half-precision operands ran on the generic multiply-add kernel, not on the matrix "
-            "cores (operands need a unit stride on one axis, 16-byte aligned rows, a reduction that is a multiple of 64)",
+            "cores (operands need a unit stride on one axis, 16-byte aligned rows, a reduction that is a multiple of 8)",
             RuntimeWarning,
             stacklevel=3,
         )

@@ -166,8 +166,8 @@ struct TileLoader {
     uint32_t num_records;    // wave-uniform: lane offsets >= this bring zeros
     int64_t step;            // bytes from one slice to the next
     int slices_left;         // slices after the one being fetched
-    uint32_t last_records;   // row-contiguous: `num_records` of the last slice (its K-rows past the reduction range
-                             // bring zeros)
+    uint32_t last_records;   // `num_records` of the last slice: its K-rows past the reduction range bring zeros (row-
+                             // contiguous), or its last row ends where the reduction range does (K-contiguous)
     int wave_index;          // wave-uniform
 
     // `stride`: bytes between rows (K-contiguous) or between K-rows (row-contiguous). Rows >= valid_rows are never
@@ -177,7 +177,8 @@ struct TileLoader {
     // 128..191 but lie `split_rows` rows after them, i.e. tile row n is memory row
     // (n / 128) * 64 + n % 64 + (n / 64 % 2) * split_rows (the gate and up halves of a gated layer's weight).
     // `k_count`: reduction indices from the first one of slice 0 to the end of the reduction range; a row-contiguous
-    // operand gets zeros for the K-rows of its last slice that lie past it.
+    // operand gets zeros for the K-rows of its last slice that lie past it. Of a K-contiguous operand only the last
+    // row gets zeros there: what the other rows bring is the start of the next row, to be masked in LDS.
     __device__ __forceinline__ void setup(const char *tile_base, int64_t stride, int valid_rows, int num_slices,
                                           int k_count, int wave, int lane, int split_rows = 0) {
         static_assert(kLoadsPerOperand % 2 == 0, "loads come in (even, odd) pairs");
@@ -205,10 +206,13 @@ struct TileLoader {
         pair_stride = static_cast<uint32_t>((kContiguousK ? 128 / kChunksPerRow : 4) * stride);
         const int64_t last_row = split_rows == 0 ? valid_rows - 1 : split_rows + kTile / 2 - 1;
         step = kContiguousK ? kBK * 2 : kBK * stride;
+        const int last_count = k_count - (num_slices - 1) * kBK;  // of the last slice
         if constexpr (kContiguousK) {
-            num_records = last_records = static_cast<uint32_t>(last_row * stride + kBK * 2);
+            // Whole 16-byte chunks: a chunk that crosses the range would come back as zeros.
+            last_records = static_cast<uint32_t>(last_row * stride + min((last_count + 7) & ~7, kBK) * 2);
+            num_records = num_slices == 1 ? last_records : static_cast<uint32_t>(last_row * stride + kBK * 2);
         } else {
-            last_records = static_cast<uint32_t>((k_count - (num_slices - 1) * kBK) * stride);
+            last_records = static_cast<uint32_t>(last_count * stride);
             num_records = num_slices == 1 ? last_records : 0xffffffffu;
         }
     }
@@ -926,7 +930,8 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[kTilesM][kTi
             }
 }
 
-// kMasked: the row-sparse product, whose reduction range [k_lo, k_hi) is ragged.
+// kMasked: the reduction range [k_lo, k_hi) is ragged: the row-sparse product, and any whose reduction is not a whole
+// number of slices.
 // kFusion: a GemmFusion, the epilogue to run instead of the plain store.
 template <typename T, bool kLhsContiguousK, bool kRhsContiguousK, bool kMasked, int kFusion = kFusionNone>
 __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_kernel(GemmArgs launch_args) {
@@ -1448,8 +1453,11 @@ static int launch_layout(const GemmArgs &args, hipStream_t stream) {
     const bool lhs_k = args.lhs_stride_inner == 1, rhs_k = args.rhs_stride_inner == 1;
     if (args.fusion == kFusionGatedForward) return launch_instance<T, true, true, false, kFusionGatedForward>(args, stream);
     if (args.fusion == kFusionGatedBackward) return launch_instance<T, true, true, false, kFusionGatedBackward>(args, stream);
-    // Only the row-sparse product with a map has a ragged reduction range.
-    const bool masked = args.mode == kInputRowSparse && args.expert_ends != nullptr;
+    // A ragged reduction range: the row-sparse product with a map, and a reduction that is no whole number of slices
+    // (a feed-forward size of 3416, say), whose last slice is then masked in LDS: one pass over two operands and one
+    // barrier per tile. Layer 2 forward and layer 1 input gradient at 6002 rows over 16 experts, 1280 x 3416 (6832):
+    // 2932 and 5843 us on the multiply-add kernel that such reductions went to before, 99 and 180 here.
+    const bool masked = (args.mode == kInputRowSparse && args.expert_ends != nullptr) || args.inner % kBK != 0;
 #define FM_LAUNCH(LHS, RHS) \
     return masked ? launch_instance<T, LHS, RHS, true>(args, stream) : launch_instance<T, LHS, RHS, false>(args, stream)
     if (lhs_k && rhs_k) FM_LAUNCH(true, true);
@@ -1468,9 +1476,9 @@ bool mfma_gemm_eligible(const GemmArgs &args, int dtype) {
     if (!(lhs_k || lhs_m) || !(rhs_k || rhs_n)) return false;
     if (!vector_ok(args.lhs, lhs_k ? args.lhs_stride_row : args.lhs_stride_inner)) return false;
     if (!vector_ok(args.rhs, rhs_k ? args.rhs_stride_col : args.rhs_stride_inner)) return false;
-    // The reduction axis is walked in whole 64-element tiles that must exist in memory; 16-byte chunks along the
-    // contiguous axis of a row-contiguous operand must not straddle the end of an expert's block.
-    if (args.inner <= 0 || args.inner % kBK != 0 || args.sparse_size % 8 != 0 || args.cols % 8 != 0) return false;
+    // 16-byte chunks along the reduction axis of a K-contiguous operand, and along the other axis of a row-contiguous
+    // one, must not straddle the end of the axis or of an expert's block.
+    if (args.inner <= 0 || args.inner % 8 != 0 || args.sparse_size % 8 != 0 || args.cols % 8 != 0) return false;
     if (!lhs_k && args.mode != kInputRowSparse && args.rows % 8 != 0) return false;
     // Per-lane byte offsets inside an operand tile are 32-bit.
     if (max(max(args.lhs_stride_row, args.lhs_stride_inner), max(args.rhs_stride_inner, args.rhs_stride_col)) >=
@@ -1484,7 +1492,8 @@ bool mfma_gemm_eligible(const GemmArgs &args, int dtype) {
 // The fused epilogues exist for one layout: both operands K-contiguous, output-sparse mode, T in and out, whole
 // column tiles (the activation width a multiple of 128 for the forward, of 8 for the backward).
 bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype) {
-    if (!mfma_gemm_eligible(args, dtype) || args.mode != kOutputSparse || args.out_dtype != dtype || args.accumulate)
+    if (!mfma_gemm_eligible(args, dtype) || args.mode != kOutputSparse || args.out_dtype != dtype || args.accumulate ||
+        args.inner % kBK != 0)
         return false;
     if (args.lhs_stride_inner != 1 || args.rhs_stride_inner != 1) return false;
     if (!aligned16(args.fused_out) || !aligned16(args.fused_in) || args.fused_stride % 8 != 0 || args.half % 8 != 0)
@@ -1536,8 +1545,8 @@ static size_t table_bytes(int num_ids) {
 
 size_t mfma_gemm_workspace_size(GemmArgs args) {
     if (args.rows <= 0 || args.cols <= 0 || args.inner <= 0) return 0;
-    // Dimensions that `mfma_gemm_eligible` refuses whatever the strides: such a product runs on the generic kernel,
-    // which takes no workspace.
+    // Dimensions that `mfma_gemm_eligible` refuses whatever the strides (such a product runs on the generic kernel, which
+    // takes no workspace), and reductions that are no whole number of slices (which do not split).
     if (args.inner % kBK != 0 || args.cols % 8 != 0 || (args.mode == kInputRowSparse && args.sparse_size % 8 != 0)) return 0;
     count_tiles(args);
     if (too_many_tiles(args)) return 0;
@@ -1550,6 +1559,7 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
     if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
     args.partials = nullptr;
     args.tile_table = nullptr;
+    if (args.inner % kBK != 0) workspace = nullptr;  // as mfma_gemm_workspace_size says
     const bool split = workspace != nullptr && splits_last_round(args);
     args.num_ids = count_ids(args, split);
     if (workspace != nullptr) {

@@ -39,7 +39,7 @@ enum fm_index_dtype { FM_INDEX_I16 = 0, FM_INDEX_I32 = 1, FM_INDEX_I64 = 2 };
 enum fm_status {
     /* Positive: the call succeeded and was launched, with a remark. The three grouped products return this one when
      * bf16/fp16 operands had to take the bounds-checked multiply-add kernel instead of the matrix cores (a stride
-     * that is not 1 on either axis, rows not 16-byte aligned, reduction not a multiple of 64, stride >= 2^21). */
+     * that is not 1 on either axis, rows not 16-byte aligned, reduction not a multiple of 8, stride >= 2^21). */
     FM_NOTE_GENERIC_KERNEL = 1,
     FM_OK = 0,
     FM_ERR_INVALID_ARGUMENT = -1, /* bad enum, negative size, null pointer, misaligned/unsupported stride */

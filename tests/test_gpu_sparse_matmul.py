@@ -579,6 +579,37 @@ def test_expert_boundaries_inside_a_tile(pad, dtype, device):
     assert max_rel_err(out.cpu(), expected) <= tolerance
 
 
+@pytest.mark.parametrize("inner", [8, 56, 72, 120, 136, 1000, 2104])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_reductions_of_no_whole_number_of_slices(inner, dtype, device):
+    """Reductions around one and two slices of 64 and long ones, none a multiple of 64, on the matrix-core kernel (no
+    remark about the generic one). The rows after an expert's last token hold NaN: what a row's last slice brings of
+    the next row must not reach it."""
+    import warnings
+
+    generator = torch.Generator().manual_seed(inner)
+    experts, other = 5, 264
+    case = _ragged_case(inner, experts)
+    oracle_map = fixture_sparse_map(case)
+    oracle_map.num_rows = case["expert_ends"][-1] + case["phantom_rows"]
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    real = oracle_map.real_row_mask()
+    x = _normal(oracle_map.num_rows, inner, dtype, generator)
+    weight, weight_inner = _normal(experts * other, inner, dtype, generator), _normal(experts * inner, other, dtype, generator)
+    poisoned = x.clone()
+    poisoned[~real] = float("nan")
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        outer = output_sparse_matmul(poisoned.to(device), weight.to(device).t(), sparse_map).cpu()
+        inner_out = input_inner_sparse_matmul(poisoned.to(device), weight_inner.to(device), sparse_map).cpu()
+        dense = dense_matmul(x[:296].to(device).t().contiguous().t(), weight[:264].to(device).t().contiguous()).cpu()
+    expected = moe_oracle.output_sparse_matmul(x, weight.t(), oracle_map)
+    assert max_rel_err(outer[real], expected[real]) <= _MAX_REL[dtype]
+    expected = moe_oracle.input_inner_sparse_matmul(x, weight_inner, oracle_map)
+    assert max_rel_err(inner_out[real], expected[real]) <= _MAX_REL[dtype]
+    assert max_rel_err(dense, (x[:296].float() @ weight[:264].float().t()).to(dtype)) <= _MAX_REL[dtype]
+
+
 def test_half_precision_on_the_generic_kernel_warns(device):
     """bf16 operands the matrix-core kernel cannot take (here: a reduction that is not a multiple of 64) still give the
     right product, from the multiply-add kernel, and the wrapper says so."""
