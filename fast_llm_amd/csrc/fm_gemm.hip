@@ -7,11 +7,10 @@
 //                        token axis, everything outside replaced by zero before the multiply
 // (reference semantics: fast_llm/functional/triton/sparse_linear.py:185-258, 310-385, 437-517).
 //
-// Half-precision operands with vectorisable layouts go to the MFMA kernel (fm_gemm_mfma.hip). fp32 operands go to
-// the fp32 matrix-core kernel below (tiles of v_mfma_f32_32x32x2_f32: true fp32 multiply-adds, which is what the
-// 1e-5 fp32 parity bound needs; 59-63 TFLOP/s at 16384 x 4096 x 2048 over 8 experts). Everything else
-// (half-precision operands with odd strides or sizes) goes to the generic kernel: a 64 x 64 x 16 LDS-tiled kernel of
-// scalar multiply-adds. Both compute a row block that straddles an expert boundary in one pass per expert, so they
+// Half-precision operands with vectorisable layouts go to fm_gemm_mfma.hip, fp32 ones to fm_gemm_f32.hip. Operands with
+// odd strides or sizes, fp32 products with a half-precision result and row-sparse fp32 products of K-contiguous operands
+// go to the two kernels here: a 64 x 64 x 16 LDS-tiled kernel of scalar multiply-adds (half precision) and one of fp32
+// matrix instructions (fp32). Both compute a row block that straddles an expert boundary in one pass per expert, so they
 // take any padding multiple, and both check every bound.
 #include "fm_gemm_common.h"
 
@@ -43,14 +42,13 @@ constexpr int kGenTile = 64, kGenK = 16, kGenThreads = 256;
 // The work of the tile at (row0, col0) for the expert that owns its row `first_row` (relative to row0): in the
 // products whose rows are grouped by expert, a tile that straddles an expert boundary (any padding multiple is
 // allowed) is computed in one piece per expert.
-__device__ __forceinline__ TileWork resolve_tile(const GemmArgs &args, int64_t row0, int64_t col0, int first_row,
-                                                 int tile_rows = kGenTile) {
+__device__ __forceinline__ TileWork resolve_tile(const GemmArgs &args, int64_t row0, int64_t col0, int first_row) {
     TileWork work;
     work.skip = false;
     work.k_lo = 0;
     work.k_hi = args.inner;
     work.row_lo = first_row;
-    work.row_hi = tile_rows;
+    work.row_hi = kGenTile;
     work.out_offset = row0 * args.out_stride_row + col0 * args.out_stride_col;
     const bool dense = args.expert_ends == nullptr;
     if (args.mode == kInputRowSparse) {
@@ -174,16 +172,11 @@ __global__ __launch_bounds__(kGenThreads) void grouped_gemm_generic_kernel(GemmA
 // one slice ahead and stored to LDS as [k][row], double-buffered, one barrier per slice; several workgroups share a
 // CU. Tiles lie on a fixed grid of kTile rows: one that straddles an expert boundary is computed in one pass per
 // expert, like the generic kernel's, so any padding multiple works (the reference's multiple of 128 gives one pass).
-// Two shapes: 128 x 128 x 16 for launches that fill the device (59-63 TFLOP/s at 16384 x 4096 x 2048 over 8 experts),
-// and 64 x 64 x 32 for launches of fewer 128-tiles than there are CUs (the 512-token configuration: 32 to 128 of
-// them), which are bound by the memory latency of one slice after the other: four times the workgroups, each with a
-// quarter of the multiply-adds and half the slices.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gemm_f32x16_t;
-constexpr int kF32Tile = 128, kF32SmallTile = 64, kF32Threads = 256;
-constexpr int kF32SmallLaunchTiles = 256;  // fewer 128-tiles than this (the CUs of the device): tiles of 64
+constexpr int kF32Threads = 256;
 
-template <int kTile, int kK>
-__global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_mfma_kernel(GemmArgs args) {
+__global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_any_layout_kernel(GemmArgs args) {
+    constexpr int kTile = kGenTile, kK = 32;
     constexpr int kPitch = kTile + 4;                       // floats per K-row in LDS; +4 spreads the banks
     constexpr int kPerThread = kTile * kK / kF32Threads;    // operand elements per thread and slice
     constexpr int kWaveTile = kTile / 2, kBlocks = kWaveTile / 32;  // a wavefront's part, in 32 x 32 accumulators
@@ -205,7 +198,7 @@ __global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_mfma_kernel(Gemm
     const float *lhs_all = static_cast<const float *>(args.lhs), *rhs_all = static_cast<const float *>(args.rhs);
 
     for (int first_row = 0; first_row < rows_here;) {
-        const TileWork work = resolve_tile(args, row0, col0, first_row, kTile);
+        const TileWork work = resolve_tile(args, row0, col0, first_row);
         if (work.skip) return;  // the rest of the tile lies past the last expert
         const int row_hi = work.row_hi < rows_here ? work.row_hi : static_cast<int>(rows_here);
         const float *lhs = lhs_all + work.lhs_offset, *rhs = rhs_all + work.rhs_offset;
@@ -315,6 +308,8 @@ static int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace,
     int note = FM_OK;
     if (mfma_gemm_eligible(args, dtype)) {
         if (int status = mfma_gemm_launch(args, dtype, workspace, workspace_size, stream)) return status;
+    } else if (f32_gemm_eligible(args, dtype)) {
+        if (int status = f32_gemm_launch(args, stream)) return status;
     } else {
         // Half-precision operands that the matrix-core kernel cannot take: correct, but far slower. Say so.
         if (dtype != FM_DTYPE_F32) note = FM_NOTE_GENERIC_KERNEL;
@@ -322,26 +317,14 @@ static int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace,
         if (args.mode == kInputRowSparse && args.num_experts > 1 && args.sparse_size % kGenTile != 0)
             return fail(FM_ERR_UNSUPPORTED, "%s: row_sparse_dim=%lld must be a multiple of %d", name,
                         (long long)args.sparse_size, kGenTile);
-        // fp32 operands go to the matrix cores when the row-sparse product's blocks of out are whole tiles there too:
-        // tiles of 128, or of 64 when there are fewer 128-tiles than CUs (see the kernel).
-        const auto whole_tiles = [&](int tile) {
-            return !(args.mode == kInputRowSparse && args.num_experts > 1 && args.sparse_size % tile != 0);
-        };
-        const int64_t large_tiles = ((args.rows + kF32Tile - 1) / kF32Tile) * ((args.cols + kF32Tile - 1) / kF32Tile);
-        const bool f32_small = dtype == FM_DTYPE_F32 && large_tiles < kF32SmallLaunchTiles && whole_tiles(kF32SmallTile);
-        const bool f32_mfma = dtype == FM_DTYPE_F32 && (f32_small || whole_tiles(kF32Tile));
-        const int tile = f32_small ? kF32SmallTile : (f32_mfma ? kF32Tile : kGenTile);
+        constexpr int tile = kGenTile;
         args.tiles_m = static_cast<int>((args.rows + tile - 1) / tile);
         args.tiles_n = static_cast<int>((args.cols + tile - 1) / tile);
         FM_REQUIRE(static_cast<int64_t>(args.tiles_m) * args.tiles_n < (int64_t(1) << 31), "%s: too many tiles", name);
         const int grid = args.tiles_m * args.tiles_n;
-        if (f32_small) {
-            grouped_gemm_f32_mfma_kernel<kF32SmallTile, 32><<<grid, kF32Threads, 0, stream>>>(args);
-        } else if (f32_mfma) {
-            grouped_gemm_f32_mfma_kernel<kF32Tile, 16><<<grid, kF32Threads, 0, stream>>>(args);
-        } else {
-            FM_DISPATCH_DTYPE(dtype, T, { grouped_gemm_generic_kernel<T><<<grid, kGenThreads, 0, stream>>>(args); });
-        }
+        if (dtype == FM_DTYPE_F32) grouped_gemm_f32_any_layout_kernel<<<grid, kF32Threads, 0, stream>>>(args);
+        else if (dtype == FM_DTYPE_BF16) grouped_gemm_generic_kernel<bf16_t><<<grid, kGenThreads, 0, stream>>>(args);
+        else grouped_gemm_generic_kernel<f16_t><<<grid, kGenThreads, 0, stream>>>(args);
     }
     if (int status = check_launch(name)) return status;
     return note;

@@ -42,7 +42,124 @@ struct GemmArgs {
     int64_t half;          // columns of the activation output per expert
     int num_ids;           // workgroup ids that may have a tile (set by the MFMA kernel's launcher)
     void *tile_table;      // one record per id, written by the plan kernel into the caller's workspace, or null
+    int chunk_tiles;       // consecutive tiles that go to one XCD (set by the fp32 kernel's launcher)
 };
+
+#define FM_LDS(T) __attribute__((address_space(3))) T
+
+constexpr int kBufferResourceFlags = 0x00020000;  // raw buffer, 32-bit data format, no swizzle
+
+// The same value, but the compiler cannot tell: what is computed from it is computed where it is written, not hoisted
+// out of an enclosing loop into registers that stay occupied across the loop.
+__device__ __forceinline__ int opaque(int value) {
+    asm volatile("" : "+v"(value));
+    return value;
+}
+
+// Tell the compiler that a pointer computed from tile coordinates is the same in every lane (it then lives in
+// scalar registers and the loads use the scalar-base addressing form).
+__device__ __forceinline__ const char *uniform_pointer(const char *pointer) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(pointer);
+    const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits));
+    const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32));
+    return reinterpret_cast<const char *>((static_cast<uint64_t>(high) << 32) | low);
+}
+
+// ---- which tile ----------------------------------------------------------------------------------------
+constexpr int kGroupRows = 8;
+
+// Logical order of the tiles of a product whose rows are grouped by expert (output-sparse, input-inner-sparse,
+// dense): expert after expert; within an expert its row tiles (ceil(rows_e / kTile)) are cut into ceil(count / 8)
+// groups of nearly equal size (9 row tiles: 5 + 4), and a group is walked column tile by column tile, row tiles
+// fastest. 32 consecutive tiles (what an XCD runs at one time) are then about 8 row tiles x 4 column tiles of ONE
+// expert, i.e. 8 lhs panels and 4 rhs panels shared in that XCD's L2; with groups that ignore the expert boundaries
+// most chunks straddled two experts and needed twice the rhs panels.
+// Every wavefront scans `expert_ends` 64 experts at a time; returns false if `logical` is past the last tile.
+struct RowTile {
+    int expert, tile_n, rows_valid;
+    int64_t row0;
+};
+
+__device__ __forceinline__ void place_in_expert(int local, int count, int tiles_n, int &row_tile, int &tile_n) {
+    const int groups = (count + kGroupRows - 1) / kGroupRows;
+    const int base = count / groups, larger = count % groups;  // the first `larger` groups have base + 1 row tiles
+    const int larger_tiles = larger * (base + 1) * tiles_n;
+    int first_row, rows, in_group;
+    if (local < larger_tiles) {
+        const int group = local / ((base + 1) * tiles_n);
+        rows = base + 1;
+        first_row = group * rows;
+        in_group = local - group * rows * tiles_n;
+    } else {
+        const int rest = local - larger_tiles;
+        const int group = rest / (base * tiles_n);
+        rows = base;
+        first_row = larger * (base + 1) + group * rows;
+        in_group = rest - group * rows * tiles_n;
+    }
+    row_tile = first_row + in_group % rows;
+    tile_n = in_group / rows;
+}
+
+template <int kTile>
+__device__ __forceinline__ bool locate_tile(const GemmArgs &args, int logical, RowTile &tile) {
+    const int tiles_n = args.tiles_n;
+    if (args.expert_ends == nullptr) {
+        const int count = static_cast<int>((args.rows + kTile - 1) / kTile);
+        if (logical >= count * tiles_n) return false;
+        int row_tile;
+        place_in_expert(logical, count, tiles_n, row_tile, tile.tile_n);
+        tile.expert = 0;
+        tile.row0 = static_cast<int64_t>(row_tile) * kTile;
+        tile.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.rows - tile.row0));
+        return true;
+    }
+    const int lane = opaque(static_cast<int>(threadIdx.x & 63));
+    int tiles_before = 0;  // row tiles of the experts before this block of 64
+    for (int base = 0; base < args.num_experts; base += 64) {
+        const int e = base + lane;
+        int64_t begin = 0, end = 0;
+        if (e < args.num_experts) {
+            end = min(load_index(args.expert_ends, args.index_dtype, e), args.rows);
+            begin = e > 0 ? load_index(args.expert_ends, args.index_dtype, e - 1) : 0;
+        }
+        const int count = end > begin ? static_cast<int>((end - begin + kTile - 1) / kTile) : 0;
+        int inclusive = count;
+#pragma unroll
+        for (int offset = 1; offset < 64; offset <<= 1) {
+            const int other = __shfl_up(inclusive, offset, 64);
+            if (lane >= offset) inclusive += other;
+        }
+        const int total = __shfl(inclusive, 63, 64);
+        if (logical < (tiles_before + total) * tiles_n) {
+            const uint64_t owners = __ballot((tiles_before + inclusive) * tiles_n > logical);
+            const int owner = __ffsll(static_cast<unsigned long long>(owners)) - 1;
+            const int owner_count = __shfl(count, owner, 64);
+            const int first_tile = tiles_before + __shfl(inclusive - count, owner, 64);
+            const int64_t owner_begin = __shfl(begin, owner, 64), owner_end = __shfl(end, owner, 64);
+            int row_tile;
+            place_in_expert(logical - first_tile * tiles_n, owner_count, tiles_n, row_tile, tile.tile_n);
+            tile.expert = base + owner;
+            tile.row0 = owner_begin + static_cast<int64_t>(row_tile) * kTile;
+            tile.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), owner_end - tile.row0));
+            return true;
+        }
+        tiles_before += total;
+    }
+    return false;
+}
+
+// Logical tile -> (row tile, column tile) for the row-sparse product, whose row tiles are expert-aligned by
+// construction: groups of 8 row tiles, column by column inside a group.
+__device__ __forceinline__ void tile_coordinates(int logical, int tiles_m, int tiles_n, int &tile_m, int &tile_n) {
+    const int width = kGroupRows * tiles_n;
+    const int group = logical / width;
+    const int first_m = group * kGroupRows;
+    const int group_rows = min(tiles_m - first_m, kGroupRows);
+    const int in_group = logical - group * width;
+    tile_m = first_m + in_group % group_rows;
+    tile_n = in_group / group_rows;
+}
 
 template <typename OutT>
 __device__ __forceinline__ void store_out(void *out, int64_t offset, float value, bool accumulate) {
@@ -64,5 +181,9 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype);  // with args.f
 // `workspace` (may be null: no split) must hold mfma_gemm_workspace_size(args) bytes when that is not 0.
 size_t mfma_gemm_workspace_size(GemmArgs args);
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream);
+
+// fp32 operands with a unit stride and 16-byte aligned lines (fm_gemm_f32.hip).
+bool f32_gemm_eligible(const GemmArgs &args, int dtype);
+int f32_gemm_launch(GemmArgs args, hipStream_t stream);
 
 }  // namespace fm

@@ -63,9 +63,6 @@ __device__ __forceinline__ void store_streaming(T *pointer, const Vec16x4<T> &va
     __builtin_nontemporal_store(__builtin_bit_cast(Raw, value), reinterpret_cast<Raw *>(pointer));
 }
 
-#define FM_LDS(T) __attribute__((address_space(3))) T
-#define FM_GLOBAL(T) __attribute__((address_space(1))) T
-
 template <typename T>
 struct Mfma;
 template <>
@@ -95,7 +92,6 @@ constexpr int kWaveRows = kTile / kWavesM, kWaveCols = kTile / kWavesN;  // a wa
 constexpr int kTilesM = kWaveRows / 32, kTilesN = kWaveCols / 32;        // in 32x32 MFMA accumulators
 constexpr int kChunksPerRow = kBK / 8;          // 16-byte chunks of a K-major row
 constexpr int kLoadsPerOperand = kOperandBytes / 16 / kMfmaThreads;  // 16-byte loads per lane, operand and slice
-constexpr int kBufferResourceFlags = 0x00020000;  // raw buffer, 32-bit data format, no swizzle
 constexpr int kEpiloguePadBytes = 16;  // after each staged row of the epilogue; keeps 16-byte alignment and spreads
                                        // the rows over the banks
 constexpr int kStagingBase = kOperandBytes;  // the epilogue stages rows in LDS from here up to the last lhs slot
@@ -118,22 +114,6 @@ __device__ __forceinline__ int lds_offset_k_major(int row, int chunk) {
 // A transpose load by 32 lanes touches 4 K-rows x 2 groups; the XOR sends them to 8 different bank octets.
 __device__ __forceinline__ int lds_offset_row_major(int k, int row) {
     return k * (kTile * 2) + ((((row >> 4) ^ ((k & 3) << 1)) << 5) | ((row & 15) << 1));
-}
-
-// The same value, but the compiler cannot tell: what is computed from it is computed where it is written, not hoisted
-// out of an enclosing loop into registers that stay occupied across the loop.
-__device__ __forceinline__ int opaque(int value) {
-    asm volatile("" : "+v"(value));
-    return value;
-}
-
-// Tell the compiler that a pointer computed from tile coordinates is the same in every lane (it then lives in
-// scalar registers and the loads use the scalar-base addressing form).
-__device__ __forceinline__ const char *uniform_pointer(const char *pointer) {
-    const uint64_t bits = reinterpret_cast<uint64_t>(pointer);
-    const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits));
-    const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32));
-    return reinterpret_cast<const char *>((static_cast<uint64_t>(high) << 32) | low);
 }
 
 __device__ __forceinline__ int64_t uniform_int64(int64_t value) {
@@ -325,100 +305,8 @@ struct TileWork {
     int64_t k_lo, k_hi;
 };
 
-constexpr int kXcds = 8, kGroupRows = 8, kChunkTiles = 32;
+constexpr int kXcds = 8, kChunkTiles = 32;
 constexpr int kHalfTileMaxSlices = 64;  // reductions of this many slices or more have no half tiles (see find_tile)
-
-// Logical order of the tiles of a product whose rows are grouped by expert (output-sparse, input-inner-sparse,
-// dense): expert after expert; within an expert its row tiles (ceil(rows_e / 256)) are cut into ceil(count / 8)
-// groups of nearly equal size (9 row tiles: 5 + 4), and a group is walked column tile by column tile, row tiles
-// fastest. 32 consecutive tiles (what an XCD runs at one time) are then about 8 row tiles x 4 column tiles of ONE
-// expert, i.e. 8 lhs panels and 4 rhs panels shared in that XCD's L2; with groups that ignore the expert boundaries
-// most chunks straddled two experts and needed twice the rhs panels.
-// Every wavefront scans `expert_ends` 64 experts at a time; returns false if `logical` is past the last tile.
-struct RowTile {
-    int expert, tile_n, rows_valid;
-    int64_t row0;
-};
-
-__device__ __forceinline__ void place_in_expert(int local, int count, int tiles_n, int &row_tile, int &tile_n) {
-    const int groups = (count + kGroupRows - 1) / kGroupRows;
-    const int base = count / groups, larger = count % groups;  // the first `larger` groups have base + 1 row tiles
-    const int larger_tiles = larger * (base + 1) * tiles_n;
-    int first_row, rows, in_group;
-    if (local < larger_tiles) {
-        const int group = local / ((base + 1) * tiles_n);
-        rows = base + 1;
-        first_row = group * rows;
-        in_group = local - group * rows * tiles_n;
-    } else {
-        const int rest = local - larger_tiles;
-        const int group = rest / (base * tiles_n);
-        rows = base;
-        first_row = larger * (base + 1) + group * rows;
-        in_group = rest - group * rows * tiles_n;
-    }
-    row_tile = first_row + in_group % rows;
-    tile_n = in_group / rows;
-}
-
-__device__ __forceinline__ bool locate_tile(const GemmArgs &args, int logical, RowTile &tile) {
-    const int tiles_n = args.tiles_n;
-    if (args.expert_ends == nullptr) {
-        const int count = static_cast<int>((args.rows + kTile - 1) / kTile);
-        if (logical >= count * tiles_n) return false;
-        int row_tile;
-        place_in_expert(logical, count, tiles_n, row_tile, tile.tile_n);
-        tile.expert = 0;
-        tile.row0 = static_cast<int64_t>(row_tile) * kTile;
-        tile.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.rows - tile.row0));
-        return true;
-    }
-    const int lane = opaque(static_cast<int>(threadIdx.x & 63));
-    int tiles_before = 0;  // row tiles of the experts before this block of 64
-    for (int base = 0; base < args.num_experts; base += 64) {
-        const int e = base + lane;
-        int64_t begin = 0, end = 0;
-        if (e < args.num_experts) {
-            end = min(load_index(args.expert_ends, args.index_dtype, e), args.rows);
-            begin = e > 0 ? load_index(args.expert_ends, args.index_dtype, e - 1) : 0;
-        }
-        const int count = end > begin ? static_cast<int>((end - begin + kTile - 1) / kTile) : 0;
-        int inclusive = count;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const int other = __shfl_up(inclusive, offset, 64);
-            if (lane >= offset) inclusive += other;
-        }
-        const int total = __shfl(inclusive, 63, 64);
-        if (logical < (tiles_before + total) * tiles_n) {
-            const uint64_t owners = __ballot((tiles_before + inclusive) * tiles_n > logical);
-            const int owner = __ffsll(static_cast<unsigned long long>(owners)) - 1;
-            const int owner_count = __shfl(count, owner, 64);
-            const int first_tile = tiles_before + __shfl(inclusive - count, owner, 64);
-            const int64_t owner_begin = __shfl(begin, owner, 64), owner_end = __shfl(end, owner, 64);
-            int row_tile;
-            place_in_expert(logical - first_tile * tiles_n, owner_count, tiles_n, row_tile, tile.tile_n);
-            tile.expert = base + owner;
-            tile.row0 = owner_begin + static_cast<int64_t>(row_tile) * kTile;
-            tile.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), owner_end - tile.row0));
-            return true;
-        }
-        tiles_before += total;
-    }
-    return false;
-}
-
-// Logical tile -> (row tile, column tile) for the row-sparse product, whose row tiles are expert-aligned by
-// construction: groups of 8 row tiles, column by column inside a group.
-__device__ __forceinline__ void tile_coordinates(int logical, int tiles_m, int tiles_n, int &tile_m, int &tile_n) {
-    const int width = kGroupRows * tiles_n;
-    const int group = logical / width;
-    const int first_m = group * kGroupRows;
-    const int group_rows = min(tiles_m - first_m, kGroupRows);
-    const int in_group = logical - group * width;
-    tile_m = first_m + in_group % group_rows;
-    tile_n = in_group / group_rows;
-}
 
 // Where the operands and the output of logical tile `logical` are. False: there is no such tile.
 __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, TileWork &work) {
@@ -447,7 +335,7 @@ __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, 
         return true;
     }
     RowTile tile;
-    if (!locate_tile(args, logical, tile)) return false;
+    if (!locate_tile<kTile>(args, logical, tile)) return false;
     // A tile of the fused gated forward product has 128 gate columns (and their up columns).
     const bool paired = args.fusion == kFusionGatedForward;
     const int64_t col0 = static_cast<int64_t>(tile.tile_n) * (paired ? kTile / 2 : kTile);

@@ -579,6 +579,41 @@ def test_expert_boundaries_inside_a_tile(pad, dtype, device):
     assert max_rel_err(out.cpu(), expected) <= tolerance
 
 
+# Reductions around the slices of 16 and 32, columns around the tiles of 32 and 64; with 4100 columns the launches have
+# enough tiles for the larger one.
+@pytest.mark.parametrize("inner", [4, 12, 16, 28, 36, 132])
+@pytest.mark.parametrize("other", [4, 36, 100, 4100])
+def test_fp32_tiles_and_remainders(inner, other, device):
+    """All three products and operand layouts of the fp32 matrix-core kernel, NaN in the rows after an expert's last
+    token, accumulation on top of the first results."""
+    generator = torch.Generator().manual_seed(inner + other)
+    experts, dtype = 5, torch.float32
+    oracle_map = fixture_sparse_map(case := _ragged_case(inner, experts))
+    oracle_map.num_rows = case["expert_ends"][-1] + case["phantom_rows"]
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    real = oracle_map.real_row_mask()
+    x, y = (_normal(oracle_map.num_rows, size, dtype, generator) for size in (inner, other))
+    weight, weight_inner = _normal(experts * other, inner, dtype, generator), _normal(experts * inner, other, dtype, generator)
+    expected = moe_oracle.output_sparse_matmul(x, weight.t(), oracle_map)
+    expected_inner = moe_oracle.input_inner_sparse_matmul(x, weight_inner, oracle_map)
+    expected_row = moe_oracle.input_row_sparse_matmul(x.t(), y, oracle_map)
+    x[~real] = y[~real] = float("nan")
+    x, y, weight, weight_inner = (tensor.to(device) for tensor in (x, y, weight, weight_inner))
+    for rhs in (weight.t(), weight.t().contiguous()):
+        out = output_sparse_matmul(x, rhs, sparse_map)
+        assert max_rel_err(out.cpu()[real], expected[real]) <= 1e-5
+        output_sparse_matmul(x, rhs, sparse_map, out, accumulate=True)
+        assert max_rel_err(out.cpu()[real], 2 * expected[real]) <= 1e-5
+    out = input_inner_sparse_matmul(x, weight_inner, sparse_map)
+    assert max_rel_err(out.cpu()[real], expected_inner[real]) <= 1e-5
+    out = input_row_sparse_matmul(x.t(), y, sparse_map)
+    assert max_rel_err(out.cpu(), expected_row) <= 1e-5
+    input_row_sparse_matmul(x.t(), y, sparse_map, out, accumulate=True)
+    assert max_rel_err(out.cpu(), 2 * expected_row) <= 1e-5
+    dense = dense_matmul(weight[:, :inner].t().contiguous().t(), weight_inner[:inner].contiguous())
+    assert max_rel_err(dense.cpu(), weight.cpu() @ weight_inner[:inner].cpu()) <= 1e-5
+
+
 @pytest.mark.parametrize("inner", [8, 56, 72, 120, 136, 1000, 2104])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_reductions_of_no_whole_number_of_slices(inner, dtype, device):
