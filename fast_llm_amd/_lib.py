@@ -52,6 +52,8 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_ptr] * 6 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr],
     ),
+    "fm_few_tokens_workspace_size": (_c_size, [_c_i64] * 5 + [_c_int] * 2),
+    "fm_few_tokens_forward": (_c_int, [_c_ptr] * 6 + [_c_i64] * 5 + [_c_int] * 3 + [_c_ptr, _c_size, _c_ptr]),
 }
 
 FM_ERR_INVALID_ARGUMENT, FM_ERR_UNSUPPORTED, FM_ERR_LAUNCH = -1, -2, -3

@@ -26,7 +26,12 @@ from fast_llm_amd.functional.sparse_copy import (
     copy_sparse_to_dense_forward,
 )
 from fast_llm_amd.functional.sparse_linear import output_sparse_matmul
-from fast_llm_amd.functional.utils import wrap_forward_backward
+from fast_llm_amd.functional.utils import Assert, wrap_forward_backward
+
+# Up to this many rows per expert, on average, inference takes the kernels for few tokens (`few_tokens_forward`). us there /
+# with a sparse layout: 2 of 8 experts, 4096 x 14336: 32 rows 621 / 708, 48 rows 709 / 718, 64 rows 1025 / 714; 6 of 64
+# experts, 2048 x 1408: 24 rows 272 / 341, 36 rows 325 / 343; 2 of 16 experts, 1024 x 4096: 48 rows 163 / 180.
+FEW_TOKENS_MAX_ROWS_PER_EXPERT = 40
 
 
 def _activation_tag(activation_type: ActivationType | str) -> int:
@@ -376,6 +381,48 @@ def mlp_backward(grad_output: torch.Tensor, context: list[typing.Any]) -> tuple[
 
 
 mlp_autograd = wrap_forward_backward(mlp_forward, mlp_backward)
+
+
+def few_tokens_forward(
+    input_: torch.Tensor,
+    scores: torch.Tensor,
+    top_experts: torch.Tensor,
+    weight_1: torch.Tensor,
+    weight_2: torch.Tensor,
+    num_experts: int,
+    gated: bool,
+    activation_type: ActivationType,
+) -> torch.Tensor | None:
+    """
+    `mlp_forward(..., training=False)` of `input_` [tokens, hidden] straight from the routing (`scores` and `top_experts`
+    [tokens, k], no sparse map) by the kernels for few tokens, weights in the layouts of the sparse MLP. None where they
+    are not the faster way or do not take the operands.
+    """
+    tokens, slots = top_experts.shape
+    if tokens * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts or input_.dtype not in (torch.bfloat16, torch.float16):
+        return None
+    hidden, dtype = input_.size(1), _lib.dtype_tag(input_.dtype)
+    ffn = weight_2.size(0) // num_experts
+    size = _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), dtype)
+    tensors = (input_, top_experts, scores, weight_1, weight_2)
+    if size == 0 or weight_1.dtype != input_.dtype or weight_2.dtype != input_.dtype or weight_2.size(1) != hidden:
+        return None
+    if top_experts.dtype != torch.int64 or not all(tensor.is_contiguous() for tensor in tensors):
+        return None
+    device = _lib.require_device(*tensors)
+    Assert.eq(tuple(weight_1.shape), (num_experts * ffn * (2 if gated else 1), hidden))
+    Assert.eq(input_.size(0), tokens)
+    Assert.eq(scores.shape, top_experts.shape)
+    if scores.dtype != torch.float32:
+        scores = scores.float()
+    output = torch.empty_like(input_)
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    _lib.call(
+        "fm_few_tokens_forward", device, input_.data_ptr(), top_experts.data_ptr(), scores.data_ptr(), weight_1.data_ptr(),
+        weight_2.data_ptr(), output.data_ptr(), tokens, slots, hidden, ffn, num_experts, int(gated),
+        _activation_tag(activation_type), dtype, workspace.data_ptr(), size,
+    )  # fmt: skip
+    return output
 
 
 def mlp_autograd_looped(

@@ -11,7 +11,7 @@ Weight layout as in the reference: `layer_1.weight` [experts * 2 * ffn, hidden] 
 import torch
 
 from fast_llm_amd.functional.config import ActivationType, MLPRecomputeLevel
-from fast_llm_amd.functional.mlp import mlp_autograd
+from fast_llm_amd.functional.mlp import few_tokens_forward, mlp_autograd
 from fast_llm_amd.functional.sparse_copy import get_sparse_map
 
 
@@ -173,6 +173,12 @@ class DroplessMoEMLP(torch.nn.Module):
         if top_experts is None:
             # The router has counted the tokens of every expert on its way: the map need not count them again.
             scores, top_experts, router_counts = self.route_with_counts(hidden_states, grad_scale, losses)
+        if not self.training and scores is not None:
+            output = few_tokens_forward(
+                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation
+            )  # fmt: skip
+            if output is not None:
+                return output.view_as(input_)
         sparse_map = get_sparse_map(
             top_experts, self.experts, dynamic_shape=self.dropless_dynamic_shape, router_counts=router_counts
         )

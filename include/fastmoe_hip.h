@@ -338,6 +338,24 @@ int fm_output_sparse_matmul_gated_activation_backward(const void *lhs, const voi
                                                       int64_t rhs_stride_col, int activation, int dtype,
                                                       int index_dtype, void *stream);
 
+/* Inference of the dropless MoE MLP (dispatch, layer 1, activation, layer 2, combine: reference
+ * fast_llm/functional/triton/mlp.py:207-285 with training=False) for few tokens, in three kernels that read every selected
+ * expert's weights once for all its tokens and use no sparse layout:
+ *   output[t, :] = sum_j scores[t, j] * (act(input[t, :] . W1_e^T) [* up]) . W2_e,  e = top_experts[t, j].
+ * input, output [num_tokens, hidden], weight_1 [num_experts * ffn * (2 if gated), hidden], weight_2 [num_experts * ffn,
+ * hidden], all contiguous and 16-byte aligned, of `dtype` (bf16 or fp16); top_experts [num_tokens, slots_per_token] int64,
+ * scores fp32. Entries of top_experts outside [0, num_experts) contribute nothing. Layer 1's output is rounded to `dtype`
+ * before the activation and the activation's before layer 2, as in the separate kernels; layer 2's is not rounded.
+ * `workspace`: fm_few_tokens_workspace_size(...) bytes, 16-byte aligned; that function returns 0 for what these kernels do
+ * not take (other dtypes, hidden or ffn not multiples of 8, more than 4096 (token, slot) pairs, an expert's weight of 4
+ * GiB or more), which FM_ERR_UNSUPPORTED then reports. */
+size_t fm_few_tokens_workspace_size(int64_t num_tokens, int64_t slots_per_token, int64_t hidden, int64_t ffn,
+                                    int64_t num_experts, int gated, int dtype);
+int fm_few_tokens_forward(const void *input, const void *top_experts, const void *scores, const void *weight_1,
+                          const void *weight_2, void *output, int64_t num_tokens, int64_t slots_per_token, int64_t hidden,
+                          int64_t ffn, int64_t num_experts, int gated, int activation, int dtype, void *workspace,
+                          size_t workspace_size, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,64 @@
+"""The inference kernels for few tokens against the oracle's dropless MLP."""
+
+import pytest
+import torch
+
+from fast_llm_amd.functional import mlp
+from fast_llm_amd.functional.config import ActivationType
+from oracle import moe_oracle
+from tests.helpers import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+_MAX_REL = {torch.bfloat16: 1e-2, torch.float16: 2e-3}
+
+
+def _expected(x, scores, top_experts, weight_1, weight_2, experts, gated, activation):
+    """Per expert in fp32, rounded to the operands' type where the kernels round: before and after the activation."""
+    dtype, out = x.dtype, torch.zeros(x.shape)
+    for e, (w1, w2) in enumerate(zip(weight_1.chunk(experts), weight_2.chunk(experts))):
+        token, slot = torch.where(top_experts == e)
+        layer_1 = (x[token].float() @ w1.float().t()).to(dtype).float()
+        act = moe_oracle.mlp_activation_forward(layer_1, gated, activation.value).to(dtype).float()
+        out.index_add_(0, token, (act @ w2.float()) * scores[token, slot, None])
+    return out
+
+
+# Tokens, experts and slots on each side of where the kernels change: one workgroup row per entry or per expert, mean rows
+# per expert of 10 and 24 (one, two or four groups of 16 tokens), experts with more rows than a group.
+@pytest.mark.parametrize(("tokens", "experts", "slots"), [(1, 8, 2), (3, 64, 6), (16, 4, 2), (17, 4, 1), (40, 6, 3), (65, 5, 2), (99, 5, 2)])
+# Sizes around the chunks (128 of K, 16 and 128 outputs), and more than one piece of layer 2's reduction.
+@pytest.mark.parametrize(("hidden", "ffn"), [(64, 72), (136, 128), (264, 1032), (2056, 40)])
+@pytest.mark.parametrize(("dtype", "gated", "activation"), [
+    (torch.bfloat16, True, ActivationType.silu), (torch.float16, True, ActivationType.gelu),
+    (torch.bfloat16, False, ActivationType.squared_relu),
+])  # fmt: skip
+def test_few_tokens_forward(tokens, experts, slots, hidden, ffn, dtype, gated, activation, device):
+    generator = torch.Generator().manual_seed(tokens + hidden)
+    x = torch.randn(tokens, hidden, generator=generator).to(dtype)
+    weight_1 = torch.normal(0, 0.1, (experts * ffn * (1 + gated), hidden), generator=generator).to(dtype)
+    weight_2 = torch.normal(0, 0.1, (experts * ffn, hidden), generator=generator).to(dtype)
+    # Preferred experts: some get many rows, some none.
+    logits = torch.randn(tokens, experts, generator=generator) + 2 * torch.randn(experts, generator=generator)
+    scores, top_experts = moe_oracle.topk_routing(logits, slots)
+    if tokens > 1:
+        top_experts[1, 0] = -1  # an entry that selects no expert contributes nothing
+    output = mlp.few_tokens_forward(
+        *(t.to(device) for t in (x, scores, top_experts, weight_1, weight_2)), experts, gated, activation
+    )
+    expected = _expected(x, scores, top_experts, weight_1, weight_2, experts, gated, activation)
+    assert output.dtype == dtype
+    # The sums differ from the oracle's in their order: a value next to a rounding boundary of the activation's type may
+    # fall on its other side, which the type's own bound covers.
+    assert max_rel_err(output.cpu(), expected) <= _MAX_REL[dtype]
+
+
+def test_few_tokens_forward_leaves_the_rest_to_the_sparse_layout(device):
+    def call(tokens, dtype=torch.bfloat16, ffn=64):
+        x, weight_1, weight_2 = (torch.zeros(rows, 64, dtype=dtype, device=device) for rows in (tokens, 8 * ffn, 4 * ffn))
+        scores, top_experts = torch.ones(tokens, 2, device=device), torch.zeros(tokens, 2, dtype=torch.int64, device=device)
+        return mlp.few_tokens_forward(x, scores, top_experts, weight_1, weight_2, 4, True, ActivationType.silu)
+
+    limit = mlp.FEW_TOKENS_MAX_ROWS_PER_EXPERT * 2
+    assert call(limit) is not None and call(limit + 1) is None
+    assert call(4, torch.float32) is None and call(4, ffn=60) is None
