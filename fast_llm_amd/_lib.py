@@ -17,6 +17,33 @@ FM_VERSION = 10
 
 _c_i64, _c_int, _c_ptr, _c_size = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 
+
+class MoELayer(ctypes.Structure):
+    """`fm_moe_layer` of include/fastmoe_hip.h, field for field."""
+
+    _fields_ = (
+        [
+            (name, _c_i64)
+            for name in (
+                "tokens", "hidden", "ffn", "routed_experts", "shared_experts", "experts_per_token", "gated", "activation",
+                "dtype", "grad_dtype", "with_losses", "recompute_input", "recompute_layer_1", "recompute_activation",
+                "accumulate_1", "accumulate_2",
+            )
+        ]
+        + [(name, ctypes.c_double) for name in ("auxiliary_loss_grad", "z_loss_grad")]
+        + [(name, _c_i64) for name in ("dynamic_rows", "rows", "routing_bytes", "workspace_bytes", "index_dtype", "used_rows_offset")]
+        + [
+            (name, _c_ptr)
+            for name in (
+                "logits", "noise", "input", "weight_1", "weight_2", "routing", "workspace", "sparse_input", "layer_1_output",
+                "activation_output", "layer_2_output", "output", "grad_output", "grad_layer_2_output",
+                "grad_activation_output", "grad_layer_1_output", "grad_scores", "grad_logits", "grad_input", "grad_weight_1",
+                "grad_weight_2",
+            )
+        ]
+    )  # fmt: skip
+
+
 # name -> (restype, argtypes). Mirrors include/fastmoe_hip.h one to one; tests check that every declared symbol
 # is listed here and exported by the library.
 SIGNATURES: dict[str, tuple] = {
@@ -52,6 +79,10 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_ptr] * 6 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr],
     ),
+    "fm_moe_layer_sizes": (_c_int, [_c_ptr]),
+    "fm_moe_layer_route": (_c_int, [_c_ptr, _c_ptr]),
+    "fm_moe_layer_forward": (_c_int, [_c_ptr, _c_ptr]),
+    "fm_moe_layer_backward": (_c_int, [_c_ptr, _c_ptr]),
     "fm_few_tokens_workspace_size": (_c_size, [_c_i64] * 5 + [_c_int] * 2),
     "fm_few_tokens_forward": (_c_int, [_c_ptr] * 6 + [_c_i64] * 5 + [_c_int] * 3 + [_c_ptr, _c_size, _c_ptr]),
 }

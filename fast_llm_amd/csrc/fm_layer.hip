@@ -1,0 +1,234 @@
+// The MoE layer's forward and backward as one or two host calls each: the launches of the router, the sparse map, the copies, the
+// activation and the grouped products in the order of a layer step, on the caller's stream and buffers.
+//
+// What bounds a small layer is the host: a step of 512 tokens, 256 x 512, runs 20 kernels that the device finishes in 166 us,
+// and launching them one Python call at a time took 567 us. Through these calls it takes 300.
+#include "fm_gemm_common.h"
+#include "fm_router_layout.h"
+
+namespace fm {
+
+namespace {
+
+struct Plan {
+    int64_t experts, slots, rows, used_index_size;
+    int index_dtype;
+    size_t losses, top_experts, scores, lse, statistics, sparse_rows, expert_ends, expert_pad_begins, router, routing_bytes;
+    size_t workspace_bytes;
+};
+
+constexpr int64_t kPad = 128;
+
+int make_plan(const fm_moe_layer &layer, Plan &plan) {
+    const char *name = "fm_moe_layer";
+    FM_REQUIRE(layer.tokens > 0 && layer.hidden > 0 && layer.ffn > 0 && layer.routed_experts > 0 && layer.shared_experts >= 0 &&
+                   layer.experts_per_token > 0,
+               "%s: bad shape", name);
+    FM_REQUIRE(valid_dtype(static_cast<int>(layer.dtype)), "%s: bad dtype", name);
+    plan.experts = layer.routed_experts + layer.shared_experts;
+    plan.slots = layer.experts_per_token + layer.shared_experts;
+    const int64_t entries = layer.tokens * plan.slots;
+    const int64_t most_rows = (entries + plan.experts * kPad) / kPad * kPad;
+    FM_REQUIRE(layer.dynamic_rows >= 0 && layer.dynamic_rows <= most_rows, "%s: %lld rows of at most %lld", name,
+               static_cast<long long>(layer.dynamic_rows), static_cast<long long>(most_rows));
+    plan.rows = layer.dynamic_rows > 0 ? layer.dynamic_rows : most_rows;
+    plan.index_dtype = most_rows < 32768 ? FM_INDEX_I16 : FM_INDEX_I32;
+    plan.used_index_size = plan.index_dtype == FM_INDEX_I16 ? 2 : 4;
+    size_t at = 0;
+    const auto take = [&](size_t bytes) {
+        const size_t offset = at;
+        at += (bytes + 63) / 64 * 64;
+        return offset;
+    };
+    plan.losses = take(8);  // first: the caller reads them
+    plan.top_experts = take(8 * entries);
+    plan.scores = take(4 * entries);
+    plan.lse = take(8 * layer.tokens);
+    plan.statistics = take(4 * RouterStats::size(static_cast<int>(layer.routed_experts)));
+    plan.sparse_rows = take(plan.used_index_size * entries);
+    plan.expert_ends = take(plan.used_index_size * plan.experts);
+    plan.expert_pad_begins = take(plan.used_index_size * plan.experts);
+    plan.router = take(fm_router_workspace_size(layer.tokens, layer.routed_experts));
+    plan.routing_bytes = at;
+    const int64_t ffn_1 = layer.ffn * (layer.gated ? 2 : 1);
+    const int dtype = static_cast<int>(layer.dtype);
+    plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
+    for (size_t bytes : {fm_grouped_gemm_workspace_size(plan.rows, ffn_1, layer.hidden, plan.experts, dtype),
+                         fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, layer.ffn, plan.experts, dtype),
+                         fm_grouped_gemm_workspace_size(plan.rows, layer.ffn, layer.hidden, plan.experts, dtype),
+                         fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, ffn_1, plan.experts, dtype),
+                         fm_input_row_sparse_matmul_workspace_size(layer.ffn, layer.hidden, plan.rows, plan.experts, dtype),
+                         fm_input_row_sparse_matmul_workspace_size(ffn_1, layer.hidden, plan.rows, plan.experts, dtype)})
+        if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+    return FM_OK;
+}
+
+// The calls of one layer step: the first failure ends it, a remark (the generic kernel ran) is kept.
+struct Step {
+    const fm_moe_layer &layer;
+    const Plan &plan;
+    void *stream;
+    int note = FM_OK;
+
+    char *routing(size_t offset) const { return static_cast<char *>(layer.routing) + offset; }
+    int dtype() const { return static_cast<int>(layer.dtype); }
+    int64_t ffn_1() const { return layer.ffn * (layer.gated ? 2 : 1); }
+    int keep(int status) {
+        if (status > 0) note = status;
+        return status < 0 ? status : FM_OK;
+    }
+
+    int dispatch(void *out) {
+        return fm_copy_dense_to_sparse(layer.input, nullptr, routing(plan.sparse_rows), out, layer.tokens, layer.hidden, plan.slots,
+                                       plan.rows, dtype(), FM_DTYPE_F32, plan.index_dtype, stream);
+    }
+    int combine(const void *in, const void *scores, void *out) {
+        return fm_copy_sparse_to_dense(in, scores, routing(plan.sparse_rows), out, layer.tokens, layer.hidden, plan.slots, plan.rows,
+                                       dtype(), FM_DTYPE_F32, plan.index_dtype, stream);
+    }
+    // out [rows, columns] = lhs [rows, inner] x (weight_e [columns, inner])^T
+    int output_sparse(const void *lhs, const void *weight, void *out, int64_t columns, int64_t inner) {
+        const size_t bytes = fm_grouped_gemm_workspace_size(plan.rows, columns, inner, plan.experts, dtype());
+        return keep(fm_output_sparse_matmul(lhs, weight, out, routing(plan.expert_ends), plan.rows, columns, inner, plan.experts, inner,
+                                            1, 1, inner, columns, 1, 0, dtype(), dtype(), plan.index_dtype,
+                                            bytes ? layer.workspace : nullptr, bytes, stream));
+    }
+    // out [rows, hidden] = lhs [rows, inner] x weight_e [inner, hidden]
+    int inner_sparse(const void *lhs, const void *weight, void *out, int64_t inner) {
+        const size_t bytes = fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, inner, plan.experts, dtype());
+        return keep(fm_input_inner_sparse_matmul(lhs, weight, out, routing(plan.expert_ends), plan.rows, layer.hidden, inner,
+                                                 plan.experts, inner, 1, layer.hidden, 1, layer.hidden, 1, 0, dtype(), dtype(),
+                                                 plan.index_dtype, bytes ? layer.workspace : nullptr, bytes, stream));
+    }
+    // out [experts * size, hidden] (+)= lhs^T x rhs, lhs [rows, size], rhs [rows, hidden]
+    int row_sparse(const void *lhs, const void *rhs, void *out, int64_t size, bool accumulate) {
+        const size_t bytes = fm_input_row_sparse_matmul_workspace_size(size, layer.hidden, plan.rows, plan.experts, dtype());
+        return keep(fm_input_row_sparse_matmul(lhs, rhs, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), size,
+                                               layer.hidden, plan.rows, plan.experts, 1, size, layer.hidden, 1, layer.hidden, 1,
+                                               accumulate, dtype(), static_cast<int>(layer.grad_dtype), plan.index_dtype,
+                                               bytes ? layer.workspace : nullptr, bytes, stream));
+    }
+    const void *rows_in_use() const { return routing(plan.expert_ends + (plan.experts - 1) * plan.used_index_size); }
+};
+
+#define FM_STEP(call) \
+    if (int status = (call)) return status
+
+int route(const fm_moe_layer &layer, const Plan &plan, void *stream) {
+    Step step{layer, plan, stream};
+    FM_REQUIRE(layer.logits && layer.routing && layer.workspace, "fm_moe_layer_forward: null tensor");
+    const bool losses = layer.with_losses != 0;
+    FM_STEP(fm_router_forward(layer.logits, layer.noise, step.routing(plan.top_experts), step.routing(plan.scores),
+                              losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
+                              losses ? step.routing(plan.losses) : nullptr, step.routing(plan.router),
+                              plan.routing_bytes - plan.router, layer.tokens, layer.routed_experts, layer.experts_per_token,
+                              layer.shared_experts, step.dtype(), stream));
+    FM_STEP(fm_sparse_map_from_router(reinterpret_cast<const int64_t *>(step.routing(plan.top_experts)), step.routing(plan.router),
+                                      plan.routing_bytes - plan.router, layer.tokens, plan.experts, layer.experts_per_token,
+                                      layer.shared_experts, kPad, plan.index_dtype, step.routing(plan.sparse_rows),
+                                      step.routing(plan.expert_ends), step.routing(plan.expert_pad_begins), layer.workspace,
+                                      plan.workspace_bytes, stream));
+    return FM_OK;
+}
+
+int forward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
+    Step step{layer, plan, stream};
+    FM_REQUIRE(layer.input && layer.weight_1 && layer.weight_2 && layer.routing && layer.sparse_input && layer.activation_output &&
+                   layer.layer_2_output && layer.output && layer.workspace,
+               "fm_moe_layer_forward: null tensor");
+    FM_STEP(step.dispatch(layer.sparse_input));
+    if (layer.layer_1_output == nullptr) {
+        // The product with the activation in its epilogue; FM_ERR_UNSUPPORTED tells the caller to bring a layer-1 buffer.
+        FM_STEP(fm_output_sparse_matmul_gated_activation(layer.sparse_input, layer.weight_1, nullptr, layer.activation_output,
+                                                         step.routing(plan.expert_ends), plan.rows, layer.ffn, layer.hidden,
+                                                         plan.experts, layer.hidden, 1, 1, layer.hidden,
+                                                         static_cast<int>(layer.activation), step.dtype(), plan.index_dtype, stream));
+    } else {
+        FM_STEP(step.output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, step.ffn_1(), layer.hidden));
+        FM_STEP(fm_mlp_activation_forward(layer.layer_1_output, layer.activation_output, plan.rows, layer.ffn,
+                                          static_cast<int>(layer.gated), static_cast<int>(layer.activation), step.dtype(),
+                                          step.rows_in_use(), plan.index_dtype, stream));
+    }
+    FM_STEP(step.inner_sparse(layer.activation_output, layer.weight_2, layer.layer_2_output, layer.ffn));
+    FM_STEP(step.combine(layer.layer_2_output, step.routing(plan.scores), layer.output));
+    return step.note;
+}
+
+int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
+    Step step{layer, plan, stream};
+    FM_REQUIRE(layer.logits && layer.weight_1 && layer.weight_2 && layer.routing && layer.sparse_input && layer.layer_1_output &&
+                   layer.activation_output && layer.layer_2_output && layer.grad_output && layer.grad_layer_2_output &&
+                   layer.grad_activation_output && layer.grad_layer_1_output && layer.grad_scores && layer.grad_logits &&
+                   layer.workspace && (layer.input || !(layer.recompute_input || layer.grad_input)),
+               "fm_moe_layer_backward: null tensor");
+    // The gradient of layer 2's output and of the scores.
+    FM_STEP(fm_copy_sparse_to_dense_backward(layer.layer_2_output, layer.grad_output, step.routing(plan.scores),
+                                             step.routing(plan.sparse_rows), layer.grad_layer_2_output, layer.grad_scores,
+                                             layer.tokens, layer.hidden, plan.slots, plan.rows, step.dtype(), FM_DTYPE_F32,
+                                             FM_DTYPE_F32, plan.index_dtype, stream));
+    // What the forward did not keep.
+    if (layer.recompute_input) FM_STEP(step.dispatch(layer.sparse_input));
+    if (layer.recompute_layer_1)
+        FM_STEP(step.output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, step.ffn_1(), layer.hidden));
+    // Through layer 2 and the activation.
+    FM_STEP(step.output_sparse(layer.grad_layer_2_output, layer.weight_2, layer.grad_activation_output, layer.ffn, layer.hidden));
+    FM_STEP(fm_mlp_activation_backward(layer.grad_activation_output, layer.grad_layer_1_output, layer.layer_1_output,
+                                       layer.recompute_activation ? layer.activation_output : nullptr, plan.rows, layer.ffn,
+                                       static_cast<int>(layer.gated), static_cast<int>(layer.activation), step.dtype(),
+                                       step.rows_in_use(), plan.index_dtype, stream));
+    if (layer.grad_weight_2)
+        FM_STEP(step.row_sparse(layer.activation_output, layer.grad_layer_2_output, layer.grad_weight_2, layer.ffn,
+                                layer.accumulate_2 != 0));
+    // Through layer 1. The gradient of layer 2's output has been read for the last time: that of the sparse input takes
+    // its place.
+    if (layer.grad_input) FM_STEP(step.inner_sparse(layer.grad_layer_1_output, layer.weight_1, layer.grad_layer_2_output, step.ffn_1()));
+    if (layer.grad_weight_1)
+        FM_STEP(step.row_sparse(layer.grad_layer_1_output, layer.sparse_input, layer.grad_weight_1, step.ffn_1(),
+                                layer.accumulate_1 != 0));
+    if (layer.grad_input) FM_STEP(step.combine(layer.grad_layer_2_output, nullptr, layer.grad_input));
+    const bool losses = layer.with_losses != 0;
+    FM_STEP(fm_router_backward(layer.grad_scores, step.routing(plan.scores), step.routing(plan.top_experts), layer.logits, layer.noise,
+                               losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
+                               layer.grad_logits, layer.auxiliary_loss_grad, layer.z_loss_grad, layer.tokens,
+                               layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), stream));
+    return step.note;
+}
+
+}  // namespace
+
+}  // namespace fm
+
+using namespace fm;
+
+extern "C" int fm_moe_layer_sizes(fm_moe_layer *layer) {
+    Plan plan;
+    FM_REQUIRE(layer, "fm_moe_layer_sizes: null");
+    if (int status = make_plan(*layer, plan)) return status;
+    layer->rows = plan.rows;
+    layer->routing_bytes = static_cast<int64_t>(plan.routing_bytes);
+    layer->workspace_bytes = static_cast<int64_t>(plan.workspace_bytes);
+    layer->index_dtype = plan.index_dtype;
+    layer->used_rows_offset = static_cast<int64_t>(plan.expert_ends) + (plan.experts - 1) * plan.used_index_size;
+    return FM_OK;
+}
+
+extern "C" int fm_moe_layer_route(const fm_moe_layer *layer, void *stream) {
+    Plan plan;
+    FM_REQUIRE(layer, "fm_moe_layer_route: null");
+    if (int status = make_plan(*layer, plan)) return status;
+    return route(*layer, plan, stream);
+}
+
+extern "C" int fm_moe_layer_forward(const fm_moe_layer *layer, void *stream) {
+    Plan plan;
+    FM_REQUIRE(layer, "fm_moe_layer_forward: null");
+    if (int status = make_plan(*layer, plan)) return status;
+    return forward(*layer, plan, stream);
+}
+
+extern "C" int fm_moe_layer_backward(const fm_moe_layer *layer, void *stream) {
+    Plan plan;
+    FM_REQUIRE(layer, "fm_moe_layer_backward: null");
+    if (int status = make_plan(*layer, plan)) return status;
+    return backward(*layer, plan, stream);
+}

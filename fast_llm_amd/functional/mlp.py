@@ -383,6 +383,11 @@ def mlp_backward(grad_output: torch.Tensor, context: list[typing.Any]) -> tuple[
 mlp_autograd = wrap_forward_backward(mlp_forward, mlp_backward)
 
 
+def few_tokens_expected(rows: int, num_experts: int, dtype: torch.dtype) -> bool:
+    """Whether `few_tokens_forward` is the faster way for so many (token, slot) pairs."""
+    return rows <= FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts and dtype in (torch.bfloat16, torch.float16)
+
+
 def few_tokens_forward(
     input_: torch.Tensor,
     scores: torch.Tensor,
@@ -399,7 +404,7 @@ def few_tokens_forward(
     are not the faster way or do not take the operands.
     """
     tokens, slots = top_experts.shape
-    if tokens * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts or input_.dtype not in (torch.bfloat16, torch.float16):
+    if not few_tokens_expected(tokens * slots, num_experts, input_.dtype):
         return None
     hidden, dtype = input_.size(1), _lib.dtype_tag(input_.dtype)
     ffn = weight_2.size(0) // num_experts

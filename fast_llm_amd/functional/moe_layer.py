@@ -1,0 +1,248 @@
+"""
+The whole MoE layer, from the router's linear layer to the output, with two library calls for the forward and one for the
+backward (`fm_moe_layer_route` and `fm_moe_layer_forward`, `fm_moe_layer_backward`) instead of one per kernel: the same kernels in the same order as
+`router` -> `get_sparse_map` -> `mlp_autograd`, without the host time of some twenty Python launches.
+
+Covers `MixtureOfExpertMLP._forward` (fast_llm/layers/decoder/mlp/mixture_of_experts.py:126-213) for top-k routing of the
+hidden states themselves; `layers.moe.DroplessMoEMLP` composes the other cases from the parts.
+"""
+
+import dataclasses
+
+import torch
+
+from fast_llm_amd import _lib
+from fast_llm_amd.functional.config import ActivationType, KernelConfig, MLPRecomputeLevel
+from fast_llm_amd.functional.mlp import _activation_tag
+from fast_llm_amd.tensor import param_get_and_unset_is_zero
+
+
+@dataclasses.dataclass(frozen=True)
+class MoELayerOptions:
+    routed_experts: int
+    shared_experts: int
+    experts_per_token: int
+    gated: bool
+    activation_type: ActivationType
+    recompute_level: MLPRecomputeLevel
+    dynamic_shape: bool
+
+
+def moe_layer_supported(
+    hidden_states: torch.Tensor, router: torch.Tensor, weight_1: torch.Tensor, weight_2: torch.Tensor
+) -> bool:
+    """Whether `moe_layer` takes these operands. It steps aside for what the parts offer and it does not: kernel timers,
+    kernel choices other than the default ones, gradient buffers of different types or layouts."""
+    buffer_1, buffer_2, dtype = weight_1.grad_buffer, weight_2.grad_buffer, hidden_states.dtype
+    return (
+        _lib._active_timer is None
+        and KernelConfig.fuse_activation is None
+        and KernelConfig.grouped_gemm_workspace
+        and hidden_states.dim() == 2
+        and hidden_states.size(0) > 0
+        and dtype in _lib.DTYPES
+        and router.dtype == weight_1.dtype == weight_2.dtype == dtype
+        and buffer_1.dtype == buffer_2.dtype
+        and router.is_contiguous()
+        and weight_1.is_contiguous()
+        and weight_2.is_contiguous()
+        and buffer_1.is_contiguous()
+        and buffer_2.is_contiguous()
+    )
+
+
+def _describe(
+    options: MoELayerOptions,
+    hidden_states: torch.Tensor,
+    weight_1: torch.Tensor,
+    weight_2: torch.Tensor,
+    with_losses: bool,
+    dynamic_rows: int = 0,
+) -> _lib.MoELayer:
+    tokens, hidden = hidden_states.shape
+    layer = _lib.MoELayer(
+        tokens,
+        hidden,
+        weight_2.size(0) // (options.routed_experts + options.shared_experts),
+        options.routed_experts,
+        options.shared_experts,
+        options.experts_per_token,
+        options.gated,
+        _activation_tag(options.activation_type),
+        _lib.DTYPES[hidden_states.dtype],
+    )
+    layer.with_losses, layer.dynamic_rows = with_losses, dynamic_rows
+    layer.weight_1, layer.weight_2 = weight_1.data_ptr(), weight_2.data_ptr()
+    _lib.check(_lib.lib().fm_moe_layer_sizes(_lib.ctypes.byref(layer)))
+    return layer
+
+
+def _fuses_layer_1(options: MoELayerOptions, layer: _lib.MoELayer) -> bool:
+    """Whether layer 1's product has an instance with the gated activation in its epilogue."""
+    return options.gated and layer.dtype != 0 and layer.hidden % 64 == 0 and layer.ffn % 128 == 0
+
+
+@dataclasses.dataclass
+class _Saved:
+    """What the forward keeps for the backward. An intermediate that the recompute level does not keep is None."""
+
+    logits: torch.Tensor
+    noise: torch.Tensor | None
+    routing: torch.Tensor
+    sparse_input: torch.Tensor | None
+    layer_1_output: torch.Tensor | None
+    activation_output: torch.Tensor | None
+    layer_2_output: torch.Tensor
+    dynamic_rows: int
+
+
+def _forward(
+    options: MoELayerOptions,
+    hidden_states: torch.Tensor,
+    router: torch.Tensor,
+    weight_1: torch.Tensor,
+    weight_2: torch.Tensor,
+    noise: torch.Tensor | None,
+    with_losses: bool,
+    training: bool,
+) -> tuple[torch.Tensor, torch.Tensor | None, _Saved]:
+    """(output, losses [2] or None, what the backward needs)."""
+    device = _lib.require_device(hidden_states, router, weight_1, weight_2, noise)
+    logits = torch.nn.functional.linear(hidden_states, router)
+    layer = _describe(options, hidden_states, weight_1, weight_2, with_losses)
+    new = hidden_states.new_empty
+    routing = new(layer.routing_bytes, dtype=torch.uint8)
+    layer.logits, layer.noise, layer.routing = logits.data_ptr(), _lib.ptr(noise), routing.data_ptr()
+    if options.dynamic_shape:
+        workspace = new(layer.workspace_bytes, dtype=torch.uint8)
+        layer.workspace = workspace.data_ptr()
+        _lib.call("fm_moe_layer_route", device, _lib.ctypes.byref(layer))
+        index_dtype = torch.int16 if layer.index_dtype == 0 else torch.int32
+        used_rows = routing[layer.used_rows_offset : layer.used_rows_offset + index_dtype.itemsize].view(index_dtype)
+        layer.dynamic_rows = used_rows.item()
+        _lib.check(_lib.lib().fm_moe_layer_sizes(_lib.ctypes.byref(layer)))
+    level, rows, ffn = options.recompute_level, layer.rows, layer.ffn
+    keep_layer_1 = training and not level.recompute_layer_1
+    workspace = new(layer.workspace_bytes, dtype=torch.uint8)
+    sparse_input, layer_2_output = new((rows, layer.hidden)), new((rows, layer.hidden))
+    activation_output, output = new((rows, ffn)), new(hidden_states.shape)
+    layer_1_output = None
+    if keep_layer_1 or not _fuses_layer_1(options, layer):
+        layer_1_output = new((rows, ffn * 2 if options.gated else ffn))
+        layer.layer_1_output = layer_1_output.data_ptr()
+    layer.input, layer.output, layer.workspace = hidden_states.data_ptr(), output.data_ptr(), workspace.data_ptr()
+    layer.sparse_input, layer.activation_output = sparse_input.data_ptr(), activation_output.data_ptr()
+    layer.layer_2_output = layer_2_output.data_ptr()
+    if not options.dynamic_shape:
+        _lib.call("fm_moe_layer_route", device, _lib.ctypes.byref(layer))
+    try:
+        _lib.call("fm_moe_layer_forward", device, _lib.ctypes.byref(layer))
+    except NotImplementedError:  # a shape the fused product does not tile after all
+        if layer_1_output is not None:
+            raise
+        layer_1_output = new((rows, ffn * 2))
+        layer.layer_1_output = layer_1_output.data_ptr()
+        _lib.call("fm_moe_layer_forward", device, _lib.ctypes.byref(layer))
+    saved = _Saved(
+        logits,
+        noise,
+        routing,
+        None if level.recompute_sparse_input else sparse_input,
+        layer_1_output if keep_layer_1 else None,
+        None if level.recompute_activation else activation_output,
+        layer_2_output,
+        layer.dynamic_rows,
+    )
+    return output, routing[:8].view(torch.float32) if with_losses else None, saved
+
+
+class _MoELayer(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, hidden_states, router, weight_1, weight_2, noise, options, with_losses, loss_grads):
+        output, losses, ctx.saved = _forward(
+            options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=True
+        )
+        ctx.save_for_backward(hidden_states, router)
+        ctx.weights, ctx.options, ctx.with_losses, ctx.loss_grads = (weight_1, weight_2), options, with_losses, loss_grads
+        ctx.set_materialize_grads(False)
+        if losses is not None:
+            ctx.mark_non_differentiable(losses)
+        return output, losses
+
+    @staticmethod
+    def backward(ctx, grad_output, _):
+        if grad_output is None:
+            return (None,) * 8
+        hidden_states, router = ctx.saved_tensors
+        (weight_1, weight_2), options = ctx.weights, ctx.options
+        saved, ctx.saved = ctx.saved, None  # the intermediates go when this call ends, whoever holds the graph
+        if saved is None:
+            raise RuntimeError("the layer's intermediates have been freed: backward ran already")
+        grad_output = grad_output.contiguous()
+        device = _lib.require_device(hidden_states, grad_output)
+        layer = _describe(options, hidden_states, weight_1, weight_2, ctx.with_losses, saved.dynamic_rows)
+        layer.auxiliary_loss_grad, layer.z_loss_grad = ctx.loss_grads
+        rows, hidden, ffn = layer.rows, layer.hidden, layer.ffn
+        new = hidden_states.new_empty
+        workspace = new(layer.workspace_bytes, dtype=torch.uint8)
+        sparse_input, layer_1_output, activation_output = saved.sparse_input, saved.layer_1_output, saved.activation_output
+        if sparse_input is None:
+            sparse_input, layer.recompute_input = new((rows, hidden)), True
+        if layer_1_output is None:
+            layer_1_output, layer.recompute_layer_1 = new((rows, ffn * 2 if options.gated else ffn)), True
+        if activation_output is None:
+            activation_output, layer.recompute_activation = new((rows, ffn)), True
+        grad_layer_2_output, grad_activation_output = new((rows, hidden)), new((rows, ffn))
+        grad_layer_1_output = new(layer_1_output.shape)
+        grad_scores = new(layer.tokens * (options.experts_per_token + options.shared_experts), dtype=torch.float32)
+        grad_logits = new(saved.logits.shape)
+        layer.logits, layer.noise, layer.input = saved.logits.data_ptr(), _lib.ptr(saved.noise), hidden_states.data_ptr()
+        layer.routing, layer.workspace = saved.routing.data_ptr(), workspace.data_ptr()
+        layer.sparse_input, layer.layer_1_output = sparse_input.data_ptr(), layer_1_output.data_ptr()
+        layer.activation_output, layer.layer_2_output = activation_output.data_ptr(), saved.layer_2_output.data_ptr()
+        layer.grad_output, layer.grad_layer_2_output = grad_output.data_ptr(), grad_layer_2_output.data_ptr()
+        layer.grad_activation_output = grad_activation_output.data_ptr()
+        layer.grad_layer_1_output = grad_layer_1_output.data_ptr()
+        layer.grad_scores, layer.grad_logits = grad_scores.data_ptr(), grad_logits.data_ptr()
+        grad_input = None
+        if ctx.needs_input_grad[0]:
+            grad_input = new(hidden_states.shape)
+            layer.grad_input = grad_input.data_ptr()
+        layer.grad_dtype = _lib.dtype_tag(weight_1.grad_buffer.dtype)
+        if weight_1.requires_grad:
+            layer.grad_weight_1, layer.accumulate_1 = weight_1.grad_buffer.data_ptr(), not param_get_and_unset_is_zero(weight_1)
+        if weight_2.requires_grad:
+            layer.grad_weight_2, layer.accumulate_2 = weight_2.grad_buffer.data_ptr(), not param_get_and_unset_is_zero(weight_2)
+        _lib.call("fm_moe_layer_backward", device, _lib.ctypes.byref(layer))
+        # The router's linear layer.
+        if grad_input is not None:
+            grad_input.addmm_(grad_logits, router)
+        grad_router = torch.mm(grad_logits.t(), hidden_states) if ctx.needs_input_grad[1] else None
+        return grad_input, grad_router, None, None, None, None, None, None
+
+
+def moe_layer(
+    hidden_states: torch.Tensor,
+    router: torch.Tensor,
+    weight_1: torch.Tensor,
+    weight_2: torch.Tensor,
+    options: MoELayerOptions,
+    *,
+    training: bool,
+    noise: torch.Tensor | None = None,
+    with_losses: bool = False,
+    auxiliary_loss_grad: float = 0.0,
+    z_loss_grad: float = 0.0,
+) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """
+    `hidden_states` [tokens, hidden] -> (output, [load-balancing loss, z-loss] or None). Weight layouts as in
+    `layers.moe.DroplessMoEMLP`; the expert weights' gradients go to their grad buffers. The two loss gradients are those
+    of `functional.routing.router` and need `with_losses`. Without `training` nothing is kept for a backward.
+    """
+    hidden_states = hidden_states.contiguous()
+    if training:
+        return _MoELayer.apply(
+            hidden_states, router, weight_1, weight_2, noise, options, with_losses, (auxiliary_loss_grad, z_loss_grad)
+        )
+    with torch.no_grad():
+        return _forward(options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=False)[:2]

@@ -228,9 +228,15 @@ def router(
         raise ValueError("a loss that is not computed has no gradient")
     flat = logits.flatten(0, -2)
     flat_noise = None if noise is None else noise.flatten(0, -2)
-    scores, top_experts, losses, workspace = _Router.apply(
-        flat, flat_noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad, with_losses
-    )
+    if logits.requires_grad and torch.is_grad_enabled():
+        scores, top_experts, losses, workspace = _Router.apply(
+            flat, flat_noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad, with_losses
+        )
+    else:
+        scores, top_experts, losses, _, _, counts = router_forward(
+            flat.contiguous(), None if noise is None else flat_noise.contiguous(), experts_per_token, shared_experts, with_losses
+        )
+        workspace = counts.workspace
     shape = logits.shape[:-1] + (shared_experts + experts_per_token,)
     load_balancing_loss, z_loss = (losses[0], losses[1]) if with_losses else (None, None)
     result = (scores.view(shape), top_experts.view(shape), load_balancing_loss, z_loss)

@@ -11,7 +11,8 @@ Weight layout as in the reference: `layer_1.weight` [experts * 2 * ffn, hidden] 
 import torch
 
 from fast_llm_amd.functional.config import ActivationType, MLPRecomputeLevel
-from fast_llm_amd.functional.mlp import few_tokens_forward, mlp_autograd
+from fast_llm_amd.functional.mlp import few_tokens_expected, few_tokens_forward, mlp_autograd
+from fast_llm_amd.functional.moe_layer import MoELayerOptions, moe_layer, moe_layer_supported
 from fast_llm_amd.functional.sparse_copy import get_sparse_map
 
 
@@ -170,10 +171,15 @@ class DroplessMoEMLP(torch.nn.Module):
         """`scores`/`top_experts` may be passed to bypass the router (tests pin the routing that way)."""
         hidden_states = input_.flatten(0, -2)
         router_counts = None
+        few_tokens = not self.training and few_tokens_expected(
+            hidden_states.size(0) * (self.shared_experts + self.experts_per_token), self.experts, hidden_states.dtype
+        )
+        if top_experts is None and not few_tokens and self._is_one_call(hidden_states):
+            return self._forward_in_one_call(hidden_states, grad_scale, losses).view_as(input_)
         if top_experts is None:
             # The router has counted the tokens of every expert on its way: the map need not count them again.
             scores, top_experts, router_counts = self.route_with_counts(hidden_states, grad_scale, losses)
-        if not self.training and scores is not None:
+        if few_tokens and scores is not None:
             output = few_tokens_forward(
                 hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation
             )  # fmt: skip
@@ -199,6 +205,51 @@ class DroplessMoEMLP(torch.nn.Module):
             sparse_map=sparse_map,
         )
         return output.view_as(input_)
+
+    def _is_one_call(self, hidden_states: torch.Tensor) -> bool:
+        """Whether router and MLP have no step in between that `moe_layer` does not know."""
+        return (
+            self.routing == ROUTING_TOPK
+            and self.router_normalization is None
+            and self.router_scale is None
+            and self.router_input_scale == 1.0
+            and self.router_per_expert_scale is None
+            and moe_layer_supported(hidden_states, self.router, self.layer_1, self.layer_2)
+        )
+
+    def _forward_in_one_call(
+        self, hidden_states: torch.Tensor, grad_scale: float | None, losses: dict | None
+    ) -> torch.Tensor:
+        noise = None
+        if self.training and self.jitter_eps > 0.0:
+            noise = hidden_states.new_empty(hidden_states.size(0), self.unshared_experts)
+            noise.uniform_(1.0 - self.jitter_eps, 1.0 + self.jitter_eps)
+        trained = self.training and grad_scale is not None
+        output, loss_values = moe_layer(
+            hidden_states,
+            self.router,
+            self.layer_1,
+            self.layer_2,
+            MoELayerOptions(
+                self.unshared_experts,
+                self.shared_experts,
+                self.experts_per_token,
+                self.gated,
+                self.activation,
+                self.recompute_level,
+                self.dropless_dynamic_shape,
+            ),
+            training=self.training,
+            noise=noise,
+            with_losses=trained or losses is not None,
+            auxiliary_loss_grad=self.unshared_experts * self.auxiliary_loss_coefficient * grad_scale if trained else 0.0,
+            z_loss_grad=self.z_loss_coefficient * grad_scale if trained else 0.0,
+        )
+        if losses is not None:
+            losses.setdefault(LOAD_BALANCING_LOSS, []).append(loss_values[0])
+            if self.z_loss_coefficient > 0.0:
+                losses.setdefault(ROUTER_Z_LOSS, []).append(loss_values[1])
+        return output
 
     # ---- Hugging Face Mixtral layout ----------------------------------------------------------------------
     # The reference's Mixtral converter (fast_llm/models/gpt/conversion/mixtral.py:65-82) maps, per block,

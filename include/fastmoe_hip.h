@@ -356,6 +356,46 @@ int fm_few_tokens_forward(const void *input, const void *top_experts, const void
                           int64_t ffn, int64_t num_experts, int gated, int activation, int dtype, void *workspace,
                           size_t workspace_size, void *stream);
 
+/* The layer between the router's logits and its output in one call each way: the entry points above in the order of
+ * `MixtureOfExpertMLP._forward_dropless` (fast_llm/layers/decoder/mlp/mixture_of_experts.py:184-213) and `mlp_backward`
+ * (fast_llm/functional/triton/mlp.py:314-415), experts padded to 128 rows. fm_moe_layer_route runs the router and the sparse
+ * map, fm_moe_layer_forward the rest. Same kernels and results as the single calls, except that the gradient of the scores
+ * stays fp32 on its way to the router. All tensors are contiguous device memory of `dtype` unless said otherwise; nothing of
+ * a call is kept after it. */
+typedef struct {
+    /* Shape and options, set by the caller. */
+    int64_t tokens, hidden, ffn, routed_experts, shared_experts, experts_per_token;
+    int64_t gated, activation /* fm_activation */, dtype /* fm_dtype */, grad_dtype /* of the weight gradients */;
+    int64_t with_losses;   /* the router's losses are computed; must be the same in the backward */
+    int64_t recompute_input, recompute_layer_1, recompute_activation; /* backward: the forward did not keep it */
+    int64_t accumulate_1, accumulate_2;                               /* add to the weight gradients */
+    double auxiliary_loss_grad, z_loss_grad;                          /* as fm_router_backward */
+    int64_t dynamic_rows; /* sparse rows; 0: the static worst case. Known after fm_moe_layer_route: what it leaves in
+                           * `routing` at used_rows_offset (`index_dtype`) */
+    /* Set by fm_moe_layer_sizes: sparse rows, bytes of the two untyped buffers below, and where the map's last expert ends. */
+    int64_t rows, routing_bytes, workspace_bytes, index_dtype /* fm_index_dtype */, used_rows_offset;
+    /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned, kept for the
+     * backward) starts with the two losses (fp32) if there are losses; `workspace` is free again after the call.
+     * layer_1_output [rows, ffn * (2 if gated)] may be null where the backward recomputes it or does not follow: layer 1
+     * then runs with the gated activation in its epilogue, FM_ERR_UNSUPPORTED if it cannot. */
+    const void *logits, *noise, *input, *weight_1, *weight_2;
+    void *routing, *workspace;
+    void *sparse_input /* [rows, hidden] */, *layer_1_output, *activation_output /* [rows, ffn] */,
+        *layer_2_output /* [rows, hidden] */, *output /* [tokens, hidden] */;
+    /* Backward: the forward's tensors (recomputed ones as space to write), its output's gradient, space for the gradients of
+     * layer 2's output [rows, hidden] (overwritten with that of the sparse input), of the activation [rows, ffn] and of layer
+     * 1's output, and of the scores [tokens, shared_experts + experts_per_token] fp32; results. grad_weight_1, grad_weight_2
+     * and grad_input may be null: not computed. */
+    const void *grad_output;
+    void *grad_layer_2_output, *grad_activation_output, *grad_layer_1_output, *grad_scores;
+    void *grad_logits, *grad_input, *grad_weight_1, *grad_weight_2;
+} fm_moe_layer;
+
+int fm_moe_layer_sizes(fm_moe_layer *layer);
+int fm_moe_layer_route(const fm_moe_layer *layer, void *stream);
+int fm_moe_layer_forward(const fm_moe_layer *layer, void *stream);
+int fm_moe_layer_backward(const fm_moe_layer *layer, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

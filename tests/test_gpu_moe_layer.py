@@ -1,0 +1,89 @@
+"""The layer in two library calls (`functional.moe_layer`) against its composition from the single functions, which a
+kernel timer selects and the oracle tests pin."""
+
+import pytest
+import torch
+
+from fast_llm_amd import _lib
+from fast_llm_amd.functional.config import ActivationType, MLPRecomputeLevel
+from fast_llm_amd.layers.moe import DroplessMoEMLP
+from tests.helpers import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(layer, batches, composed):
+    layer.router.grad = None
+    layer.layer_1.param_grad_is_zero = layer.layer_2.param_grad_is_zero = True
+    outputs, input_grads, losses = [], [], {}
+    for x in batches:
+        x.grad = None
+        if composed:
+            with _lib.KernelTimer():
+                output = layer(x, grad_scale=0.5, losses=losses)
+        else:
+            output = layer(x, grad_scale=0.5, losses=losses)
+        output.backward(torch.ones_like(output) / output.numel() ** 0.5)
+        outputs.append(output.detach())
+        input_grads.append(x.grad)
+    return {
+        "outputs": outputs,
+        "losses": [value for values in losses.values() for value in values],
+        "weight_grads": [layer.layer_1.grad_buffer.clone(), layer.layer_2.grad_buffer.clone()],
+        "input_grads": input_grads,
+        "router_grad": [layer.router.grad],
+    }
+
+
+@pytest.mark.parametrize("recompute_level", list(MLPRecomputeLevel))
+@pytest.mark.parametrize(
+    ("hidden", "ffn", "options"),
+    [
+        (128, 256, dict(dtype=torch.bfloat16)),
+        # No instance with the activation in the product's epilogue; one shared expert; both losses trained; jitter.
+        (72, 40, dict(dtype=torch.float16, shared_experts=1, z_loss_coefficient=0.1, activation=ActivationType.gelu)),
+        (64, 192, dict(dtype=torch.bfloat16, gated=False, full_precision_gradients=True, dropless_dynamic_shape=True)),
+        (64, 128, dict(dtype=torch.float32, dropless_dynamic_shape=True)),
+    ],
+)
+def test_layer_in_two_calls_matches_the_composition(recompute_level, hidden, ffn, options, device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(hidden, ffn, 7, 2, recompute_level=recompute_level, init_std=0.2, device=device, **options)
+    batches = [torch.randn(tokens, hidden, device=device, dtype=options["dtype"], requires_grad=True) for tokens in (300, 77)]
+    one, composed = _step(layer, batches, False), _step(layer, batches, True)
+    for name in ("outputs", "losses", "weight_grads"):
+        assert all(torch.equal(a, b) for a, b in zip(one[name], composed[name], strict=True)), name
+    # The gradient of the scores is not rounded on its way to the router and the router's input gradient is added before
+    # the rounding: half a unit in the last place each.
+    bound = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}[options["dtype"]]
+    for name in ("input_grads", "router_grad"):
+        assert all(max_rel_err(a, b) <= bound for a, b in zip(one[name], composed[name], strict=True)), name
+    layer.eval()
+    with torch.no_grad():
+        x = torch.cat(batches)
+        output = layer(x)
+        with _lib.KernelTimer():
+            assert torch.equal(output, layer(x))
+
+
+def test_layer_in_two_calls_with_jitter_frozen_weights_and_no_input_gradient(device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 4, 2, jitter_eps=0.1, device=device)
+    x = torch.randn(100, 64, device=device, dtype=torch.bfloat16)
+    results = []
+    for composed in (False, True):
+        torch.manual_seed(1)
+        results.append(_step(layer, [x], composed))
+    assert torch.equal(results[0]["outputs"][0], results[1]["outputs"][0])
+    assert results[0]["input_grads"] == [None]
+    assert max_rel_err(results[0]["router_grad"][0], results[1]["router_grad"][0]) <= 1e-2
+    before = layer.layer_1.grad_buffer.clone()
+    layer.layer_1.requires_grad_(False)
+    layer.layer_1.grad_buffer.fill_(3)
+    result = _step(layer, [x.requires_grad_()], False)
+    assert (layer.layer_1.grad_buffer == 3).all() and before.abs().max() > 0
+    assert result["input_grads"][0].abs().max() > 0
+    output = layer(x)
+    output.sum().backward(retain_graph=True)
+    with pytest.raises(RuntimeError, match="backward ran already"):
+        output.sum().backward()
