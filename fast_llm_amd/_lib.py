@@ -31,16 +31,17 @@ class MoELayer(ctypes.Structure):
             )
         ]
         + [(name, ctypes.c_double) for name in ("auxiliary_loss_grad", "z_loss_grad")]
-        + [(name, _c_i64) for name in ("dynamic_rows", "rows", "routing_bytes", "workspace_bytes", "index_dtype", "used_rows_offset")]
+        + [(name, _c_i64) for name in ("dynamic_rows", "rows", "routing_bytes", "workspace_bytes", "index_dtype", "used_rows_offset", "router_linear")]
         + [
             (name, _c_ptr)
             for name in (
                 "logits", "noise", "input", "weight_1", "weight_2", "routing", "workspace", "sparse_input", "layer_1_output",
                 "activation_output", "layer_2_output", "output", "grad_output", "grad_layer_2_output",
                 "grad_activation_output", "grad_layer_1_output", "grad_scores", "grad_logits", "grad_input", "grad_weight_1",
-                "grad_weight_2",
+                "grad_weight_2", "router", "grad_router",
             )
         ]
+        + [("router_input_grad", _c_i64)]
     )  # fmt: skip
 
 
@@ -79,6 +80,8 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_ptr] * 6 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr],
     ),
+    "fm_router_linear_backward_workspace_size": (_c_size, [_c_i64] * 3 + [_c_int]),
+    "fm_router_linear_backward": (_c_int, [_c_ptr] * 5 + [_c_i64] * 3 + [_c_int, _c_ptr, _c_size, _c_ptr]),
     "fm_moe_layer_sizes": (_c_int, [_c_ptr]),
     "fm_moe_layer_route": (_c_int, [_c_ptr, _c_ptr]),
     "fm_moe_layer_forward": (_c_int, [_c_ptr, _c_ptr]),

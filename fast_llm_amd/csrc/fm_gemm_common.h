@@ -42,6 +42,8 @@ struct GemmArgs {
     int64_t half;          // columns of the activation output per expert
     int num_ids;           // workgroup ids that may have a tile (set by the MFMA kernel's launcher)
     void *tile_table;      // one record per id, written by the plan kernel into the caller's workspace, or null
+    int64_t piece_length;  // row-sparse mode without a map: group e reduces over [e, e + 1) * piece_length instead of
+                           // everything (0: everything)
     int chunk_tiles;       // consecutive tiles that go to one XCD (set by the fp32 kernel's launcher)
 };
 

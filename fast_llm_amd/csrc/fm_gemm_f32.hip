@@ -143,6 +143,9 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
             k_hi = load_index(args.expert_pad_begins, args.index_dtype, expert);
             k_lo = max(k_lo, static_cast<int64_t>(0));
             k_hi = min(k_hi, args.inner);
+        } else if (args.piece_length > 0) {
+            k_lo = expert * args.piece_length;
+            k_hi = min(k_lo + args.piece_length, args.inner);
         }
         lhs_offset = row * args.lhs_stride_row + k_lo * args.lhs_stride_inner;
         rhs_offset = col0 * args.rhs_stride_col + k_lo * args.rhs_stride_inner;

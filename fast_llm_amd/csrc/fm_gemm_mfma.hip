@@ -260,9 +260,9 @@ __device__ __forceinline__ u32x4_t load_fragment(FM_LDS(char) * lds, const int (
     // `lds + offset`, every fragment address costs an addition of zero in the main loop.
     (void)lds;
     if constexpr (kContiguousK) {
-        return *(FM_LDS(u32x4_t) *)static_cast<uint32_t>(bases[kstep] + (slot * kOperandBytes + i * 32 * kBK * 2));
+        return *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(bases[kstep] + (slot * kOperandBytes + i * 32 * kBK * 2));
     } else {
-        FM_LDS(char) *address = (FM_LDS(char) *)static_cast<uint32_t>(bases[i] + (slot * kOperandBytes + kstep * 16 * kTile * 2));
+        FM_LDS(char) *address = (FM_LDS(char) *)static_cast<uintptr_t>(bases[i] + (slot * kOperandBytes + kstep * 16 * kTile * 2));
         const i16x4_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<FM_LDS(i16x4_t) *>(address));
         const i16x4_t high =
             __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<FM_LDS(i16x4_t) *>(address + 4 * kTile * 2));
@@ -328,6 +328,9 @@ __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, 
             work.k_hi = load_index(args.expert_pad_begins, args.index_dtype, expert);
             work.k_lo = max(work.k_lo, static_cast<int64_t>(0));
             work.k_hi = min(work.k_hi, args.inner);
+        } else if (args.piece_length > 0) {
+            work.k_lo = expert * args.piece_length;
+            work.k_hi = min(work.k_lo + args.piece_length, args.inner);
         }
         work.lhs_offset = row_in_expert * args.lhs_stride_row;
         work.rhs_offset = col0 * args.rhs_stride_col;

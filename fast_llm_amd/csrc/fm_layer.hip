@@ -14,7 +14,7 @@ struct Plan {
     int64_t experts, slots, rows, used_index_size;
     int index_dtype;
     size_t losses, top_experts, scores, lse, statistics, sparse_rows, expert_ends, expert_pad_begins, router, routing_bytes;
-    size_t workspace_bytes;
+    size_t workspace_bytes, router_linear_bytes;
 };
 
 constexpr int64_t kPad = 128;
@@ -52,8 +52,9 @@ int make_plan(const fm_moe_layer &layer, Plan &plan) {
     plan.routing_bytes = at;
     const int64_t ffn_1 = layer.ffn * (layer.gated ? 2 : 1);
     const int dtype = static_cast<int>(layer.dtype);
+    plan.router_linear_bytes = fm_router_linear_backward_workspace_size(layer.tokens, layer.routed_experts, layer.hidden, dtype);
     plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
-    for (size_t bytes : {fm_grouped_gemm_workspace_size(plan.rows, ffn_1, layer.hidden, plan.experts, dtype),
+    for (size_t bytes : {plan.router_linear_bytes, fm_grouped_gemm_workspace_size(plan.rows, ffn_1, layer.hidden, plan.experts, dtype),
                          fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, layer.ffn, plan.experts, dtype),
                          fm_grouped_gemm_workspace_size(plan.rows, layer.ffn, layer.hidden, plan.experts, dtype),
                          fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, ffn_1, plan.experts, dtype),
@@ -159,7 +160,7 @@ int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     FM_REQUIRE(layer.logits && layer.weight_1 && layer.weight_2 && layer.routing && layer.sparse_input && layer.layer_1_output &&
                    layer.activation_output && layer.layer_2_output && layer.grad_output && layer.grad_layer_2_output &&
                    layer.grad_activation_output && layer.grad_layer_1_output && layer.grad_scores && layer.grad_logits &&
-                   layer.workspace && (layer.input || !(layer.recompute_input || layer.grad_input)),
+                   layer.workspace && (layer.input || !(layer.recompute_input || layer.router)),
                "fm_moe_layer_backward: null tensor");
     // The gradient of layer 2's output and of the scores.
     FM_STEP(fm_copy_sparse_to_dense_backward(layer.layer_2_output, layer.grad_output, step.routing(plan.scores),
@@ -191,6 +192,10 @@ int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
                                losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
                                layer.grad_logits, layer.auxiliary_loss_grad, layer.z_loss_grad, layer.tokens,
                                layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), stream));
+    if (layer.router != nullptr)
+        FM_STEP(step.keep(fm_router_linear_backward(layer.grad_logits, layer.input, layer.router, layer.router_input_grad ? layer.grad_input : nullptr, layer.grad_router,
+                                                    layer.tokens, layer.routed_experts, layer.hidden, step.dtype(), layer.workspace,
+                                                    plan.workspace_bytes, stream)));
     return step.note;
 }
 
@@ -208,6 +213,7 @@ extern "C" int fm_moe_layer_sizes(fm_moe_layer *layer) {
     layer->routing_bytes = static_cast<int64_t>(plan.routing_bytes);
     layer->workspace_bytes = static_cast<int64_t>(plan.workspace_bytes);
     layer->index_dtype = plan.index_dtype;
+    layer->router_linear = plan.router_linear_bytes > 0;
     layer->used_rows_offset = static_cast<int64_t>(plan.expert_ends) + (plan.experts - 1) * plan.used_index_size;
     return FM_OK;
 }

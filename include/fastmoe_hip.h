@@ -356,6 +356,15 @@ int fm_few_tokens_forward(const void *input, const void *top_experts, const void
                           int64_t ffn, int64_t num_experts, int gated, int activation, int dtype, void *workspace,
                           size_t workspace_size, void *stream);
 
+/* Backward of the router's linear layer, logits = input [num_tokens, hidden] x weight [num_experts, hidden]^T:
+ * grad_weight = grad_logits^T x input (may be null: not computed) and grad_input += grad_logits x weight (may be null). All
+ * contiguous and 16-byte aligned, of `dtype`. The workspace size is 0 for what the kernels do not take (experts or hidden not a
+ * multiple of 16 bytes), which FM_ERR_UNSUPPORTED then reports. Deterministic. */
+size_t fm_router_linear_backward_workspace_size(int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype);
+int fm_router_linear_backward(const void *grad_logits, const void *input, const void *weight, void *grad_input,
+                              void *grad_weight, int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype,
+                              void *workspace, size_t workspace_size, void *stream);
+
 /* The layer between the router's logits and its output in one call each way: the entry points above in the order of
  * `MixtureOfExpertMLP._forward_dropless` (fast_llm/layers/decoder/mlp/mixture_of_experts.py:184-213) and `mlp_backward`
  * (fast_llm/functional/triton/mlp.py:314-415), experts padded to 128 rows. fm_moe_layer_route runs the router and the sparse
@@ -374,6 +383,7 @@ typedef struct {
                            * `routing` at used_rows_offset (`index_dtype`) */
     /* Set by fm_moe_layer_sizes: sparse rows, bytes of the two untyped buffers below, and where the map's last expert ends. */
     int64_t rows, routing_bytes, workspace_bytes, index_dtype /* fm_index_dtype */, used_rows_offset;
+    int64_t router_linear; /* whether fm_router_linear_backward takes the shape */
     /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned, kept for the
      * backward) starts with the two losses (fp32) if there are losses; `workspace` is free again after the call.
      * layer_1_output [rows, ffn * (2 if gated)] may be null where the backward recomputes it or does not follow: layer 1
@@ -389,6 +399,11 @@ typedef struct {
     const void *grad_output;
     void *grad_layer_2_output, *grad_activation_output, *grad_layer_1_output, *grad_scores;
     void *grad_logits, *grad_input, *grad_weight_1, *grad_weight_2;
+    /* Where router_linear is not 0, if `router` is not null: the backward of the router's linear layer as well
+     * (fm_router_linear_backward), into grad_router (may be null) and, with router_input_grad, added into grad_input. */
+    const void *router;
+    void *grad_router;
+    int64_t router_input_grad;
 } fm_moe_layer;
 
 int fm_moe_layer_sizes(fm_moe_layer *layer);
