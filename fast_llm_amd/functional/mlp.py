@@ -414,6 +414,8 @@ def few_tokens_forward(
         return None
     if top_experts.dtype != torch.int64 or not all(tensor.is_contiguous() for tensor in tensors):
         return None
+    if any(tensor.data_ptr() % 16 != 0 for tensor in (input_, weight_1, weight_2)):
+        return None
     device = _lib.require_device(*tensors)
     Assert.eq(tuple(weight_1.shape), (num_experts * ffn * (2 if gated else 1), hidden))
     Assert.eq(input_.size(0), tokens)

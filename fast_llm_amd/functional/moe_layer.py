@@ -1,7 +1,8 @@
 """
-The whole MoE layer, from the router's linear layer to the output, with two library calls for the forward and one for the
-backward (`fm_moe_layer_route` and `fm_moe_layer_forward`, `fm_moe_layer_backward`) instead of one per kernel: the same kernels in the same order as
-`router` -> `get_sparse_map` -> `mlp_autograd`, without the host time of some twenty Python launches.
+The whole MoE layer, from the router's linear layer to the output, with two library calls for the forward
+(`fm_moe_layer_route`, `fm_moe_layer_forward`) and one for the backward (`fm_moe_layer_backward`) instead of one per
+kernel: the same kernels in the same order as `router` -> `get_sparse_map` -> `mlp_autograd`, without the host time of
+some twenty Python launches.
 
 Covers `MixtureOfExpertMLP._forward` (fast_llm/layers/decoder/mlp/mixture_of_experts.py:126-213) for top-k routing of the
 hidden states themselves; `layers.moe.DroplessMoEMLP` composes the other cases from the parts.
@@ -14,7 +15,8 @@ import torch
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.config import ActivationType, KernelConfig, MLPRecomputeLevel
 from fast_llm_amd.functional.mlp import _activation_tag
-from fast_llm_amd.tensor import param_get_and_unset_is_zero
+from fast_llm_amd.functional.utils import ANCHOR, Assert, without_backward
+from fast_llm_amd.tensor import accumulate_gradient, param_get_and_unset_is_zero
 
 
 @dataclasses.dataclass(frozen=True)
@@ -29,25 +31,32 @@ class MoELayerOptions:
 
 
 def moe_layer_supported(
-    hidden_states: torch.Tensor, router: torch.Tensor, weight_1: torch.Tensor, weight_2: torch.Tensor
+    hidden_states: torch.Tensor,
+    router: torch.Tensor,
+    weight_1: torch.Tensor,
+    weight_2: torch.Tensor,
+    options: MoELayerOptions,
 ) -> bool:
-    """Whether `moe_layer` takes these operands. It steps aside for what the parts offer and it does not: kernel timers,
-    kernel choices other than the default ones, gradient buffers of different types or layouts."""
-    buffer_1, buffer_2, dtype = weight_1.grad_buffer, weight_2.grad_buffer, hidden_states.dtype
+    """Whether `moe_layer` takes these operands. It steps aside for what the parts offer and it does not (kernel timers,
+    kernel choices other than the default ones, logits that autocast makes another type of) and for operands that do not
+    fit together, which the parts refuse."""
+    dtype, (experts, hidden) = hidden_states.dtype, (options.routed_experts + options.shared_experts, hidden_states.size(-1))
+    ffn = weight_2.size(0) // experts
     return (
         _lib._active_timer is None
         and KernelConfig.fuse_activation is None
         and KernelConfig.grouped_gemm_workspace
+        and not torch.is_autocast_enabled("cuda")
         and hidden_states.dim() == 2
         and hidden_states.size(0) > 0
         and dtype in _lib.DTYPES
         and router.dtype == weight_1.dtype == weight_2.dtype == dtype
-        and buffer_1.dtype == buffer_2.dtype
+        and router.shape == (options.routed_experts, hidden)
+        and weight_1.shape == (experts * ffn * (2 if options.gated else 1), hidden)
+        and weight_2.shape == (experts * ffn, hidden)
         and router.is_contiguous()
         and weight_1.is_contiguous()
         and weight_2.is_contiguous()
-        and buffer_1.is_contiguous()
-        and buffer_2.is_contiguous()
     )
 
 
@@ -156,9 +165,22 @@ def _forward(
     return output, routing[:8].view(torch.float32) if with_losses else None, saved
 
 
+def _gradient_targets(weights: list[torch.Tensor]) -> list[torch.Tensor]:
+    """What the library writes the gradients of `weights` to: their buffers, or where it does not take those (two types,
+    strides), tensors in single precision that are added to them afterwards."""
+    buffers = [weight.grad_buffer for weight in weights]
+    for weight, buffer in zip(weights, buffers):
+        Assert.eq(buffer.shape, weight.shape)
+    one_type = len({_lib.dtype_tag(buffer.dtype) for buffer in buffers}) <= 1
+    direct = one_type and all(buffer.is_contiguous() for buffer in buffers)
+    return buffers if direct else [torch.empty(weight.shape, dtype=torch.float32, device=weight.device) for weight in weights]
+
+
 class _MoELayer(torch.autograd.Function):
+    # The last argument of `apply` is an empty tensor that requires a gradient: the weight gradients are side effects, the
+    # node is to be visited whatever else needs one.
     @staticmethod
-    def forward(ctx, hidden_states, router, weight_1, weight_2, noise, options, with_losses, loss_grads):
+    def forward(ctx, hidden_states, router, weight_1, weight_2, noise, options, with_losses, loss_grads, _):
         output, losses, ctx.saved = _forward(
             options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=True
         )
@@ -172,7 +194,7 @@ class _MoELayer(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, _):
         if grad_output is None:
-            return (None,) * 8
+            return (None,) * 9
         hidden_states, router = ctx.saved_tensors
         (weight_1, weight_2), options = ctx.weights, ctx.options
         saved, ctx.saved = ctx.saved, None  # the intermediates go when this call ends, whoever holds the graph
@@ -208,26 +230,35 @@ class _MoELayer(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             grad_input = new(hidden_states.shape)
             layer.grad_input = grad_input.data_ptr()
-        layer.grad_dtype = _lib.dtype_tag(weight_1.grad_buffer.dtype)
-        if weight_1.requires_grad:
-            layer.grad_weight_1, layer.accumulate_1 = weight_1.grad_buffer.data_ptr(), not param_get_and_unset_is_zero(weight_1)
-        if weight_2.requires_grad:
-            layer.grad_weight_2, layer.accumulate_2 = weight_2.grad_buffer.data_ptr(), not param_get_and_unset_is_zero(weight_2)
+        trained = [weight for weight in (weight_1, weight_2) if weight.requires_grad]
+        targets = _gradient_targets(trained)
+        for weight, target in zip(trained, targets):
+            layer.grad_dtype = _lib.DTYPES[target.dtype]
+            accumulate = target is weight.grad_buffer and not param_get_and_unset_is_zero(weight)
+            if weight is weight_1:
+                layer.grad_weight_1, layer.accumulate_1 = target.data_ptr(), accumulate
+            else:
+                layer.grad_weight_2, layer.accumulate_2 = target.data_ptr(), accumulate
         # The router's linear layer: with the rest, or in torch for sizes the library does not take. Half-precision input
         # gradients are torch's too: a reduction of 8 to 128 experts is one or two slices of the library's 256 x 256 tiles
         # (16384 tokens of 2048, 128 experts: 39 us against 33; 512 of 256, 8 experts: 17 against 5).
         grad_router = None
+        if hidden_states.data_ptr() % 16 != 0 or router.data_ptr() % 16 != 0:
+            layer.router_linear = False
         if layer.router_linear:
             layer.router, layer.router_input_grad = router.data_ptr(), layer.dtype == 0
             if ctx.needs_input_grad[1]:
                 grad_router = torch.empty_like(router)
                 layer.grad_router = grad_router.data_ptr()
         _lib.call("fm_moe_layer_backward", device, _lib.ctypes.byref(layer))
+        for weight, target in zip(trained, targets):
+            if target is not weight.grad_buffer:
+                accumulate_gradient(weight, target)
         if not layer.router_linear and ctx.needs_input_grad[1]:
             grad_router = torch.mm(grad_logits.t(), hidden_states)
         if not layer.router_input_grad and grad_input is not None:
             grad_input.addmm_(grad_logits, router)
-        return grad_input, grad_router, None, None, None, None, None, None
+        return (grad_input, grad_router) + (None,) * 7
 
 
 def moe_layer(
@@ -251,7 +282,8 @@ def moe_layer(
     hidden_states = hidden_states.contiguous()
     if training:
         return _MoELayer.apply(
-            hidden_states, router, weight_1, weight_2, noise, options, with_losses, (auxiliary_loss_grad, z_loss_grad)
+            hidden_states, router, weight_1, weight_2, noise, options, with_losses, (auxiliary_loss_grad, z_loss_grad), ANCHOR
         )
     with torch.no_grad():
-        return _forward(options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=False)[:2]
+        output, losses, _ = _forward(options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=False)
+    return without_backward(output), losses

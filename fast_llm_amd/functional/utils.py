@@ -27,6 +27,25 @@ def div(x: int, y: int) -> int:
     return x // y
 
 
+# An argument that makes autograd visit a node whatever else needs a gradient.
+ANCHOR = torch.empty(0, requires_grad=True)
+
+
+class _WithoutBackward(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, output: torch.Tensor, _: torch.Tensor) -> torch.Tensor:
+        return output.view_as(output)
+
+    @staticmethod
+    def backward(ctx, grad_output: torch.Tensor):
+        raise RuntimeError("the layer ran in inference mode (`training=False`): it kept nothing for a backward")
+
+
+def without_backward(output: torch.Tensor) -> torch.Tensor:
+    """`output`, computed outside autograd: a backward that reaches it raises instead of losing its gradient silently."""
+    return _WithoutBackward.apply(output, ANCHOR) if torch.is_grad_enabled() else output
+
+
 class _ForwardBackwardPair(torch.autograd.Function):
     """One autograd node for every wrapped pair: the pair itself travels as the first argument. The last argument is
     an empty tensor that requires a gradient, so that autograd visits the node even when none of the caller's tensors
@@ -64,11 +83,10 @@ def wrap_forward_backward(
     Keyword arguments are passed on positionally, in the order the caller wrote them (the reference's convention,
     fast_llm/functional/utils.py:52-54: the caller's keyword order must match `forward`'s positional order).
     """
-    anchor = torch.empty(0, requires_grad=True)
     pair = (forward, backward)
 
     def differentiable(*args, **kwargs):
-        return _ForwardBackwardPair.apply(pair, *args, *kwargs.values(), anchor)
+        return _ForwardBackwardPair.apply(pair, *args, *kwargs.values(), ANCHOR)
 
     return differentiable
 

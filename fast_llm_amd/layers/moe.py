@@ -25,7 +25,7 @@ def attach_grad_buffer(weight: torch.Tensor, dtype: torch.dtype | None = None) -
 
 
 from fast_llm_amd.functional.routing import router, sinkhorn_routing, topk_routing  # noqa: E402, F401  (re-exported)
-from fast_llm_amd.functional.utils import AuxiliaryLoss  # noqa: E402
+from fast_llm_amd.functional.utils import AuxiliaryLoss, without_backward  # noqa: E402
 
 LOAD_BALANCING_LOSS, ROUTER_Z_LOSS = "load_balancing_loss", "router_z_loss"  # layers/decoder/mlp/config.py:24-26
 ROUTING_TOPK, ROUTING_SINKHORN = "aux_loss", "sinkhorn"  # `RoutingType`, layers/decoder/mlp/config.py:29-31
@@ -184,7 +184,7 @@ class DroplessMoEMLP(torch.nn.Module):
                 hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation
             )  # fmt: skip
             if output is not None:
-                return output.view_as(input_)
+                return without_backward(output).view_as(input_)
         sparse_map = get_sparse_map(
             top_experts, self.experts, dynamic_shape=self.dropless_dynamic_shape, router_counts=router_counts
         )
@@ -214,7 +214,18 @@ class DroplessMoEMLP(torch.nn.Module):
             and self.router_scale is None
             and self.router_input_scale == 1.0
             and self.router_per_expert_scale is None
-            and moe_layer_supported(hidden_states, self.router, self.layer_1, self.layer_2)
+            and moe_layer_supported(hidden_states, self.router, self.layer_1, self.layer_2, self._one_call_options())
+        )
+
+    def _one_call_options(self) -> MoELayerOptions:
+        return MoELayerOptions(
+            self.unshared_experts,
+            self.shared_experts,
+            self.experts_per_token,
+            self.gated,
+            self.activation,
+            self.recompute_level,
+            self.dropless_dynamic_shape,
         )
 
     def _forward_in_one_call(
@@ -230,15 +241,7 @@ class DroplessMoEMLP(torch.nn.Module):
             self.router,
             self.layer_1,
             self.layer_2,
-            MoELayerOptions(
-                self.unshared_experts,
-                self.shared_experts,
-                self.experts_per_token,
-                self.gated,
-                self.activation,
-                self.recompute_level,
-                self.dropless_dynamic_shape,
-            ),
+            self._one_call_options(),
             training=self.training,
             noise=noise,
             with_losses=trained or losses is not None,

@@ -87,3 +87,63 @@ def test_layer_in_two_calls_with_jitter_frozen_weights_and_no_input_gradient(dev
     output.sum().backward(retain_graph=True)
     with pytest.raises(RuntimeError, match="backward ran already"):
         output.sum().backward()
+
+
+def test_layer_in_two_calls_refuses_and_accepts_what_the_composition_does(device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device, dtype=torch.float32)
+    x = torch.randn(100, 64, device=device)
+    # Autocast makes the logits half as wide as the library's call takes them.
+    with torch.autocast("cuda", torch.bfloat16):
+        output = layer(x)
+        with _lib.KernelTimer():
+            assert torch.equal(output, layer(x))
+    # Nothing that autograd knows needs a gradient, but the backward runs; buffers of two types, one with strides.
+    for parameter in (layer.router, layer.layer_1, layer.layer_2):
+        parameter.requires_grad_(False)
+    layer(x).backward(x)
+    layer.layer_1.requires_grad_(True), layer.layer_2.requires_grad_(True)
+    results = []
+    for direct in (True, False):
+        if not direct:
+            layer.layer_1.grad_buffer = torch.empty_like(layer.layer_1, dtype=torch.bfloat16)
+            layer.layer_2.grad_buffer = layer.layer_2.detach().t().contiguous().t()
+        layer.layer_1.param_grad_is_zero = layer.layer_2.param_grad_is_zero = True
+        for _ in range(2):
+            layer(x).backward(x)
+        results.append([layer.layer_1.grad_buffer, layer.layer_2.grad_buffer])
+    assert all(max_rel_err(a, b) <= 1e-2 for a, b in zip(*results))
+    layer.layer_1.grad_buffer = layer.layer_1.detach().double()
+    with pytest.raises(ValueError, match="dtype"):
+        layer(x).backward(x)
+    # A weight that does not fit is refused.
+    whole, layer.layer_1 = layer.layer_1, torch.nn.Parameter(layer.layer_1.detach()[:-8].clone())
+    with pytest.raises((AssertionError, ValueError)):
+        layer(x)
+    layer.layer_1 = whole
+
+
+@pytest.mark.parametrize("tokens", [8, 512])  # the kernels for few tokens; the layer in two calls
+def test_inference_without_gradient_buffers_at_odd_addresses_and_with_a_backward(tokens, device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device).eval()
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
+    del layer.layer_1.grad_buffer, layer.layer_2.grad_buffer
+    with torch.no_grad():
+        expected = layer(x)
+        odd = torch.empty(tokens * 64 + 1, device=device, dtype=torch.bfloat16)[1:].view(tokens, 64).copy_(x)
+        assert max_rel_err(layer(odd), expected) <= 1e-2
+    output = layer(x)
+    assert torch.equal(output, expected)
+    with pytest.raises(RuntimeError, match="kept nothing"):
+        output.sum().backward()
+
+
+def test_training_step_with_an_input_at_an_odd_address(device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device)
+    x = torch.randn(300, 64, device=device, dtype=torch.bfloat16)
+    odd = torch.empty(300 * 64 + 1, device=device, dtype=torch.bfloat16)[1:].view(300, 64).copy_(x)
+    results = [_step(layer, [value.requires_grad_()], False) for value in (x, odd)]
+    for name in ("outputs", "input_grads", "router_grad", "weight_grads"):
+        assert all(max_rel_err(a, b) <= 1e-2 for a, b in zip(results[0][name], results[1][name])), name
