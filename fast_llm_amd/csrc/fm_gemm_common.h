@@ -1,6 +1,8 @@
 // Arguments and small device helpers shared by the grouped-GEMM kernels.
 #pragma once
 
+#include <atomic>
+
 #include "fm_common.h"
 
 namespace fm {
@@ -183,6 +185,13 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype);  // with args.f
 // `workspace` (may be null: no split) must hold mfma_gemm_workspace_size(args) bytes when that is not 0.
 size_t mfma_gemm_workspace_size(GemmArgs args);
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream);
+
+// Allows `kernel` that many bytes of dynamic LDS. `configured`: the kernel's own bit mask of devices done.
+int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured);
+
+// Row-sparse products of experts of few rows (fm_gemm_row_sparse.hip), of those that `mfma_gemm_eligible` accepts.
+bool row_sparse_gemm_chosen(const GemmArgs &args, int dtype);
+int row_sparse_gemm_launch(GemmArgs args, int dtype, hipStream_t stream);
 
 // fp32 operands with a unit stride and 16-byte aligned lines (fm_gemm_f32.hip).
 bool f32_gemm_eligible(const GemmArgs &args, int dtype);

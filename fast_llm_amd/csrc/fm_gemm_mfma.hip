@@ -38,8 +38,6 @@
 #include "fm_activation_math.h"
 #include "fm_gemm_common.h"
 
-#include <atomic>
-
 namespace fm {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
@@ -1307,7 +1305,7 @@ __global__ __launch_bounds__(64) void grouped_gemm_reduce_kernel(GemmArgs args) 
 // ---- host side -----------------------------------------------------------------------------------------
 // Kernels that use more dynamic LDS than the default limit need the attribute set once per device; `configured` is the
 // kernel's own bit mask of devices done (setting it twice from racing threads is harmless).
-static int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured) {
+int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured) {
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return fail(FM_ERR_LAUNCH, "hipGetDevice failed");
     const uint64_t bit = uint64_t(1) << (device & 63);
@@ -1446,6 +1444,7 @@ size_t mfma_gemm_workspace_size(GemmArgs args) {
 }
 
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
+    if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
     count_tiles(args);
     if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
     args.partials = nullptr;

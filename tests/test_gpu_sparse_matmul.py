@@ -747,3 +747,30 @@ def test_random_launches_of_many_rounds(block, device):
         out = input_row_sparse_matmul(x.t(), y, sparse_map)
         expected = moe_oracle.input_row_sparse_matmul(x.t().float(), y.float(), oracle_map)
         assert max_rel_err(out, expected) <= _MAX_REL[dtype], case
+
+
+# Weight gradients of experts of few rows (tiles of 128 x 256, slices of 32 rows, two slices ahead): every remainder of a slice,
+# around the pipeline's depth, an expert without rows and one row; column tiles whole, partial and of one chunk.
+@pytest.mark.parametrize("sparse_dim", [8, 120, 128, 136, 264])
+@pytest.mark.parametrize("dense_dim", [8, 248, 256, 520])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weight_gradients_of_few_rows(sparse_dim, dense_dim, dtype, device):
+    tokens = [0, 1, 31, 32, 33, 64, 65, 95, 97, 130, 257, 7]
+    ends = torch.cumsum((torch.tensor(tokens) + 127) // 128 * 128, 0)
+    oracle_map = fixture_sparse_map({"expert_ends": ends.tolist(), "tokens_per_expert": tokens, "phantom_rows": 128})
+    oracle_map.num_rows = int(ends[-1]) + 128
+    sparse_map = to_device_map(oracle_map, device, torch.int16)
+    generator = torch.Generator().manual_seed(sparse_dim + dense_dim)
+    y = _normal(oracle_map.num_rows, sparse_dim + 8, dtype, generator).to(device)[:, :sparse_dim]
+    x = _normal(oracle_map.num_rows, dense_dim, dtype, generator).to(device)
+    padding = ~oracle_map.real_row_mask().to(device)
+    expected = moe_oracle.input_row_sparse_matmul(y.cpu().t(), x.cpu(), oracle_map)
+    y[padding], x[padding] = float("nan"), float("nan")
+    out = torch.full((len(tokens) * sparse_dim, dense_dim + 16), 3.0, dtype=dtype, device=device)
+    input_row_sparse_matmul(y.t(), x, sparse_map, out=out[:, :dense_dim])
+    assert max_rel_err(out[:, :dense_dim].cpu(), expected) <= _MAX_REL[dtype]
+    assert (out[:, dense_dim:] == 3.0).all()
+    # The same bits as on tiles of 256 x 256, which add to what is there: the order of a sum does not depend on the tile.
+    added = torch.zeros(len(tokens) * sparse_dim, dense_dim, dtype=dtype, device=device)
+    input_row_sparse_matmul(y.t(), x, sparse_map, out=added, accumulate=True)
+    assert torch.equal(out[:, :dense_dim], added)
