@@ -293,7 +293,7 @@ __global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_any_layout_kerne
 // =========================================================================================================
 // Host dispatch
 // =========================================================================================================
-static int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace, size_t workspace_size, void *stream_) {
+int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace, size_t workspace_size, void *stream_) {
     FM_REQUIRE(valid_dtype(dtype) && valid_dtype(args.out_dtype), "%s: bad dtype", name);
     FM_REQUIRE(valid_index_dtype(args.index_dtype), "%s: bad index_dtype %d", name, args.index_dtype);
     FM_REQUIRE(args.rows >= 0 && args.cols >= 0 && args.inner >= 0 && args.sparse_size >= 0 && args.num_experts >= 1,
@@ -400,7 +400,7 @@ extern "C" size_t fm_input_row_sparse_matmul_workspace_size(int64_t row_sparse_d
 }
 
 // ---- grouped products with the gated activation fused into the epilogue ------------------------------------
-static int run_fused_gemm(const char *name, GemmArgs args, int dtype, void *stream) {
+int fm::run_fused_gemm(const char *name, GemmArgs args, int dtype, void *stream) {
     FM_REQUIRE(valid_dtype(dtype) && valid_index_dtype(args.index_dtype), "%s: bad dtype", name);
     FM_REQUIRE(args.activation >= FM_ACT_GELU && args.activation <= FM_ACT_IDENTITY, "%s: bad activation %d", name,
                args.activation);

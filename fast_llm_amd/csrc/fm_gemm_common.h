@@ -23,7 +23,8 @@ struct GemmArgs {
     const void *rhs;
     void *out;
     const void *expert_ends;        // null: dense product
-    const void *expert_pad_begins;  // row-sparse mode only
+    const void *expert_pad_begins;  // row-sparse mode: where a reduction ends; the others: where the rows to compute end (null: at
+                                    // `expert_ends`, padding rows too)
     int64_t lhs_stride_row, lhs_stride_inner, rhs_stride_inner, rhs_stride_col, out_stride_row, out_stride_col;
     int64_t rows;         // rows of out
     int64_t cols;         // columns of out
@@ -46,6 +47,7 @@ struct GemmArgs {
     void *tile_table;      // one record per id, written by the plan kernel into the caller's workspace, or null
     int64_t piece_length;  // row-sparse mode without a map: group e reduces over [e, e + 1) * piece_length instead of
                            // everything (0: everything)
+    int planned;           // `tile_table` (and `partials`) have been set up by mfma_gemm_plan
     int chunk_tiles;       // consecutive tiles that go to one XCD (set by the fp32 kernel's launcher)
 };
 
@@ -79,6 +81,13 @@ constexpr int kGroupRows = 8;
 // expert, i.e. 8 lhs panels and 4 rhs panels shared in that XCD's L2; with groups that ignore the expert boundaries
 // most chunks straddled two experts and needed twice the rhs panels.
 // Every wavefront scans `expert_ends` 64 experts at a time; returns false if `logical` is past the last tile.
+// The rows of an expert end where its padding begins, if the caller says where that is.
+__device__ __forceinline__ void rows_of_expert(const GemmArgs &args, int expert, int64_t &begin, int64_t &end) {
+    const void *ends = args.expert_pad_begins != nullptr ? args.expert_pad_begins : args.expert_ends;
+    end = min(load_index(ends, args.index_dtype, expert), args.rows);
+    begin = expert > 0 ? load_index(args.expert_ends, args.index_dtype, expert - 1) : 0;
+}
+
 struct RowTile {
     int expert, tile_n, rows_valid;
     int64_t row0;
@@ -123,10 +132,7 @@ __device__ __forceinline__ bool locate_tile(const GemmArgs &args, int logical, R
     for (int base = 0; base < args.num_experts; base += 64) {
         const int e = base + lane;
         int64_t begin = 0, end = 0;
-        if (e < args.num_experts) {
-            end = min(load_index(args.expert_ends, args.index_dtype, e), args.rows);
-            begin = e > 0 ? load_index(args.expert_ends, args.index_dtype, e - 1) : 0;
-        }
+        if (e < args.num_experts) rows_of_expert(args, e, begin, end);
         const int count = end > begin ? static_cast<int>((end - begin + kTile - 1) / kTile) : 0;
         int inclusive = count;
 #pragma unroll
@@ -185,6 +191,17 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype);  // with args.f
 // `workspace` (may be null: no split) must hold mfma_gemm_workspace_size(args) bytes when that is not 0.
 size_t mfma_gemm_workspace_size(GemmArgs args);
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream);
+
+// Tile tables of several products that follow one another on `stream`, in one launch: sets `planned`, `tile_table` and `partials`
+// of those that want them (they share the space for pieces). `workspace`: mfma_gemm_plan_size(...) bytes, 64-byte aligned, kept
+// until the last of them has run. A product with a table has to run as `run_gemm` (or the fused product) would have run it.
+constexpr int kMaxPlanned = 5;
+size_t mfma_gemm_plan_size(const GemmArgs *products, int count, int dtype);
+int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, size_t workspace_size, hipStream_t stream);
+
+// What the entry points of fm_gemm.hip check, dispatch and launch.
+int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace, size_t workspace_size, void *stream);
+int run_fused_gemm(const char *name, GemmArgs args, int dtype, void *stream);
 
 // Allows `kernel` that many bytes of dynamic LDS. `configured`: the kernel's own bit mask of devices done.
 int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured);

@@ -403,10 +403,7 @@ __device__ __forceinline__ int count_row_tiles(const GemmArgs &args) {
     for (int base = 0; base < args.num_experts; base += 64) {
         const int e = base + lane;
         int64_t begin = 0, end = 0;
-        if (e < args.num_experts) {
-            end = min(load_index(args.expert_ends, args.index_dtype, e), args.rows);
-            begin = e > 0 ? load_index(args.expert_ends, args.index_dtype, e - 1) : 0;
-        }
+        if (e < args.num_experts) rows_of_expert(args, e, begin, end);
         int count = end > begin ? static_cast<int>((end - begin + kTile - 1) / kTile) : 0;
 #pragma unroll
         for (int offset = 32; offset > 0; offset >>= 1) count += __shfl_xor(count, offset, 64);
@@ -512,8 +509,15 @@ struct alignas(64) TableHeader {
 };
 static_assert(sizeof(TableHeader) == 64 && sizeof(TableHeader) == sizeof(TileRecord), "the header is record -1");
 
+// The products whose tables are written together, one per blockIdx.y.
+struct PlannedProducts {
+    GemmArgs products[kMaxPlanned];
+};
+
 // One wavefront per id; the wavefront of id 0 also leaves the split plan of the launch in the table's header.
-__global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(GemmArgs args, TileRecord *table) {
+__global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(PlannedProducts planned) {
+    const GemmArgs &args = planned.products[blockIdx.y];
+    TileRecord *table = static_cast<TileRecord *>(args.tile_table);
     const int id = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (id >= args.num_ids) return;
     if (id == 0 && args.partials != nullptr) {
@@ -1313,10 +1317,6 @@ static int launch_instance(const GemmArgs &args, hipStream_t stream) {
     auto kernel = grouped_gemm_mfma_kernel<T, kLhsK, kRhsK, kMasked, kFusion>;
     static std::atomic<uint64_t> configured{0};
     if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
-    // With a workspace, one wavefront per id first writes the id's tile record (and, when the last round may be
-    // split, the plan of the split).
-    if (args.tile_table != nullptr)
-        grouped_gemm_plan_kernel<<<(args.num_ids + 3) / 4, 256, 0, stream>>>(args, static_cast<TileRecord *>(args.tile_table));
     // One workgroup per CU walks the ids (see the kernel).
     kernel<<<min(args.num_ids, kRound), kMfmaThreads, kLdsBytes, stream>>>(args);
     if (args.partials != nullptr) {
@@ -1424,37 +1424,107 @@ static size_t table_bytes(int num_ids) {
     return (sizeof(TableHeader) + static_cast<size_t>(num_ids) * sizeof(TileRecord) + 255) / 256 * 256;
 }
 
-size_t mfma_gemm_workspace_size(GemmArgs args) {
-    if (args.rows <= 0 || args.cols <= 0 || args.inner <= 0) return 0;
+// Where the pieces and the table of one product go. False: it wants neither, or cannot run here.
+struct TableSpace {
+    bool split;
+    size_t table_bytes;
+};
+static bool table_space(GemmArgs &args, TableSpace &space) {
+    if (args.rows <= 0 || args.cols <= 0 || args.inner <= 0) return false;
     // Dimensions that `mfma_gemm_eligible` refuses whatever the strides (such a product runs on the generic kernel, which
     // takes no workspace), and reductions that are no whole number of slices (which do not split).
-    if (args.inner % kBK != 0 || args.cols % 8 != 0 || (args.mode == kInputRowSparse && args.sparse_size % 8 != 0)) return 0;
+    if (args.inner % kBK != 0 || args.cols % 8 != 0 || (args.mode == kInputRowSparse && args.sparse_size % 8 != 0)) return false;
     count_tiles(args);
-    if (too_many_tiles(args)) return 0;
-    const bool split = splits_last_round(args);
-    return (split ? kPartialBytes : 0) + table_bytes(count_ids(args, split));
+    if (too_many_tiles(args)) return false;
+    space.split = splits_last_round(args);
+    args.num_ids = count_ids(args, space.split);
+    space.table_bytes = table_bytes(args.num_ids);
+    return true;
+}
+
+size_t mfma_gemm_workspace_size(GemmArgs args) {
+    TableSpace space;
+    return table_space(args, space) ? (space.split ? kPartialBytes : 0) + space.table_bytes : 0;
+}
+
+// A launch of at most one round that does not split: every workgroup finds its one tile itself (a scan of the expert map, a
+// few thousand cycles) sooner than a kernel launched in front of it could tell it.
+static bool wants_table(const GemmArgs &args, bool split) { return split || args.num_ids > kRound; }
+
+static int launch_plan(const GemmArgs *products, int count, hipStream_t stream) {
+    PlannedProducts planned;
+    int most_ids = 0;
+    for (int i = 0; i < count; ++i) {
+        planned.products[i] = products[i];
+        most_ids = max(most_ids, products[i].num_ids);
+    }
+    grouped_gemm_plan_kernel<<<dim3((most_ids + 3) / 4, count), 256, 0, stream>>>(planned);
+    return FM_OK;
+}
+
+size_t mfma_gemm_plan_size(const GemmArgs *products, int count, int dtype) {
+    if (dtype == FM_DTYPE_F32) return 0;
+    size_t bytes = 0;
+    bool any_split = false;
+    for (int i = 0; i < count; ++i) {
+        GemmArgs args = products[i];
+        TableSpace space;
+        if (!table_space(args, space)) continue;
+        any_split = any_split || space.split;
+        bytes += space.table_bytes;
+    }
+    return bytes + (any_split ? kPartialBytes : 0);
+}
+
+int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
+    if (count > kMaxPlanned || workspace_size < mfma_gemm_plan_size(products, count, dtype) ||
+        reinterpret_cast<uintptr_t>(workspace) % 64 != 0)
+        return fail(FM_ERR_INVALID_ARGUMENT, "grouped gemm: %d products to plan in %zu bytes at %p", count, workspace_size, workspace);
+    GemmArgs planned[kMaxPlanned];
+    int num_planned = 0;
+    size_t at = 0;
+    const auto plan = [&](bool split_ones) {
+        for (int i = 0; i < count; ++i) {
+            GemmArgs args = products[i];
+            TableSpace space;
+            const bool eligible = args.fusion == kFusionNone ? mfma_gemm_eligible(args, dtype) : mfma_gemm_fusion_eligible(args, dtype);
+            if (!eligible || row_sparse_gemm_chosen(args, dtype) || !table_space(args, space) || !wants_table(args, space.split)) continue;
+            if (space.split != split_ones) continue;
+            if (split_ones && at == 0) at = kPartialBytes;
+            args.partials = space.split ? static_cast<float *>(workspace) : nullptr;
+            args.tile_table = static_cast<char *>(workspace) + at + sizeof(TableHeader);
+            args.planned = 1;
+            at += space.table_bytes;
+            products[i] = planned[num_planned++] = args;
+        }
+    };
+    plan(true);  // first, so that the space for pieces is in front of all tables
+    plan(false);
+    return num_planned > 0 ? launch_plan(planned, num_planned, stream) : FM_OK;
 }
 
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
-    if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
-    count_tiles(args);
-    if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
-    args.partials = nullptr;
-    args.tile_table = nullptr;
-    if (args.inner % kBK != 0) workspace = nullptr;  // as mfma_gemm_workspace_size says
-    const bool split = workspace != nullptr && splits_last_round(args);
-    args.num_ids = count_ids(args, split);
-    if (workspace != nullptr) {
-        const size_t needed = (split ? kPartialBytes : 0) + table_bytes(args.num_ids);
-        if (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0)
-            return fail(FM_ERR_INVALID_ARGUMENT,
-                        "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
-                        workspace_size, workspace);
-        if (split) args.partials = static_cast<float *>(workspace);
-        args.tile_table = static_cast<char *>(workspace) + (split ? kPartialBytes : 0) + sizeof(TableHeader);
-        // A launch of at most one round that does not split: every workgroup finds its one tile itself (a scan of the
-        // expert map, a few thousand cycles) sooner than a kernel launched in front of it could tell it.
-        if (!split && args.num_ids <= kRound) args.tile_table = nullptr;
+    if (!args.planned) {
+        if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
+        count_tiles(args);
+        if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
+        args.partials = nullptr;
+        args.tile_table = nullptr;
+        if (args.inner % kBK != 0) workspace = nullptr;  // as mfma_gemm_workspace_size says
+        const bool split = workspace != nullptr && splits_last_round(args);
+        args.num_ids = count_ids(args, split);
+        if (workspace != nullptr) {
+            const size_t needed = (split ? kPartialBytes : 0) + table_bytes(args.num_ids);
+            if (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0)
+                return fail(FM_ERR_INVALID_ARGUMENT,
+                            "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
+                            workspace_size, workspace);
+            if (split) args.partials = static_cast<float *>(workspace);
+            if (wants_table(args, split)) {
+                args.tile_table = static_cast<char *>(workspace) + (split ? kPartialBytes : 0) + sizeof(TableHeader);
+                if (int status = launch_plan(&args, 1, stream)) return status;
+            }
+        }
     }
     return dtype == FM_DTYPE_BF16 ? launch_layout<bf16_t>(args, stream) : launch_layout<f16_t>(args, stream);
 }

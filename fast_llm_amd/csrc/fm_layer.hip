@@ -50,17 +50,8 @@ int make_plan(const fm_moe_layer &layer, Plan &plan) {
     plan.expert_pad_begins = take(plan.used_index_size * plan.experts);
     plan.router = take(fm_router_workspace_size(layer.tokens, layer.routed_experts));
     plan.routing_bytes = at;
-    const int64_t ffn_1 = layer.ffn * (layer.gated ? 2 : 1);
-    const int dtype = static_cast<int>(layer.dtype);
-    plan.router_linear_bytes = fm_router_linear_backward_workspace_size(layer.tokens, layer.routed_experts, layer.hidden, dtype);
-    plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
-    for (size_t bytes : {plan.router_linear_bytes, fm_grouped_gemm_workspace_size(plan.rows, ffn_1, layer.hidden, plan.experts, dtype),
-                         fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, layer.ffn, plan.experts, dtype),
-                         fm_grouped_gemm_workspace_size(plan.rows, layer.ffn, layer.hidden, plan.experts, dtype),
-                         fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, ffn_1, plan.experts, dtype),
-                         fm_input_row_sparse_matmul_workspace_size(layer.ffn, layer.hidden, plan.rows, plan.experts, dtype),
-                         fm_input_row_sparse_matmul_workspace_size(ffn_1, layer.hidden, plan.rows, plan.experts, dtype)})
-        if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+    plan.router_linear_bytes = fm_router_linear_backward_workspace_size(layer.tokens, layer.routed_experts, layer.hidden, static_cast<int>(layer.dtype));
+    plan.workspace_bytes = 0;  // the rest of it: see plan_workspace
     return FM_OK;
 }
 
@@ -88,29 +79,72 @@ struct Step {
                                        dtype(), FM_DTYPE_F32, plan.index_dtype, stream);
     }
     // out [rows, columns] = lhs [rows, inner] x (weight_e [columns, inner])^T
-    int output_sparse(const void *lhs, const void *weight, void *out, int64_t columns, int64_t inner) {
-        const size_t bytes = fm_grouped_gemm_workspace_size(plan.rows, columns, inner, plan.experts, dtype());
-        return keep(fm_output_sparse_matmul(lhs, weight, out, routing(plan.expert_ends), plan.rows, columns, inner, plan.experts, inner,
-                                            1, 1, inner, columns, 1, 0, dtype(), dtype(), plan.index_dtype,
-                                            bytes ? layer.workspace : nullptr, bytes, stream));
+    GemmArgs output_sparse(const void *lhs, const void *weight, void *out, int64_t columns, int64_t inner) const {
+        return GemmArgs{lhs, weight, out, routing(plan.expert_ends), nullptr, inner, 1, 1, inner, columns, 1,
+                        plan.rows, columns, inner, columns, static_cast<int>(plan.experts), kOutputSparse, 0, plan.index_dtype, dtype()};
     }
     // out [rows, hidden] = lhs [rows, inner] x weight_e [inner, hidden]
-    int inner_sparse(const void *lhs, const void *weight, void *out, int64_t inner) {
-        const size_t bytes = fm_grouped_gemm_workspace_size(plan.rows, layer.hidden, inner, plan.experts, dtype());
-        return keep(fm_input_inner_sparse_matmul(lhs, weight, out, routing(plan.expert_ends), plan.rows, layer.hidden, inner,
-                                                 plan.experts, inner, 1, layer.hidden, 1, layer.hidden, 1, 0, dtype(), dtype(),
-                                                 plan.index_dtype, bytes ? layer.workspace : nullptr, bytes, stream));
+    GemmArgs inner_sparse(const void *lhs, const void *weight, void *out, int64_t inner) const {
+        const int64_t hidden = layer.hidden;
+        return GemmArgs{lhs, weight, out, routing(plan.expert_ends), nullptr, inner, 1, hidden, 1, hidden, 1,
+                        plan.rows, hidden, inner, inner, static_cast<int>(plan.experts), kInputInnerSparse, 0, plan.index_dtype, dtype()};
     }
     // out [experts * size, hidden] (+)= lhs^T x rhs, lhs [rows, size], rhs [rows, hidden]
-    int row_sparse(const void *lhs, const void *rhs, void *out, int64_t size, bool accumulate) {
-        const size_t bytes = fm_input_row_sparse_matmul_workspace_size(size, layer.hidden, plan.rows, plan.experts, dtype());
-        return keep(fm_input_row_sparse_matmul(lhs, rhs, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), size,
-                                               layer.hidden, plan.rows, plan.experts, 1, size, layer.hidden, 1, layer.hidden, 1,
-                                               accumulate, dtype(), static_cast<int>(layer.grad_dtype), plan.index_dtype,
-                                               bytes ? layer.workspace : nullptr, bytes, stream));
+    GemmArgs row_sparse(const void *lhs, const void *rhs, void *out, int64_t size, bool accumulate) const {
+        const int64_t hidden = layer.hidden;
+        return GemmArgs{lhs, rhs, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), 1, size, hidden, 1, hidden, 1,
+                        size * plan.experts, hidden, plan.rows, size, static_cast<int>(plan.experts), kInputRowSparse, accumulate,
+                        plan.index_dtype, static_cast<int>(layer.grad_dtype)};
     }
+    GemmArgs layer_1() const {
+        GemmArgs args = output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, ffn_1(), layer.hidden);
+        if (layer.gated && layer.layer_1_output == nullptr) {  // the activation in the product's epilogue
+            args.fusion = kFusionGatedForward;
+            args.activation = static_cast<int>(layer.activation);
+            args.fused_out = layer.activation_output;
+            args.fused_stride = args.half = layer.ffn;
+        }
+        return args;
+    }
+    enum { kLayer1 = 0, kLayer2 = 1, kGradActivation = 1, kGradWeight2 = 2, kGradInput = 3, kGradWeight1 = 4 };
+    // The products of a forward, and of a backward.
+    void forward_products(GemmArgs *products) const {
+        products[kLayer1] = layer_1();
+        products[kLayer2] = inner_sparse(layer.activation_output, layer.weight_2, layer.layer_2_output, layer.ffn);
+    }
+    void backward_products(GemmArgs *products) const {
+        products[kLayer1] = layer_1();
+        products[kGradActivation] = output_sparse(layer.grad_layer_2_output, layer.weight_2, layer.grad_activation_output, layer.ffn, layer.hidden);
+        products[kGradWeight2] = row_sparse(layer.activation_output, layer.grad_layer_2_output, layer.grad_weight_2, layer.ffn, layer.accumulate_2 != 0);
+        products[kGradInput] = inner_sparse(layer.grad_layer_1_output, layer.weight_1, layer.grad_layer_2_output, ffn_1());
+        products[kGradWeight1] = row_sparse(layer.grad_layer_1_output, layer.sparse_input, layer.grad_weight_1, ffn_1(), layer.accumulate_1 != 0);
+    }
+    // One launch for the tile tables of all products that are wanted: each launch of its own took 7 us.
+    int plan_tables(GemmArgs *products, const bool *wanted, int count) const {
+        GemmArgs chosen[kMaxPlanned];
+        int which[kMaxPlanned], num = 0;
+        for (int i = 0; i < count; ++i)
+            if (wanted[i]) chosen[num] = products[i], which[num++] = i;
+        if (dtype() == FM_DTYPE_F32) return FM_OK;
+        const int status = mfma_gemm_plan(chosen, num, dtype(), layer.workspace, plan.workspace_bytes, static_cast<hipStream_t>(stream));
+        for (int i = 0; i < num; ++i) products[which[i]] = chosen[i];
+        return status;
+    }
+    int product(const GemmArgs &args) { return keep(run_gemm("fm_moe_layer", args, dtype(), nullptr, 0, stream)); }
     const void *rows_in_use() const { return routing(plan.expert_ends + (plan.experts - 1) * plan.used_index_size); }
 };
+
+void plan_workspace(const fm_moe_layer &layer, Plan &plan) {
+    const Step step{layer, plan, nullptr};
+    plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
+    GemmArgs products[kMaxPlanned];
+    step.forward_products(products);
+    size_t bytes = mfma_gemm_plan_size(products, 2, step.dtype());
+    step.backward_products(products);
+    for (size_t other : {plan.router_linear_bytes, mfma_gemm_plan_size(products, 5, step.dtype())})
+        if (other > bytes) bytes = other;
+    if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+}
 
 #define FM_STEP(call) \
     if (int status = (call)) return status
@@ -137,20 +171,22 @@ int forward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     FM_REQUIRE(layer.input && layer.weight_1 && layer.weight_2 && layer.routing && layer.sparse_input && layer.activation_output &&
                    layer.layer_2_output && layer.output && layer.workspace,
                "fm_moe_layer_forward: null tensor");
+    FM_REQUIRE(layer.gated || layer.layer_1_output, "fm_moe_layer_forward: layer 1 without a gate needs its output");
+    GemmArgs products[2];
+    step.forward_products(products);
+    const bool wanted[2] = {true, true};
+    FM_STEP(step.plan_tables(products, wanted, 2));
     FM_STEP(step.dispatch(layer.sparse_input));
-    if (layer.layer_1_output == nullptr) {
-        // The product with the activation in its epilogue; FM_ERR_UNSUPPORTED tells the caller to bring a layer-1 buffer.
-        FM_STEP(fm_output_sparse_matmul_gated_activation(layer.sparse_input, layer.weight_1, nullptr, layer.activation_output,
-                                                         step.routing(plan.expert_ends), plan.rows, layer.ffn, layer.hidden,
-                                                         plan.experts, layer.hidden, 1, 1, layer.hidden,
-                                                         static_cast<int>(layer.activation), step.dtype(), plan.index_dtype, stream));
+    if (products[Step::kLayer1].fusion != kFusionNone) {
+        // FM_ERR_UNSUPPORTED tells the caller to bring a layer-1 buffer.
+        FM_STEP(run_fused_gemm("fm_moe_layer_forward", products[Step::kLayer1], step.dtype(), stream));
     } else {
-        FM_STEP(step.output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, step.ffn_1(), layer.hidden));
+        FM_STEP(step.product(products[Step::kLayer1]));
         FM_STEP(fm_mlp_activation_forward(layer.layer_1_output, layer.activation_output, plan.rows, layer.ffn,
                                           static_cast<int>(layer.gated), static_cast<int>(layer.activation), step.dtype(),
                                           step.rows_in_use(), plan.index_dtype, stream));
     }
-    FM_STEP(step.inner_sparse(layer.activation_output, layer.weight_2, layer.layer_2_output, layer.ffn));
+    FM_STEP(step.product(products[Step::kLayer2]));
     FM_STEP(step.combine(layer.layer_2_output, step.routing(plan.scores), layer.output));
     return step.note;
 }
@@ -162,6 +198,11 @@ int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
                    layer.grad_activation_output && layer.grad_layer_1_output && layer.grad_scores && layer.grad_logits &&
                    layer.workspace && (layer.input || !(layer.recompute_input || layer.router)),
                "fm_moe_layer_backward: null tensor");
+    GemmArgs products[kMaxPlanned];
+    step.backward_products(products);
+    const bool wanted[kMaxPlanned] = {layer.recompute_layer_1 != 0, true, layer.grad_weight_2 != nullptr, layer.grad_input != nullptr,
+                                      layer.grad_weight_1 != nullptr};
+    FM_STEP(step.plan_tables(products, wanted, kMaxPlanned));
     // The gradient of layer 2's output and of the scores.
     FM_STEP(fm_copy_sparse_to_dense_backward(layer.layer_2_output, layer.grad_output, step.routing(plan.scores),
                                              step.routing(plan.sparse_rows), layer.grad_layer_2_output, layer.grad_scores,
@@ -169,23 +210,18 @@ int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
                                              FM_DTYPE_F32, plan.index_dtype, stream));
     // What the forward did not keep.
     if (layer.recompute_input) FM_STEP(step.dispatch(layer.sparse_input));
-    if (layer.recompute_layer_1)
-        FM_STEP(step.output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, step.ffn_1(), layer.hidden));
+    if (layer.recompute_layer_1) FM_STEP(step.product(products[Step::kLayer1]));
     // Through layer 2 and the activation.
-    FM_STEP(step.output_sparse(layer.grad_layer_2_output, layer.weight_2, layer.grad_activation_output, layer.ffn, layer.hidden));
+    FM_STEP(step.product(products[Step::kGradActivation]));
     FM_STEP(fm_mlp_activation_backward(layer.grad_activation_output, layer.grad_layer_1_output, layer.layer_1_output,
                                        layer.recompute_activation ? layer.activation_output : nullptr, plan.rows, layer.ffn,
                                        static_cast<int>(layer.gated), static_cast<int>(layer.activation), step.dtype(),
                                        step.rows_in_use(), plan.index_dtype, stream));
-    if (layer.grad_weight_2)
-        FM_STEP(step.row_sparse(layer.activation_output, layer.grad_layer_2_output, layer.grad_weight_2, layer.ffn,
-                                layer.accumulate_2 != 0));
+    if (layer.grad_weight_2) FM_STEP(step.product(products[Step::kGradWeight2]));
     // Through layer 1. The gradient of layer 2's output has been read for the last time: that of the sparse input takes
     // its place.
-    if (layer.grad_input) FM_STEP(step.inner_sparse(layer.grad_layer_1_output, layer.weight_1, layer.grad_layer_2_output, step.ffn_1()));
-    if (layer.grad_weight_1)
-        FM_STEP(step.row_sparse(layer.grad_layer_1_output, layer.sparse_input, layer.grad_weight_1, step.ffn_1(),
-                                layer.accumulate_1 != 0));
+    if (layer.grad_input) FM_STEP(step.product(products[Step::kGradInput]));
+    if (layer.grad_weight_1) FM_STEP(step.product(products[Step::kGradWeight1]));
     if (layer.grad_input) FM_STEP(step.combine(layer.grad_layer_2_output, nullptr, layer.grad_input));
     const bool losses = layer.with_losses != 0;
     FM_STEP(fm_router_backward(layer.grad_scores, step.routing(plan.scores), step.routing(plan.top_experts), layer.logits, layer.noise,
@@ -209,6 +245,7 @@ extern "C" int fm_moe_layer_sizes(fm_moe_layer *layer) {
     Plan plan;
     FM_REQUIRE(layer, "fm_moe_layer_sizes: null");
     if (int status = make_plan(*layer, plan)) return status;
+    plan_workspace(*layer, plan);
     layer->rows = plan.rows;
     layer->routing_bytes = static_cast<int64_t>(plan.routing_bytes);
     layer->workspace_bytes = static_cast<int64_t>(plan.workspace_bytes);
@@ -222,6 +259,7 @@ extern "C" int fm_moe_layer_route(const fm_moe_layer *layer, void *stream) {
     Plan plan;
     FM_REQUIRE(layer, "fm_moe_layer_route: null");
     if (int status = make_plan(*layer, plan)) return status;
+    plan_workspace(*layer, plan);
     return route(*layer, plan, stream);
 }
 
@@ -229,6 +267,7 @@ extern "C" int fm_moe_layer_forward(const fm_moe_layer *layer, void *stream) {
     Plan plan;
     FM_REQUIRE(layer, "fm_moe_layer_forward: null");
     if (int status = make_plan(*layer, plan)) return status;
+    plan_workspace(*layer, plan);
     return forward(*layer, plan, stream);
 }
 
@@ -236,5 +275,6 @@ extern "C" int fm_moe_layer_backward(const fm_moe_layer *layer, void *stream) {
     Plan plan;
     FM_REQUIRE(layer, "fm_moe_layer_backward: null");
     if (int status = make_plan(*layer, plan)) return status;
+    plan_workspace(*layer, plan);
     return backward(*layer, plan, stream);
 }
