@@ -135,16 +135,26 @@ struct Step {
     const void *rows_in_use() const { return routing(plan.expert_ends + (plan.experts - 1) * plan.used_index_size); }
 };
 
+// From the shape alone, whatever buffers the caller has filled in: it asks for the size before it has them. A forward runs layer
+// 1 with or without its output, whose tables differ; a backward always has the output.
 void plan_workspace(const fm_moe_layer &layer, Plan &plan) {
-    const Step step{layer, plan, nullptr};
+    fm_moe_layer kept = layer, fused = layer;
+    kept.layer_1_output = kept.routing = &kept;  // any address: nothing is launched
+    fused.layer_1_output = nullptr, fused.routing = &fused;
+    const Step with_output{kept, plan, nullptr}, without{fused, plan, nullptr};
+    const int dtype = with_output.dtype();
     plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
+    const auto at_least = [&](size_t bytes) {
+        if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+    };
+    at_least(plan.router_linear_bytes);
     GemmArgs products[kMaxPlanned];
-    step.forward_products(products);
-    size_t bytes = mfma_gemm_plan_size(products, 2, step.dtype());
-    step.backward_products(products);
-    for (size_t other : {plan.router_linear_bytes, mfma_gemm_plan_size(products, 5, step.dtype())})
-        if (other > bytes) bytes = other;
-    if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+    with_output.forward_products(products);
+    at_least(mfma_gemm_plan_size(products, 2, dtype));
+    without.forward_products(products);
+    at_least(mfma_gemm_plan_size(products, 2, dtype));
+    with_output.backward_products(products);
+    at_least(mfma_gemm_plan_size(products, kMaxPlanned, dtype));
 }
 
 #define FM_STEP(call) \

@@ -157,3 +157,20 @@ def test_enums_mirror_the_reference():
     assert MLPRecomputeLevel("activation_and_input").recompute_sparse_input
     assert ActivationType.silu.value == "silu" and f"{ActivationType.gelu}" == "gelu"
     assert KernelConfig.POINTWISE_BLOCK_SIZE == 1024
+
+
+@pytest.mark.parametrize("gated", [0, 1])
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize(("hidden", "ffn", "tokens"), [(2048, 2176, 300), (2048, 192, 2100), (4096, 14336, 8192), (128, 256, 77)])
+def test_layer_sizes_come_from_the_shape_alone(library, hidden, ffn, tokens, dtype, gated):
+    """The caller asks for the workspace before it has the buffers of the call: with or without layer 1's output, in the forward
+    or in the backward, the size is the same."""
+    sizes = set()
+    for buffers in ((), ("layer_1_output",), ("layer_1_output", "routing", "grad_output", "grad_input", "grad_weight_1", "grad_weight_2")):
+        layer = _lib.MoELayer(tokens, hidden, ffn, 7, 0, 2, gated, 1, dtype)
+        layer.recompute_layer_1 = len(buffers) > 1
+        for name in buffers:
+            setattr(layer, name, 64)
+        _lib.check(library.fm_moe_layer_sizes(ctypes.byref(layer)))
+        sizes.add((layer.rows, layer.routing_bytes, layer.workspace_bytes))
+    assert len(sizes) == 1
