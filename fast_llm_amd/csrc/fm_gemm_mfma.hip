@@ -304,7 +304,8 @@ struct TileWork {
 };
 
 constexpr int kXcds = 8, kChunkTiles = 32;
-constexpr int kHalfTileMaxSlices = 64;  // reductions of this many slices or more have no half tiles (see find_tile)
+// Reductions of this many slices or more have no half tiles (see finish_tile): with up to kFewRows rows per expert, and with more.
+constexpr int kFewRows = 1024, kHalfTileMaxSlicesFewRows = 128, kHalfTileMaxSlices = 64;
 
 // Where the operands and the output of logical tile `logical` are. False: there is no such tile.
 __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, TileWork &work) {
@@ -476,7 +477,8 @@ struct alignas(64) TileRecord {
     int k_lo, k_hi;    // reduction range (a piece of it for a split tile; ragged for the row-sparse product)
     int piece_slot;    // >= 0: a piece of a split reduction, stored to that workspace slot
     int found;         // 0: the id has no tile (and no later id has one)
-    int unused[2];
+    int half_slices;   // a half tile if the reduction has fewer slices than this
+    int unused;
 };
 static_assert(sizeof(TileRecord) == 64, "one s_load_dwordx16 per record");
 
@@ -487,6 +489,8 @@ __device__ __forceinline__ bool compute_tile_record(const GemmArgs &args, int id
     const bool found = tile_of_block(args, id, logical, piece, piece_slices, piece_slot) && resolve_tile(args, logical, work);
     record.found = __builtin_amdgcn_readfirstlane(found);
     if (!record.found) return false;
+    record.half_slices = args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts ? kHalfTileMaxSlicesFewRows : kHalfTileMaxSlices;
+    record.unused = 0;
     record.piece_slot = __builtin_amdgcn_readfirstlane(piece_slot);
     if (record.piece_slot >= 0) {  // a piece of a tile whose reduction is split (never the row-sparse product)
         work.k_lo = static_cast<int64_t>(piece) * piece_slices * kBK;
@@ -525,8 +529,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(PlannedProducts 
         if ((threadIdx.x & 63) == 0) reinterpret_cast<TableHeader *>(table)[-1].plan = plan;
     }
     TileRecord record;
-    record.unused[0] = record.unused[1] = 0;
     if (!compute_tile_record(args, id, record)) {
+        record.half_slices = record.unused = 0;
         record.lhs_offset = record.rhs_offset = record.out_offset = record.fused_offset = 0;
         record.rows_valid = record.cols_valid = record.k_lo = record.k_hi = 0;
         record.piece_slot = -1;
@@ -727,11 +731,11 @@ template <typename T, int kActivation>
 __device__ __forceinline__ void store_tile_gated_forward(const f32x16_t (&acc)[kTilesM][kTilesN], FM_LDS(char) * lds,
                                                          T *layer_1, T *activation_out, int64_t stride,
                                                          int64_t activation_stride, int64_t half, int rows_valid,
-                                                         int wave, int lane) {
+                                                         int wave, int lane, int row_base, int blocks) {
     static_assert(kTilesN == 4 && kWaveCols == 128, "two gate and two up accumulators per row block");
     constexpr int kColumns = kWaveCols / 2, kRowBytes = kColumns * sizeof(T) + kEpiloguePadBytes;
     constexpr int kLanesPerRow = kColumns * sizeof(T) / 16, kRowsPerRead = 64 / kLanesPerRow, kReads = 32 / kRowsPerRead;
-    const int wave_m = wave / kWavesN, wave_n = wave % kWavesN;
+    const int wave_n = wave % kWavesN;
     FM_LDS(char) *staging = lds + wave * (32 * kRowBytes);
     FM_LDS(char) *write_base = staging + (lane & 31) * kRowBytes + (lane >> 5) * 4 * sizeof(T);
     const int read_row = lane / kLanesPerRow, read_column = lane % kLanesPerRow * 8;
@@ -762,7 +766,8 @@ __device__ __forceinline__ void store_tile_gated_forward(const f32x16_t (&acc)[k
     };
 #pragma unroll
     for (int i = 0; i < kTilesM; ++i) {
-        const int first_row = wave_m * kWaveRows + i * 32 + read_row;
+        if (i >= blocks) break;  // wave-uniform
+        const int first_row = row_base + i * 32 + read_row;
         if (layer_1 != nullptr) {
             pass(layer_1, stride, first_row, [&](int j, int v) { return from_float<T>(acc[i][j][v]); });
             pass(layer_1 + half, stride, first_row, [&](int j, int v) { return from_float<T>(acc[i][j + 2][v]); });
@@ -880,9 +885,12 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
         // some ten slices of each other) the panels are then fetched again by those that follow. Measured at 64
         // slices and more: L2-miss traffic 5.6 -> 3.0 and 4.6 -> 3.2 (FETCH_SIZE, layer-1 forward and input gradient of
         // the Mixtral-like workload) and the launches 2 to 4 % faster with full-cost last tiles; at 12 to 44 slices
-        // the half tiles win by 1.5 to 5 %.
-        tile.half = kFusion == kFusionNone && tile.piece_slot < 0 && work.rows_valid <= kTile / 2 &&
-                    tile.num_slices < kHalfTileMaxSlices;
+        // the half tiles win by 1.5 to 5 %. Where experts have few row tiles, the half tiles are a larger part of the work and
+        // an XCD's 32 tiles share less: with 64 slices (4096) 698 -> 658 us at 383 rows per expert (8 experts of 4096 x 14336,
+        // layer 1), 1042 -> 983 at 600, 1557 -> 1552 at 1000, 2939 -> 3006 at 2048; with 224 slices 334 -> 335, 501 -> 501,
+        // with 448 962 -> 986 at 600.
+        tile.half = kFusion != kFusionGatedBackward && tile.piece_slot < 0 && work.rows_valid <= kTile / 2 &&
+                    tile.num_slices < work.half_slices;
     };
     auto find_tile = [&](int id, Tile &tile) -> bool {
         if (args.tile_table != nullptr) {
@@ -1230,7 +1238,8 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
             FM_DISPATCH_ACTIVATION(args.activation, kActivation,
                                    store_tile_gated_forward<T, kActivation>(
                                        acc, staging, layer_1, static_cast<T *>(args.fused_out) + work.fused_offset,
-                                       args.out_stride_row, args.fused_stride, args.half, work.rows_valid, wave, lane));
+                                       args.out_stride_row, args.fused_stride, args.half, work.rows_valid, wave, lane,
+                                       wave_row_base, wave_row_blocks));
         } else if constexpr (kFusion == kFusionGatedBackward) {
             T *recomputed = args.fused_out == nullptr ? nullptr : static_cast<T *>(args.fused_out) + work.fused_offset;
             FM_DISPATCH_ACTIVATION(args.activation, kActivation,
