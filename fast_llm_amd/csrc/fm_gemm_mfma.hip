@@ -385,7 +385,10 @@ __device__ __forceinline__ int logical_of_block(int pid) {
 // kernels computes the same one.
 constexpr int kMaxPartials = 512;          // workspace slots of 256 x 256 floats
 constexpr int kMinPieceSlices = 16;        // do not cut a reduction into pieces shorter than this
-constexpr int kPieceOverheadSlices = 8;    // set-up, prologue and epilogue of a piece, in slice times
+// What a round of pieces costs over its multiplications, in slice times (about 1.5 us): set-up, prologue and epilogue, writing
+// and reading 64 MiB of accumulators, the launch that adds them. 160 tiles of 107 slices in three pieces are two rounds of 36: 187
+// us, 184 unsplit; 80 such tiles in one round of three pieces 102 us, 159 unsplit; 160 tiles of 54 slices 133 and 102.
+constexpr int kPieceOverheadSlices = 17;
 constexpr int kPartialFloats = kTile * kTile;
 
 struct SplitPlan {
@@ -422,12 +425,12 @@ __device__ __forceinline__ SplitPlan plan_split(const GemmArgs &args, bool with_
     plan.tail = total % kRound;
     plan.whole = total - plan.tail;
     plan.pieces = 1;
-    const int num_slices = static_cast<int>(args.inner / kBK);
+    const int num_slices = static_cast<int>((args.inner + kBK - 1) / kBK);
     plan.piece_slices = num_slices;
     int best = num_slices;
     if (plan.tail > 0 && with_pieces) {
 #pragma unroll
-        for (int split = 2; split <= 8; split *= 2) {
+        for (int split : {2, 3, 4, 8}) {
             if (plan.tail * split > kMaxPartials || num_slices / split < kMinPieceSlices) continue;
             const int length = ((num_slices + split - 1) / split + 1) / 2 * 2;  // even: slices are multiplied in pairs
             const int pieces = (num_slices + length - 1) / length;
@@ -1415,10 +1418,15 @@ static bool too_many_tiles(const GemmArgs &args) {
     return static_cast<int64_t>(args.tiles_m) * args.tiles_n >= (int64_t(1) << 31) - 2 * kRound - kMaxPartials;
 }
 
+// A reduction that is no whole number of slices is masked, and splits only in launches that leave a quarter of the CUs idle
+// even by the upper bound of their tiles: the table and the launch that adds the pieces cost 10 us, which those without idle CUs
+// do not get back (375 rows of 16 experts, 1280 x 3416: 103 -> 109 and 184 -> 188 us; 200 rows 105 -> 74 and 190 -> 106; 20 rows
+// 85 -> 69 and 158 -> 99).
 static bool splits_last_round(const GemmArgs &args) {
     constexpr int kMaxRoundsToSplit = 16;
-    return args.fusion == kFusionNone && args.mode != kInputRowSparse && args.inner / kBK >= 2 * kMinPieceSlices &&
-           static_cast<int64_t>(args.tiles_m) * args.tiles_n <= kMaxRoundsToSplit * kRound;
+    const int64_t most = args.inner % kBK == 0 ? kMaxRoundsToSplit * kRound : kRound * 3 / 4;
+    return args.fusion == kFusionNone && args.mode != kInputRowSparse && (args.inner + kBK - 1) / kBK >= 2 * kMinPieceSlices &&
+           static_cast<int64_t>(args.tiles_m) * args.tiles_n <= most;
 }
 
 // Whole rounds of one chunk per XCD; when the last round is split its pieces come after the whole tiles, at most
@@ -1441,11 +1449,12 @@ struct TableSpace {
 static bool table_space(GemmArgs &args, TableSpace &space) {
     if (args.rows <= 0 || args.cols <= 0 || args.inner <= 0) return false;
     // Dimensions that `mfma_gemm_eligible` refuses whatever the strides (such a product runs on the generic kernel, which
-    // takes no workspace), and reductions that are no whole number of slices (which do not split).
-    if (args.inner % kBK != 0 || args.cols % 8 != 0 || (args.mode == kInputRowSparse && args.sparse_size % 8 != 0)) return false;
+    // takes no workspace).
+    if (args.inner % 8 != 0 || args.cols % 8 != 0 || (args.mode == kInputRowSparse && args.sparse_size % 8 != 0)) return false;
     count_tiles(args);
     if (too_many_tiles(args)) return false;
     space.split = splits_last_round(args);
+    if (!space.split && args.inner % kBK != 0) return false;
     args.num_ids = count_ids(args, space.split);
     space.table_bytes = table_bytes(args.num_ids);
     return true;
@@ -1519,7 +1528,8 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
         if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
         args.partials = nullptr;
         args.tile_table = nullptr;
-        if (args.inner % kBK != 0) workspace = nullptr;  // as mfma_gemm_workspace_size says
+        TableSpace space;
+        if (!table_space(args, space)) workspace = nullptr;
         const bool split = workspace != nullptr && splits_last_round(args);
         args.num_ids = count_ids(args, split);
         if (workspace != nullptr) {

@@ -4,6 +4,7 @@
 import pytest
 import torch
 
+from fast_llm_amd.functional.config import KernelConfig
 from fast_llm_amd.functional.sparse_linear import (
     InputSparseLinear,
     OutputSparseLinear,
@@ -774,3 +775,29 @@ def test_weight_gradients_of_few_rows(sparse_dim, dense_dim, dtype, device):
     added = torch.zeros(len(tokens) * sparse_dim, dense_dim, dtype=dtype, device=device)
     input_row_sparse_matmul(y.t(), x, sparse_map, out=added, accumulate=True)
     assert torch.equal(out[:, :dense_dim], added)
+
+
+# Reductions of no whole number of slices that are cut into pieces (few tiles; 2, 3, 4 and 8 pieces at these tile counts), with
+# the last piece masked, against the unsplit sums that a call without a workspace takes.
+@pytest.mark.parametrize(("experts", "inner", "other"), [(3, 2056, 264), (2, 4104, 2600), (5, 3416, 1280), (16, 2104, 1280), (1, 8200, 72)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_reductions_of_no_whole_number_of_slices(experts, inner, other, dtype, device, monkeypatch):
+    tokens = [(37 * e) % 200 + 1 for e in range(experts)]
+    ends = torch.cumsum((torch.tensor(tokens) + 127) // 128 * 128, 0)
+    oracle_map = fixture_sparse_map({"expert_ends": ends.tolist(), "tokens_per_expert": tokens, "phantom_rows": 0})
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    generator = torch.Generator().manual_seed(inner)
+    x = _normal(oracle_map.num_rows, inner, dtype, generator)
+    weight = _normal(experts * inner, other, dtype, generator)
+    weight_t = _normal(experts * other, inner, dtype, generator)
+    results = []
+    for workspace in (True, False):
+        monkeypatch.setattr(KernelConfig, "grouped_gemm_workspace", workspace)
+        results.append(
+            (input_inner_sparse_matmul(x.to(device), weight.to(device), sparse_map),
+             output_sparse_matmul(x.to(device), weight_t.to(device).t(), sparse_map))
+        )  # fmt: skip
+    expected = (moe_oracle.input_inner_sparse_matmul(x, weight, oracle_map), moe_oracle.output_sparse_matmul(x, weight_t.t(), oracle_map))
+    for split, whole, reference in zip(*results, expected):
+        assert max_rel_err(split.cpu(), reference) <= _MAX_REL[dtype]
+        assert max_rel_err(whole.cpu(), reference) <= _MAX_REL[dtype]
