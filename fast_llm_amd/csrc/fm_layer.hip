@@ -235,10 +235,10 @@ int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     if (layer.grad_weight_1) FM_STEP(step.product(products[Step::kGradWeight1]));
     if (layer.grad_input) FM_STEP(step.combine(layer.grad_layer_2_output, nullptr, layer.grad_input));
     const bool losses = layer.with_losses != 0;
-    FM_STEP(fm_router_backward(layer.grad_scores, step.routing(plan.scores), step.routing(plan.top_experts), layer.logits, layer.noise,
-                               losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
-                               layer.grad_logits, layer.auxiliary_loss_grad, layer.z_loss_grad, layer.tokens,
-                               layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), stream));
+    FM_STEP(router_backward(layer.grad_scores, step.routing(plan.scores), step.routing(plan.top_experts), layer.logits, layer.noise,
+                            losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
+                            layer.grad_logits, layer.auxiliary_loss_grad, layer.z_loss_grad, layer.tokens,
+                            layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), true, stream));
     if (layer.router != nullptr)
         FM_STEP(step.keep(fm_router_linear_backward(layer.grad_logits, layer.input, layer.router, layer.router_input_grad ? layer.grad_input : nullptr, layer.grad_router,
                                                     layer.tokens, layer.routed_experts, layer.hidden, step.dtype(), layer.workspace,

@@ -1,4 +1,5 @@
-// What the router's forward kernel leaves in its workspace, shared with the sparse-map kernels that consume it.
+// What the router's forward kernel leaves in its workspace, shared with the sparse-map kernels that consume it, and the
+// router's backward as the layer calls it.
 #pragma once
 
 #include <stddef.h>
@@ -33,5 +34,12 @@ inline int64_t router_tokens_per_block(int64_t tokens) {
 inline size_t router_counts_bytes(int64_t tokens, int64_t experts) {
     return sizeof(int32_t) * static_cast<size_t>(router_blocks(tokens)) * static_cast<size_t>(experts);
 }
+
+// `fm_router_backward`. With `round_grad_scores` the gradients of the scores are rounded to `dtype` first: the type in which
+// the combine's backward hands them over where the layer runs one call after the other.
+int router_backward(const void *grad_scores, const void *scores, const void *top_experts, const void *logits, const void *noise,
+                    const void *lse, const void *statistics, void *grad_logits, double auxiliary_loss_grad, double z_loss_grad,
+                    int64_t num_tokens, int64_t num_experts, int64_t experts_per_token, int64_t shared_experts, int dtype,
+                    bool round_grad_scores, void *stream);
 
 }  // namespace fm

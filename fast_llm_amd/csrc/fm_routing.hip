@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
     const float *__restrict__ grad_scores, const float *__restrict__ scores, const int64_t *__restrict__ top_experts,
     const T *__restrict__ logits, const T *__restrict__ noise, const float *__restrict__ lse,
     const float *__restrict__ statistics, T *__restrict__ grad_logits, float aux_scale, float z_scale, int64_t tokens,
-    int experts, int k, int shared) {
+    int experts, int k, int shared, bool round_grad_scores) {
     constexpr int kTokens = RouterShape<kGroup, kPerLane>::kTokens;
     const int lane = threadIdx.x & (kGroup - 1), group = (threadIdx.x & 63) / kGroup;
     const int64_t mine = (static_cast<int64_t>(blockIdx.x) * (kRoutingThreads / 64) + (threadIdx.x >> 6)) * kTokens + group;
@@ -331,7 +331,8 @@ __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
     }
     const float lse_routed = with_losses ? lse[2 * token] : 0.f, lse_raw = with_losses ? lse[2 * token + 1] : 0.f;
     const float score = lane < k ? scores[token * slots + shared + lane] : 0.f;
-    const float grad_score = lane < k ? grad_scores[token * slots + shared + lane] : 0.f;
+    float grad_score = lane < k ? grad_scores[token * slots + shared + lane] : 0.f;
+    if (round_grad_scores) grad_score = to_float(from_float<T>(grad_score));
     const int expert = lane < k ? static_cast<int>(top_experts[token * slots + shared + lane]) : -1;
 
     // Load balancing.
@@ -430,7 +431,7 @@ static void launch_router_forward(const void *logits, const void *noise, void *t
 static int run_router_backward(const char *name, const void *grad_scores, const void *scores, const void *top_experts,
                                const void *logits, const void *noise, const void *lse, const void *statistics,
                                void *grad_logits, float aux_scale, float z_scale, int64_t tokens, int experts, int k,
-                               int shared, int dtype, hipStream_t stream) {
+                               int shared, int dtype, bool round_grad_scores, hipStream_t stream) {
     FM_DISPATCH_DTYPE(dtype, T, {
         FM_DISPATCH_ROUTER_SHAPE(experts, kGroup, kPerLane, {
             constexpr int64_t kTokens = RouterShape<kGroup, kPerLane>::kTokens * (kRoutingThreads / 64);
@@ -438,7 +439,7 @@ static int run_router_backward(const char *name, const void *grad_scores, const 
                 static_cast<const float *>(grad_scores), static_cast<const float *>(scores),
                 static_cast<const int64_t *>(top_experts), static_cast<const T *>(logits), static_cast<const T *>(noise),
                 static_cast<const float *>(lse), static_cast<const float *>(statistics), static_cast<T *>(grad_logits),
-                aux_scale, z_scale, tokens, experts, k, shared);
+                aux_scale, z_scale, tokens, experts, k, shared, round_grad_scores);
         })
     });
     return check_launch(name);
@@ -472,7 +473,7 @@ extern "C" int fm_topk_routing_backward(const void *grad_scores, const void *sco
     FM_REQUIRE(grad_scores && scores && top_experts && grad_logits, "%s: null tensor", name);
     return run_router_backward(name, grad_scores, scores, top_experts, nullptr, nullptr, nullptr, nullptr, grad_logits,
                                0.f, 0.f, num_tokens, static_cast<int>(num_experts),
-                               static_cast<int>(experts_per_token), 0, dtype, static_cast<hipStream_t>(stream));
+                               static_cast<int>(experts_per_token), 0, dtype, false, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int fm_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
@@ -508,11 +509,11 @@ extern "C" int fm_router_forward(const void *logits, const void *noise, void *to
     return check_launch(name);
 }
 
-extern "C" int fm_router_backward(const void *grad_scores, const void *scores, const void *top_experts,
-                                  const void *logits, const void *noise, const void *lse, const void *statistics,
-                                  void *grad_logits, double auxiliary_loss_grad, double z_loss_grad,
-                                  int64_t num_tokens, int64_t num_experts, int64_t experts_per_token,
-                                  int64_t shared_experts, int dtype, void *stream_) {
+int fm::router_backward(const void *grad_scores, const void *scores, const void *top_experts, const void *logits,
+                        const void *noise, const void *lse, const void *statistics, void *grad_logits,
+                        double auxiliary_loss_grad, double z_loss_grad, int64_t num_tokens, int64_t num_experts,
+                        int64_t experts_per_token, int64_t shared_experts, int dtype, bool round_grad_scores,
+                        void *stream_) {
     const char *name = "fm_router_backward";
     if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, shared_experts, dtype))
         return status;
@@ -526,5 +527,16 @@ extern "C" int fm_router_backward(const void *grad_scores, const void *scores, c
     const float z_scale = static_cast<float>(2.0 * z_loss_grad / count);
     return run_router_backward(name, grad_scores, scores, top_experts, logits, noise, lse, statistics, grad_logits,
                                aux_scale, z_scale, num_tokens, static_cast<int>(num_experts),
-                               static_cast<int>(experts_per_token), static_cast<int>(shared_experts), dtype, stream);
+                               static_cast<int>(experts_per_token), static_cast<int>(shared_experts), dtype,
+                               round_grad_scores, stream);
+}
+
+extern "C" int fm_router_backward(const void *grad_scores, const void *scores, const void *top_experts,
+                                  const void *logits, const void *noise, const void *lse, const void *statistics,
+                                  void *grad_logits, double auxiliary_loss_grad, double z_loss_grad,
+                                  int64_t num_tokens, int64_t num_experts, int64_t experts_per_token,
+                                  int64_t shared_experts, int dtype, void *stream) {
+    return router_backward(grad_scores, scores, top_experts, logits, noise, lse, statistics, grad_logits,
+                           auxiliary_loss_grad, z_loss_grad, num_tokens, num_experts, experts_per_token, shared_experts,
+                           dtype, false, stream);
 }

@@ -257,7 +257,8 @@ class _MoELayer(torch.autograd.Function):
         if not layer.router_linear and ctx.needs_input_grad[1]:
             grad_router = torch.mm(grad_logits.t(), hidden_states)
         if not layer.router_input_grad and grad_input is not None:
-            grad_input.addmm_(grad_logits, router)
+            # Rounded, then added: what autograd makes of the two gradients where the layer is composed of its parts.
+            grad_input.add_(torch.mm(grad_logits, router))
         return (grad_input, grad_router) + (None,) * 7
 
 

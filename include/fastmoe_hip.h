@@ -369,9 +369,9 @@ int fm_router_linear_backward(const void *grad_logits, const void *input, const 
 /* The layer between the router's logits and its output in one call each way: the entry points above in the order of
  * `MixtureOfExpertMLP._forward_dropless` (fast_llm/layers/decoder/mlp/mixture_of_experts.py:184-213) and `mlp_backward`
  * (fast_llm/functional/triton/mlp.py:314-415), experts padded to 128 rows. fm_moe_layer_route runs the router and the sparse
- * map, fm_moe_layer_forward the rest. Same kernels and results as the single calls, except that the gradient of the scores
- * stays fp32 on its way to the router. All tensors are contiguous device memory of `dtype` unless said otherwise; nothing of
- * a call is kept after it. */
+ * map, fm_moe_layer_forward the rest. Same kernels and results as the single calls: the gradient of the scores, too, is
+ * rounded to `dtype` on its way to the router. All tensors are contiguous device memory of `dtype` unless said otherwise;
+ * nothing of a call is kept after it. */
 typedef struct {
     /* Shape and options, set by the caller. */
     int64_t tokens, hidden, ffn, routed_experts, shared_experts, experts_per_token;

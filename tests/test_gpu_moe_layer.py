@@ -53,8 +53,7 @@ def test_layer_in_two_calls_matches_the_composition(recompute_level, hidden, ffn
     one, composed = _step(layer, batches, False), _step(layer, batches, True)
     for name in ("outputs", "losses", "weight_grads"):
         assert all(torch.equal(a, b) for a, b in zip(one[name], composed[name], strict=True)), name
-    # The gradient of the scores is not rounded on its way to the router and the router's input gradient is added before
-    # the rounding: half a unit in the last place each.
+    # The router's linear layer sums in another order, and in fp32 its input gradient is added as it is summed.
     bound = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}[options["dtype"]]
     for name in ("input_grads", "router_grad"):
         assert all(max_rel_err(a, b) <= bound for a, b in zip(one[name], composed[name], strict=True)), name
@@ -64,6 +63,35 @@ def test_layer_in_two_calls_matches_the_composition(recompute_level, hidden, ffn
         output = layer(x)
         with _lib.KernelTimer():
             assert torch.equal(output, layer(x))
+
+
+# Preferred experts: input feature 0 carries log p_e in the router's weight, so its gradient is the largest of the token's by far,
+# and what is rounded on the way to it shows in single elements.
+@pytest.mark.parametrize("zipf", [0.6, 1.2])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("hidden", "experts", "options"), [
+    (2048, 64, dict(shared_experts=1, recompute_level=MLPRecomputeLevel.full)), (4096, 8, dict()),
+    (2048, 60, dict(jitter_eps=0.1, z_loss_coefficient=0.01)),
+])  # fmt: skip
+def test_layer_in_two_calls_rounds_where_the_composition_does(hidden, experts, options, dtype, zipf, device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(hidden, 512, experts + options.get("shared_experts", 0), 4, dtype=dtype, device=device, **options)
+    probabilities = torch.arange(1, experts + 1, device=device) ** -zipf
+    with torch.no_grad():
+        layer.router[:, 0] = (probabilities / probabilities.sum()).log()
+    x = torch.randn(701, hidden, device=device, dtype=dtype)
+    x[:, 0] = 1
+    results = []
+    for composed in (False, True):
+        torch.manual_seed(1)
+        results.append(_step(layer, [x.requires_grad_()], composed))
+    one, other = results
+    for name in ("outputs", "losses", "weight_grads", "input_grads"):
+        assert all(torch.equal(a, b) for a, b in zip(one[name], other[name], strict=True)), name
+    # The router's weight gradient: sums of the same products in another order, rounded once. A unit in the last place of the
+    # element, and 1e-5 of the largest for the order.
+    a, b = one["router_grad"][0].double(), other["router_grad"][0].double()
+    assert ((a - b).abs() <= torch.finfo(dtype).eps * b.abs() + 1e-5 * b.abs().max()).all()
 
 
 def test_layer_in_two_calls_with_jitter_frozen_weights_and_no_input_gradient(device):
