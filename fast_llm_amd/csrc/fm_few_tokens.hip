@@ -120,6 +120,8 @@ __device__ __forceinline__ void multiply_rows(__amdgpu_buffer_rsrc_t weight, __a
         // The next chunk is on its way while this one is multiplied; past the end it is zeros and touches no memory.
         fetch_rows(k0 + kWaves * kChunk);
         fetch_tokens(k0 + kWaves * kChunk, next);
+        // The lanes read what others wrote: the hardware keeps a wavefront's LDS operations in order, and this the compiler.
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
 #pragma unroll
@@ -128,6 +130,7 @@ __device__ __forceinline__ void multiply_rows(__amdgpu_buffer_rsrc_t weight, __a
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) sums[r][g] = mfma(T(), fragment, now[g][s], sums[r][g]);
             }
+        asm volatile("" ::: "memory");  // and the next chunk's writes stay behind these reads
     };
     fetch_rows(wave * kChunk);
     fetch_tokens(wave * kChunk, tokens[0]);
