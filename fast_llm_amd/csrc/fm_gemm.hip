@@ -10,7 +10,7 @@
 // Half-precision operands with vectorisable layouts go to fm_gemm_mfma.hip, fp32 ones to fm_gemm_f32.hip. Operands with
 // odd strides or sizes, fp32 products with a half-precision result and row-sparse fp32 products of K-contiguous operands
 // go to the two kernels here: a 64 x 64 x 16 LDS-tiled kernel of scalar multiply-adds (half precision) and one of fp32
-// matrix instructions (fp32). Both compute a row block that straddles an expert boundary in one pass per expert, so they
+// matrix instructions on tiles of 128 x 128 or 64 x 64 (fp32). Both compute a row block that straddles an expert boundary in one pass per expert, so they
 // take any padding multiple, and both check every bound.
 #include "fm_gemm_common.h"
 
@@ -42,13 +42,14 @@ constexpr int kGenTile = 64, kGenK = 16, kGenThreads = 256;
 // The work of the tile at (row0, col0) for the expert that owns its row `first_row` (relative to row0): in the
 // products whose rows are grouped by expert, a tile that straddles an expert boundary (any padding multiple is
 // allowed) is computed in one piece per expert.
-__device__ __forceinline__ TileWork resolve_tile(const GemmArgs &args, int64_t row0, int64_t col0, int first_row) {
+__device__ __forceinline__ TileWork resolve_tile(const GemmArgs &args, int64_t row0, int64_t col0, int first_row,
+                                                 int tile_rows = kGenTile) {
     TileWork work;
     work.skip = false;
     work.k_lo = 0;
     work.k_hi = args.inner;
     work.row_lo = first_row;
-    work.row_hi = kGenTile;
+    work.row_hi = tile_rows;
     work.out_offset = row0 * args.out_stride_row + col0 * args.out_stride_col;
     const bool dense = args.expert_ends == nullptr;
     if (args.mode == kInputRowSparse) {
@@ -172,11 +173,13 @@ __global__ __launch_bounds__(kGenThreads) void grouped_gemm_generic_kernel(GemmA
 // one slice ahead and stored to LDS as [k][row], double-buffered, one barrier per slice; several workgroups share a
 // CU. Tiles lie on a fixed grid of kTile rows: one that straddles an expert boundary is computed in one pass per
 // expert, like the generic kernel's, so any padding multiple works (the reference's multiple of 128 gives one pass).
+// Two shapes: 128 x 128 x 16, which reads an operand half as often, and 64 x 64 x 32 for what would leave CUs idle on those
+// (f32_large_tiles).
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gemm_f32x16_t;
-constexpr int kF32Threads = 256;
+constexpr int kF32Threads = 256, kF32LargeTile = 128, kF32SmallTile = 64;
 
+template <int kTile, int kK>
 __global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_any_layout_kernel(GemmArgs args) {
-    constexpr int kTile = kGenTile, kK = 32;
     constexpr int kPitch = kTile + 4;                       // floats per K-row in LDS; +4 spreads the banks
     constexpr int kPerThread = kTile * kK / kF32Threads;    // operand elements per thread and slice
     constexpr int kWaveTile = kTile / 2, kBlocks = kWaveTile / 32;  // a wavefront's part, in 32 x 32 accumulators
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_any_layout_kerne
     const float *lhs_all = static_cast<const float *>(args.lhs), *rhs_all = static_cast<const float *>(args.rhs);
 
     for (int first_row = 0; first_row < rows_here;) {
-        const TileWork work = resolve_tile(args, row0, col0, first_row);
+        const TileWork work = resolve_tile(args, row0, col0, first_row, kTile);
         if (work.skip) return;  // the rest of the tile lies past the last expert
         const int row_hi = work.row_hi < rows_here ? work.row_hi : static_cast<int>(rows_here);
         const float *lhs = lhs_all + work.lhs_offset, *rhs = rhs_all + work.rhs_offset;
@@ -293,6 +296,21 @@ __global__ __launch_bounds__(kF32Threads) void grouped_gemm_f32_any_layout_kerne
 // =========================================================================================================
 // Host dispatch
 // =========================================================================================================
+// Whether an fp32 product of any layout runs on tiles of 128 x 128 instead of 64 x 64. 256 of the large ones, one per CU, take
+// as long as the small ones of 155 (2046 reduction indices) to 180 (510) of them, and there is no large launch between two
+// whole rounds. us, large / small, 8 experts: 1024 tokens, 2 slots, columns x reduction 1282 x 2046 277 / 400, 1666 x 2046 543 /
+// 500, 2050 x 2046 547 / 599, 3074 x 2046 559 / 802, 1666 x 510 181 / 145, 2050 x 510 183 / 173, 3074 x 510 194 / 231; 4096
+// tokens 3074 x 2046 1909 / 2692, 514 x 2046 546 / 504.
+static bool f32_large_tiles(const GemmArgs &args) {
+    if (args.mode == kInputRowSparse && args.num_experts > 1 && args.sparse_size % kF32LargeTile != 0) return false;
+    const int64_t tiles_m = (args.rows + kF32LargeTile - 1) / kF32LargeTile, tiles_n = (args.cols + kF32LargeTile - 1) / kF32LargeTile;
+    // Buffers of a map have room for a whole tile of padding per expert, of which half is expected to be in use.
+    const bool padded = args.mode != kInputRowSparse && args.expert_ends != nullptr;
+    const int64_t tiles = max(tiles_m - (padded ? args.num_experts / 2 : 0), int64_t(1)) * tiles_n;
+    constexpr int64_t kCus = 256, kSmallPerRound = 165;
+    return (tiles + kCus - 1) / kCus * kSmallPerRound <= tiles;
+}
+
 int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace, size_t workspace_size, void *stream_) {
     FM_REQUIRE(valid_dtype(dtype) && valid_dtype(args.out_dtype), "%s: bad dtype", name);
     FM_REQUIRE(valid_index_dtype(args.index_dtype), "%s: bad index_dtype %d", name, args.index_dtype);
@@ -317,12 +335,15 @@ int run_gemm(const char *name, GemmArgs args, int dtype, void *workspace, size_t
         if (args.mode == kInputRowSparse && args.num_experts > 1 && args.sparse_size % kGenTile != 0)
             return fail(FM_ERR_UNSUPPORTED, "%s: row_sparse_dim=%lld must be a multiple of %d", name,
                         (long long)args.sparse_size, kGenTile);
-        constexpr int tile = kGenTile;
+        const bool large = dtype == FM_DTYPE_F32 && f32_large_tiles(args);
+        const int tile = large ? kF32LargeTile : kGenTile;
         args.tiles_m = static_cast<int>((args.rows + tile - 1) / tile);
         args.tiles_n = static_cast<int>((args.cols + tile - 1) / tile);
         FM_REQUIRE(static_cast<int64_t>(args.tiles_m) * args.tiles_n < (int64_t(1) << 31), "%s: too many tiles", name);
         const int grid = args.tiles_m * args.tiles_n;
-        if (dtype == FM_DTYPE_F32) grouped_gemm_f32_any_layout_kernel<<<grid, kF32Threads, 0, stream>>>(args);
+        static_assert(kF32SmallTile == kGenTile, "one grid for both kernels");
+        if (large) grouped_gemm_f32_any_layout_kernel<kF32LargeTile, 16><<<grid, kF32Threads, 0, stream>>>(args);
+        else if (dtype == FM_DTYPE_F32) grouped_gemm_f32_any_layout_kernel<kF32SmallTile, 32><<<grid, kF32Threads, 0, stream>>>(args);
         else if (dtype == FM_DTYPE_BF16) grouped_gemm_generic_kernel<bf16_t><<<grid, kGenThreads, 0, stream>>>(args);
         else grouped_gemm_generic_kernel<f16_t><<<grid, kGenThreads, 0, stream>>>(args);
     }

@@ -615,6 +615,37 @@ def test_fp32_tiles_and_remainders(inner, other, device):
     assert max_rel_err(dense.cpu(), weight.cpu() @ weight_inner[:inner].cpu()) <= 1e-5
 
 
+# fp32 operands of odd sizes, K-contiguous row-sparse ones and a half-precision result, in launches of more than 165 tiles of 128 x
+# 128, with expert boundaries on and off the tiles' grid.
+@pytest.mark.parametrize("pad", [128, 8])
+@pytest.mark.parametrize("other", [1282, 1666])
+def test_fp32_products_of_any_layout_in_large_launches(pad, other, device):
+    tokens = [500, 0, 129, 871, 700]
+    ends = torch.cumsum((torch.tensor(tokens) + pad - 1) // pad * pad, 0)
+    oracle_map = fixture_sparse_map({"expert_ends": ends.tolist(), "tokens_per_expert": tokens})
+    oracle_map.num_rows = int(ends[-1]) + 128
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    used, padding = _used_rows(oracle_map), ~oracle_map.real_row_mask()
+    generator = torch.Generator().manual_seed(other)
+    x = _normal(oracle_map.num_rows, 70, torch.float32, generator)
+    weight = _normal(5 * other, 70, torch.float32, generator)
+    out = output_sparse_matmul(x.to(device), weight.to(device).t(), sparse_map)
+    expected = moe_oracle.output_sparse_matmul(x.double(), weight.t().double(), oracle_map)
+    assert max_rel_err(out[:used].cpu(), expected[:used]) <= _MAX_REL[torch.float32]
+    weight = _normal(5 * 70, other, torch.float32, generator)
+    out = input_inner_sparse_matmul(x.to(device), weight.to(device), sparse_map)
+    expected = moe_oracle.input_inner_sparse_matmul(x.double(), weight.double(), oracle_map)
+    assert max_rel_err(out[:used].cpu(), expected[:used]) <= _MAX_REL[torch.float32]
+    y, z = (_normal(oracle_map.num_rows, size, torch.float32, generator) for size in (384, other))
+    expected = moe_oracle.input_row_sparse_matmul(y.t().double(), z.double(), oracle_map)
+    y[padding] = z[padding] = float("nan")
+    along_k = [t.t().contiguous().to(device).t() for t in (y, z)]
+    assert max_rel_err(input_row_sparse_matmul(along_k[0].t(), along_k[1], sparse_map).cpu(), expected) <= _MAX_REL[torch.float32]
+    out = torch.empty(expected.shape, dtype=torch.bfloat16, device=device)
+    input_row_sparse_matmul(y.to(device).t(), z.to(device), sparse_map, out=out)
+    assert max_rel_err(out.cpu(), expected) <= _MAX_REL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("inner", [8, 56, 72, 120, 136, 1000, 2104])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_reductions_of_no_whole_number_of_slices(inner, dtype, device):
