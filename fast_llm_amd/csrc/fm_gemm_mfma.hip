@@ -391,6 +391,22 @@ constexpr int kMinPieceSlices = 16;        // do not cut a reduction into pieces
 constexpr int kPieceOverheadSlices = 17;
 constexpr int kPartialFloats = kTile * kTile;
 
+// Slices per piece of a reduction cut into `split` pieces (even: slices are multiplied in pairs; the last piece may have fewer),
+// 0 if they would be too short.
+__host__ __device__ inline int piece_slices(int num_slices, int split) {
+    if (num_slices / split < kMinPieceSlices) return 0;
+    return ((num_slices + split - 1) / split + 1) / 2 * 2;
+}
+
+// Whether plan_split can find a cut worth its cost, whatever the number of tiles: 36 slices, 38 and more.
+inline bool can_split(int num_slices) {
+    for (int split : {2, 3, 4, 8}) {
+        const int length = piece_slices(num_slices, split);
+        if (length > 0 && length + kPieceOverheadSlices < num_slices) return true;
+    }
+    return false;
+}
+
 struct SplitPlan {
     int tiles_m;       // row tiles that exist
     int whole;         // logical tiles [0, whole) are computed by one workgroup each
@@ -431,8 +447,8 @@ __device__ __forceinline__ SplitPlan plan_split(const GemmArgs &args, bool with_
     if (plan.tail > 0 && with_pieces) {
 #pragma unroll
         for (int split : {2, 3, 4, 8}) {
-            if (plan.tail * split > kMaxPartials || num_slices / split < kMinPieceSlices) continue;
-            const int length = ((num_slices + split - 1) / split + 1) / 2 * 2;  // even: slices are multiplied in pairs
+            const int length = piece_slices(num_slices, split);
+            if (plan.tail * split > kMaxPartials || length == 0) continue;
             const int pieces = (num_slices + length - 1) / length;
             const int cost = (plan.tail * pieces + kRound - 1) / kRound * (length + kPieceOverheadSlices);
             if (cost < best) {
@@ -1425,7 +1441,7 @@ static bool too_many_tiles(const GemmArgs &args) {
 static bool splits_last_round(const GemmArgs &args) {
     constexpr int kMaxRoundsToSplit = 16;
     const int64_t most = args.inner % kBK == 0 ? kMaxRoundsToSplit * kRound : kRound * 3 / 4;
-    return args.fusion == kFusionNone && args.mode != kInputRowSparse && (args.inner + kBK - 1) / kBK >= 2 * kMinPieceSlices &&
+    return args.fusion == kFusionNone && args.mode != kInputRowSparse && can_split(static_cast<int>((args.inner + kBK - 1) / kBK)) &&
            static_cast<int64_t>(args.tiles_m) * args.tiles_n <= most;
 }
 

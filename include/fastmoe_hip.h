@@ -254,9 +254,9 @@ int fm_mlp_activation_backward(const void *grad_output, void *grad_input, const 
  * (`fm_input_row_sparse_matmul_workspace_size(...)` for the row-sparse product). With it, a small kernel first writes
  * where every tile of the launch lies, so that the workgroups of the product look their tiles up instead of each
  * scanning the expert map (same tiles, same results); and a launch of few, long tiles (at most 16 rounds of 256
- * tiles of 256 x 256, reduction of 2048 or more; 192 tiles where it is no multiple of 64) of the output-sparse and
- * input-inner-sparse products, which would
- * leave most CUs idle in its last round, cuts the reductions of that round's tiles into 2, 3, 4 or 8 pieces that fill
+ * tiles of 256 x 256, 192 tiles where the reduction is no multiple of 64; a reduction of 36, 38 or more 64-element
+ * slices) of the output-sparse and input-inner-sparse products, which would leave most
+ * CUs idle in its last round, cuts the reductions of that round's tiles into 2, 3, 4 or 8 pieces that fill
  * the CUs and adds the pieces in piece order. Whether that split happens depends on the dimensions and on whether a
  * workspace is passed, on nothing else (not on the stream, the device's free memory or earlier calls): NULL with
  * size 0 selects the unsplit sums, which differ from the split ones in the last bits; a non-null workspace smaller

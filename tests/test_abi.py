@@ -174,3 +174,24 @@ def test_layer_sizes_come_from_the_shape_alone(library, hidden, ffn, tokens, dty
         _lib.check(library.fm_moe_layer_sizes(ctypes.byref(layer)))
         sizes.add((layer.rows, layer.routing_bytes, layer.workspace_bytes))
     assert len(sizes) == 1
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+def test_space_for_pieces_only_where_a_reduction_can_be_cut(library, dtype):
+    """A cut costs 17 slices over its multiplications and its pieces have an even number of slices, 16 or more: fewer than 36
+    slices, and 37, are never cut. A launch that cannot be cut reserves no space for pieces and launches nothing to add them."""
+    partials = 512 * 256 * 256 * 4
+    rows, columns, experts = 1024, 512, 8  # few tiles: what is left to decide is the reduction
+
+    def cuts(inner):
+        return library.fm_grouped_gemm_workspace_size(rows, columns, inner, experts, dtype) >= partials
+
+    def worth_it(slices):
+        lengths = [(-(-slices // split) + 1) // 2 * 2 for split in (2, 3, 4, 8) if slices // split >= 16]
+        return any(length + 17 < slices for length in lengths)
+
+    assert [slices for slices in range(1, 300) if worth_it(slices)] == [36, *range(38, 300)]
+    for slices in range(1, 300):
+        assert cuts(64 * slices) == worth_it(slices), slices
+        if slices > 1:
+            assert cuts(64 * slices - 8) == worth_it(slices), slices
