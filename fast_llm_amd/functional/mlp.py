@@ -410,7 +410,9 @@ def few_tokens_forward(
     ffn = weight_2.size(0) // num_experts
     size = _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), dtype)
     tensors = (input_, top_experts, scores, weight_1, weight_2)
-    if size == 0 or weight_1.dtype != input_.dtype or weight_2.dtype != input_.dtype or weight_2.size(1) != hidden:
+    if size == 0 or weight_1.dtype != input_.dtype or weight_2.dtype != input_.dtype:
+        return None
+    if tuple(weight_2.shape) != (num_experts * ffn, hidden):  # the products of the sparse layout refuse it
         return None
     if top_experts.dtype != torch.int64 or not all(tensor.is_contiguous() for tensor in tensors):
         return None

@@ -5,6 +5,7 @@ import torch
 
 from fast_llm_amd.functional import mlp
 from fast_llm_amd.functional.config import ActivationType
+from fast_llm_amd.layers.moe import DroplessMoEMLP
 from oracle import moe_oracle
 from tests.helpers import max_rel_err
 
@@ -62,3 +63,11 @@ def test_few_tokens_forward_leaves_the_rest_to_the_sparse_layout(device):
     limit = mlp.FEW_TOKENS_MAX_ROWS_PER_EXPERT * 2
     assert call(limit) is not None and call(limit + 1) is None
     assert call(4, torch.float32) is None and call(4, ffn=60) is None
+
+
+def test_few_tokens_refuse_a_weight_that_does_not_fit(device):
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device).eval()
+    x = torch.randn(16, 64, device=device, dtype=torch.bfloat16)
+    layer.layer_2 = torch.nn.Parameter(torch.cat([layer.layer_2.detach(), layer.layer_2.detach()[:4]]))
+    with torch.no_grad(), pytest.raises((AssertionError, ValueError)):
+        layer(x)
