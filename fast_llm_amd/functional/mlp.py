@@ -383,9 +383,31 @@ def mlp_backward(grad_output: torch.Tensor, context: list[typing.Any]) -> tuple[
 mlp_autograd = wrap_forward_backward(mlp_forward, mlp_backward)
 
 
-def few_tokens_expected(rows: int, num_experts: int, dtype: torch.dtype) -> bool:
-    """Whether `few_tokens_forward` is the faster way for so many (token, slot) pairs."""
-    return rows <= FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts and dtype in (torch.bfloat16, torch.float16)
+def few_tokens_supported(
+    input_: torch.Tensor, slots: int, weight_1: torch.Tensor, weight_2: torch.Tensor, num_experts: int, gated: bool
+) -> bool:
+    """Whether the kernels for few tokens are the faster way for `slots` experts per row of `input_` and take these operands:
+    half precision, contiguous, 16-byte aligned, of sizes that fit together and that the library accepts. Everything else
+    runs in the sparse layout, which also refuses what does not fit."""
+    dtype, ffn = input_.dtype, weight_2.size(0) // num_experts
+    if input_.dim() != 2 or input_.size(0) * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts:
+        return False
+    tokens, hidden = input_.shape
+    return (
+        dtype in (torch.bfloat16, torch.float16)
+        and weight_1.dtype == weight_2.dtype == dtype
+        and weight_1.shape == (num_experts * ffn * (2 if gated else 1), hidden)
+        and weight_2.shape == (num_experts * ffn, hidden)
+        and all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in (input_, weight_1, weight_2))
+        and _few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, gated, dtype) > 0
+    )
+
+
+def _few_tokens_workspace_size(
+    tokens: int, slots: int, hidden: int, ffn: int, num_experts: int, gated: bool, dtype: torch.dtype
+) -> int:
+    """0: sizes that the kernels do not take."""
+    return _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), _lib.dtype_tag(dtype))
 
 
 def few_tokens_forward(
@@ -401,35 +423,26 @@ def few_tokens_forward(
     """
     `mlp_forward(..., training=False)` of `input_` [tokens, hidden] straight from the routing (`scores` and `top_experts`
     [tokens, k], no sparse map) by the kernels for few tokens, weights in the layouts of the sparse MLP. None where they
-    are not the faster way or do not take the operands.
+    are not the faster way or do not take the operands (`few_tokens_supported`, and contiguous `scores` and `top_experts`).
     """
     tokens, slots = top_experts.shape
-    if not few_tokens_expected(tokens * slots, num_experts, input_.dtype):
+    if not few_tokens_supported(input_, slots, weight_1, weight_2, num_experts, gated):
         return None
-    hidden, dtype = input_.size(1), _lib.dtype_tag(input_.dtype)
-    ffn = weight_2.size(0) // num_experts
-    size = _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), dtype)
-    tensors = (input_, top_experts, scores, weight_1, weight_2)
-    if size == 0 or weight_1.dtype != input_.dtype or weight_2.dtype != input_.dtype:
+    if top_experts.dtype != torch.int64 or not top_experts.is_contiguous() or not scores.is_contiguous():
         return None
-    if tuple(weight_2.shape) != (num_experts * ffn, hidden):  # the products of the sparse layout refuse it
-        return None
-    if top_experts.dtype != torch.int64 or not all(tensor.is_contiguous() for tensor in tensors):
-        return None
-    if any(tensor.data_ptr() % 16 != 0 for tensor in (input_, weight_1, weight_2)):
-        return None
-    device = _lib.require_device(*tensors)
-    Assert.eq(tuple(weight_1.shape), (num_experts * ffn * (2 if gated else 1), hidden))
+    device = _lib.require_device(input_, top_experts, scores, weight_1, weight_2)
     Assert.eq(input_.size(0), tokens)
     Assert.eq(scores.shape, top_experts.shape)
     if scores.dtype != torch.float32:
         scores = scores.float()
+    hidden, ffn = input_.size(1), weight_2.size(0) // num_experts
+    size = _few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, gated, input_.dtype)
     output = torch.empty_like(input_)
     workspace = torch.empty(size, dtype=torch.uint8, device=device)
     _lib.call(
         "fm_few_tokens_forward", device, input_.data_ptr(), top_experts.data_ptr(), scores.data_ptr(), weight_1.data_ptr(),
         weight_2.data_ptr(), output.data_ptr(), tokens, slots, hidden, ffn, num_experts, int(gated),
-        _activation_tag(activation_type), dtype, workspace.data_ptr(), size,
+        _activation_tag(activation_type), _lib.dtype_tag(input_.dtype), workspace.data_ptr(), size,
     )  # fmt: skip
     return output
 

@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from fast_llm_amd import _lib
 from fast_llm_amd.functional import mlp
 from fast_llm_amd.functional.config import ActivationType
 from fast_llm_amd.layers.moe import DroplessMoEMLP
@@ -71,3 +72,28 @@ def test_few_tokens_refuse_a_weight_that_does_not_fit(device):
     layer.layer_2 = torch.nn.Parameter(torch.cat([layer.layer_2.detach(), layer.layer_2.detach()[:4]]))
     with torch.no_grad(), pytest.raises((AssertionError, ValueError)):
         layer(x)
+
+
+# The kernels take 4096 (token, slot) pairs, sizes that are multiples of 8 and aligned, contiguous inputs: what they do not take
+# goes through the layer in two calls, not one launch at a time.
+@pytest.mark.parametrize(("tokens", "ffn", "odd", "expected"), [
+    (512, 64, None, "fm_few_tokens_forward"), (513, 64, None, "fm_moe_layer_forward"), (641, 64, None, "fm_moe_layer_forward"),
+    (16, 60, None, "fm_moe_layer_forward"), (16, 64, "address", "fm_moe_layer_forward"), (16, 64, "strides", "fm_moe_layer_forward"),
+])  # fmt: skip
+def test_inference_takes_one_of_two_routes(tokens, ffn, odd, expected, device, monkeypatch):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, ffn, 128, 8, device=device).eval()
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
+    if odd == "address":
+        x = torch.empty(tokens * 64 + 1, device=device, dtype=torch.bfloat16)[1:].view(tokens, 64).copy_(x)
+    elif odd == "strides":
+        x = x.t().contiguous().t()
+    calls, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args, **kwargs: (calls.append(name), call(name, *args, **kwargs)))
+    with torch.no_grad():
+        output = layer(x)
+        assert calls[-1] == expected
+        scores, top_experts = layer.route(x)
+        operands = (t.cpu() for t in (x, scores, top_experts, layer.layer_1, layer.layer_2))
+        reference = _expected(*operands, 128, True, ActivationType.silu)
+    assert max_rel_err(output.cpu(), reference) <= _MAX_REL[torch.bfloat16]
