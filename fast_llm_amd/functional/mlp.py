@@ -28,10 +28,17 @@ from fast_llm_amd.functional.sparse_copy import (
 from fast_llm_amd.functional.sparse_linear import output_sparse_matmul
 from fast_llm_amd.functional.utils import Assert, wrap_forward_backward
 
-# Up to this many rows per expert, on average, inference takes the kernels for few tokens (`few_tokens_forward`). us there /
-# with a sparse layout: 2 of 8 experts, 4096 x 14336: 32 rows 621 / 708, 48 rows 709 / 718, 64 rows 1025 / 714; 6 of 64
-# experts, 2048 x 1408: 24 rows 272 / 341, 36 rows 325 / 343; 2 of 16 experts, 1024 x 4096: 48 rows 163 / 180.
+# The kernels for few tokens (`few_tokens_forward`) read an expert's weights again for every 16 to 64 of its rows; past this many
+# rows per expert, on average, they are never the faster way.
 FEW_TOKENS_MAX_ROWS_PER_EXPERT = 40
+# Where the layer stops taking them, in rows per expert of (a layer without, with shared experts). The host knows the mean only:
+# an expert that is preferred, or shared by all tokens, has many times as many rows, and its passes are as long a tail as it has
+# few workgroups to share them (ffn / 32). us there / in the sparse layout (layer in two calls), routing unbiased and by a Zipf law
+# with exponent 1.2: 2 of 8 experts, 4096 x 14336, 20 rows 525 / 645, 599 / 645, 40 rows 702 / 651, 742 / 659; with a shared expert 20
+# rows 653 / 719, 701 / 719, 40 rows 811 / 731, 869 / 730; 6 of 64, 2048 x 1408, 20 rows 269 / 297, 376 / 296, 24 rows 294 / 298, 415 / 299;
+# with a shared expert 10 rows 311 / 316, 356 / 315, 20 rows 396 / 327, 427 / 325; 8 of 128, 2048 x 768, 20 rows 316 / 334, 413 / 365;
+# with a shared expert 10 rows 356 / 383, 419 / 383, 20 rows 443 / 392, 509 / 381; 2 of 16, 1024 x 4096, 30 rows 144 / 164, 165 / 171.
+FEW_TOKENS_ROWS_NARROW, FEW_TOKENS_ROWS_WIDE, FEW_TOKENS_WIDE_FFN = (20, 10), (32, 24), 2048
 
 
 def _activation_tag(activation_type: ActivationType | str) -> int:
@@ -383,30 +390,30 @@ def mlp_backward(grad_output: torch.Tensor, context: list[typing.Any]) -> tuple[
 mlp_autograd = wrap_forward_backward(mlp_forward, mlp_backward)
 
 
-def few_tokens_supported(
+def few_tokens_expected(tokens: int, slots: int, shared_experts: int, num_experts: int, ffn: int) -> bool:
+    """Whether a layer whose tokens visit `slots` experts, the shared ones among them, is to take `few_tokens_forward`."""
+    limits = FEW_TOKENS_ROWS_WIDE if ffn >= FEW_TOKENS_WIDE_FFN else FEW_TOKENS_ROWS_NARROW
+    return tokens * slots <= limits[shared_experts > 0] * num_experts
+
+
+def few_tokens_workspace_size(
     input_: torch.Tensor, slots: int, weight_1: torch.Tensor, weight_2: torch.Tensor, num_experts: int, gated: bool
-) -> bool:
-    """Whether the kernels for few tokens are the faster way for `slots` experts per row of `input_` and take these operands:
-    half precision, contiguous, 16-byte aligned, of sizes that fit together and that the library accepts. Everything else
-    runs in the sparse layout, which also refuses what does not fit."""
-    dtype, ffn = input_.dtype, weight_2.size(0) // num_experts
-    if input_.dim() != 2 or input_.size(0) * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts:
-        return False
-    tokens, hidden = input_.shape
-    return (
-        dtype in (torch.bfloat16, torch.float16)
-        and weight_1.dtype == weight_2.dtype == dtype
-        and weight_1.shape == (num_experts * ffn * (2 if gated else 1), hidden)
-        and weight_2.shape == (num_experts * ffn, hidden)
-        and all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in (input_, weight_1, weight_2))
-        and _few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, gated, dtype) > 0
-    )
-
-
-def _few_tokens_workspace_size(
-    tokens: int, slots: int, hidden: int, ffn: int, num_experts: int, gated: bool, dtype: torch.dtype
 ) -> int:
-    """0: sizes that the kernels do not take."""
+    """Bytes that the kernels for few tokens need for `slots` experts per row of `input_`. 0 where they cannot be the faster way
+    or do not take these operands: half precision, contiguous, 16-byte aligned, of sizes that fit together and that the library
+    accepts. Everything else runs in the sparse layout, which also refuses what does not fit."""
+    dtype, ffn = input_.dtype, weight_2.size(0) // num_experts
+    if dtype not in (torch.bfloat16, torch.float16) or input_.dim() != 2:
+        return 0
+    tokens, hidden = input_.shape
+    if (
+        tokens * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts
+        or not weight_1.dtype == weight_2.dtype == dtype
+        or weight_1.shape != (num_experts * ffn * (2 if gated else 1), hidden)
+        or weight_2.shape != (num_experts * ffn, hidden)
+        or not all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in (input_, weight_1, weight_2))
+    ):
+        return 0
     return _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), _lib.dtype_tag(dtype))
 
 
@@ -419,14 +426,19 @@ def few_tokens_forward(
     num_experts: int,
     gated: bool,
     activation_type: ActivationType,
+    workspace_size: int | None = None,
 ) -> torch.Tensor | None:
     """
     `mlp_forward(..., training=False)` of `input_` [tokens, hidden] straight from the routing (`scores` and `top_experts`
     [tokens, k], no sparse map) by the kernels for few tokens, weights in the layouts of the sparse MLP. None where they
-    are not the faster way or do not take the operands (`few_tokens_supported`, and contiguous `scores` and `top_experts`).
+    are not the faster way or do not take the operands (`few_tokens_workspace_size`, which a caller that has asked already
+    passes on, and contiguous `scores` and `top_experts`).
     """
     tokens, slots = top_experts.shape
-    if not few_tokens_supported(input_, slots, weight_1, weight_2, num_experts, gated):
+    size = workspace_size
+    if size is None:
+        size = few_tokens_workspace_size(input_, slots, weight_1, weight_2, num_experts, gated)
+    if size == 0:
         return None
     if top_experts.dtype != torch.int64 or not top_experts.is_contiguous() or not scores.is_contiguous():
         return None
@@ -436,7 +448,6 @@ def few_tokens_forward(
     if scores.dtype != torch.float32:
         scores = scores.float()
     hidden, ffn = input_.size(1), weight_2.size(0) // num_experts
-    size = _few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, gated, input_.dtype)
     output = torch.empty_like(input_)
     workspace = torch.empty(size, dtype=torch.uint8, device=device)
     _lib.call(

@@ -11,7 +11,7 @@ Weight layout as in the reference: `layer_1.weight` [experts * 2 * ffn, hidden] 
 import torch
 
 from fast_llm_amd.functional.config import ActivationType, MLPRecomputeLevel
-from fast_llm_amd.functional.mlp import few_tokens_forward, few_tokens_supported, mlp_autograd
+from fast_llm_amd.functional.mlp import few_tokens_expected, few_tokens_forward, few_tokens_workspace_size, mlp_autograd
 from fast_llm_amd.functional.moe_layer import MoELayerOptions, moe_layer, moe_layer_supported
 from fast_llm_amd.functional.sparse_copy import get_sparse_map
 
@@ -171,10 +171,14 @@ class DroplessMoEMLP(torch.nn.Module):
         """`scores`/`top_experts` may be passed to bypass the router (tests pin the routing that way)."""
         hidden_states = input_.flatten(0, -2)
         router_counts = None
-        slots = self.shared_experts + self.experts_per_token if top_experts is None else top_experts.size(-1)
-        few_tokens = not self.training and few_tokens_supported(
-            hidden_states, slots, self.layer_1, self.layer_2, self.experts, self.gated
-        )
+        few_tokens = 0  # bytes that the kernels for few tokens need, where they are the route
+        if not self.training:
+            slots = self.shared_experts + self.experts_per_token if top_experts is None else top_experts.size(-1)
+            ffn = self.layer_2.size(0) // self.experts
+            if few_tokens_expected(hidden_states.size(0), slots, self.shared_experts, self.experts, ffn):
+                few_tokens = few_tokens_workspace_size(
+                    hidden_states, slots, self.layer_1, self.layer_2, self.experts, self.gated
+                )
         if top_experts is None and not few_tokens and self._is_one_call(hidden_states):
             return self._forward_in_one_call(hidden_states, grad_scale, losses).view_as(input_)
         if top_experts is None:
@@ -182,7 +186,7 @@ class DroplessMoEMLP(torch.nn.Module):
             scores, top_experts, router_counts = self.route_with_counts(hidden_states, grad_scale, losses)
         if few_tokens and scores is not None:
             output = few_tokens_forward(
-                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation
+                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation, few_tokens
             )  # fmt: skip
             if output is not None:
                 return without_backward(output).view_as(input_)

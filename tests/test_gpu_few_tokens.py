@@ -77,7 +77,8 @@ def test_few_tokens_refuse_a_weight_that_does_not_fit(device):
 # The kernels take 4096 (token, slot) pairs, sizes that are multiples of 8 and aligned, contiguous inputs: what they do not take
 # goes through the layer in two calls, not one launch at a time.
 @pytest.mark.parametrize(("tokens", "ffn", "odd", "expected"), [
-    (512, 64, None, "fm_few_tokens_forward"), (513, 64, None, "fm_moe_layer_forward"), (641, 64, None, "fm_moe_layer_forward"),
+    (320, 64, None, "fm_few_tokens_forward"), (321, 64, None, "fm_moe_layer_forward"),  # 20 rows per expert
+    (512, 2048, None, "fm_few_tokens_forward"), (513, 2048, None, "fm_moe_layer_forward"), (641, 64, None, "fm_moe_layer_forward"),
     (16, 60, None, "fm_moe_layer_forward"), (16, 64, "address", "fm_moe_layer_forward"), (16, 64, "strides", "fm_moe_layer_forward"),
 ])  # fmt: skip
 def test_inference_takes_one_of_two_routes(tokens, ffn, odd, expected, device, monkeypatch):
@@ -97,3 +98,14 @@ def test_inference_takes_one_of_two_routes(tokens, ffn, odd, expected, device, m
         operands = (t.cpu() for t in (x, scores, top_experts, layer.layer_1, layer.layer_2))
         reference = _expected(*operands, 128, True, ActivationType.silu)
     assert max_rel_err(output.cpu(), reference) <= _MAX_REL[torch.bfloat16]
+
+
+def test_layers_with_a_shared_expert_leave_the_few_token_kernels_sooner(device, monkeypatch):
+    """A shared expert has a row for every token, many times the mean, and its weights are read again for each 16 to 64."""
+    layer = DroplessMoEMLP(64, 64, 17, 2, shared_experts=1, device=device).eval()
+    calls, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args, **kwargs: (calls.append(name), call(name, *args, **kwargs)))
+    with torch.no_grad():
+        for tokens, expected in ((56, "fm_few_tokens_forward"), (57, "fm_moe_layer_forward")):  # 10 rows per expert
+            layer(torch.randn(tokens, 64, device=device, dtype=torch.bfloat16))
+            assert calls[-1] == expected
