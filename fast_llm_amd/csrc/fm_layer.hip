@@ -162,7 +162,7 @@ void plan_workspace(const fm_moe_layer &layer, Plan &plan) {
 
 int route(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     Step step{layer, plan, stream};
-    FM_REQUIRE(layer.logits && layer.routing && layer.workspace, "fm_moe_layer_forward: null tensor");
+    FM_REQUIRE(layer.logits && layer.routing && layer.workspace, "fm_moe_layer_route: null tensor");
     const bool losses = layer.with_losses != 0;
     FM_STEP(fm_router_forward(layer.logits, layer.noise, step.routing(plan.top_experts), step.routing(plan.scores),
                               losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
@@ -266,26 +266,36 @@ extern "C" int fm_moe_layer_sizes(fm_moe_layer *layer) {
     return FM_OK;
 }
 
-extern "C" int fm_moe_layer_route(const fm_moe_layer *layer, void *stream) {
-    Plan plan;
-    FM_REQUIRE(layer, "fm_moe_layer_route: null");
+// The plan of a call, and that the caller's buffers are of the sizes which fm_moe_layer_sizes gave it for this very shape: the
+// parts are told how large they are, so none of them would notice.
+static int plan_call(const char *name, const fm_moe_layer *layer, Plan &plan) {
+    FM_REQUIRE(layer, "%s: null", name);
     if (int status = make_plan(*layer, plan)) return status;
     plan_workspace(*layer, plan);
+    FM_REQUIRE(layer->rows == plan.rows && layer->routing_bytes >= static_cast<int64_t>(plan.routing_bytes) &&
+                   layer->workspace_bytes >= static_cast<int64_t>(plan.workspace_bytes),
+               "%s: %lld rows, %lld bytes of routing and %lld of workspace, needs %lld, %zu and %zu (fm_moe_layer_sizes, after the last "
+               "change of the shape)", name, static_cast<long long>(layer->rows), static_cast<long long>(layer->routing_bytes),
+               static_cast<long long>(layer->workspace_bytes), static_cast<long long>(plan.rows), plan.routing_bytes, plan.workspace_bytes);
+    FM_REQUIRE(reinterpret_cast<uintptr_t>(layer->routing) % 64 == 0 && reinterpret_cast<uintptr_t>(layer->workspace) % 64 == 0,
+               "%s: routing and workspace must be 64-byte aligned", name);
+    return FM_OK;
+}
+
+extern "C" int fm_moe_layer_route(const fm_moe_layer *layer, void *stream) {
+    Plan plan;
+    if (int status = plan_call("fm_moe_layer_route", layer, plan)) return status;
     return route(*layer, plan, stream);
 }
 
 extern "C" int fm_moe_layer_forward(const fm_moe_layer *layer, void *stream) {
     Plan plan;
-    FM_REQUIRE(layer, "fm_moe_layer_forward: null");
-    if (int status = make_plan(*layer, plan)) return status;
-    plan_workspace(*layer, plan);
+    if (int status = plan_call("fm_moe_layer_forward", layer, plan)) return status;
     return forward(*layer, plan, stream);
 }
 
 extern "C" int fm_moe_layer_backward(const fm_moe_layer *layer, void *stream) {
     Plan plan;
-    FM_REQUIRE(layer, "fm_moe_layer_backward: null");
-    if (int status = make_plan(*layer, plan)) return status;
-    plan_workspace(*layer, plan);
+    if (int status = plan_call("fm_moe_layer_backward", layer, plan)) return status;
     return backward(*layer, plan, stream);
 }

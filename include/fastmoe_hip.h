@@ -382,11 +382,12 @@ typedef struct {
     double auxiliary_loss_grad, z_loss_grad;                          /* as fm_router_backward */
     int64_t dynamic_rows; /* sparse rows; 0: the static worst case. Known after fm_moe_layer_route: what it leaves in
                            * `routing` at used_rows_offset (`index_dtype`) */
-    /* Set by fm_moe_layer_sizes: sparse rows, bytes of the two untyped buffers below, and where the map's last expert ends. */
+    /* Set by fm_moe_layer_sizes: sparse rows, bytes of the two untyped buffers below, and where the map's last expert ends. The
+     * other calls refuse a struct whose shape has changed since (FM_ERR_INVALID_ARGUMENT). */
     int64_t rows, routing_bytes, workspace_bytes, index_dtype /* fm_index_dtype */, used_rows_offset;
     int64_t router_linear; /* whether fm_router_linear_backward takes the shape */
     /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned, kept for the
-     * backward) starts with the two losses (fp32) if there are losses; `workspace` is free again after the call.
+     * backward) starts with the two losses (fp32) if there are losses; `workspace` (64-byte aligned) is free again after the call.
      * layer_1_output [rows, ffn * (2 if gated)] may be null where the backward recomputes it or does not follow: layer 1
      * then runs with the gated activation in its epilogue, FM_ERR_UNSUPPORTED if it cannot. */
     const void *logits, *noise, *input, *weight_1, *weight_2;

@@ -195,3 +195,34 @@ def test_space_for_pieces_only_where_a_reduction_can_be_cut(library, dtype):
         assert cuts(64 * slices) == worth_it(slices), slices
         if slices > 1:
             assert cuts(64 * slices - 8) == worth_it(slices), slices
+
+
+@pytest.mark.parametrize("call", ["fm_moe_layer_route", "fm_moe_layer_forward", "fm_moe_layer_backward"])
+def test_layer_refuses_sizes_of_another_shape(library, call):
+    """The three calls compute offsets and workspace from the struct: one whose shape has changed since fm_moe_layer_sizes, or
+    whose buffers are misaligned, is refused before anything is launched."""
+    layer = _lib.MoELayer(100, 128, 256, 7, 0, 2, 1, 1, 1)
+    for name in ("logits", "input", "weight_1", "weight_2", "routing", "workspace", "sparse_input", "layer_1_output",
+                 "activation_output", "layer_2_output", "output", "grad_output", "grad_layer_2_output",
+                 "grad_activation_output", "grad_layer_1_output", "grad_scores", "grad_logits"):  # fmt: skip
+        setattr(layer, name, 4096)
+
+    def refused(what):
+        return getattr(library, call)(ctypes.byref(layer), None) == _lib.FM_ERR_INVALID_ARGUMENT and what in library.fm_last_error()
+
+    assert refused(b"fm_moe_layer_sizes")  # never asked
+    _lib.check(library.fm_moe_layer_sizes(ctypes.byref(layer)))
+    for name in ("routing", "workspace"):
+        setattr(layer, name, 4096 + 16)
+        assert refused(b"aligned")
+        setattr(layer, name, 4096)
+    for field, value in (("tokens", 1000), ("routed_experts", 64), ("dynamic_rows", 128), ("shared_experts", 1), ("ffn", 1 << 20)):
+        before = getattr(layer, field)
+        setattr(layer, field, value)
+        # A wider layer needs more only where its products' tables grow.
+        asked = _lib.MoELayer.from_buffer_copy(layer)
+        _lib.check(library.fm_moe_layer_sizes(ctypes.byref(asked)))
+        needed = [(asked.rows, layer.rows), (asked.routing_bytes, layer.routing_bytes), (asked.workspace_bytes, layer.workspace_bytes)]
+        assert needed[0][0] != needed[0][1] or any(now > had for now, had in needed[1:])
+        assert refused(b"fm_moe_layer_sizes")
+        setattr(layer, field, before)
