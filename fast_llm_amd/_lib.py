@@ -13,7 +13,7 @@ import torch
 
 LIBRARY_PATH = pathlib.Path(__file__).resolve().parent / "csrc" / "libfastmoe_hip.so"
 
-FM_VERSION = 10
+FM_VERSION = 11
 
 _c_i64, _c_int, _c_ptr, _c_size = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 
@@ -35,7 +35,7 @@ class MoELayer(ctypes.Structure):
         + [
             (name, _c_ptr)
             for name in (
-                "logits", "noise", "input", "weight_1", "weight_2", "routing", "workspace", "sparse_input", "layer_1_output",
+                "logits", "noise", "input", "weight_1", "weight_2", "routing", "workspace", "losses", "sparse_input", "layer_1_output",
                 "activation_output", "layer_2_output", "output", "grad_output", "grad_layer_2_output",
                 "grad_activation_output", "grad_layer_1_output", "grad_scores", "grad_logits", "grad_input", "grad_weight_1",
                 "grad_weight_2", "router", "grad_router",

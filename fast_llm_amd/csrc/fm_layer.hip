@@ -13,7 +13,7 @@ namespace {
 struct Plan {
     int64_t experts, slots, rows, used_index_size;
     int index_dtype;
-    size_t losses, top_experts, scores, lse, statistics, sparse_rows, expert_ends, expert_pad_begins, router, routing_bytes;
+    size_t top_experts, scores, lse, statistics, sparse_rows, expert_ends, expert_pad_begins, router, routing_bytes;
     size_t workspace_bytes, router_linear_bytes;
 };
 
@@ -40,7 +40,6 @@ int make_plan(const fm_moe_layer &layer, Plan &plan) {
         at += (bytes + 63) / 64 * 64;
         return offset;
     };
-    plan.losses = take(8);  // first: the caller reads them
     plan.top_experts = take(8 * entries);
     plan.scores = take(4 * entries);
     plan.lse = take(8 * layer.tokens);
@@ -162,11 +161,11 @@ void plan_workspace(const fm_moe_layer &layer, Plan &plan) {
 
 int route(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     Step step{layer, plan, stream};
-    FM_REQUIRE(layer.logits && layer.routing && layer.workspace, "fm_moe_layer_route: null tensor");
     const bool losses = layer.with_losses != 0;
+    FM_REQUIRE(layer.logits && layer.routing && layer.workspace && (layer.losses || !losses), "fm_moe_layer_route: null tensor");
     FM_STEP(fm_router_forward(layer.logits, layer.noise, step.routing(plan.top_experts), step.routing(plan.scores),
                               losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
-                              losses ? step.routing(plan.losses) : nullptr, step.routing(plan.router),
+                              losses ? layer.losses : nullptr, step.routing(plan.router),
                               plan.routing_bytes - plan.router, layer.tokens, layer.routed_experts, layer.experts_per_token,
                               layer.shared_experts, step.dtype(), stream));
     FM_STEP(fm_sparse_map_from_router(reinterpret_cast<const int64_t *>(step.routing(plan.top_experts)), step.routing(plan.router),

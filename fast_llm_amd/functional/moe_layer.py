@@ -121,6 +121,8 @@ def _forward(
     layer = _describe(options, hidden_states, weight_1, weight_2, with_losses)
     new = hidden_states.new_empty
     routing = new(layer.routing_bytes, dtype=torch.uint8)
+    losses = new(2, dtype=torch.float32) if with_losses else None  # of its own: a caller may keep it long
+    layer.losses = _lib.ptr(losses)
     layer.logits, layer.noise, layer.routing = logits.data_ptr(), _lib.ptr(noise), routing.data_ptr()
     if options.dynamic_shape:
         workspace = new(layer.workspace_bytes, dtype=torch.uint8)
@@ -162,7 +164,7 @@ def _forward(
         layer_2_output,
         layer.dynamic_rows,
     )
-    return output, routing[:8].view(torch.float32) if with_losses else None, saved
+    return output, losses, saved
 
 
 def _gradient_targets(weights: list[torch.Tensor]) -> list[torch.Tensor]:

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FM_VERSION 10
+#define FM_VERSION 11
 
 /* Element type of activations, weights and outputs. */
 enum fm_dtype { FM_DTYPE_F32 = 0, FM_DTYPE_BF16 = 1, FM_DTYPE_F16 = 2 };
@@ -386,12 +386,13 @@ typedef struct {
      * other calls refuse a struct whose shape has changed since (FM_ERR_INVALID_ARGUMENT). */
     int64_t rows, routing_bytes, workspace_bytes, index_dtype /* fm_index_dtype */, used_rows_offset;
     int64_t router_linear; /* whether fm_router_linear_backward takes the shape */
-    /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned, kept for the
-     * backward) starts with the two losses (fp32) if there are losses; `workspace` (64-byte aligned) is free again after the call.
+    /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned) is kept for the
+     * backward; `workspace` (64-byte aligned) is free again after the call; `losses` [2] fp32 (null without them) as
+     * fm_router_forward.
      * layer_1_output [rows, ffn * (2 if gated)] may be null where the backward recomputes it or does not follow: layer 1
      * then runs with the gated activation in its epilogue, FM_ERR_UNSUPPORTED if it cannot. */
     const void *logits, *noise, *input, *weight_1, *weight_2;
-    void *routing, *workspace;
+    void *routing, *workspace, *losses;
     void *sparse_input /* [rows, hidden] */, *layer_1_output, *activation_output /* [rows, ffn] */,
         *layer_2_output /* [rows, hidden] */, *output /* [tokens, hidden] */;
     /* Backward: the forward's tensors (recomputed ones as space to write), its output's gradient, space for the gradients of

@@ -202,7 +202,7 @@ def test_layer_refuses_sizes_of_another_shape(library, call):
     """The three calls compute offsets and workspace from the struct: one whose shape has changed since fm_moe_layer_sizes, or
     whose buffers are misaligned, is refused before anything is launched."""
     layer = _lib.MoELayer(100, 128, 256, 7, 0, 2, 1, 1, 1)
-    for name in ("logits", "input", "weight_1", "weight_2", "routing", "workspace", "sparse_input", "layer_1_output",
+    for name in ("logits", "input", "weight_1", "weight_2", "routing", "workspace", "losses", "sparse_input", "layer_1_output",
                  "activation_output", "layer_2_output", "output", "grad_output", "grad_layer_2_output",
                  "grad_activation_output", "grad_layer_1_output", "grad_scores", "grad_logits"):  # fmt: skip
         setattr(layer, name, 4096)

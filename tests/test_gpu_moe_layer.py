@@ -195,3 +195,11 @@ def test_layer_in_two_calls_with_tile_tables(recompute_level, hidden, ffn, token
     bound = {torch.float32: 1e-5, torch.bfloat16: 1e-2}[dtype]  # as in test_layer_in_two_calls_matches_the_composition
     for name in ("input_grads", "router_grad"):
         assert all(max_rel_err(a, b) <= bound for a, b in zip(results[0][name], results[1][name], strict=True)), name
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_collected_losses_keep_no_buffer_of_the_layer(training, device):
+    layer = DroplessMoEMLP(64, 128, 8, 2, z_loss_coefficient=0.1, device=device).train(training)
+    losses = {}
+    layer(torch.randn(2000, 64, device=device, dtype=torch.bfloat16), grad_scale=1.0, losses=losses)
+    assert all(value.untyped_storage().nbytes() <= 64 for values in losses.values() for value in values) and len(losses) == 2
