@@ -215,6 +215,8 @@ class DroplessMoEMLP(torch.nn.Module):
         """Whether router and MLP have no step in between that `moe_layer` does not know."""
         return (
             self.routing == ROUTING_TOPK
+            # A routing of the caller's own (a subclass's or an instance's) is run, not passed by.
+            and getattr(self.route_with_counts, "__func__", None) is DroplessMoEMLP.route_with_counts
             and self.router_normalization is None
             and self.router_scale is None
             and self.router_input_scale == 1.0

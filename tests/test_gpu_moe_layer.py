@@ -203,3 +203,23 @@ def test_collected_losses_keep_no_buffer_of_the_layer(training, device):
     losses = {}
     layer(torch.randn(2000, 64, device=device, dtype=torch.bfloat16), grad_scale=1.0, losses=losses)
     assert all(value.untyped_storage().nbytes() <= 64 for values in losses.values() for value in values) and len(losses) == 2
+
+
+@pytest.mark.parametrize("tokens", [8, 512])
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("subclass", [False, True])
+def test_replaced_routing_is_honoured(tokens, training, subclass, device):
+    def first_experts(self, hidden_states, grad_scale=None, losses=None):
+        experts = torch.arange(2, device=hidden_states.device).expand(hidden_states.size(0), 2).contiguous()
+        return torch.full(experts.shape, 0.5, device=hidden_states.device), experts, None
+
+    torch.manual_seed(0)
+    layer_class = type("FirstExperts", (DroplessMoEMLP,), {"route_with_counts": first_experts}) if subclass else DroplessMoEMLP
+    layer = layer_class(64, 128, 8, 2, device=device).train(training)
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
+    scores, experts, _ = first_experts(layer, x)
+    with torch.no_grad():
+        expected = layer(x, scores, experts)
+        if not subclass:
+            layer.route_with_counts = lambda *args: first_experts(layer, *args)
+        assert torch.equal(layer(x), expected)
