@@ -195,9 +195,9 @@ class _MoELayer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, _):
-        if grad_output is None:
-            return (None,) * 9
         hidden_states, router = ctx.saved_tensors
+        if grad_output is None:  # nothing depends on the output: the losses still train the router, the buffers become zero
+            grad_output = torch.zeros_like(hidden_states)
         (weight_1, weight_2), options = ctx.weights, ctx.options
         saved, ctx.saved = ctx.saved, None  # the intermediates go when this call ends, whoever holds the graph
         if saved is None:

@@ -223,3 +223,32 @@ def test_replaced_routing_is_honoured(tokens, training, subclass, device):
         if not subclass:
             layer.route_with_counts = lambda *args: first_experts(layer, *args)
         assert torch.equal(layer(x), expected)
+
+
+def test_undefined_output_gradient_trains_the_router_and_clears_the_buffers(device):
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 8, 2, auxiliary_loss_coefficient=1.0, z_loss_coefficient=1.0, device=device, dtype=torch.float32)
+    x = torch.randn(100, 64, device=device, requires_grad=True)
+    results = []
+    for composed in (False, True):
+        layer.router.grad = x.grad = None
+        layer.layer_1.param_grad_is_zero = layer.layer_2.param_grad_is_zero = True
+        layer.layer_1.grad_buffer.fill_(7), layer.layer_2.grad_buffer.fill_(7)
+        if composed:
+            with _lib.KernelTimer():
+                output = layer(x, grad_scale=1.0)
+        else:
+            output = layer(x, grad_scale=1.0)
+        NoGradient.apply(output).sum().backward()
+        results.append((layer.router.grad, x.grad))
+        assert not layer.layer_1.grad_buffer.any() and not layer.layer_2.grad_buffer.any()
+    assert all(max_rel_err(a, b) <= 1e-5 and b.abs().max() > 0 for a, b in zip(*results))
