@@ -46,6 +46,12 @@ def without_backward(output: torch.Tensor) -> torch.Tensor:
     return _WithoutBackward.apply(output, ANCHOR) if torch.is_grad_enabled() else output
 
 
+def forward_mode() -> bool:
+    """Whether forward-mode differentiation is on. The autograd functions refuse inputs with a tangent; what runs outside them
+    would lose it silently and steps aside."""
+    return torch.autograd.forward_ad._current_level >= 0
+
+
 class _ForwardBackwardPair(torch.autograd.Function):
     """One autograd node for every wrapped pair: the pair itself travels as the first argument. The last argument is
     an empty tensor that requires a gradient, so that autograd visits the node even when none of the caller's tensors

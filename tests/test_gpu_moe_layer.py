@@ -252,3 +252,19 @@ def test_undefined_output_gradient_trains_the_router_and_clears_the_buffers(devi
         results.append((layer.router.grad, x.grad))
         assert not layer.layer_1.grad_buffer.any() and not layer.layer_2.grad_buffer.any()
     assert all(max_rel_err(a, b) <= 1e-5 and b.abs().max() > 0 for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("tokens", [8, 512])
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("which", ["input", "router"])
+def test_tangents_are_refused_not_lost(tokens, training, which, device):
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device).train(training)
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x if which == "input" else layer.router.detach(), torch.ones_like(x if which == "input" else layer.router))
+        with pytest.raises(RuntimeError, match="jvp|forward"):
+            if which == "input":
+                layer(dual)
+            else:
+                torch.func.functional_call(layer, {"router": dual}, (x,))
+        layer(x)  # without a tangent nothing is lost
