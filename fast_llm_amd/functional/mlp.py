@@ -26,7 +26,7 @@ from fast_llm_amd.functional.sparse_copy import (
     copy_sparse_to_dense_forward,
 )
 from fast_llm_amd.functional.sparse_linear import output_sparse_matmul
-from fast_llm_amd.functional.utils import Assert, forward_mode, wrap_forward_backward
+from fast_llm_amd.functional.utils import Assert, is_traced, wrap_forward_backward
 
 # The kernels for few tokens (`few_tokens_forward`) read an expert's weights again for every 16 to 64 of its rows; past this many
 # rows per expert, on average, they are never the faster way.
@@ -403,7 +403,7 @@ def few_tokens_workspace_size(
     or do not take these operands: half precision, contiguous, 16-byte aligned, of sizes that fit together and that the library
     accepts. Everything else runs in the sparse layout, which also refuses what does not fit."""
     dtype, ffn = input_.dtype, weight_2.size(0) // num_experts
-    if dtype not in (torch.bfloat16, torch.float16) or input_.dim() != 2 or forward_mode():
+    if dtype not in (torch.bfloat16, torch.float16) or input_.dim() != 2 or is_traced():
         return 0
     tokens, hidden = input_.shape
     if (

@@ -15,7 +15,7 @@ import torch
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.config import ActivationType, KernelConfig, MLPRecomputeLevel
 from fast_llm_amd.functional.mlp import _activation_tag
-from fast_llm_amd.functional.utils import ANCHOR, Assert, forward_mode, without_backward
+from fast_llm_amd.functional.utils import ANCHOR, Assert, is_traced, without_backward
 from fast_llm_amd.tensor import accumulate_gradient, param_get_and_unset_is_zero
 
 
@@ -38,7 +38,7 @@ def moe_layer_supported(
     options: MoELayerOptions,
 ) -> bool:
     """Whether `moe_layer` takes these operands. It steps aside for what the parts offer and it does not (kernel timers,
-    kernel choices other than the default ones, logits that autocast makes another type of, tangents) and for operands that do not
+    kernel choices other than the default ones, logits that autocast makes another type of, tracers) and for operands that do not
     fit together, which the parts refuse."""
     dtype, (experts, hidden) = hidden_states.dtype, (options.routed_experts + options.shared_experts, hidden_states.size(-1))
     ffn = weight_2.size(0) // experts
@@ -47,7 +47,7 @@ def moe_layer_supported(
         and KernelConfig.fuse_activation is None
         and KernelConfig.grouped_gemm_workspace
         and not torch.is_autocast_enabled("cuda")
-        and not forward_mode()
+        and not is_traced()
         and hidden_states.dim() == 2
         and hidden_states.size(0) > 0
         and dtype in _lib.DTYPES

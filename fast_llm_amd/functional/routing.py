@@ -11,7 +11,7 @@ import dataclasses
 import torch
 
 from fast_llm_amd import _lib
-from fast_llm_amd.functional.utils import forward_mode
+from fast_llm_amd.functional.utils import is_traced
 
 
 @dataclasses.dataclass
@@ -229,7 +229,7 @@ def router(
         raise ValueError("a loss that is not computed has no gradient")
     flat = logits.flatten(0, -2)
     flat_noise = None if noise is None else noise.flatten(0, -2)
-    if (logits.requires_grad and torch.is_grad_enabled()) or forward_mode():
+    if (logits.requires_grad and torch.is_grad_enabled()) or is_traced():
         scores, top_experts, losses, workspace = _Router.apply(
             flat, flat_noise, experts_per_token, shared_experts, auxiliary_loss_grad, z_loss_grad, with_losses
         )

@@ -46,10 +46,10 @@ def without_backward(output: torch.Tensor) -> torch.Tensor:
     return _WithoutBackward.apply(output, ANCHOR) if torch.is_grad_enabled() else output
 
 
-def forward_mode() -> bool:
-    """Whether forward-mode differentiation is on. The autograd functions refuse inputs with a tangent; what runs outside them
-    would lose it silently and steps aside."""
-    return torch.autograd.forward_ad._current_level >= 0
+def is_traced() -> bool:
+    """Whether forward-mode differentiation or `torch.jit`'s tracer looks at what runs. They know the autograd functions and
+    refuse or record them; a tangent or a result of what runs outside them would be lost silently, so that steps aside."""
+    return torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing()
 
 
 class _ForwardBackwardPair(torch.autograd.Function):

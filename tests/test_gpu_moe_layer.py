@@ -268,3 +268,12 @@ def test_tangents_are_refused_not_lost(tokens, training, which, device):
             else:
                 torch.func.functional_call(layer, {"router": dual}, (x,))
         layer(x)  # without a tangent nothing is lost
+
+
+@pytest.mark.parametrize("tokens", [8, 512])
+def test_traces_are_refused_not_wrong(tokens, device):
+    """A tracer would record the space for the output and not the library calls that fill it."""
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device).eval()
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="requires grad"):
+        torch.jit.trace(layer, x, check_trace=False)
