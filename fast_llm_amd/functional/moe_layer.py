@@ -96,9 +96,7 @@ def _fuses_layer_1(options: MoELayerOptions, layer: _lib.MoELayer) -> bool:
 class _Saved:
     """What the forward keeps for the backward. An intermediate that the recompute level does not keep is None."""
 
-    logits: torch.Tensor
-    noise: torch.Tensor | None
-    routing: torch.Tensor
+    router: tuple[torch.Tensor, torch.Tensor | None, torch.Tensor]  # logits, noise, routing: autograd saves these
     sparse_input: torch.Tensor | None
     layer_1_output: torch.Tensor | None
     activation_output: torch.Tensor | None
@@ -156,9 +154,7 @@ def _forward(
         layer.layer_1_output = layer_1_output.data_ptr()
         _lib.call("fm_moe_layer_forward", device, _lib.ctypes.byref(layer))
     saved = _Saved(
-        logits,
-        noise,
-        routing,
+        (logits, noise, routing),
         None if level.recompute_sparse_input else sparse_input,
         layer_1_output if keep_layer_1 else None,
         None if level.recompute_activation else activation_output,
@@ -187,7 +183,9 @@ class _MoELayer(torch.autograd.Function):
         output, losses, ctx.saved = _forward(
             options, hidden_states, router, weight_1, weight_2, noise, with_losses, training=True
         )
-        ctx.save_for_backward(hidden_states, router)
+        # As the router's own nodes do: saved-tensor hooks see its tensors. The MLP's intermediates are the layer's.
+        ctx.save_for_backward(hidden_states, router, *ctx.saved.router)
+        ctx.saved.router = None
         ctx.weights, ctx.options, ctx.with_losses, ctx.loss_grads = (weight_1, weight_2), options, with_losses, loss_grads
         ctx.set_materialize_grads(False)
         if losses is not None:
@@ -196,7 +194,7 @@ class _MoELayer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, _):
-        hidden_states, router = ctx.saved_tensors
+        hidden_states, router, logits, noise, routing = ctx.saved_tensors
         if grad_output is None:  # nothing depends on the output: the losses still train the router, the buffers become zero
             grad_output = torch.zeros_like(hidden_states)
         (weight_1, weight_2), options = ctx.weights, ctx.options
@@ -220,9 +218,9 @@ class _MoELayer(torch.autograd.Function):
         grad_layer_2_output, grad_activation_output = new((rows, hidden)), new((rows, ffn))
         grad_layer_1_output = new(layer_1_output.shape)
         grad_scores = new(layer.tokens * (options.experts_per_token + options.shared_experts), dtype=torch.float32)
-        grad_logits = new(saved.logits.shape)
-        layer.logits, layer.noise, layer.input = saved.logits.data_ptr(), _lib.ptr(saved.noise), hidden_states.data_ptr()
-        layer.routing, layer.workspace = saved.routing.data_ptr(), workspace.data_ptr()
+        grad_logits = new(logits.shape)
+        layer.logits, layer.noise, layer.input = logits.data_ptr(), _lib.ptr(noise), hidden_states.data_ptr()
+        layer.routing, layer.workspace = routing.data_ptr(), workspace.data_ptr()
         layer.sparse_input, layer.layer_1_output = sparse_input.data_ptr(), layer_1_output.data_ptr()
         layer.activation_output, layer.layer_2_output = activation_output.data_ptr(), saved.layer_2_output.data_ptr()
         layer.grad_output, layer.grad_layer_2_output = grad_output.data_ptr(), grad_layer_2_output.data_ptr()

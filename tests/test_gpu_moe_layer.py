@@ -277,3 +277,27 @@ def test_traces_are_refused_not_wrong(tokens, device):
     x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16)
     with torch.no_grad(), pytest.raises(RuntimeError, match="requires grad"):
         torch.jit.trace(layer, x, check_trace=False)
+
+
+def test_saved_tensor_hooks_see_what_the_router_saves(device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(64, 128, 8, 2, device=device, dtype=torch.float32)
+    x = torch.randn(300, 64, device=device, requires_grad=True)
+    results, packed = [], []
+
+    def pack(tensor):
+        packed.append(tuple(tensor.shape))
+        return tensor.cpu()
+
+    for hooks in (False, True):
+        layer.router.grad = x.grad = None
+        layer.layer_1.param_grad_is_zero = layer.layer_2.param_grad_is_zero = True
+        if hooks:
+            with torch.autograd.graph.saved_tensors_hooks(pack, lambda tensor: tensor.to(device)):
+                output = layer(x, grad_scale=1.0)
+        else:
+            output = layer(x, grad_scale=1.0)
+        output.backward(torch.ones_like(output))
+        results.append((x.grad, layer.router.grad, layer.layer_1.grad_buffer.clone(), layer.layer_2.grad_buffer.clone()))
+    assert {(300, 64), (8, 64), (300, 8)} <= set(packed) and len(packed) > 3  # input, router, logits, and what was selected
+    assert all(torch.equal(a, b) for a, b in zip(*results))
