@@ -31,7 +31,7 @@ class MoELayer(ctypes.Structure):
             )
         ]
         + [(name, ctypes.c_double) for name in ("auxiliary_loss_grad", "z_loss_grad")]
-        + [(name, _c_i64) for name in ("dynamic_rows", "rows", "routing_bytes", "workspace_bytes", "index_dtype", "used_rows_offset", "router_linear")]
+        + [(name, _c_i64) for name in ("dynamic_rows", "rows", "routing_bytes", "workspace_bytes", "index_dtype", "used_rows_offset", "forward_workspace_bytes", "router_linear")]
         + [
             (name, _c_ptr)
             for name in (
@@ -41,7 +41,7 @@ class MoELayer(ctypes.Structure):
                 "grad_weight_2", "router", "grad_router",
             )
         ]
-        + [("router_input_grad", _c_i64)]
+        + [("router_input_grad", _c_i64), ("backward_part", _c_i64)]
     )  # fmt: skip
 
 

@@ -14,7 +14,8 @@ struct Plan {
     int64_t experts, slots, rows, used_index_size;
     int index_dtype;
     size_t top_experts, scores, lse, statistics, sparse_rows, expert_ends, expert_pad_begins, router, routing_bytes;
-    size_t workspace_bytes, router_linear_bytes;
+    size_t workspace_bytes, router_linear_bytes;  // of a backward
+    size_t forward_workspace_bytes;
 };
 
 constexpr int64_t kPad = 128;
@@ -50,7 +51,7 @@ int make_plan(const fm_moe_layer &layer, Plan &plan) {
     plan.router = take(fm_router_workspace_size(layer.tokens, layer.routed_experts));
     plan.routing_bytes = at;
     plan.router_linear_bytes = fm_router_linear_backward_workspace_size(layer.tokens, layer.routed_experts, layer.hidden, static_cast<int>(layer.dtype));
-    plan.workspace_bytes = 0;  // the rest of it: see plan_workspace
+    plan.workspace_bytes = plan.forward_workspace_bytes = 0;  // see plan_workspace
     return FM_OK;
 }
 
@@ -120,13 +121,13 @@ struct Step {
         products[kGradWeight1] = row_sparse(layer.grad_layer_1_output, layer.sparse_input, layer.grad_weight_1, ffn_1(), layer.accumulate_1 != 0);
     }
     // One launch for the tile tables of all products that are wanted: each launch of its own took 7 us.
-    int plan_tables(GemmArgs *products, const bool *wanted, int count) const {
+    int plan_tables(GemmArgs *products, const bool *wanted, int count, size_t workspace_bytes) const {
         GemmArgs chosen[kMaxPlanned];
         int which[kMaxPlanned], num = 0;
         for (int i = 0; i < count; ++i)
             if (wanted[i]) chosen[num] = products[i], which[num++] = i;
         if (dtype() == FM_DTYPE_F32) return FM_OK;
-        const int status = mfma_gemm_plan(chosen, num, dtype(), layer.workspace, plan.workspace_bytes, static_cast<hipStream_t>(stream));
+        const int status = mfma_gemm_plan(chosen, num, dtype(), layer.workspace, workspace_bytes, static_cast<hipStream_t>(stream));
         for (int i = 0; i < num; ++i) products[which[i]] = chosen[i];
         return status;
     }
@@ -142,18 +143,13 @@ void plan_workspace(const fm_moe_layer &layer, Plan &plan) {
     fused.layer_1_output = nullptr, fused.routing = &fused;
     const Step with_output{kept, plan, nullptr}, without{fused, plan, nullptr};
     const int dtype = with_output.dtype();
-    plan.workspace_bytes = fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts);
-    const auto at_least = [&](size_t bytes) {
-        if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
-    };
-    at_least(plan.router_linear_bytes);
     GemmArgs products[kMaxPlanned];
     with_output.forward_products(products);
-    at_least(mfma_gemm_plan_size(products, 2, dtype));
+    plan.forward_workspace_bytes = max(fm_sparse_map_from_router_workspace_size(layer.tokens, plan.experts), mfma_gemm_plan_size(products, 2, dtype));
     without.forward_products(products);
-    at_least(mfma_gemm_plan_size(products, 2, dtype));
+    plan.forward_workspace_bytes = max(plan.forward_workspace_bytes, mfma_gemm_plan_size(products, 2, dtype));
     with_output.backward_products(products);
-    at_least(mfma_gemm_plan_size(products, kMaxPlanned, dtype));
+    plan.workspace_bytes = max(max(plan.router_linear_bytes, mfma_gemm_plan_size(products, kMaxPlanned, dtype)), size_t(256));
 }
 
 #define FM_STEP(call) \
@@ -172,7 +168,7 @@ int route(const fm_moe_layer &layer, const Plan &plan, void *stream) {
                                       plan.routing_bytes - plan.router, layer.tokens, plan.experts, layer.experts_per_token,
                                       layer.shared_experts, kPad, plan.index_dtype, step.routing(plan.sparse_rows),
                                       step.routing(plan.expert_ends), step.routing(plan.expert_pad_begins), layer.workspace,
-                                      plan.workspace_bytes, stream));
+                                      plan.forward_workspace_bytes, stream));
     return FM_OK;
 }
 
@@ -185,7 +181,7 @@ int forward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     GemmArgs products[2];
     step.forward_products(products);
     const bool wanted[2] = {true, true};
-    FM_STEP(step.plan_tables(products, wanted, 2));
+    FM_STEP(step.plan_tables(products, wanted, 2, plan.forward_workspace_bytes));
     FM_STEP(step.dispatch(layer.sparse_input));
     if (products[Step::kLayer1].fusion != kFusionNone) {
         // FM_ERR_UNSUPPORTED tells the caller to bring a layer-1 buffer.
@@ -201,23 +197,29 @@ int forward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     return step.note;
 }
 
-int backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
+// The gradients of layer 2's output and of the scores: the only step of a backward that reads layer 2's output.
+int combine_backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
+    const Step step{layer, plan, stream};
+    FM_REQUIRE(layer.routing && layer.layer_2_output && layer.grad_output && layer.grad_layer_2_output && layer.grad_scores,
+               "fm_moe_layer_backward: null tensor");
+    return fm_copy_sparse_to_dense_backward(layer.layer_2_output, layer.grad_output, step.routing(plan.scores),
+                                            step.routing(plan.sparse_rows), layer.grad_layer_2_output, layer.grad_scores,
+                                            layer.tokens, layer.hidden, plan.slots, plan.rows, step.dtype(), FM_DTYPE_F32,
+                                            FM_DTYPE_F32, plan.index_dtype, stream);
+}
+
+int rest_of_backward(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     Step step{layer, plan, stream};
     FM_REQUIRE(layer.logits && layer.weight_1 && layer.weight_2 && layer.routing && layer.sparse_input && layer.layer_1_output &&
-                   layer.activation_output && layer.layer_2_output && layer.grad_output && layer.grad_layer_2_output &&
-                   layer.grad_activation_output && layer.grad_layer_1_output && layer.grad_scores && layer.grad_logits &&
-                   layer.workspace && (layer.input || !(layer.recompute_input || layer.router)),
+                   layer.activation_output && layer.grad_layer_2_output && layer.grad_activation_output &&
+                   layer.grad_layer_1_output && layer.grad_scores && layer.grad_logits && layer.workspace &&
+                   (layer.input || !(layer.recompute_input || layer.router)),
                "fm_moe_layer_backward: null tensor");
     GemmArgs products[kMaxPlanned];
     step.backward_products(products);
     const bool wanted[kMaxPlanned] = {layer.recompute_layer_1 != 0, true, layer.grad_weight_2 != nullptr, layer.grad_input != nullptr,
                                       layer.grad_weight_1 != nullptr};
-    FM_STEP(step.plan_tables(products, wanted, kMaxPlanned));
-    // The gradient of layer 2's output and of the scores.
-    FM_STEP(fm_copy_sparse_to_dense_backward(layer.layer_2_output, layer.grad_output, step.routing(plan.scores),
-                                             step.routing(plan.sparse_rows), layer.grad_layer_2_output, layer.grad_scores,
-                                             layer.tokens, layer.hidden, plan.slots, plan.rows, step.dtype(), FM_DTYPE_F32,
-                                             FM_DTYPE_F32, plan.index_dtype, stream));
+    FM_STEP(step.plan_tables(products, wanted, kMaxPlanned, plan.workspace_bytes));
     // What the forward did not keep.
     if (layer.recompute_input) FM_STEP(step.dispatch(layer.sparse_input));
     if (layer.recompute_layer_1) FM_STEP(step.product(products[Step::kLayer1]));
@@ -259,6 +261,7 @@ extern "C" int fm_moe_layer_sizes(fm_moe_layer *layer) {
     layer->rows = plan.rows;
     layer->routing_bytes = static_cast<int64_t>(plan.routing_bytes);
     layer->workspace_bytes = static_cast<int64_t>(plan.workspace_bytes);
+    layer->forward_workspace_bytes = static_cast<int64_t>(plan.forward_workspace_bytes);
     layer->index_dtype = plan.index_dtype;
     layer->router_linear = plan.router_linear_bytes > 0;
     layer->used_rows_offset = static_cast<int64_t>(plan.expert_ends) + (plan.experts - 1) * plan.used_index_size;
@@ -272,10 +275,12 @@ static int plan_call(const char *name, const fm_moe_layer *layer, Plan &plan) {
     if (int status = make_plan(*layer, plan)) return status;
     plan_workspace(*layer, plan);
     FM_REQUIRE(layer->rows == plan.rows && layer->routing_bytes >= static_cast<int64_t>(plan.routing_bytes) &&
-                   layer->workspace_bytes >= static_cast<int64_t>(plan.workspace_bytes),
-               "%s: %lld rows, %lld bytes of routing and %lld of workspace, needs %lld, %zu and %zu (fm_moe_layer_sizes, after the last "
-               "change of the shape)", name, static_cast<long long>(layer->rows), static_cast<long long>(layer->routing_bytes),
-               static_cast<long long>(layer->workspace_bytes), static_cast<long long>(plan.rows), plan.routing_bytes, plan.workspace_bytes);
+                   layer->workspace_bytes >= static_cast<int64_t>(plan.workspace_bytes) &&
+                   layer->forward_workspace_bytes >= static_cast<int64_t>(plan.forward_workspace_bytes),
+               "%s: %lld rows, %lld bytes of routing, %lld and %lld of workspace, needs %lld, %zu, %zu and %zu (fm_moe_layer_sizes, after "
+               "the last change of the shape)", name, static_cast<long long>(layer->rows), static_cast<long long>(layer->routing_bytes),
+               static_cast<long long>(layer->forward_workspace_bytes), static_cast<long long>(layer->workspace_bytes),
+               static_cast<long long>(plan.rows), plan.routing_bytes, plan.forward_workspace_bytes, plan.workspace_bytes);
     FM_REQUIRE(reinterpret_cast<uintptr_t>(layer->routing) % 64 == 0 && reinterpret_cast<uintptr_t>(layer->workspace) % 64 == 0,
                "%s: routing and workspace must be 64-byte aligned", name);
     return FM_OK;
@@ -295,6 +300,9 @@ extern "C" int fm_moe_layer_forward(const fm_moe_layer *layer, void *stream) {
 
 extern "C" int fm_moe_layer_backward(const fm_moe_layer *layer, void *stream) {
     Plan plan;
-    if (int status = plan_call("fm_moe_layer_backward", layer, plan)) return status;
-    return backward(*layer, plan, stream);
+    const char *name = "fm_moe_layer_backward";
+    if (int status = plan_call(name, layer, plan)) return status;
+    FM_REQUIRE(layer->backward_part >= 0 && layer->backward_part <= 2, "%s: part %lld", name, static_cast<long long>(layer->backward_part));
+    if (layer->backward_part != 2) FM_STEP(combine_backward(*layer, plan, stream));
+    return layer->backward_part != 1 ? rest_of_backward(*layer, plan, stream) : FM_OK;
 }

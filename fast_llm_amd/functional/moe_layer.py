@@ -124,7 +124,7 @@ def _forward(
     layer.losses = _lib.ptr(losses)
     layer.logits, layer.noise, layer.routing = logits.data_ptr(), _lib.ptr(noise), routing.data_ptr()
     if options.dynamic_shape:
-        workspace = new(layer.workspace_bytes, dtype=torch.uint8)
+        workspace = new(layer.forward_workspace_bytes, dtype=torch.uint8)
         layer.workspace = workspace.data_ptr()
         _lib.call("fm_moe_layer_route", device, _lib.ctypes.byref(layer))
         index_dtype = torch.int16 if layer.index_dtype == 0 else torch.int32
@@ -133,8 +133,10 @@ def _forward(
         _lib.check(_lib.lib().fm_moe_layer_sizes(_lib.ctypes.byref(layer)))
     level, rows, ffn = options.recompute_level, layer.rows, layer.ffn
     keep_layer_1 = training and not level.recompute_layer_1
-    workspace = new(layer.workspace_bytes, dtype=torch.uint8)
-    sparse_input, layer_2_output = new((rows, layer.hidden)), new((rows, layer.hidden))
+    workspace = new(layer.forward_workspace_bytes, dtype=torch.uint8)
+    sparse_input = new((rows, layer.hidden))
+    # Layer 1 is the only one to read the sparse input: where nobody keeps it, layer 2's output takes its place.
+    layer_2_output = new((rows, layer.hidden)) if training and not level.recompute_sparse_input else sparse_input
     activation_output, output = new((rows, ffn)), new(hidden_states.shape)
     layer_1_output = None
     if keep_layer_1 or not _fuses_layer_1(options, layer):
@@ -175,6 +177,11 @@ def _gradient_targets(weights: list[torch.Tensor]) -> list[torch.Tensor]:
     return buffers if direct else [torch.empty(weight.shape, dtype=torch.float32, device=weight.device) for weight in weights]
 
 
+# Layer 2's output from this size on is let go before the backward makes the rest of its buffers, at the price of a library call
+# more; what is smaller is not worth the host time that small layers are bound by.
+_LARGE_BUFFER = 32 << 20
+
+
 class _MoELayer(torch.autograd.Function):
     # The last argument of `apply` is an empty tensor that requires a gradient: the weight gradients are side effects, the
     # node is to be visited whatever else needs one.
@@ -207,6 +214,15 @@ class _MoELayer(torch.autograd.Function):
         layer.auxiliary_loss_grad, layer.z_loss_grad = ctx.loss_grads
         rows, hidden, ffn = layer.rows, layer.hidden, layer.ffn
         new = hidden_states.new_empty
+        grad_layer_2_output = new((rows, hidden))
+        grad_scores = new(layer.tokens * (options.experts_per_token + options.shared_experts), dtype=torch.float32)
+        layer.routing, layer.layer_2_output = routing.data_ptr(), saved.layer_2_output.data_ptr()
+        layer.grad_output, layer.grad_layer_2_output = grad_output.data_ptr(), grad_layer_2_output.data_ptr()
+        layer.grad_scores = grad_scores.data_ptr()
+        if saved.layer_2_output.nbytes >= _LARGE_BUFFER:
+            layer.backward_part = 1
+            _lib.call("fm_moe_layer_backward", device, _lib.ctypes.byref(layer))
+            saved.layer_2_output, layer.backward_part = None, 2
         workspace = new(layer.workspace_bytes, dtype=torch.uint8)
         sparse_input, layer_1_output, activation_output = saved.sparse_input, saved.layer_1_output, saved.activation_output
         if sparse_input is None:
@@ -215,18 +231,13 @@ class _MoELayer(torch.autograd.Function):
             layer_1_output, layer.recompute_layer_1 = new((rows, ffn * 2 if options.gated else ffn)), True
         if activation_output is None:
             activation_output, layer.recompute_activation = new((rows, ffn)), True
-        grad_layer_2_output, grad_activation_output = new((rows, hidden)), new((rows, ffn))
-        grad_layer_1_output = new(layer_1_output.shape)
-        grad_scores = new(layer.tokens * (options.experts_per_token + options.shared_experts), dtype=torch.float32)
+        grad_activation_output, grad_layer_1_output = new((rows, ffn)), new(layer_1_output.shape)
         grad_logits = new(logits.shape)
         layer.logits, layer.noise, layer.input = logits.data_ptr(), _lib.ptr(noise), hidden_states.data_ptr()
-        layer.routing, layer.workspace = routing.data_ptr(), workspace.data_ptr()
-        layer.sparse_input, layer.layer_1_output = sparse_input.data_ptr(), layer_1_output.data_ptr()
-        layer.activation_output, layer.layer_2_output = activation_output.data_ptr(), saved.layer_2_output.data_ptr()
-        layer.grad_output, layer.grad_layer_2_output = grad_output.data_ptr(), grad_layer_2_output.data_ptr()
+        layer.workspace, layer.sparse_input = workspace.data_ptr(), sparse_input.data_ptr()
+        layer.layer_1_output, layer.activation_output = layer_1_output.data_ptr(), activation_output.data_ptr()
         layer.grad_activation_output = grad_activation_output.data_ptr()
-        layer.grad_layer_1_output = grad_layer_1_output.data_ptr()
-        layer.grad_scores, layer.grad_logits = grad_scores.data_ptr(), grad_logits.data_ptr()
+        layer.grad_layer_1_output, layer.grad_logits = grad_layer_1_output.data_ptr(), grad_logits.data_ptr()
         grad_input = None
         if ctx.needs_input_grad[0]:
             grad_input = new(hidden_states.shape)
@@ -252,6 +263,8 @@ class _MoELayer(torch.autograd.Function):
                 grad_router = torch.empty_like(router)
                 layer.grad_router = grad_router.data_ptr()
         _lib.call("fm_moe_layer_backward", device, _lib.ctypes.byref(layer))
+        del saved, sparse_input, layer_1_output, activation_output, workspace
+        del grad_layer_2_output, grad_activation_output, grad_layer_1_output
         for weight, target in zip(trained, targets):
             if target is not weight.grad_buffer:
                 accumulate_gradient(weight, target)

@@ -384,13 +384,15 @@ typedef struct {
                            * `routing` at used_rows_offset (`index_dtype`) */
     /* Set by fm_moe_layer_sizes: sparse rows, bytes of the two untyped buffers below, and where the map's last expert ends. The
      * other calls refuse a struct whose shape has changed since (FM_ERR_INVALID_ARGUMENT). */
-    int64_t rows, routing_bytes, workspace_bytes, index_dtype /* fm_index_dtype */, used_rows_offset;
+    int64_t rows, routing_bytes, workspace_bytes /* of a backward */, index_dtype /* fm_index_dtype */, used_rows_offset;
+    int64_t forward_workspace_bytes; /* of fm_moe_layer_route and fm_moe_layer_forward */
     int64_t router_linear; /* whether fm_router_linear_backward takes the shape */
     /* Forward. `logits` and `noise` (may be null) [tokens, routed_experts]; `routing` (64-byte aligned) is kept for the
      * backward; `workspace` (64-byte aligned) is free again after the call; `losses` [2] fp32 (null without them) as
      * fm_router_forward.
      * layer_1_output [rows, ffn * (2 if gated)] may be null where the backward recomputes it or does not follow: layer 1
-     * then runs with the gated activation in its epilogue, FM_ERR_UNSUPPORTED if it cannot. */
+     * then runs with the gated activation in its epilogue, FM_ERR_UNSUPPORTED if it cannot. layer_2_output may be the
+     * buffer of sparse_input where that is not kept. */
     const void *logits, *noise, *input, *weight_1, *weight_2;
     void *routing, *workspace, *losses;
     void *sparse_input /* [rows, hidden] */, *layer_1_output, *activation_output /* [rows, ffn] */,
@@ -407,6 +409,9 @@ typedef struct {
     const void *router;
     void *grad_router;
     int64_t router_input_grad;
+    /* Backward: 1: only the gradients of layer 2's output and of the scores, after which layer_2_output and grad_output are not
+     * read again and may go before the other buffers are made; 2: the rest; 0: both. */
+    int64_t backward_part;
 } fm_moe_layer;
 
 int fm_moe_layer_sizes(fm_moe_layer *layer);

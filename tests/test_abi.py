@@ -172,7 +172,7 @@ def test_layer_sizes_come_from_the_shape_alone(library, hidden, ffn, tokens, dty
         for name in buffers:
             setattr(layer, name, 64)
         _lib.check(library.fm_moe_layer_sizes(ctypes.byref(layer)))
-        sizes.add((layer.rows, layer.routing_bytes, layer.workspace_bytes))
+        sizes.add((layer.rows, layer.routing_bytes, layer.workspace_bytes, layer.forward_workspace_bytes))
     assert len(sizes) == 1
 
 
