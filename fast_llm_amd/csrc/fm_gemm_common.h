@@ -48,7 +48,7 @@ struct GemmArgs {
     int64_t piece_length;  // row-sparse mode without a map: group e reduces over [e, e + 1) * piece_length instead of
                            // everything (0: everything)
     int planned;           // `tile_table` (and `partials`) have been set up by mfma_gemm_plan
-    int chunk_tiles;       // consecutive tiles that go to one XCD (set by the fp32 kernel's launcher)
+    int chunk_tiles;       // consecutive tiles that go to one XCD (set by the launchers of the fp32 and the few-row kernels)
 };
 
 #define FM_LDS(T) __attribute__((address_space(3))) T
@@ -74,13 +74,6 @@ __device__ __forceinline__ const char *uniform_pointer(const char *pointer) {
 // ---- which tile ----------------------------------------------------------------------------------------
 constexpr int kGroupRows = 8;
 
-// Logical order of the tiles of a product whose rows are grouped by expert (output-sparse, input-inner-sparse,
-// dense): expert after expert; within an expert its row tiles (ceil(rows_e / kTile)) are cut into ceil(count / 8)
-// groups of nearly equal size (9 row tiles: 5 + 4), and a group is walked column tile by column tile, row tiles
-// fastest. 32 consecutive tiles (what an XCD runs at one time) are then about 8 row tiles x 4 column tiles of ONE
-// expert, i.e. 8 lhs panels and 4 rhs panels shared in that XCD's L2; with groups that ignore the expert boundaries
-// most chunks straddled two experts and needed twice the rhs panels.
-// Every wavefront scans `expert_ends` 64 experts at a time; returns false if `logical` is past the last tile.
 // The rows of an expert end where its padding begins, if the caller says where that is.
 __device__ __forceinline__ void rows_of_expert(const GemmArgs &args, int expert, int64_t &begin, int64_t &end) {
     const void *ends = args.expert_pad_begins != nullptr ? args.expert_pad_begins : args.expert_ends;
@@ -88,6 +81,13 @@ __device__ __forceinline__ void rows_of_expert(const GemmArgs &args, int expert,
     begin = expert > 0 ? load_index(args.expert_ends, args.index_dtype, expert - 1) : 0;
 }
 
+// Logical order of the tiles of a product whose rows are grouped by expert (output-sparse, input-inner-sparse,
+// dense): expert after expert; within an expert its row tiles (ceil(rows_e / kTile)) are cut into ceil(count / 8)
+// groups of nearly equal size (9 row tiles: 5 + 4), and a group is walked column tile by column tile, row tiles
+// fastest. 32 consecutive tiles (what an XCD runs at one time) are then about 8 row tiles x 4 column tiles of ONE
+// expert, i.e. 8 lhs panels and 4 rhs panels shared in that XCD's L2; with groups that ignore the expert boundaries
+// most chunks straddled two experts and needed twice the rhs panels.
+// Every wavefront scans `expert_ends` 64 experts at a time; returns false if `logical` is past the last tile.
 struct RowTile {
     int expert, tile_n, rows_valid;
     int64_t row0;

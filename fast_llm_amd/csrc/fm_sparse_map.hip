@@ -366,7 +366,7 @@ extern "C" int fm_sparse_map_static(const int64_t *top_experts, int64_t num_rows
                     kStaticScratchBytes);
     void *workspace = nullptr;
     if (int status = static_scratch_of_current_device(static_cast<hipStream_t>(stream), &workspace)) return status;
-    // Nothing to clear: the histogram kernel writes every count the other two kernels read.
+    // Nothing to clear: the histogram kernel writes every count that the other kernel reads.
     return run_sparse_map("fm_sparse_map_static", top_experts, num_rows_dense, num_experts_per_token, num_experts,
                           pad_to_multiple, index_dtype, sparse_rows, expert_ends, expert_pad_begins, workspace,
                           static_cast<hipStream_t>(stream));

@@ -1,6 +1,6 @@
 """
 The whole MoE layer, from the router's linear layer to the output, with two library calls for the forward
-(`fm_moe_layer_route`, `fm_moe_layer_forward`) and one for the backward (`fm_moe_layer_backward`) instead of one per
+(`fm_moe_layer_route`, `fm_moe_layer_forward`) and one or two for the backward (`fm_moe_layer_backward`) instead of one per
 kernel: the same kernels in the same order as `router` -> `get_sparse_map` -> `mlp_autograd`, without the host time of
 some twenty Python launches.
 

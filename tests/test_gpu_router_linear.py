@@ -9,8 +9,8 @@ from tests.helpers import max_rel_err
 pytestmark = pytest.mark.gpu
 
 
-# Tokens around a wavefront's 32 and a workgroup's 256, several pieces; experts around the workgroup's 64 and 128; columns
-# around its 64.
+# One piece of the token axis and many (pieces are whole slices of 64 tokens, 128 at least), with a last slice of every kind;
+# experts and columns around the tiles of 32 (fp32) and 256.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize(
     ("tokens", "experts", "hidden"),

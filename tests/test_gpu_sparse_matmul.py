@@ -350,7 +350,8 @@ def test_every_slice_count_through_the_pipeline(slices, other, device):
 
 # Few tiles and a long reduction: the tiles of the last round of workgroups are cut along the reduction axis and their
 # pieces added by a second kernel. (experts, reduction size, other size): 4 pieces of 18 slices with a shorter, odd last
-# one; whole tiles followed by more than 256 pieces; 2 pieces.
+# one; many tiles of 35 slices, too few to cut; 64 slices; 32 slices, too few. (Which cuts there are, and that they happen:
+# test_every_kind_of_cut.)
 @pytest.mark.parametrize(("experts", "inner", "other"), [(9, 4160, 320), (70, 2240, 600), (40, 4096, 256), (3, 2048, 264)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_split_reduction_of_last_round(experts, inner, other, dtype, device):
@@ -808,8 +809,8 @@ def test_weight_gradients_of_few_rows(sparse_dim, dense_dim, dtype, device):
     assert torch.equal(out[:, :dense_dim], added)
 
 
-# Reductions of no whole number of slices that are cut into pieces (few tiles; 2, 3, 4 and 8 pieces at these tile counts), with
-# the last piece masked, against the unsplit sums that a call without a workspace takes.
+# Reductions of no whole number of slices, cut into 4, 3 and 8 pieces with the last one masked, and (33 slices) too short to be cut,
+# against the unsplit sums that a call without a workspace takes.
 @pytest.mark.parametrize(("experts", "inner", "other"), [(3, 2056, 264), (2, 4104, 2600), (5, 3416, 1280), (16, 2104, 1280), (1, 8200, 72)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_split_reductions_of_no_whole_number_of_slices(experts, inner, other, dtype, device, monkeypatch):
@@ -832,3 +833,43 @@ def test_split_reductions_of_no_whole_number_of_slices(experts, inner, other, dt
     for split, whole, reference in zip(*results, expected):
         assert max_rel_err(split.cpu(), reference) <= _MAX_REL[dtype]
         assert max_rel_err(whole.cpu(), reference) <= _MAX_REL[dtype]
+
+
+# Every cut that the plan knows: 2, 3, 4 and 8 pieces of a round's few tiles; whole tiles before them; more pieces than CUs (two
+# rounds of pieces); the same of reductions that are no whole number of slices, whose last piece is masked; and what is too short
+# or has too many tiles to be cut. Against the unsplit sums that a call without a workspace takes: where there is a cut the bits
+# differ. Operands are drawn on the GPU and the checker is the oracle evaluated there in fp32.
+@pytest.mark.parametrize(("tokens", "inner", "other", "cut"), [
+    ((3, 150, 77), 36 * 64, 264, True), ((3, 150, 77), 39 * 64, 264, True),  # 2 pieces, the second one shorter
+    ((3, 150, 77), 50 * 64, 264, True), ((200, 0, 130), 72 * 64, 520, True), ((40,), 128 * 64, 72, True),  # 3, 4, 8
+    ((1200, 900, 2), 64 * 64, 9000, True),  # 10 x 36 tiles: 256 whole ones, the other 104 in 2 pieces each
+    ((1280, 1280), 128 * 64, 3328, True),  # 130 tiles in 3 pieces each
+    ((3, 150, 77), 35 * 64, 264, False), ((3, 150, 77), 37 * 64, 264, False),
+    ((5, 38, 75, 112, 149), 3416, 1280, True), ((1, 38), 4104, 2600, True), ((1,), 8200, 72, True), ((3, 150, 77), 2440, 264, True),
+    ((1, 38, 75), 2056, 264, False), ((2000, 600), 4104, 4200, False),
+])  # fmt: skip
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_kind_of_cut(tokens, inner, other, cut, dtype, device, monkeypatch):
+    tokens = list(tokens)
+    experts = len(tokens)
+    ends = torch.cumsum((torch.tensor(tokens) + 127) // 128 * 128, 0)
+    oracle_map = fixture_sparse_map({"expert_ends": ends.tolist(), "tokens_per_expert": tokens})
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    generator = torch.Generator(device=device).manual_seed(inner)
+
+    def normal(*shape):
+        return torch.empty(shape, dtype=dtype, device=device).normal_(0, _STD, generator=generator)
+
+    x, weight, weight_t = normal(oracle_map.num_rows, inner), normal(experts * inner, other), normal(experts * other, inner)
+    results = []
+    for workspace in (True, False):
+        monkeypatch.setattr(KernelConfig, "grouped_gemm_workspace", workspace)
+        results.append((input_inner_sparse_matmul(x, weight, sparse_map), output_sparse_matmul(x, weight_t.t(), sparse_map)))
+    expected = (
+        moe_oracle.input_inner_sparse_matmul(x.float(), weight.float(), oracle_map),
+        moe_oracle.output_sparse_matmul(x.float(), weight_t.t().float(), oracle_map),
+    )
+    for split, whole, reference in zip(*results, expected):
+        assert max_rel_err(split, reference) <= _MAX_REL[dtype]
+        assert max_rel_err(whole, reference) <= _MAX_REL[dtype]
+        assert torch.equal(split, whole) == (not cut)
