@@ -4,7 +4,7 @@
 // the rest of the router's front end around it; and the backward of both with respect to the logits.
 #include <type_traits>
 
-#include "fm_common.h"
+#include "fm_gemm_common.h"
 #include "fm_router_layout.h"
 
 namespace fm {
@@ -209,6 +209,7 @@ __global__ __launch_bounds__(kRouterMaxThreads) void router_forward_kernel(
         }
     }
 
+    if (block_counts == nullptr) return;
     // Sums of the workgroup's tokens: over the groups of a wavefront, then over the wavefronts in their order.
 #pragma unroll
     for (int offset = kGroup; offset < 64; offset <<= 1) {
@@ -234,7 +235,6 @@ __global__ __launch_bounds__(kRouterMaxThreads) void router_forward_kernel(
         if (kStatistics && lane == 0) wave_sums[experts] = z_sum;
     }
     __syncthreads();
-    if (block_counts == nullptr) return;
     for (int c = threadIdx.x; c < columns; c += blockDim.x) {
         if (c < experts) {
             int32_t total = 0;
@@ -387,6 +387,7 @@ __global__ __launch_bounds__(kRoutingThreads) void router_backward_kernel(
     else if (experts <= 64) { constexpr int kGroup = 64, kPerLane = 1; __VA_ARGS__; }                   \
     else if (experts <= 128) { constexpr int kGroup = 64, kPerLane = 2; __VA_ARGS__; }                  \
     else if (experts <= 256) { constexpr int kGroup = 64, kPerLane = 4; __VA_ARGS__; }                  \
+    else if (experts <= 512) { constexpr int kGroup = 64, kPerLane = 8; __VA_ARGS__; }                  \
     else { constexpr int kGroup = 64, kPerLane = kMaxPerLane; __VA_ARGS__; }
 
 }  // namespace fm
@@ -415,17 +416,29 @@ static int check_router_shape(const char *name, int64_t num_tokens, int64_t num_
 namespace fm {
 
 template <typename T, int kGroup, int kPerLane, bool kStatistics>
-static void launch_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
+static int launch_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
                                   int32_t *block_counts, float *block_sums, int64_t tokens, int experts, int k,
                                   int shared, hipStream_t stream) {
-    // 16 wavefronts per workgroup (there is one workgroup per CU at most), 4 where their sums would fill LDS.
-    const int threads = experts <= 256 ? kRouterMaxThreads : kRouterMaxThreads / 4;
-    const int columns = kStatistics ? RouterStats::size(experts) : experts;
-    router_forward_kernel<T, kGroup, kPerLane, kStatistics>
-        <<<router_blocks(tokens), threads, sizeof(float) * (threads / 64) * columns, stream>>>(
-            static_cast<const T *>(logits), static_cast<const T *>(noise), static_cast<int64_t *>(top_experts),
-            static_cast<float *>(scores), static_cast<float *>(lse), block_counts, block_sums, tokens,
-            router_tokens_per_block(tokens), experts, k, shared);
+    constexpr int kTokens = RouterShape<kGroup, kPerLane>::kTokens;
+    const auto kernel = router_forward_kernel<T, kGroup, kPerLane, kStatistics>;
+    // Where nobody wants counts a wavefront has its tokens once and no workgroup is asked what it did.
+    int blocks = static_cast<int>((tokens + kTokens * 4 - 1) / (kTokens * 4)), threads = 256;
+    int64_t per_block = kTokens * 4;
+    size_t lds = 0;
+    if (block_counts != nullptr) {
+        // One workgroup per CU at most, so 16 wavefronts, whose sums take up to 131 KB of its 160 (1024 experts).
+        blocks = router_blocks(tokens), per_block = router_tokens_per_block(tokens), threads = kRouterMaxThreads;
+        lds = sizeof(float) * (threads / 64) * (kStatistics ? RouterStats::size(experts) : experts);
+    }
+    if (lds > 64 * 1024) {
+        static std::atomic<uint64_t> configured{0};
+        constexpr int kMost = static_cast<int>(sizeof(float)) * (kRouterMaxThreads / 64) * (2 * 64 * kMaxPerLane + 1);
+        if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kMost, configured)) return status;
+    }
+    kernel<<<blocks, threads, lds, stream>>>(static_cast<const T *>(logits), static_cast<const T *>(noise),
+                                             static_cast<int64_t *>(top_experts), static_cast<float *>(scores),
+                                             static_cast<float *>(lse), block_counts, block_sums, tokens, per_block, experts, k, shared);
+    return FM_OK;
 }
 
 static int run_router_backward(const char *name, const void *grad_scores, const void *scores, const void *top_experts,
@@ -455,10 +468,10 @@ extern "C" int fm_topk_routing(const void *logits, void *top_experts, void *scor
     FM_REQUIRE(logits && top_experts && scores, "%s: null tensor", name);
     FM_DISPATCH_DTYPE(dtype, T, {
         FM_DISPATCH_ROUTER_SHAPE(num_experts, kGroup, kPerLane, {
-            launch_router_forward<T, kGroup, kPerLane, false>(logits, nullptr, top_experts, scores, nullptr, nullptr, nullptr,
-                                                              num_tokens, static_cast<int>(num_experts),
-                                                              static_cast<int>(experts_per_token), 0,
-                                                              static_cast<hipStream_t>(stream));
+            if (int status = launch_router_forward<T, kGroup, kPerLane, false>(
+                    logits, nullptr, top_experts, scores, nullptr, nullptr, nullptr, num_tokens, static_cast<int>(num_experts),
+                    static_cast<int>(experts_per_token), 0, static_cast<hipStream_t>(stream)))
+                return status;
         })
     });
     return check_launch(name);
@@ -498,8 +511,9 @@ extern "C" int fm_router_forward(const void *logits, const void *noise, void *to
         FM_DISPATCH_ROUTER_SHAPE(experts, kGroup, kPerLane, {
             auto launch = with_statistics ? launch_router_forward<T, kGroup, kPerLane, true>
                                           : launch_router_forward<T, kGroup, kPerLane, false>;
-            launch(logits, noise, top_experts, scores, lse, block_counts, block_sums, num_tokens, experts,
-                   static_cast<int>(experts_per_token), shared, stream);
+            if (int status = launch(logits, noise, top_experts, scores, lse, block_counts, block_sums, num_tokens, experts,
+                                    static_cast<int>(experts_per_token), shared, stream))
+                return status;
         })
     });
     if (with_statistics)
