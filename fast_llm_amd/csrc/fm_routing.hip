@@ -421,12 +421,14 @@ static int launch_router_forward(const void *logits, const void *noise, void *to
                                   int shared, hipStream_t stream) {
     constexpr int kTokens = RouterShape<kGroup, kPerLane>::kTokens;
     const auto kernel = router_forward_kernel<T, kGroup, kPerLane, kStatistics>;
-    // Where nobody wants counts a wavefront has its tokens once and no workgroup is asked what it did.
+    // Where nobody wants counts a wavefront has its tokens once and no workgroup is asked what it did: top 8 of 131072 tokens of
+    // 512 experts 159 us, 971 when 256 workgroups of 4 wavefronts walked over them.
     int blocks = static_cast<int>((tokens + kTokens * 4 - 1) / (kTokens * 4)), threads = 256;
     int64_t per_block = kTokens * 4;
     size_t lds = 0;
     if (block_counts != nullptr) {
-        // One workgroup per CU at most, so 16 wavefronts, whose sums take up to 131 KB of its 160 (1024 experts).
+        // One workgroup per CU at most, so 16 wavefronts, whose sums take up to 131 KB of its 160 (1024 experts). 131072 tokens
+        // of 512 experts 298 us, 1130 with 4 wavefronts.
         blocks = router_blocks(tokens), per_block = router_tokens_per_block(tokens), threads = kRouterMaxThreads;
         lds = sizeof(float) * (threads / 64) * (kStatistics ? RouterStats::size(experts) : experts);
     }
