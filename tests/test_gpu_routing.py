@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 # (tokens, experts, k): the reference's sparse-map test shapes plus the benchmark configurations' routers.
-_SHAPES = [(2048, 8, 2), (2048, 6, 2), (2048, 8, 8), (256, 8, 2), (5627, 8, 2), (2048, 64, 2), (512, 64, 6), (300, 128, 8), (7, 1000, 64), (1, 1, 1)]
+_SHAPES = [(2048, 8, 2), (2048, 6, 2), (2048, 8, 8), (256, 8, 2), (5627, 8, 2), (2048, 64, 2), (512, 64, 6), (300, 128, 8), (7, 1000, 64), (1, 1, 1),
+           (1003, 512, 8), (515, 513, 4)]
 
 
 def _distinct_logits(tokens, experts, dtype, generator):
@@ -42,8 +43,8 @@ def test_topk_routing_forward(tokens, experts, k, dtype, device):
 
 
 # Each side of the numbers of experts at which the kernels change how many lanes share a token (8, 16, 32, 64) and how
-# many logits a lane holds (128, 256), and of the token counts at which workgroups take more than 16 tokens (4096).
-@pytest.mark.parametrize("experts", [2, 9, 16, 17, 32, 33, 65, 129, 256, 257])
+# many logits a lane holds (128, 256, 512), and of the token counts at which workgroups take more than 16 tokens (4096).
+@pytest.mark.parametrize("experts", [2, 9, 16, 17, 32, 33, 65, 129, 256, 257, 512, 513, 1022])
 @pytest.mark.parametrize("tokens", [1, 17, 4096, 4111])
 def test_router_group_and_block_edges(tokens, experts, device):
     k, shared = min(experts, 5), 2

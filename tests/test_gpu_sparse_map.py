@@ -46,7 +46,7 @@ def test_benchmark_configurations(name, device):
 @pytest.mark.parametrize(
     ("tokens", "experts", "top_k", "pad"),
     [(1, 1, 1, 128), (1, 8, 8, 128), (3, 2, 1, 1), (1025, 3, 2, 64), (4096, 1, 1, 128), (777, 130, 5, 32),
-     (300, 1024, 4, 8), (64, 1000, 64, 16), (100000, 7, 3, 128)],
+     (300, 1024, 4, 8), (64, 1000, 64, 16), (100000, 7, 3, 128), (30000, 513, 2, 8), (5000, 65, 5, 128), (40000, 1024, 8, 128)],
 )
 def test_edge_shapes(tokens, experts, top_k, pad, device):
     torch.manual_seed(tokens + experts)
