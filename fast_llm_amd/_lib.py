@@ -158,7 +158,9 @@ class KernelTimer:
     Device-time of every kernel-library call made while the timer is active, from HIP events recorded on the launch
     stream right before and after the call. Used by the benchmark; costs two event records per call (each one a
     marker in the stream that the next kernel waits behind: some 3 us of device time per timed call). `only` restricts
-    the timer to the entry points whose name contains it.
+    the timer to the entry points whose name contains it. `layers.moe.DroplessMoEMLP` runs composed of its parts while a
+    timer is active, one entry point after the other: the same kernels and results, except that the products compute
+    padding rows as well and write a tile table each.
     """
 
     def __init__(self, only: str | None = None):

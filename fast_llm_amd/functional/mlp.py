@@ -402,19 +402,24 @@ def few_tokens_workspace_size(
     """Bytes that the kernels for few tokens need for `slots` experts per row of `input_`. 0 where they cannot be the faster way
     or do not take these operands: half precision, contiguous, 16-byte aligned, of sizes that fit together and that the library
     accepts. Everything else runs in the sparse layout, which also refuses what does not fit."""
-    dtype, ffn = input_.dtype, weight_2.size(0) // num_experts
-    if dtype not in (torch.bfloat16, torch.float16) or input_.dim() != 2 or is_traced():
+    dtype, rows_2 = input_.dtype, weight_2.size(0)
+    ffn = rows_2 // num_experts
+    if (dtype is not torch.bfloat16 and dtype is not torch.float16) or input_.dim() != 2 or is_traced():
         return 0
     tokens, hidden = input_.shape
     if (
         tokens * slots > FEW_TOKENS_MAX_ROWS_PER_EXPERT * num_experts
-        or not weight_1.dtype == weight_2.dtype == dtype
-        or weight_1.shape != (num_experts * ffn * (2 if gated else 1), hidden)
-        or weight_2.shape != (num_experts * ffn, hidden)
-        or not all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in (input_, weight_1, weight_2))
+        or weight_1.dtype is not dtype
+        or weight_2.dtype is not dtype
+        or weight_1.size(0) != (2 * rows_2 if gated else rows_2)
+        or weight_1.size(1) != hidden
+        or weight_2.size(1) != hidden
+        or rows_2 % num_experts != 0
+        or not (input_.is_contiguous() and weight_1.is_contiguous() and weight_2.is_contiguous())
+        or (input_.data_ptr() | weight_1.data_ptr() | weight_2.data_ptr()) % 16 != 0
     ):
         return 0
-    return _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), _lib.dtype_tag(dtype))
+    return _lib.lib().fm_few_tokens_workspace_size(tokens, slots, hidden, ffn, num_experts, int(gated), _lib.DTYPES[dtype])
 
 
 def few_tokens_forward(
