@@ -270,7 +270,8 @@ bool f32_gemm_eligible(const GemmArgs &args, int dtype) {
         return false;
     // 16-byte chunks must not straddle the end of an axis or of an expert's block.
     if (args.inner <= 0 || args.inner % 4 != 0 || args.sparse_size % 4 != 0 || args.cols % 4 != 0) return false;
-    if (!lhs_k && args.mode != kInputRowSparse && args.rows % 4 != 0) return false;
+    // Rows along the contiguous axis: an expert may start at any of them, and the last chunk would then end past the last row.
+    if (!lhs_k && args.mode != kInputRowSparse && (args.rows % 4 != 0 || args.expert_ends != nullptr)) return false;
     if (args.inner >= (int64_t(1) << 30)) return false;
     // Per-lane byte offsets inside a slice are below 2^31: at most 64 lines.
     return max(max(args.lhs_stride_row, args.lhs_stride_inner), max(args.rhs_stride_inner, args.rhs_stride_col)) < (int64_t(1) << 21);

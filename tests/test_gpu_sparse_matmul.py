@@ -616,6 +616,24 @@ def test_fp32_tiles_and_remainders(inner, other, device):
     assert max_rel_err(dense.cpu(), weight.cpu() @ weight_inner[:inner].cpu()) <= 1e-5
 
 
+# Activations whose rows lie along the contiguous axis, with experts that start at any row, the last one within four rows of the end:
+# nothing past the operand's last element is read (it is the last of its allocation's rows and columns here).
+@pytest.mark.parametrize("ends", [[125, 128], [64, 65, 127, 128], [128, 256]])
+def test_fp32_rows_along_the_contiguous_axis(ends, device):
+    tokens = [end - begin for begin, end in zip([0] + ends, ends)]
+    oracle_map = fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": tokens})
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    generator = torch.Generator().manual_seed(0)
+    x = _normal(ends[-1], 64, torch.float32, generator)
+    along_rows = x.t().contiguous().to(device).t()
+    weight = _normal(len(ends) * 36, 64, torch.float32, generator)
+    expected = moe_oracle.output_sparse_matmul(x.double(), weight.t().double(), oracle_map)
+    assert max_rel_err(output_sparse_matmul(along_rows, weight.to(device).t(), sparse_map).cpu(), expected) <= 1e-5
+    weight = _normal(len(ends) * 64, 36, torch.float32, generator)
+    expected = moe_oracle.input_inner_sparse_matmul(x.double(), weight.double(), oracle_map)
+    assert max_rel_err(input_inner_sparse_matmul(along_rows, weight.to(device), sparse_map).cpu(), expected) <= 1e-5
+
+
 # fp32 operands of odd sizes, K-contiguous row-sparse ones and a half-precision result, in launches of more than 165 tiles of 128 x
 # 128, with expert boundaries on and off the tiles' grid.
 @pytest.mark.parametrize("pad", [128, 8])
