@@ -716,7 +716,7 @@ def test_one_expert_of_more_than_4_gib(device):
     """An expert whose rows span more than 4 GiB of a row-major operand (528 384 rows of 4096 bf16 values = 4.33 GB,
     after a first expert of 256 rows): byte offsets inside one expert's block exceed 32 bits in all three products,
     along the rows of the output-sparse and inner-sparse products and along the reduction of the row-sparse one
-    (8256 slices of 64). Operands are drawn on the GPU and the checker is the oracle evaluated there in fp32: on the CPU
+    (8256 slices of 64). Operands are drawn on the GPU and the reference is the oracle evaluated there in fp32: on the CPU
     it would take minutes."""
     dtype, wide, narrow = torch.bfloat16, 4096, 256
     case = {"expert_ends": [256, 256 + 528384], "tokens_per_expert": [200, 528300]}
@@ -759,7 +759,7 @@ def test_one_expert_of_more_than_4_gib(device):
 def test_random_launches_of_many_rounds(block, device):
     """Random ragged layouts large enough for launches of several rounds of workgroups (hundreds to thousands of tiles:
     the tile table, a workgroup walking from tile to tile, half tiles, experts without tokens, split last rounds),
-    all three products. Operands are drawn on the GPU and the checker is the oracle evaluated there in fp32."""
+    all three products. Operands are drawn on the GPU and the reference is the oracle evaluated there in fp32."""
     for seed in range(30 * block, 30 * (block + 1)):
         generator = torch.Generator().manual_seed(5000 + seed)
 
@@ -856,7 +856,7 @@ def test_split_reductions_of_no_whole_number_of_slices(experts, inner, other, dt
 # Every cut that the plan knows: 2, 3, 4 and 8 pieces of a round's few tiles; whole tiles before them; more pieces than CUs (two
 # rounds of pieces); the same of reductions that are no whole number of slices, whose last piece is masked; and what is too short
 # or has too many tiles to be cut. Against the unsplit sums that a call without a workspace takes: where there is a cut the bits
-# differ. Operands are drawn on the GPU and the checker is the oracle evaluated there in fp32.
+# differ. Operands are drawn on the GPU and the reference is the oracle evaluated there in fp32.
 @pytest.mark.parametrize(("tokens", "inner", "other", "cut"), [
     ((3, 150, 77), 36 * 64, 264, True), ((3, 150, 77), 39 * 64, 264, True),  # 2 pieces, the second one shorter
     ((3, 150, 77), 50 * 64, 264, True), ((200, 0, 130), 72 * 64, 520, True), ((40,), 128 * 64, 72, True),  # 3, 4, 8
