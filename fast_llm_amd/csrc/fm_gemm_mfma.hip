@@ -532,14 +532,17 @@ struct alignas(64) TableHeader {
 };
 static_assert(sizeof(TableHeader) == 64 && sizeof(TableHeader) == sizeof(TileRecord), "the header is record -1");
 
-// The products whose tables are written together, one per blockIdx.y.
+// The products whose tables are written together, one per blockIdx.y. One alone has an instance of its own: five products' arguments
+// are 1.2 KB that every launch brings along.
+template <int kCount>
 struct PlannedProducts {
-    GemmArgs products[kMaxPlanned];
+    GemmArgs products[kCount];
 };
 
 // One wavefront per id; the wavefront of id 0 also leaves the split plan of the launch in the table's header.
-__global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(PlannedProducts planned) {
-    const GemmArgs &args = planned.products[blockIdx.y];
+template <int kCount>
+__global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(PlannedProducts<kCount> planned) {
+    const GemmArgs &args = planned.products[kCount == 1 ? 0 : blockIdx.y];
     TileRecord *table = static_cast<TileRecord *>(args.tile_table);
     const int id = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (id >= args.num_ids) return;
@@ -1485,14 +1488,20 @@ size_t mfma_gemm_workspace_size(GemmArgs args) {
 // few thousand cycles) sooner than a kernel launched in front of it could tell it.
 static bool wants_table(const GemmArgs &args, bool split) { return split || args.num_ids > kRound; }
 
-static int launch_plan(const GemmArgs *products, int count, hipStream_t stream) {
-    PlannedProducts planned;
+template <int kCount>
+static void launch_plan_of(const GemmArgs *products, int count, hipStream_t stream) {
+    PlannedProducts<kCount> planned;
     int most_ids = 0;
     for (int i = 0; i < count; ++i) {
         planned.products[i] = products[i];
         most_ids = max(most_ids, products[i].num_ids);
     }
-    grouped_gemm_plan_kernel<<<dim3((most_ids + 3) / 4, count), 256, 0, stream>>>(planned);
+    grouped_gemm_plan_kernel<kCount><<<dim3((most_ids + 3) / 4, count), 256, 0, stream>>>(planned);
+}
+
+static int launch_plan(const GemmArgs *products, int count, hipStream_t stream) {
+    if (count == 1) launch_plan_of<1>(products, count, stream);
+    else launch_plan_of<kMaxPlanned>(products, count, stream);
     return FM_OK;
 }
 
