@@ -185,8 +185,10 @@ class DroplessMoEMLP(torch.nn.Module):
             # The router has counted the tokens of every expert on its way: the map need not count them again.
             scores, top_experts, router_counts = self.route_with_counts(hidden_states, grad_scale, losses)
         if few_tokens and scores is not None:
+            # A routing of the caller's own may select another number of experts than the size is for.
+            workspace_size = few_tokens if top_experts.size(-1) == slots else None
             output = few_tokens_forward(
-                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation, few_tokens
+                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation, workspace_size
             )  # fmt: skip
             if output is not None:
                 return without_backward(output).view_as(input_)

@@ -208,9 +208,10 @@ def test_collected_losses_keep_no_buffer_of_the_layer(training, device):
 @pytest.mark.parametrize("tokens", [8, 512])
 @pytest.mark.parametrize("training", [False, True])
 @pytest.mark.parametrize("subclass", [False, True])
-def test_replaced_routing_is_honoured(tokens, training, subclass, device):
+@pytest.mark.parametrize("selected", [1, 2, 3])
+def test_replaced_routing_is_honoured(tokens, training, subclass, selected, device):
     def first_experts(self, hidden_states, grad_scale=None, losses=None):
-        experts = torch.arange(2, device=hidden_states.device).expand(hidden_states.size(0), 2).contiguous()
+        experts = torch.arange(selected, device=hidden_states.device).expand(hidden_states.size(0), selected).contiguous()
         return torch.full(experts.shape, 0.5, device=hidden_states.device), experts, None
 
     torch.manual_seed(0)
