@@ -5,6 +5,7 @@ Autograd glue and argument checks (reference: fast_llm/functional/utils.py:13-56
 import typing
 
 import torch
+from torch.autograd import forward_ad
 
 
 class Assert:
@@ -49,7 +50,7 @@ def without_backward(output: torch.Tensor) -> torch.Tensor:
 def is_traced() -> bool:
     """Whether forward-mode differentiation or `torch.jit`'s tracer looks at what runs. They know the autograd functions and
     refuse or record them; a tangent or a result of what runs outside them would be lost silently, so that steps aside."""
-    return torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing()
+    return forward_ad._current_level >= 0 or torch.jit.is_tracing()
 
 
 class _ForwardBackwardPair(torch.autograd.Function):

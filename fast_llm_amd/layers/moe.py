@@ -172,13 +172,11 @@ class DroplessMoEMLP(torch.nn.Module):
         hidden_states = input_.flatten(0, -2)
         router_counts = None
         few_tokens = 0  # bytes that the kernels for few tokens need, where they are the route
+        layer_1, layer_2 = self.layer_1, self.layer_2  # looking a parameter up takes a module half a microsecond
         if not self.training:
             slots = self.shared_experts + self.experts_per_token if top_experts is None else top_experts.size(-1)
-            ffn = self.layer_2.size(0) // self.experts
-            if few_tokens_expected(hidden_states.size(0), slots, self.shared_experts, self.experts, ffn):
-                few_tokens = few_tokens_workspace_size(
-                    hidden_states, slots, self.layer_1, self.layer_2, self.experts, self.gated
-                )
+            if few_tokens_expected(hidden_states.size(0), slots, self.shared_experts, self.experts, layer_2.size(0) // self.experts):
+                few_tokens = few_tokens_workspace_size(hidden_states, slots, layer_1, layer_2, self.experts, self.gated)
         if top_experts is None and not few_tokens and self._is_one_call(hidden_states):
             return self._forward_in_one_call(hidden_states, grad_scale, losses).view_as(input_)
         if top_experts is None:
@@ -188,7 +186,7 @@ class DroplessMoEMLP(torch.nn.Module):
             # A routing of the caller's own may select another number of experts than the size is for.
             workspace_size = few_tokens if top_experts.size(-1) == slots else None
             output = few_tokens_forward(
-                hidden_states, scores, top_experts, self.layer_1, self.layer_2, self.experts, self.gated, self.activation, workspace_size
+                hidden_states, scores, top_experts, layer_1, layer_2, self.experts, self.gated, self.activation, workspace_size
             )  # fmt: skip
             if output is not None:
                 return without_backward(output).view_as(input_)
@@ -198,9 +196,9 @@ class DroplessMoEMLP(torch.nn.Module):
         output = mlp_autograd(
             hidden_states,
             scores,
-            self.layer_1,
+            layer_1,
             None,
-            self.layer_2,
+            layer_2,
             None,
             gated=self.gated,
             activation_type=self.activation,
