@@ -1,26 +1,18 @@
-// Grouped matrix products of fp32 operands on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32: true fp32
-// multiply-adds, which is what the 1e-5 fp32 parity bound needs).
-//
-// An MFMA of this kind keeps the matrix pipe busy for 64 cycles and needs two 256-byte operand fragments, so neither
-// LDS nor address arithmetic is near a limit; what has to be hidden is memory latency, and many small workgroups per CU
-// hide it better than deep pipelines: eight of them (16 KiB of LDS, at most 64 registers per lane), each one slice
-// ahead. Tiles of 128 x 128 with two or three workgroups per CU and two to four slots were slower at every size tried,
-// and so were fewer workgroups with more slots. Forward and backward products of 4096 rows over 8 experts, 1024 x 2816
-// (5632): 5350 us for the six on tiles of 128 x 128 x 16 fetched element by element through registers, 2120 here (88 to
-// 116 TFLOP/s of rows that exist; padding is another 12 %; the device's library reaches 153 on a dense product).
+// Grouped matrix products of fp32 operands on the gfx950 matrix cores, by one of two instructions:
+//   * v_mfma_f32_32x32x16_bf16 on operands split into three bf16 parts each (`grouped_gemm_f32_split_kernel`, below): six
+//     products of parts instead of one of values at 16 times the rate of fp32 multiply-adds;
+//   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for reductions so short that start and epilogue are all there is.
+// Forward and backward products of 4096 rows over 8 experts, 1024 x 2816 (5632): 2111 us for the six on fp32 multiply-adds, 1403 on
+// split operands.
 //   * Operand slices (kBK reduction indices) go straight from global memory into LDS (`buffer_load ... lds`, 16 bytes
-//     per lane), one slice ahead of the multiplications, one barrier per slice. Lanes that have nothing to fetch (rows past the tile's last one, indices past the reduction range) are sent out of the buffer's range and
-//     bring zeros.
+//     per lane), at least one slice ahead of the multiplications, one barrier per slice. Lanes that have nothing to fetch (rows
+//     past the tile's last one, indices past the reduction range) are sent out of the buffer's range and bring zeros.
 //   * An operand may be contiguous along K (activations, `weight.t()`): stored [row][K], fragments are 128-bit reads of
 //     four K values of one row; or along its other axis (`weight`, `activations.t()`): stored [K][row] as in memory,
-//     fragments are four 32-bit reads. A group of eight K values is split over the wavefront's halves as 0..3 and 4..7;
+//     fragments are 32-bit reads. A group of K values is split over the wavefront's halves, first half and second half;
 //     both layouts agree on that, and the order of a sum is free. Chunks are XOR-swizzled on the global side so that
 //     fragment reads hit all banks.
 //   * Tiles never straddle experts (they are enumerated per expert from `expert_ends`), so any padding multiple works.
-// Two tiles, by how many there are (see `f32_gemm_launch`):
-//   64 x 64, 4 wavefronts of 32 x 32;
-//   32 x 32, the 4 wavefronts take a quarter of every slice each and add up in LDS: four times the workgroups, for
-//   launches whose outputs are too few to fill the CUs otherwise.
 #include "fm_gemm_common.h"
 
 namespace fm {
@@ -29,11 +21,15 @@ namespace f32 {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2_t;
+typedef __attribute__((__vector_size__(8 * sizeof(bf16_t)))) bf16_t bf16x8_t;
+typedef __attribute__((__vector_size__(2 * sizeof(bf16_t)))) bf16_t bf16x2_t;
 
 constexpr int kThreads = 256;
 
 // One operand's slice in LDS and the loads that fill it.
-template <int kTile, int kBK, bool kContiguousK>
+// `kGroup`: reduction indices that a wavefront multiplies at a time, the first half of them in its lanes 0..31.
+template <int kTile, int kBK, int kGroup, bool kContiguousK>
 struct Operand {
     static constexpr int kBytes = kTile * kBK * 4;
     static constexpr int kLoads = kBytes / 16 / kThreads;              // 16-byte loads per lane and slice
@@ -46,7 +42,7 @@ struct Operand {
             constexpr int kLinesPer256 = kBK >= 64 ? 1 : 64 / kBK;
             return c ^ ((line / kLinesPer256) & (kChunks < 16 ? kChunks - 1 : 15));
         } else {
-            return c ^ (kChunks > 8 ? ((line >> 2) & 1) << 3 : 0);
+            return c ^ (kChunks > 8 ? (line / (kGroup / 2) & 1) << 3 : 0);
         }
     }
 
@@ -89,20 +85,20 @@ struct Operand {
         k_left -= kBK;
     }
 
-    // The lane's four K values (8 q + 4 half + 0 .. 3) of row `row`, from the slot at byte address `slot`.
-    static __device__ __forceinline__ void fragment(int slot, int row, int q, int half, float (&values)[4]) {
+    // The lane's K values (kGroup (q + half / 2) + 0, 1, ...) of row `row`, from the slot at byte address `slot`.
+    static __device__ __forceinline__ void fragment(int slot, int row, int q, int half, float (&values)[kGroup / 2]) {
         if constexpr (kContiguousK) {
-            const int address = slot + (row * kChunks + swizzled(row, 2 * q + half)) * 16;
-            const f32x4_t vector = *(FM_LDS(f32x4_t) *)static_cast<uintptr_t>(address);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) values[i] = vector[i];
-        } else {
+            for (int c = 0; c < kGroup / 8; ++c) {
+                const int address = slot + (row * kChunks + swizzled(row, (2 * q + half) * (kGroup / 8) + c)) * 16;
+                const f32x4_t vector = *(FM_LDS(f32x4_t) *)static_cast<uintptr_t>(address);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int k = 8 * q + 4 * half + i;
-                const int address = slot + k * kTile * 4 + swizzled(k, row >> 2) * 16 + (row & 3) * 4;
-                values[i] = *(FM_LDS(float) *)static_cast<uintptr_t>(address);
+                for (int i = 0; i < 4; ++i) values[4 * c + i] = vector[i];
             }
+        } else {
+            const int address = slot + (kGroup * q + kGroup / 2 * half) * kTile * 4 + ((row >> 2) ^ (kChunks > 8 ? half << 3 : 0)) * 16 + (row & 3) * 4;
+#pragma unroll
+            for (int i = 0; i < kGroup / 2; ++i) values[i] = *(FM_LDS(float) *)static_cast<uintptr_t>(address + i * kTile * 4);
         }
     }
 };
@@ -112,32 +108,31 @@ __device__ __forceinline__ void wait_for_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNewest) : "memory");
 }
 
-template <int kTile, int kBK, int kStages, bool kLhsK, bool kRhsK>
-__global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs args) {
-    constexpr int kWavesK = kTile == 32 ? 4 : 1, kWavesN = kTile == 32 ? 1 : 2;
-    constexpr int kWaveTile = kTile / kWavesN, kBlocks = kWaveTile / 32;
-    typedef Operand<kTile, kBK, kLhsK> Lhs;
-    typedef Operand<kTile, kBK, kRhsK> Rhs;
-    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
-    constexpr int kSteps = kBK / 8 / kWavesK;  // groups of eight K values per wavefront and slice
-    extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
-    const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
+// Where a workgroup's tile and its operands lie.
+struct TileOperands {
+    int64_t lhs_offset, rhs_offset, out_offset;  // elements
+    int rows_valid, cols_valid, k_count;
+    bool exists;
+};
 
+template <int kTileM, int kTileN>
+__device__ __forceinline__ TileOperands find_tile(const GemmArgs &args) {
+    TileOperands found;
+    found.exists = false;
     // Consecutive workgroup ids go to the 8 XCDs in turn; an XCD gets runs of `chunk_tiles` consecutive logical tiles.
     const int pid = blockIdx.x, local = pid / 8;
     const int logical = (local / args.chunk_tiles * 8 + pid % 8) * args.chunk_tiles + local % args.chunk_tiles;
-    int64_t lhs_offset, rhs_offset, out_offset, k_lo = 0, k_hi = args.inner;
-    int rows_valid, cols_valid;
+    int64_t k_lo = 0, k_hi = args.inner;
     if (args.mode == kInputRowSparse) {
-        if (logical >= args.tiles_m * args.tiles_n) return;
+        if (logical >= args.tiles_m * args.tiles_n) return found;
         int tile_m, tile_n;
         tile_coordinates(logical, args.tiles_m, args.tiles_n, tile_m, tile_n);
-        const int tiles_per_expert = static_cast<int>((args.sparse_size + kTile - 1) / kTile);
+        const int tiles_per_expert = static_cast<int>((args.sparse_size + kTileM - 1) / kTileM);
         const int expert = tile_m / tiles_per_expert;
-        const int64_t row = static_cast<int64_t>(tile_m - expert * tiles_per_expert) * kTile;
-        const int64_t col0 = static_cast<int64_t>(tile_n) * kTile;
-        rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.sparse_size - row));
-        cols_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.cols - col0));
+        const int64_t row = static_cast<int64_t>(tile_m - expert * tiles_per_expert) * kTileM;
+        const int64_t col0 = static_cast<int64_t>(tile_n) * kTileN;
+        found.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTileM), args.sparse_size - row));
+        found.cols_valid = static_cast<int>(min(static_cast<int64_t>(kTileN), args.cols - col0));
         if (args.expert_ends != nullptr) {
             k_lo = expert > 0 ? load_index(args.expert_ends, args.index_dtype, expert - 1) : 0;
             k_hi = load_index(args.expert_pad_begins, args.index_dtype, expert);
@@ -147,26 +142,50 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
             k_lo = expert * args.piece_length;
             k_hi = min(k_lo + args.piece_length, args.inner);
         }
-        lhs_offset = row * args.lhs_stride_row + k_lo * args.lhs_stride_inner;
-        rhs_offset = col0 * args.rhs_stride_col + k_lo * args.rhs_stride_inner;
-        out_offset = (expert * args.sparse_size + row) * args.out_stride_row + col0;
+        found.lhs_offset = row * args.lhs_stride_row + k_lo * args.lhs_stride_inner;
+        found.rhs_offset = col0 * args.rhs_stride_col + k_lo * args.rhs_stride_inner;
+        found.out_offset = (expert * args.sparse_size + row) * args.out_stride_row + col0;
     } else {
         RowTile tile;
-        if (!locate_tile<kTile>(args, logical, tile)) return;
-        const int64_t col0 = static_cast<int64_t>(tile.tile_n) * kTile;
-        rows_valid = tile.rows_valid;
-        cols_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.cols - col0));
-        lhs_offset = tile.row0 * args.lhs_stride_row;
-        out_offset = tile.row0 * args.out_stride_row + col0;
-        rhs_offset = args.mode == kOutputSparse
+        if (!locate_tile<kTileM>(args, logical, tile)) return found;
+        const int64_t col0 = static_cast<int64_t>(tile.tile_n) * kTileN;
+        found.rows_valid = tile.rows_valid;
+        found.cols_valid = static_cast<int>(min(static_cast<int64_t>(kTileN), args.cols - col0));
+        found.lhs_offset = tile.row0 * args.lhs_stride_row;
+        found.out_offset = tile.row0 * args.out_stride_row + col0;
+        found.rhs_offset = args.mode == kOutputSparse
                          ? (static_cast<int64_t>(tile.expert) * args.sparse_size + col0) * args.rhs_stride_col
                          : static_cast<int64_t>(tile.expert) * args.sparse_size * args.rhs_stride_inner + col0 * args.rhs_stride_col;
     }
-    const int k_count = __builtin_amdgcn_readfirstlane(static_cast<int>(max(k_hi - k_lo, static_cast<int64_t>(0))));
-    const int num_slices = (k_count + kBK - 1) / kBK;
-    rows_valid = __builtin_amdgcn_readfirstlane(rows_valid);
-    cols_valid = __builtin_amdgcn_readfirstlane(cols_valid);
+    found.k_count = __builtin_amdgcn_readfirstlane(static_cast<int>(max(k_hi - k_lo, static_cast<int64_t>(0))));
+    found.rows_valid = __builtin_amdgcn_readfirstlane(found.rows_valid);
+    found.cols_valid = __builtin_amdgcn_readfirstlane(found.cols_valid);
+    found.exists = true;
+    return found;
+}
 
+// fp32 multiply-adds. An MFMA of this kind keeps the matrix pipe busy for 64 cycles and needs two 256-byte operand fragments, so
+// neither LDS nor address arithmetic is near a limit; what has to be hidden is memory latency, and many small workgroups per CU
+// hide it better than deep pipelines: eight of them (16 KiB of LDS, at most 64 registers per lane), each one slice ahead.
+//   64 x 64, 4 wavefronts of 32 x 32;
+//   32 x 32, the 4 wavefronts take a quarter of every slice each and add up in LDS: four times the workgroups, for
+//   launches whose outputs are too few to fill the CUs otherwise.
+template <int kTile, int kBK, int kStages, bool kLhsK, bool kRhsK>
+__global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs args) {
+    constexpr int kWavesK = kTile == 32 ? 4 : 1, kWavesN = kTile == 32 ? 1 : 2;
+    constexpr int kWaveTile = kTile / kWavesN, kBlocks = kWaveTile / 32;
+    typedef Operand<kTile, kBK, 8, kLhsK> Lhs;
+    typedef Operand<kTile, kBK, 8, kRhsK> Rhs;
+    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
+    constexpr int kSteps = kBK / 8 / kWavesK;  // groups of eight K values per wavefront and slice
+    extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
+    const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
+
+    const TileOperands tile = find_tile<kTile, kTile>(args);
+    if (!tile.exists) return;
+    const int k_count = tile.k_count, rows_valid = tile.rows_valid, cols_valid = tile.cols_valid;
+    const int64_t lhs_offset = tile.lhs_offset, rhs_offset = tile.rhs_offset, out_offset = tile.out_offset;
+    const int num_slices = (k_count + kBK - 1) / kBK;
     const int lane = threadIdx.x & 63, half = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wave_m = kWavesK > 1 ? 0 : wave / kWavesN, wave_n = kWavesK > 1 ? 0 : wave % kWavesN;
     const int first_step = kWavesK > 1 ? wave * kSteps : 0;
@@ -254,6 +273,243 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
     }
 }
 
+// ---- operands split into bf16 parts ---------------------------------------------------------------------------------------
+// A value is the sum of three bf16 (8 significant bits each): the nearest to it, to the rest, and to the rest of that. Of the nine
+// products of two values' parts, the six above 2^-25 of the whole are taken, in fp32 accumulators of their own for the five small
+// kinds, so that the large sum is rounded once per 16 reduction indices (every 2 on fp32 multiply-adds) and results are nearer to
+// 64 bits than those: relative 1.9e-7 against 5.7e-7 (layer 1, 1024 reduction indices), 1.6e-7 against 4.8e-7 (layer 2, 2816),
+// 1.3e-7 against 4.1e-7 (weight gradients, 512), and for all shapes and products measured.
+//
+// The parts carry what fp32 does down to 2^-110, where the third meets the end of bf16's range (2^-133), and up to where bf16
+// rounds to infinity. A result that is NaN, infinite or below 2^-90 (and not zero) may have met either: its tile is
+// computed again by fp32 multiply-adds, which such results are taken from. (An operand below 2^-110 among
+// larger ones loses what lies below 2^-134, which no sum of normal size shows.)
+//
+// Every wavefront splits the fragments it multiplies: 7.3 vector instructions per MFMA of 32 cycles, interleaved with the MFMAs of
+// the fragments before (two wavefronts per SIMD; 6 such instructions cost an MFMA nothing, and the residual as a bf16 dot product,
+// half as many instructions, 5 cycles each of the matrix pipe). Splitting once per workgroup instead would move 6 bytes per
+// element through LDS both ways, which is as long as the MFMAs take. The device then runs at 1.84 GHz: power.
+// A wavefront computes 64 x 64 of the tile; the four of them are
+//   128 x 128: 2 x 2 of the tile, slices of 16;
+//   128 x 64: 2 of the tile x 2 halves of a slice of 32;
+//   64 x 64: 4 quarters of a slice of 64
+// (halves and quarters add up in LDS), by how many tiles there are: see `f32_gemm_launch`.
+
+__device__ __forceinline__ void split(const float (&values)[8], bf16x8_t (&parts)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float rest_0 = values[2 * i], rest_1 = values[2 * i + 1];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const bf16x2_t pair = __builtin_convertvector((f32x2_t{rest_0, rest_1}), bf16x2_t);
+            parts[p][2 * i] = pair[0];
+            parts[p][2 * i + 1] = pair[1];
+            const uint32_t bits = __builtin_bit_cast(uint32_t, pair);
+            rest_0 -= __builtin_bit_cast(float, bits << 16);
+            rest_1 -= __builtin_bit_cast(float, bits & 0xffff0000u);
+        }
+    }
+}
+
+// Six times: one MFMA, seven vector instructions.
+__device__ __forceinline__ void interleave() {
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 7, 0);
+    }
+}
+
+constexpr int kNanInfOrSubnormal = 0x001 | 0x002 | 0x004 | 0x200 | 0x010 | 0x080;  // classes of v_cmp_class
+
+template <int kTileM, int kTileN, int kStages, bool kLhsK, bool kRhsK>
+__global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f32_split_kernel(GemmArgs args) {
+    constexpr int kWavesM = kTileM / 64, kWavesN = kTileN / 64, kWavesK = 4 / (kWavesM * kWavesN), kBK = 16 * kWavesK;
+    typedef Operand<kTileM, kBK, 16, kLhsK> Lhs;
+    typedef Operand<kTileN, kBK, 16, kRhsK> Rhs;
+    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
+    extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
+    const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
+    const TileOperands tile = find_tile<kTileM, kTileN>(args);
+    if (!tile.exists) return;
+    const int num_slices = (tile.k_count + kBK - 1) / kBK;
+    const int lane = threadIdx.x & 63, half = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_k = wave % kWavesK, wave_m = wave / kWavesK / kWavesN, wave_n = wave / kWavesK % kWavesN;
+    const int lhs_row = wave_m * 64 + (lane & 31), rhs_row = wave_n * 64 + (lane & 31);
+
+    // Slice t sits in slot t % kStages; slices past the last one are fetched as zeros.
+    Lhs lhs;
+    Rhs rhs;
+    int fetch_slot;
+    const auto fetch_slice = [&]() {
+        lhs.fetch(lds + fetch_slot, wave);
+        rhs.fetch(lds + fetch_slot + Lhs::kBytes, wave);
+        fetch_slot = fetch_slot == (kStages - 1) * kSlotBytes ? 0 : fetch_slot + kSlotBytes;
+    };
+    const auto start = [&]() {
+        lhs.setup(reinterpret_cast<const char *>(static_cast<const float *>(args.lhs) + tile.lhs_offset),
+                  (kLhsK ? args.lhs_stride_row : args.lhs_stride_inner) * 4, tile.rows_valid, tile.k_count, wave, lane);
+        rhs.setup(reinterpret_cast<const char *>(static_cast<const float *>(args.rhs) + tile.rhs_offset),
+                  (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 4, tile.cols_valid, tile.k_count, wave, lane);
+        fetch_slot = 0;
+#pragma unroll
+        for (int s = 0; s < kStages - 1; ++s) fetch_slice();
+    };
+    // Every wavefront has waited for its loads of the slice after those in flight, and has read the slice before it: that
+    // slice is visible after the barrier, and the slot of the one before can be filled.
+    const auto next_slice = [&]() {
+        wait_for_loads<(kStages - 2) * kLoads>();
+        __syncthreads();
+        fetch_slice();
+    };
+    float a[2][8], b[2][8];
+    const auto read = [&](int slot, int i) {
+        Lhs::fragment(lds + slot, lhs_row + i * 32, wave_k, half, a[i]);
+        Rhs::fragment(lds + slot + Lhs::kBytes, rhs_row + i * 32, wave_k, half, b[i]);
+    };
+    // Operands swapped in all MFMAs: a lane holds one row of a block of 32 x 32 and groups of four consecutive columns.
+    f32x16_t acc[2][2];
+    {
+        f32x16_t small[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = small[i][j][v] = 0.f;
+        bf16x8_t a_parts[2][3], b_parts[2][3];
+        const auto multiply = [&](int i, int j) {
+#pragma unroll
+            for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+                for (int p = 0; p <= sum; ++p) {
+                    f32x16_t &target = sum == 0 ? acc[i][j] : small[i][j];
+                    target = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b_parts[j][sum - p], a_parts[i][p], target, 0, 0, 0);
+                }
+        };
+        start();
+        next_slice();
+        read(0, 0);
+        read(0, 1);
+        split(a[0], a_parts[0]);
+        split(b[0], b_parts[0]);
+        int next = 0;  // slot of the slice to read
+        for (int t = 0; t < num_slices; ++t) {
+            // Here the first fragments of slice t are split, the second ones read.
+            next = next == (kStages - 1) * kSlotBytes ? 0 : next + kSlotBytes;
+            next_slice();
+            read(next, 0);
+            split(b[1], b_parts[1]);
+            multiply(0, 0);
+            interleave();
+            split(a[1], a_parts[1]);
+            multiply(0, 1);
+            interleave();
+            read(next, 1);
+            bf16x8_t a_next[3], b_next[3];
+            split(a[0], a_next);
+            multiply(1, 0);
+            interleave();
+            split(b[0], b_next);
+            multiply(1, 1);
+            interleave();
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                a_parts[0][p] = a_next[p];
+                b_parts[0][p] = b_next[p];
+            }
+        }
+        wait_for_loads<0>();  // the zero-filling loads past the end still write LDS
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] += small[i][j];
+    }
+
+    // The sums over the wavefronts that share a reduction, in wavefront order; each then holds kHeld of its four blocks.
+    constexpr int kHeld = 4 / kWavesK;
+    const auto add_shares = [&]() {
+        if constexpr (kWavesK > 1) {
+            static_assert(kStages * kSlotBytes >= 4 * 4 * 4096 || kWavesK == 1, "space for four wavefronts' blocks");
+            const auto share = [&](int from, int g) { return (FM_LDS(f32x4_t) *)static_cast<uintptr_t>(lds + ((from * 16 + g) * 64 + lane) * 16); };
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < 16; ++g) {
+                const f32x16_t &block = acc[g / 8][g / 4 % 2];
+                *share(wave, g) = f32x4_t{block[g % 4 * 4], block[g % 4 * 4 + 1], block[g % 4 * 4 + 2], block[g % 4 * 4 + 3]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < 4 * kHeld; ++g) {
+                f32x4_t sum = *share(wave - wave_k, wave_k * 4 * kHeld + g);
+#pragma unroll
+                for (int w = 1; w < kWavesK; ++w) sum += *share(wave - wave_k + w, wave_k * 4 * kHeld + g);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[g / 8][g / 4 % 2][g % 4 * 4 + v] = sum[v];
+            }
+        }
+    };
+    add_shares();
+    const auto in_doubt = [](float value) { return __builtin_amdgcn_classf(value * 0x1p-36f, kNanInfOrSubnormal); };
+    bool again = false;
+#pragma unroll
+    for (int held = 0; held < kHeld; ++held)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) again |= in_doubt(acc[held / 2][held % 2][v]);
+    if (__syncthreads_or(again)) {
+        f32x16_t first[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                first[i][j] = acc[i][j];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+            }
+        start();
+        int slot = 0;
+        for (int t = 0; t < num_slices; ++t) {
+            next_slice();
+            read(slot, 0);
+            read(slot, 1);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][k], a[i][k], acc[i][j], 0, 0, 0);
+            slot = slot == (kStages - 1) * kSlotBytes ? 0 : slot + kSlotBytes;
+        }
+        wait_for_loads<0>();
+        add_shares();
+        // What was in no doubt stays: the other rows and columns of the tile, padding with whatever it holds, change nobody's result.
+#pragma unroll
+        for (int held = 0; held < kHeld; ++held)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float value = first[held / 2][held % 2][v];
+                if (!in_doubt(value)) acc[held / 2][held % 2][v] = value;
+            }
+    }
+#pragma unroll
+    for (int held = 0; held < kHeld; ++held) {
+        const int block = wave_k * kHeld + held;
+        const int row = wave_m * 64 + block / 2 * 32 + (lane & 31);
+        if (row >= tile.rows_valid) continue;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int column = wave_n * 64 + block % 2 * 32 + 8 * g + 4 * half;
+            if (column >= tile.cols_valid) continue;  // a multiple of 4
+            const f32x16_t &from = acc[held / 2][held % 2];
+            f32x4_t value = f32x4_t{from[4 * g], from[4 * g + 1], from[4 * g + 2], from[4 * g + 3]};
+            float *target = static_cast<float *>(args.out) + tile.out_offset + row * args.out_stride_row + column;
+            if (args.accumulate) value += *reinterpret_cast<const f32x4_t *>(target);
+            *reinterpret_cast<f32x4_t *>(target) = value;
+        }
+    }
+}
+
 }  // namespace f32
 
 bool f32_gemm_eligible(const GemmArgs &args, int dtype) {
@@ -273,8 +529,31 @@ bool f32_gemm_eligible(const GemmArgs &args, int dtype) {
     // Rows along the contiguous axis: an expert may start at any of them, and the last chunk would then end past the last row.
     if (!lhs_k && args.mode != kInputRowSparse && (args.rows % 4 != 0 || args.expert_ends != nullptr)) return false;
     if (args.inner >= (int64_t(1) << 30)) return false;
-    // Per-lane byte offsets inside a slice are below 2^31: at most 64 lines.
+    // Per-lane byte offsets inside a slice are below 2^31: at most 128 lines.
     return max(max(args.lhs_stride_row, args.lhs_stride_inner), max(args.rhs_stride_inner, args.rhs_stride_col)) < (int64_t(1) << 21);
+}
+
+template <int kTileM, int kTileN, int kStages>
+static int launch_f32_split(GemmArgs args, int64_t tiles, hipStream_t stream) {
+    const bool lhs_k = args.lhs_stride_inner == 1, rhs_k = args.rhs_stride_inner == 1;
+    const auto kernel = lhs_k ? (rhs_k ? f32::grouped_gemm_f32_split_kernel<kTileM, kTileN, kStages, true, true>
+                                       : f32::grouped_gemm_f32_split_kernel<kTileM, kTileN, kStages, true, false>)
+                              : (rhs_k ? f32::grouped_gemm_f32_split_kernel<kTileM, kTileN, kStages, false, true>
+                                       : f32::grouped_gemm_f32_split_kernel<kTileM, kTileN, kStages, false, false>);
+    // Runs of 16 tiles per XCD (8 row tiles x 2 column tiles): with 32 the XCDs end further apart, with 8 the panels are read more often
+    // (six products, us: 1490, 1467, 1477).
+    args.chunk_tiles = static_cast<int>(min(int64_t(16), (tiles + 7) / 8));
+    const int64_t round = 8 * static_cast<int64_t>(args.chunk_tiles);
+    const int64_t grid = (tiles + round - 1) / round * round;
+    if (grid >= (int64_t(1) << 31)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
+    constexpr int kBK = 16 * 4 * 64 * 64 / (kTileM * kTileN), kLds = kStages * (kTileM + kTileN) * kBK * 4;
+    static_assert(kLds <= 80 * 1024, "two workgroups per CU");
+    if constexpr (kLds > 64 * 1024) {
+        static std::atomic<uint64_t> configured[4];
+        if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLds, configured[2 * lhs_k + rhs_k])) return status;
+    }
+    kernel<<<static_cast<uint32_t>(grid), f32::kThreads, kLds, stream>>>(args);
+    return FM_OK;
 }
 
 template <int kTile, int kBK, int kStages>
@@ -295,25 +574,49 @@ static int launch_f32_tile(GemmArgs args, int64_t tiles, hipStream_t stream) {
     return FM_OK;
 }
 
-// Fewer tiles of 64 x 64 than this (six per CU; an upper bound of the tiles that exist is counted): tiles of 32 x 32.
-// us, 64 / 32: 160 tiles 20 / 13, 400 tiles 100 / 47, 560 tiles 55 / 27, 640 tiles 15.5 / 14.3, 1056 tiles 36 / 34, 1120
-// tiles 24 / 26, 1408 tiles 295 / 265, 2048 tiles 23 / 29, 3872 tiles 238 / 254.
-constexpr int64_t kF32LargeTiles = 1536;
+// Which tile, by upper bounds of how many there are (a map's padding counted). us, 8 or 16 experts, 2 slots:
+//   * forward and input gradients, 128 x 128 / 128 x 64 / 64 x 64 on split operands (fp32 multiply-adds): 384 tiles of 128 x 64
+//     (256 reduction indices) 18 / 14 / 14 (14), 768 (2816) 213 / 175 / 166 (285), 1032 (320) 24 / 22 / 22 (29), 2048 (768) 100 / 94 / 106
+//     (140), 2112 (1024) 170 / 160 / 177 (243), 4224 (1024) 315 / 331 / 357 (447), 5632 (1024) 325 / 355 / 394 (492). Below 128 tiles of
+//     64 x 64 four times as many of 32 x 32 are faster without splitting: 56 tiles (1024) 16.5 (13.5).
+//   * weight gradients on 128 x 128 from one per CU on: 1408 tiles (512) 138, 128 x 64 152, fp32 220; 128 tiles (512) 29 / 20 (26).
+//   * reductions over few rows are all start and epilogue, and eight workgroups per CU have the most in flight: means of 8 / 16 / 32
+//     / 50 / 64 / 128 rows 113 (87), 24 (22), 60 (54), 74 (75), 72 (76), 46 (66). A map's buffer has a tile of 128 rows of padding per
+//     expert on top of the mean.
+// The fp32 kernel's own tiles, 64 x 64 / 32 x 32: 1056 tiles of 64 x 64 36 / 34, 1120 24 / 26, 1408 295 / 265, 2048 23 / 29, 3872 238 / 254.
+constexpr int64_t kF32FewTiles = 128, kF32MiddleTiles = 1024, kF32ManyTiles = 2560, kF32LargeTiles = 1536;
+constexpr int64_t kF32ShortReduction = 128 + 48;
 
 int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
     // Upper bounds of the numbers of tiles (the surplus ids have none).
-    const auto count = [&](int tile) {
+    const auto count = [&](int tile_m, int tile_n) {
         if (args.mode == kInputRowSparse)
-            args.tiles_m = static_cast<int>((args.sparse_size + tile - 1) / tile) * args.num_experts;
+            args.tiles_m = static_cast<int>((args.sparse_size + tile_m - 1) / tile_m) * args.num_experts;
         else
-            args.tiles_m = static_cast<int>((args.rows + tile - 1) / tile + (args.num_experts > 1 ? args.num_experts : 0));
-        args.tiles_n = static_cast<int>((args.cols + tile - 1) / tile);
+            args.tiles_m = static_cast<int>((args.rows + tile_m - 1) / tile_m + (args.num_experts > 1 ? args.num_experts : 0));
+        args.tiles_n = static_cast<int>((args.cols + tile_n - 1) / tile_n);
         return static_cast<int64_t>(args.tiles_m) * args.tiles_n;
     };
-    const int64_t large = count(64);
-    if (large >= kF32LargeTiles) return launch_f32_tile<64, 16, 2>(args, large, stream);
-    const int64_t small = count(32);
-    return launch_f32_tile<32, 32, 2>(args, small, stream);
+    if (args.mode == kInputRowSparse) {
+        const int64_t reduction = args.piece_length > 0 ? args.piece_length : args.inner / args.num_experts;
+        if (reduction >= kF32ShortReduction && args.sparse_size >= 64 && args.cols >= 64) {
+            if (const int64_t tiles = count(128, 128); tiles >= 256) return launch_f32_split<128, 128, 3>(args, tiles, stream);
+            const int64_t tiles = count(128, 64);
+            return launch_f32_split<128, 64, 3>(args, tiles, stream);
+        }
+    } else if (count(64, 64) > kF32FewTiles) {
+        const int64_t tiles = count(128, 64);
+        if (tiles >= kF32ManyTiles) {
+            const int64_t large = count(128, 128);
+            return launch_f32_split<128, 128, 3>(args, large, stream);
+        }
+        if (tiles > kF32MiddleTiles) return launch_f32_split<128, 64, 3>(args, tiles, stream);
+        const int64_t small = count(64, 64);
+        return launch_f32_split<64, 64, 2>(args, small, stream);
+    }
+    if (const int64_t tiles = count(64, 64); tiles >= kF32LargeTiles) return launch_f32_tile<64, 16, 2>(args, tiles, stream);
+    const int64_t tiles = count(32, 32);
+    return launch_f32_tile<32, 32, 2>(args, tiles, stream);
 }
 
 }  // namespace fm
