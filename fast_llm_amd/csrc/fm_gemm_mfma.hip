@@ -131,9 +131,11 @@ __device__ __forceinline__ int64_t uniform_int64(int64_t value) {
 // complete in order) and passes a barrier first.
 // `kHalves` (row-contiguous only): loads 0..3 of a wavefront fill the first 32 K-rows of the slot and loads 4..7 the
 // last 32, so that either half of a slot can be refilled on its own (see the pipeline of the kernel).
-template <bool kContiguousK, bool kHalves = false>
+// `kRotates` (K-contiguous, whole slices only): the slices are taken from some slice on and then from the first one.
+template <bool kContiguousK, bool kHalves = false, bool kRotates = false>
 struct TileLoader {
     static_assert(!(kContiguousK && kHalves), "only a row-contiguous slice splits into halves along K");
+    static_assert(kContiguousK || !kRotates, "rotation is for K-contiguous operands");
     // The 1 KiB block of an operand slot that load j of wavefront `wave` fills.
     static __device__ __forceinline__ int block_of(int wave, int j) {
         return kHalves ? (j >> 2) * (2 * kLoadsPerOperand) + wave * (kLoadsPerOperand / 2) + (j & 3) : wave * kLoadsPerOperand + j;
@@ -147,6 +149,9 @@ struct TileLoader {
     uint32_t last_records;   // `num_records` of the last slice: its K-rows past the reduction range bring zeros (row-
                              // contiguous), or its last row ends where the reduction range does (K-contiguous)
     int wave_index;          // wave-uniform
+    // kRotates: `fetch_base` stays at the tile's first element, and the descriptor's range at the tile's last one.
+    int slice_offset;        // wave-uniform: bytes from there to the slice being fetched
+    int wrap_at;             // `slices_left` at the operand's last slice; the next one is its first
 
     // `stride`: bytes between rows (K-contiguous) or between K-rows (row-contiguous). Rows >= valid_rows are never
     // stored; a K-contiguous operand gets zeros for them (they lie past the range of the buffer descriptor), a
@@ -158,9 +163,11 @@ struct TileLoader {
     // operand gets zeros for the K-rows of its last slice that lie past it. Of a K-contiguous operand only the last
     // row gets zeros there: what the other rows bring is the start of the next row, to be masked in LDS.
     __device__ __forceinline__ void setup(const char *tile_base, int64_t stride, int valid_rows, int num_slices,
-                                          int k_count, int wave, int lane, int split_rows = 0) {
+                                          int k_count, int wave, int lane, int split_rows = 0, int first_slice = 0) {
         static_assert(kLoadsPerOperand % 2 == 0, "loads come in (even, odd) pairs");
         fetch_base = tile_base;
+        wrap_at = first_slice;
+        slice_offset = first_slice * (kBK * 2);
         slices_left = num_slices - 1;
         wave_index = wave;
 #pragma unroll
@@ -185,7 +192,9 @@ struct TileLoader {
         const int64_t last_row = split_rows == 0 ? valid_rows - 1 : split_rows + kTile / 2 - 1;
         step = kContiguousK ? kBK * 2 : kBK * stride;
         const int last_count = k_count - (num_slices - 1) * kBK;  // of the last slice
-        if constexpr (kContiguousK) {
+        if constexpr (kRotates) {
+            num_records = static_cast<uint32_t>(last_row * stride + k_count * 2);
+        } else if constexpr (kContiguousK) {
             // Whole 16-byte chunks: a chunk that crosses the range would come back as zeros.
             last_records = static_cast<uint32_t>(last_row * stride + min((last_count + 7) & ~7, kBK) * 2);
             num_records = num_slices == 1 ? last_records : static_cast<uint32_t>(last_row * stride + kBK * 2);
@@ -199,6 +208,13 @@ struct TileLoader {
     // load fills LDS with zeros without touching memory: the pipeline can run a slice too far without a branch.
     __device__ __forceinline__ void advance() {
         // Said to be wave-uniform once more: loop-carried values otherwise end up in vector registers.
+        if constexpr (kRotates) {
+            // An empty range at offset 0: the offset may be taken off the range before a lane's own is compared with it.
+            slice_offset = __builtin_amdgcn_readfirstlane(slices_left == wrap_at || slices_left <= 0 ? 0 : slice_offset + kBK * 2);
+            num_records = __builtin_amdgcn_readfirstlane(slices_left <= 0 ? 0u : num_records);
+            slices_left = __builtin_amdgcn_readfirstlane(slices_left - 1);
+            return;
+        }
         fetch_base = uniform_pointer(fetch_base + step);
         slices_left = __builtin_amdgcn_readfirstlane(slices_left - 1);
         num_records = __builtin_amdgcn_readfirstlane(slices_left < 0 ? 0u : (slices_left == 0 ? last_records : num_records));
@@ -219,6 +235,13 @@ struct TileLoader {
         // itself, with the load's part as an immediate (one scalar instruction per load instead of two).
         const int wave_address = __builtin_amdgcn_readfirstlane(slot_address + block_of(wave_index, 0) * 1024);
         // M0 is not handed out by the register allocator and nothing else in this file uses it.
+        if constexpr (kRotates) {
+            asm volatile("s_add_i32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds"
+                         :
+                         : "s"(wave_address), "v"(lane_offset), "s"(resource), "n"((block_of(0, j) - block_of(0, 0)) * 1024), "s"(slice_offset)
+                         : "memory", "scc");
+            return;
+        }
         asm volatile("s_add_i32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                      :
                      : "s"(wave_address), "v"(lane_offset), "s"(resource), "n"((block_of(0, j) - block_of(0, 0)) * 1024)
@@ -300,6 +323,7 @@ struct TileWork {
     int64_t lhs_offset, rhs_offset, out_offset;  // elements
     int64_t fused_offset;                        // of the tile in `fused_out`, elements
     int rows_valid, cols_valid;
+    int expert;
     int64_t k_lo, k_hi;
 };
 
@@ -322,6 +346,7 @@ __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, 
         const int expert = tile_m / tiles_per_expert;
         const int64_t row_in_expert = static_cast<int64_t>(tile_m - expert * tiles_per_expert) * kTile;
         work.rows_valid = static_cast<int>(min(static_cast<int64_t>(kTile), args.sparse_size - row_in_expert));
+        work.expert = expert;
         if (args.expert_ends != nullptr) {
             work.k_lo = expert > 0 ? load_index(args.expert_ends, args.index_dtype, expert - 1) : 0;
             work.k_hi = load_index(args.expert_pad_begins, args.index_dtype, expert);
@@ -343,6 +368,7 @@ __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, 
     const int64_t col0 = static_cast<int64_t>(tile.tile_n) * (paired ? kTile / 2 : kTile);
     work.cols_valid = paired ? kTile : static_cast<int>(min(static_cast<int64_t>(kTile), args.cols - col0));
     work.rows_valid = tile.rows_valid;
+    work.expert = tile.expert;
     work.lhs_offset = tile.row0 * args.lhs_stride_row;
     work.out_offset = tile.row0 * args.out_stride_row + col0;
     work.fused_offset = tile.row0 * args.fused_stride + col0;
@@ -497,9 +523,28 @@ struct alignas(64) TileRecord {
     int piece_slot;    // >= 0: a piece of a split reduction, stored to that workspace slot
     int found;         // 0: the id has no tile (and no later id has one)
     int half_slices;   // a half tile if the reduction has fewer slices than this
-    int unused;
+    int first_slice;   // the slice that the reduction starts with (see first_slice_of)
 };
 static_assert(sizeof(TileRecord) == 64, "one s_load_dwordx16 per record");
+
+// Which slice of the reduction axis the tiles of an expert start with, where both operands are K-contiguous and the axis is whole
+// slices. The CUs take slices at about the same pace, and 128 bytes of rows that are a few KiB apart lie in few of the memory's
+// channels: with every expert's weights read from slice 0 on, all CUs ask the same channels at the same time. Experts that run at
+// the same time are spread evenly over the axis instead (the fractional parts of multiples of the golden ratio). Per tile it would
+// be worse: the tiles of an expert share its activations in L2. Row-contiguous weights, 512 bytes of every row at a time, are no
+// faster for it, and neither is a launch that is bound by its MFMAs (kFewRows). Layer 1 (and layer 2's input gradient), us: 44 rows for each of
+// 128 experts of 2048 x 768 218 -> 168 (125 -> 111), 94 for each of 64 of 2048 x 1408 200 -> 158 (106 -> 99), 125 of the 128 228 -> 218 and
+// 218 -> 186 (120 -> 119), 469 of the 64 361 -> 348 (210 -> 210); 1024 of the 128 783 -> 789 (409 -> 409) without the bound.
+__host__ __device__ inline bool starts_anywhere(const GemmArgs &args) {
+    return args.mode != kInputRowSparse && args.num_experts > 1 && args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts &&
+           args.lhs_stride_inner == 1 && args.rhs_stride_inner == 1 && args.inner % kBK == 0;
+}
+
+__device__ __forceinline__ int first_slice_of(const GemmArgs &args, int expert) {
+    if (!starts_anywhere(args)) return 0;
+    const uint32_t fraction = (static_cast<uint32_t>(expert) * 40503u) & 0xffffu;  // 40503 / 65536 = 0.618...
+    return static_cast<int>((fraction * static_cast<uint64_t>(args.inner / kBK)) >> 16);
+}
 
 // Wave-uniform result; every lane of the wavefront must call it.
 __device__ __forceinline__ bool compute_tile_record(const GemmArgs &args, int id, TileRecord &record) {
@@ -509,8 +554,8 @@ __device__ __forceinline__ bool compute_tile_record(const GemmArgs &args, int id
     record.found = __builtin_amdgcn_readfirstlane(found);
     if (!record.found) return false;
     record.half_slices = args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts ? kHalfTileMaxSlicesFewRows : kHalfTileMaxSlices;
-    record.unused = 0;
     record.piece_slot = __builtin_amdgcn_readfirstlane(piece_slot);
+    record.first_slice = record.piece_slot >= 0 ? 0 : __builtin_amdgcn_readfirstlane(first_slice_of(args, work.expert));
     if (record.piece_slot >= 0) {  // a piece of a tile whose reduction is split (never the row-sparse product)
         work.k_lo = static_cast<int64_t>(piece) * piece_slices * kBK;
         work.k_hi = min(work.k_hi, work.k_lo + static_cast<int64_t>(piece_slices) * kBK);
@@ -552,7 +597,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_plan_kernel(PlannedProducts<
     }
     TileRecord record;
     if (!compute_tile_record(args, id, record)) {
-        record.half_slices = record.unused = 0;
+        record.half_slices = record.first_slice = 0;
         record.lhs_offset = record.rhs_offset = record.out_offset = record.fused_offset = 0;
         record.rows_valid = record.cols_valid = record.k_lo = record.k_hi = 0;
         record.piece_slot = -1;
@@ -845,7 +890,9 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[kTilesM][kTi
 // kMasked: the reduction range [k_lo, k_hi) is ragged: the row-sparse product, and any whose reduction is not a whole
 // number of slices.
 // kFusion: a GemmFusion, the epilogue to run instead of the plain store.
-template <typename T, bool kLhsContiguousK, bool kRhsContiguousK, bool kMasked, int kFusion = kFusionNone>
+// kRotates: the reductions of an expert's tiles start with a slice of its own (`first_slice_of`). An instance of its own, since the
+// main loop has five scalar instructions more per slice for it: 0.3 % of the launches that are bound by their MFMAs.
+template <typename T, bool kLhsContiguousK, bool kRhsContiguousK, bool kMasked, int kFusion, bool kRotates>
 __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_kernel(GemmArgs launch_args) {
     static_assert(kFusion == kFusionNone || (kRhsContiguousK && !kMasked), "fused epilogues: output-sparse, K-major rhs");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
@@ -880,8 +927,9 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
     // Loads that may still be on their way at the barrier before the last K-step and at the one after K-step 0.
     constexpr int kBarrierNewest = kSchedule == kScheduleSplit ? 6 : (kSchedule == kScheduleLate ? 8 : 16);
     constexpr int kMidBarrierNewest = 18;
-    typedef TileLoader<kLhsContiguousK> LhsLoader;
-    typedef TileLoader<kRhsContiguousK, kRhsHalves> RhsLoader;
+    static_assert(!kRotates || (kLhsContiguousK && kRhsContiguousK && !kMasked), "whole slices of K-contiguous operands");
+    typedef TileLoader<kLhsContiguousK, false, kRotates> LhsLoader;
+    typedef TileLoader<kRhsContiguousK, kRhsHalves, kRotates> RhsLoader;
     struct Tile {
         TileRecord work;
         int piece_slot;   // >= 0: a piece of a split reduction, stored to that workspace slot
@@ -1135,11 +1183,12 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
                           (work.rhs_offset + next.k_first * args.rhs_stride_inner) * static_cast<int64_t>(sizeof(T));
         lhs_loader.setup(uniform_pointer(lhs),
                          (kLhsContiguousK ? args.lhs_stride_row : args.lhs_stride_inner) * sizeof(T), work.rows_valid,
-                         next.num_slices, work.k_hi - next.k_first, wave, lane);
+                         next.num_slices, work.k_hi - next.k_first, wave, lane, 0, kRotates ? work.first_slice : 0);
         rhs_loader.setup(uniform_pointer(rhs),
                          (kRhsContiguousK ? args.rhs_stride_col : args.rhs_stride_inner) * sizeof(T), work.cols_valid,
                          next.num_slices, work.k_hi - next.k_first, wave, lane,
-                         kFusion == kFusionGatedForward ? static_cast<int>(args.half) : 0);
+                         kFusion == kFusionGatedForward ? static_cast<int>(args.half) : 0,
+                         kRotates ? work.first_slice : 0);
     };
     constexpr int kFirstLhsSlot = kLhsBase + (kLhsStages - 1) * kOperandBytes;
     auto first_loads = [&](const Tile &next) {
@@ -1343,9 +1392,12 @@ int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured) 
     return FM_OK;
 }
 
-template <typename T, bool kLhsK, bool kRhsK, bool kMasked, int kFusion = kFusionNone>
+template <typename T, bool kLhsK, bool kRhsK, bool kMasked, int kFusion = kFusionNone, bool kRotates = false>
 static int launch_instance(const GemmArgs &args, hipStream_t stream) {
-    auto kernel = grouped_gemm_mfma_kernel<T, kLhsK, kRhsK, kMasked, kFusion>;
+    if constexpr (kLhsK && kRhsK && !kMasked && !kRotates) {
+        if (starts_anywhere(args)) return launch_instance<T, kLhsK, kRhsK, kMasked, kFusion, true>(args, stream);
+    }
+    auto kernel = grouped_gemm_mfma_kernel<T, kLhsK, kRhsK, kMasked, kFusion, kRotates>;
     static std::atomic<uint64_t> configured{0};
     if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
     // One workgroup per CU walks the ids (see the kernel).
