@@ -13,7 +13,7 @@ import torch
 
 LIBRARY_PATH = pathlib.Path(__file__).resolve().parent / "csrc" / "libfastmoe_hip.so"
 
-FM_VERSION = 11
+FM_VERSION = 12
 
 _c_i64, _c_int, _c_ptr, _c_size = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 
@@ -80,6 +80,7 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_ptr] * 6 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr],
     ),
+    "fm_router_linear_forward": (_c_int, [_c_ptr] * 3 + [_c_i64] * 3 + [_c_int, _c_ptr]),
     "fm_router_linear_backward_workspace_size": (_c_size, [_c_i64] * 3 + [_c_int]),
     "fm_router_linear_backward": (_c_int, [_c_ptr] * 5 + [_c_i64] * 3 + [_c_int, _c_ptr, _c_size, _c_ptr]),
     "fm_moe_layer_sizes": (_c_int, [_c_ptr]),

@@ -15,6 +15,7 @@ import torch
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.config import ActivationType, KernelConfig, MLPRecomputeLevel
 from fast_llm_amd.functional.mlp import _activation_tag
+from fast_llm_amd.functional.routing import router_logits
 from fast_llm_amd.functional.utils import ANCHOR, Assert, is_traced, without_backward
 from fast_llm_amd.tensor import accumulate_gradient, param_get_and_unset_is_zero
 
@@ -116,7 +117,7 @@ def _forward(
 ) -> tuple[torch.Tensor, torch.Tensor | None, _Saved]:
     """(output, losses [2] or None, what the backward needs)."""
     device = _lib.require_device(hidden_states, router, weight_1, weight_2, noise)
-    logits = torch.nn.functional.linear(hidden_states, router)
+    logits = router_logits(hidden_states, router)
     layer = _describe(options, hidden_states, weight_1, weight_2, with_losses)
     new = hidden_states.new_empty
     routing = new(layer.routing_bytes, dtype=torch.uint8)

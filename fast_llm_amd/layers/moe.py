@@ -24,7 +24,7 @@ def attach_grad_buffer(weight: torch.Tensor, dtype: torch.dtype | None = None) -
     return weight
 
 
-from fast_llm_amd.functional.routing import router, sinkhorn_routing, topk_routing  # noqa: E402, F401  (re-exported)
+from fast_llm_amd.functional.routing import router, router_linear, sinkhorn_routing, topk_routing  # noqa: E402, F401  (re-exported)
 from fast_llm_amd.functional.utils import AuxiliaryLoss, without_backward  # noqa: E402
 
 LOAD_BALANCING_LOSS, ROUTER_Z_LOSS = "load_balancing_loss", "router_z_loss"  # layers/decoder/mlp/config.py:24-26
@@ -116,7 +116,7 @@ class DroplessMoEMLP(torch.nn.Module):
             router_input = router_input * self.router_scale
         if self.router_input_scale != 1.0:
             router_input = router_input * self.router_input_scale
-        logits = torch.nn.functional.linear(router_input, self.router)
+        logits = router_linear(router_input, self.router)
         noise = None
         if self.training and self.jitter_eps > 0.0:
             noise = torch.empty_like(logits).uniform_(1.0 - self.jitter_eps, 1.0 + self.jitter_eps)

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FM_VERSION 11
+#define FM_VERSION 12
 
 /* Element type of activations, weights and outputs. */
 enum fm_dtype { FM_DTYPE_F32 = 0, FM_DTYPE_BF16 = 1, FM_DTYPE_F16 = 2 };
@@ -356,6 +356,12 @@ int fm_few_tokens_forward(const void *input, const void *top_experts, const void
                           const void *weight_2, void *output, int64_t num_tokens, int64_t slots_per_token, int64_t hidden,
                           int64_t ffn, int64_t num_experts, int gated, int activation, int dtype, void *workspace,
                           size_t workspace_size, void *stream);
+
+/* The router's linear layer, logits [num_tokens, num_experts] = input [num_tokens, hidden] x weight [num_experts, hidden]^T, for few
+ * tokens: meant for up to 64 tiles of 16 tokens x 16 experts, correct for any number. All contiguous, of `dtype`, sums in fp32;
+ * input and weight 16-byte aligned and hidden a multiple of 16 bytes (FM_ERR_UNSUPPORTED). Deterministic. */
+int fm_router_linear_forward(const void *input, const void *weight, void *logits, int64_t num_tokens, int64_t num_experts,
+                             int64_t hidden, int dtype, void *stream);
 
 /* Backward of the router's linear layer, logits = input [num_tokens, hidden] x weight [num_experts, hidden]^T:
  * grad_weight = grad_logits^T x input (may be null: not computed) and grad_input += grad_logits x weight (may be null). All

@@ -1,0 +1,53 @@
+"""The router's logits by the kernel for few tokens, against 64 bits, and their gradients."""
+
+import pytest
+import torch
+
+from fast_llm_amd.functional import routing
+
+pytestmark = pytest.mark.gpu
+
+# Unit roundoff of the type a logit is rounded to: half a unit of the last of 24, 8 and 11 significant bits.
+_ROUND = {torch.float32: 2**-24, torch.bfloat16: 2**-8, torch.float16: 2**-11}
+
+
+@pytest.mark.parametrize("dtype", list(_ROUND))
+@pytest.mark.parametrize(("tokens", "experts"), [(1, 1), (1, 8), (15, 16), (17, 17), (33, 60), (64, 128), (1024, 8)])
+@pytest.mark.parametrize("hidden", [8, 32, 40, 264, 2056, 4096])
+def test_logits(dtype, tokens, experts, hidden, device):
+    generator = torch.Generator(device).manual_seed(tokens + experts + hidden)
+    x, weight = (torch.randn((rows, hidden), generator=generator, device=device).to(dtype) for rows in (tokens, experts))
+    assert routing._few_logits(x, weight)
+    logits = routing.router_logits(x, weight)
+    assert logits.dtype == dtype and logits.shape == (tokens, experts)
+    exact = x.double() @ weight.double().t()
+    # One rounding of the result, and at most hidden + 8 of partial sums in fp32.
+    bound = _ROUND[dtype] * exact.abs() + (hidden + 8) * 2**-24 * (x.double().abs() @ weight.double().abs().t())
+    assert ((logits.double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", list(_ROUND))
+def test_gradients_are_those_of_linear(dtype, device):
+    torch.manual_seed(0)
+    x, weight = (torch.randn((rows, 72), device=device, dtype=dtype, requires_grad=True) for rows in (50, 24))
+    grad = torch.randn((50, 24), device=device, dtype=dtype)
+    results = []
+    for function in (routing.router_linear, torch.nn.functional.linear):
+        x.grad = weight.grad = None
+        logits = function(x, weight)
+        logits.backward(grad)
+        results.append((x.grad, weight.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    with torch.no_grad():
+        assert torch.equal(routing.router_linear(x, weight), routing.router_logits(x, weight))
+
+
+def test_what_the_kernel_does_not_take(device):
+    x, weight = torch.randn((30, 68), device=device), torch.randn((8, 68), device=device)
+    for operands in ((x[:, :66], weight[:, :66]), (x.t().contiguous().t(), weight), (x[:0], weight), (x[1:, 1:], weight[:, 1:])):
+        assert not routing._few_logits(*operands)
+        assert torch.equal(routing.router_linear(*operands), torch.nn.functional.linear(*operands))
+    many = torch.randn((16 * routing._MAX_LOGIT_TILES + 1, 68), device=device)
+    assert not routing._few_logits(many, weight) and routing._few_logits(many[1:], weight)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert routing.router_linear(x, weight).dtype == torch.bfloat16
