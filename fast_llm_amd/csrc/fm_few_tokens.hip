@@ -90,11 +90,13 @@ __device__ __forceinline__ int find_rows(const Args &args, int which, int *list,
 // writes hit all banks; one wavefront's LDS operations execute in order, so no barrier). Loads shaped like the fragments,
 // 64 bytes of each of 16 rows, took 326 us for the 1.9 GB of 8 experts of 4096 x 28672 and 8 tokens where these take 242
 // (7.8 TB/s).
+// The wavefronts' chunks are taken four by four, from trip `first_trip` (below their number) on and then from the first one.
 // `row_offset[i]`: byte offset of the lane's 16 bytes in the rows 4 i + l / 16 at k = 0 (kOutOfRange: no such row).
 template <typename T, int kSets, int kGroups>
 __device__ __forceinline__ void multiply_rows(__amdgpu_buffer_rsrc_t weight, __amdgpu_buffer_rsrc_t x,
                                               const uint32_t (&row_offset)[kSets * 4], const uint32_t (&token_offset)[kGroups],
-                                              FM_LDS(char) * lds, int length, int wave, int lane, f32x4_t (&sums)[kSets][kGroups]) {
+                                              FM_LDS(char) * lds, int length, int first_trip, int wave, int lane,
+                                              f32x4_t (&sums)[kSets][kGroups]) {
     constexpr int kChunk = 128, kSteps = kChunk / 32;
     const int load_k = (lane & 15) * 8, lane_k = (lane >> 4) * 8, load_row = lane >> 4, row = lane & 15;
     u32x4_t raw[kSets * 4], tokens[2][kGroups][kSteps];
@@ -111,15 +113,15 @@ __device__ __forceinline__ void multiply_rows(__amdgpu_buffer_rsrc_t weight, __a
             for (int g = 0; g < kGroups; ++g)
                 values[g][s] = load(x, k0 + s * 32 + lane_k < length ? token_offset[g] + (k0 + s * 32 + lane_k) * 2 : kOutOfRange);
     };
-    const auto chunk = [&](int k0, u32x4_t(&now)[kGroups][kSteps], u32x4_t(&next)[kGroups][kSteps]) {
+    const auto chunk = [&](int next_k0, u32x4_t(&now)[kGroups][kSteps], u32x4_t(&next)[kGroups][kSteps]) {
 #pragma unroll
         for (int i = 0; i < kSets * 4; ++i) {
             const int r = (4 * i + load_row) & 15;
             *(FM_LDS(u32x4_t) *)(lds + (i / 4) * 4096 + r * 256 + (((lane & 15) ^ r) << 4)) = raw[i];
         }
         // The next chunk is on its way while this one is multiplied; past the end it is zeros and touches no memory.
-        fetch_rows(k0 + kWaves * kChunk);
-        fetch_tokens(k0 + kWaves * kChunk, next);
+        fetch_rows(next_k0);
+        fetch_tokens(next_k0, next);
         // The lanes read what others wrote: the hardware keeps a wavefront's LDS operations in order, and this the compiler.
         asm volatile("" ::: "memory");
 #pragma unroll
@@ -132,13 +134,29 @@ __device__ __forceinline__ void multiply_rows(__amdgpu_buffer_rsrc_t weight, __a
             }
         asm volatile("" ::: "memory");  // and the next chunk's writes stay behind these reads
     };
-    fetch_rows(wave * kChunk);
-    fetch_tokens(wave * kChunk, tokens[0]);
-    for (int k0 = wave * kChunk; k0 < length; k0 += 2 * kWaves * kChunk) {
-        chunk(k0, tokens[0], tokens[1]);
-        chunk(k0 + kWaves * kChunk, tokens[1], tokens[0]);
+    const int trips = (length + kWaves * kChunk - 1) / (kWaves * kChunk);
+    int trip = first_trip, left = trips;
+    const auto next_chunk = [&]() {  // where this wavefront's next chunk starts; past the end after the last one
+        if (left <= 0) return length;
+        const int k0 = (trip * kWaves + wave) * kChunk;
+        trip = trip + 1 == trips ? 0 : trip + 1;
+        --left;
+        return k0;
+    };
+    const int first = next_chunk();
+    fetch_rows(first);
+    fetch_tokens(first, tokens[0]);
+    for (int t = 0; t < trips; t += 2) {
+        chunk(next_chunk(), tokens[0], tokens[1]);
+        chunk(next_chunk(), tokens[1], tokens[0]);
     }
 }
+
+// Weight rows of up to this many elements are read from another place on by every workgroup: the workgroups keep about the same
+// pace, and 1 KiB of rows that are 4 KiB or less apart lie in few of the memory's channels. Whole pass in us, from the start / so:
+// 96 tokens over 128 experts of 2048 x 768 225.7 / 220.5, 16 over 64 of 2048 x 1408 170.5 / 167, 40 over 32 of 1024 x 2816 113.5 / 112;
+// rows of 4096 are better read in one go: one token over 8 experts of 4096 x 14336 127 / 132, 3000 x 4096 250 / 251.
+constexpr int kMaxRotatedRow = 2048;
 
 // kSets x 16 weight rows per workgroup: half of them gate rows and the others the up rows that go with them, or (not
 // gated) consecutive rows.
@@ -164,6 +182,7 @@ __global__ __launch_bounds__(kThreads) void few_tokens_layer_1_kernel(Args args)
         row_offset[i] = f < ffn ? static_cast<uint32_t>(((f + set / kOutputSets * ffn) * static_cast<int64_t>(hidden) + (lane & 15) * 8) * 2)
                                 : kOutOfRange;
     }
+    const int first_trip = hidden <= kMaxRotatedRow ? blockIdx.x % ((hidden + kWaves * 128 - 1) / (kWaves * 128)) : 0;
     const auto activate = [&](float value) {
         float result;
         FM_DISPATCH_ACTIVATION(args.activation_type, kActivation, result = activation_forward<kActivation>(value));
@@ -186,7 +205,7 @@ __global__ __launch_bounds__(kThreads) void few_tokens_layer_1_kernel(Args args)
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) sums[r][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             FM_LDS(char) *chunks = (FM_LDS(char) *)reinterpret_cast<char *>(partial) + wave * kSets * 4096;
-            multiply_rows<T, kSets, kGroups>(weight, x, row_offset, token_offset, chunks, hidden, wave, lane, sums);
+            multiply_rows<T, kSets, kGroups>(weight, x, row_offset, token_offset, chunks, hidden, first_trip, wave, lane, sums);
             __syncthreads();
 
 

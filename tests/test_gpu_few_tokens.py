@@ -55,6 +55,25 @@ def test_few_tokens_forward(tokens, experts, slots, hidden, ffn, dtype, gated, a
     assert max_rel_err(output.cpu(), expected) <= _MAX_REL[dtype]
 
 
+# One to four trips of 512 along the rows, whole or not, which workgroups start at different places, and longer rows, which they do not.
+@pytest.mark.parametrize("hidden", [8, 512, 520, 1024, 1288, 2048, 2056])
+@pytest.mark.parametrize("tokens", [1, 20, 70])
+def test_every_part_of_a_row_counts_once(hidden, tokens, device):
+    """Small whole numbers, whose sums are exact in any order; layer 2 picks its rows out."""
+    generator = torch.Generator().manual_seed(hidden + tokens)
+    experts, ffn = 3, 200
+    x, weight_1 = (torch.randint(-1, 2, (rows, hidden), generator=generator).bfloat16() for rows in (tokens, experts * ffn))
+    weight_2 = torch.zeros(experts, ffn, max(hidden, ffn))
+    weight_2[:] = torch.eye(ffn, max(hidden, ffn))
+    weight_2 = weight_2[:, :, :hidden].reshape(experts * ffn, hidden).bfloat16()
+    top_experts = torch.randint(0, experts, (tokens, 1), generator=generator)
+    output = mlp.few_tokens_forward(
+        *(t.to(device) for t in (x, torch.ones(tokens, 1), top_experts, weight_1, weight_2)), experts, False, ActivationType.identity
+    )
+    layer_1 = torch.einsum("th,tfh->tf", x.float(), weight_1.float().view(experts, ffn, hidden)[top_experts[:, 0]]).bfloat16()
+    assert torch.equal(output.cpu()[:, :ffn], layer_1[:, :hidden])
+
+
 def test_few_tokens_forward_leaves_the_rest_to_the_sparse_layout(device):
     def call(tokens, dtype=torch.bfloat16, ffn=64):
         x, weight_1, weight_2 = (torch.zeros(rows, 64, dtype=dtype, device=device) for rows in (tokens, 8 * ffn, 4 * ffn))
