@@ -241,9 +241,9 @@ int rest_of_backward(const fm_moe_layer &layer, const Plan &plan, void *stream) 
                             layer.grad_logits, layer.auxiliary_loss_grad, layer.z_loss_grad, layer.tokens,
                             layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), true, stream));
     if (layer.router != nullptr)
-        FM_STEP(step.keep(fm_router_linear_backward(layer.grad_logits, layer.input, layer.router, layer.router_input_grad ? layer.grad_input : nullptr, layer.grad_router,
-                                                    layer.tokens, layer.routed_experts, layer.hidden, step.dtype(), layer.workspace,
-                                                    plan.workspace_bytes, stream)));
+        FM_STEP(step.keep(router_linear_backward(layer.grad_logits, layer.input, layer.router, layer.router_input_grad ? layer.grad_input : nullptr,
+                                                 layer.grad_router, layer.router_input_grad == 2, layer.tokens, layer.routed_experts,
+                                                 layer.hidden, step.dtype(), layer.workspace, plan.workspace_bytes, stream)));
     return step.note;
 }
 

@@ -42,4 +42,10 @@ int router_backward(const void *grad_scores, const void *scores, const void *top
                     int64_t num_tokens, int64_t num_experts, int64_t experts_per_token, int64_t shared_experts, int dtype,
                     bool round_grad_scores, void *stream);
 
+// `fm_router_linear_backward`. With `round_product` (half precision, up to 128 experts) what is added to grad_input is rounded to
+// `dtype` first: the two gradients of the layer's input as autograd adds them where the layer runs one call after the other.
+int router_linear_backward(const void *grad_logits, const void *input, const void *weight, void *grad_input, void *grad_weight,
+                           bool round_product, int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype, void *workspace,
+                           size_t workspace_size, void *stream);
+
 }  // namespace fm

@@ -5,7 +5,8 @@
 // row-sparse grouped product whose groups are pieces of the token axis, enough of them for a tile per CU, into fp32 partial
 // results that a small kernel adds in their order. 16384 tokens of 2048 and 128 experts: 28 us with the addition; the device
 // library's product of these operands takes 134 to 180.
-// The input gradient is a grouped product without groups.
+// The input gradient is a grouped product without groups in fp32. In half precision it reduces over at most 128 experts: the bytes
+// of the gradient that it is added to are the bound, which a kernel reads and writes once (see router_input_grad_kernel).
 //
 // The logits of few tokens are latency and nothing else: a workgroup computes 16 tokens x 16 experts, its wavefronts a part of the
 // hidden axis each, fragments straight from memory into registers, all loads of eight steps under way at once, and one exchange
@@ -13,6 +14,7 @@
 // 4096 and 8 experts 4.8 (7.4), 64 tokens 7.6 (7.6), 96 of 2048 and 128 experts 5.5 (5.4), 512 of 256 and 8 experts in single
 // precision 3.3 (3.7); 1531 of 4096 and 8 experts 7.8 (6.0). Calling that library takes 19 us of the host's time, this 8.
 #include "fm_gemm_common.h"
+#include "fm_router_layout.h"
 
 namespace fm {
 
@@ -119,6 +121,90 @@ __global__ __launch_bounds__(64 * kLogitWaves) void router_logits_kernel(const T
     }
 }
 
+// ---- input gradient ------------------------------------------------------------------------------------------------------------
+// grad_input += grad_logits x weight; with kRoundProduct the product is rounded before it is added, as where autograd adds the two
+// gradients of a layer's input. A workgroup has 128 columns of the weight in LDS as the MFMAs want them (kSteps x 32 experts, a step
+// per wavefront; the K-rows that a lane loads are transposed in blocks of 8 x 8, one v_perm_b32 per two values), and its wavefronts
+// walk kInputGradTokens tokens each, 16 at a time: a lane holds eight consecutive columns of four of them, 16 lanes 256 bytes of a
+// row. us, a product and an addition of torch in brackets: 16384 tokens of 2048 and 128 experts 31 (53), 64 experts 24 (48; 5.5
+// TB/s), 8192 of 4096 and 8 experts 22 (54; 6 TB/s), 1999 of 2048 and 128 experts 9 (22), 512 of 512 and 8 experts 5 (22, the
+// host's time). With the columns in registers there is one wavefront per SIMD from 65 experts on: 54 us for the first of these.
+constexpr int kInputGradTokens = 64, kInputGradMaxExperts = 128;
+
+template <typename T, int kSteps, bool kRoundProduct>
+__global__ __launch_bounds__(256, 4) void router_input_grad_kernel(const T *__restrict__ grad_logits, const T *__restrict__ weight,
+                                                                   T *__restrict__ grad_input, int64_t tokens, int experts, int hidden) {
+    static_assert(kSteps <= 4, "a step per wavefront");
+    __shared__ u32x4_t columns[kSteps][8][64];  // [step][i][lane]: column i of the lane's eight, experts 32 step + 8 group + 0 .. 7
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, group = lane >> 4;
+    const int column = blockIdx.x * 128 + (lane & 15) * 8;
+    const bool exists = column < hidden;  // a multiple of 8
+    if (wave < kSteps) {
+        u32x4_t raw[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int expert = wave * 32 + group * 8 + j;
+            raw[j] = u32x4_t{0, 0, 0, 0};
+            if (exists && expert < experts) raw[j] = *reinterpret_cast<const u32x4_t *>(weight + static_cast<int64_t>(expert) * hidden + column);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            u32x4_t one;
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                one[p] = __builtin_amdgcn_perm(raw[2 * p + 1][i / 2], raw[2 * p][i / 2], i % 2 ? 0x07060302u : 0x05040100u);
+            columns[wave][i][lane] = one;
+        }
+    }
+    __syncthreads();
+    const int64_t first = (static_cast<int64_t>(blockIdx.y) * 4 + wave) * kInputGradTokens;
+    for (int64_t token0 = first; token0 < min(first + kInputGradTokens, tokens); token0 += 16) {
+        asm volatile("" ::: "memory");  // the columns are read from LDS every time, not kept in registers
+        T *target = grad_input + (token0 + group * 4) * hidden + column;
+        const T *row = grad_logits + min(token0 + (lane & 15), tokens - 1) * experts + group * 8;
+        u32x4_t logits[kSteps], before[4];
+#pragma unroll
+        for (int step = 0; step < kSteps; ++step) {
+            logits[step] = u32x4_t{0, 0, 0, 0};
+            if (step * 32 + group * 8 < experts) logits[step] = *reinterpret_cast<const u32x4_t *>(row + step * 32);  // a multiple of 8
+        }
+        const int64_t left = exists ? tokens - token0 - group * 4 : 0;  // of the lane's four tokens
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r < left) before[r] = *reinterpret_cast<const u32x4_t *>(target + static_cast<int64_t>(r) * hidden);
+        f32x4_t sums[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sums[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int step = 0; step < kSteps; ++step)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sums[i] = multiply(T(), logits[step], columns[step][i][lane], sums[i]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (r >= left) continue;
+            Vec16<T> value = __builtin_bit_cast(Vec16<T>, before[r]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float product = kRoundProduct ? to_float(from_float<T>(sums[i][r])) : sums[i][r];
+                value.v[i] = from_float<T>(to_float(value.v[i]) + product);
+            }
+            store16(target + static_cast<int64_t>(r) * hidden, value);
+        }
+    }
+}
+
+template <typename T, bool kRoundProduct>
+static void launch_input_grad(const void *grad_logits, const void *weight, void *grad_input, int64_t tokens, int experts, int hidden,
+                              hipStream_t stream) {
+    const int64_t rows = 4 * kInputGradTokens;
+    const dim3 grid((hidden + 127) / 128, static_cast<uint32_t>((tokens + rows - 1) / rows));
+    const auto kernel = experts <= 32   ? router_input_grad_kernel<T, 1, kRoundProduct>
+                        : experts <= 64 ? router_input_grad_kernel<T, 2, kRoundProduct>
+                                        : router_input_grad_kernel<T, 4, kRoundProduct>;
+    kernel<<<grid, 256, 0, stream>>>(static_cast<const T *>(grad_logits), static_cast<const T *>(weight), static_cast<T *>(grad_input),
+                                     tokens, experts, hidden);
+}
+
 }  // namespace router_linear
 
 }  // namespace fm
@@ -153,15 +239,20 @@ extern "C" size_t fm_router_linear_backward_workspace_size(int64_t num_tokens, i
     return sizeof(float) * router_linear::plan_pieces(num_tokens, num_experts, hidden, dtype).count * num_experts * hidden;
 }
 
-extern "C" int fm_router_linear_backward(const void *grad_logits, const void *input, const void *weight, void *grad_input,
-                                         void *grad_weight, int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype,
-                                         void *workspace, size_t workspace_size, void *stream_) {
+int fm::router_linear_backward(const void *grad_logits, const void *input, const void *weight, void *grad_input, void *grad_weight,
+                               bool round_product, int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype,
+                               void *workspace, size_t workspace_size, void *stream_) {
     const char *name = "fm_router_linear_backward";
     const size_t needed = fm_router_linear_backward_workspace_size(num_tokens, num_experts, hidden, dtype);
     if (needed == 0)
         return fail(FM_ERR_UNSUPPORTED, "%s: experts and hidden must be multiples of 16 bytes, got %lld and %lld", name,
                     static_cast<long long>(num_experts), static_cast<long long>(hidden));
     FM_REQUIRE(grad_logits && aligned16(grad_logits), "%s: null or misaligned grad_logits", name);
+    // fp32, more experts: a grouped product. Tokens: the grid's y.
+    const bool own_input_grad =
+        dtype != FM_DTYPE_F32 && num_experts <= router_linear::kInputGradMaxExperts && num_tokens < (int64_t(1) << 23);
+    if (round_product && grad_input && !own_input_grad)
+        return fail(FM_ERR_UNSUPPORTED, "%s: the product of this size is not rounded before it is added", name);
     if (grad_weight) {
         FM_REQUIRE(input && aligned16(input) && workspace && aligned16(workspace) && workspace_size >= needed,
                    "%s: null or misaligned tensor, or a workspace of less than %zu bytes", name, needed);
@@ -182,6 +273,23 @@ extern "C" int fm_router_linear_backward(const void *grad_logits, const void *in
     }
     if (grad_input == nullptr) return FM_OK;
     FM_REQUIRE(weight && aligned16(weight) && aligned16(grad_input), "%s: null or misaligned tensor", name);
+    if (own_input_grad) {
+        const auto launch = [&](auto zero) {
+            using T = decltype(zero);
+            const auto run = round_product ? router_linear::launch_input_grad<T, true> : router_linear::launch_input_grad<T, false>;
+            run(grad_logits, weight, grad_input, num_tokens, static_cast<int>(num_experts), static_cast<int>(hidden),
+                static_cast<hipStream_t>(stream_));
+        };
+        dtype == FM_DTYPE_BF16 ? launch(bf16_t()) : launch(f16_t());
+        return check_launch(name);
+    }
     return fm_output_sparse_matmul(grad_logits, weight, grad_input, nullptr, num_tokens, hidden, num_experts, 1, num_experts, 1, hidden, 1,
                                    hidden, 1, 1, dtype, dtype, FM_INDEX_I32, nullptr, 0, stream_);
+}
+
+extern "C" int fm_router_linear_backward(const void *grad_logits, const void *input, const void *weight, void *grad_input,
+                                         void *grad_weight, int64_t num_tokens, int64_t num_experts, int64_t hidden, int dtype,
+                                         void *workspace, size_t workspace_size, void *stream) {
+    return router_linear_backward(grad_logits, input, weight, grad_input, grad_weight, false, num_tokens, num_experts, hidden, dtype,
+                                  workspace, workspace_size, stream);
 }

@@ -253,13 +253,16 @@ class _MoELayer(torch.autograd.Function):
             else:
                 layer.grad_weight_2, layer.accumulate_2 = target.data_ptr(), accumulate
         # The router's linear layer: with the rest, or in torch for sizes the library does not take. Half-precision input
-        # gradients are torch's too: a reduction of 8 to 128 experts is one or two slices of the library's 256 x 256 tiles
-        # (16384 tokens of 2048, 128 experts: 39 us against 33; 512 of 256, 8 experts: 17 against 5).
+        # gradients of more than 128 experts are torch's too: there the library has 256 x 256 tiles for them.
         grad_router = None
         if hidden_states.data_ptr() % 16 != 0 or router.data_ptr() % 16 != 0:
             layer.router_linear = False
         if layer.router_linear:
-            layer.router, layer.router_input_grad = router.data_ptr(), layer.dtype == 0
+            layer.router = router.data_ptr()
+            if layer.dtype == 0:
+                layer.router_input_grad = 1
+            elif options.routed_experts <= 128 and layer.tokens < 2**23:
+                layer.router_input_grad = 2  # rounded as torch's is
             if ctx.needs_input_grad[1]:
                 grad_router = torch.empty_like(router)
                 layer.grad_router = grad_router.data_ptr()

@@ -411,7 +411,9 @@ typedef struct {
     void *grad_layer_2_output, *grad_activation_output, *grad_layer_1_output, *grad_scores;
     void *grad_logits, *grad_input, *grad_weight_1, *grad_weight_2;
     /* Where router_linear is not 0, if `router` is not null: the backward of the router's linear layer as well
-     * (fm_router_linear_backward), into grad_router (may be null) and, with router_input_grad, added into grad_input. */
+     * (fm_router_linear_backward), into grad_router (may be null) and, with router_input_grad, added into grad_input: 1: as
+     * there; 2: the product rounded before it is added, as where autograd adds the two gradients of the layer's input (half
+     * precision, up to 128 experts, fewer than 2^23 tokens; otherwise FM_ERR_UNSUPPORTED). */
     const void *router;
     void *grad_router;
     int64_t router_input_grad;

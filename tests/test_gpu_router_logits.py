@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from fast_llm_amd import _lib
 from fast_llm_amd.functional import routing
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +52,24 @@ def test_what_the_kernel_does_not_take(device):
     assert not routing._few_logits(many, weight) and routing._few_logits(many[1:], weight)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert routing.router_linear(x, weight).dtype == torch.bfloat16
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("experts", [8, 32, 40, 64, 72, 128])
+@pytest.mark.parametrize(("tokens", "hidden"), [(1, 8), (15, 128), (17, 136), (64, 120), (257, 520), (300, 2056)])
+def test_input_gradient_is_added(dtype, experts, tokens, hidden, device):
+    """In place, nothing beside it touched, one rounding of the sum."""
+    generator = torch.Generator(device).manual_seed(experts + tokens)
+    normal = lambda *shape: torch.randn(shape, generator=generator, device=device).to(dtype)  # noqa: E731
+    grad_logits, weight, around = normal(tokens, experts), normal(experts, hidden), normal(tokens + 2, hidden)
+    grad_input = around.clone()[1:-1]
+    whole = grad_input._base
+    _lib.call(
+        "fm_router_linear_backward", device, grad_logits.data_ptr(), None, weight.data_ptr(), grad_input.data_ptr(), None,
+        tokens, experts, hidden, _lib.dtype_tag(dtype), None, 0,
+    )  # fmt: skip
+    assert torch.equal(whole[0], around[0]) and torch.equal(whole[-1], around[-1])
+    exact = around[1:-1].double() + grad_logits.double() @ weight.double()
+    # At most experts + 8 roundings of partial sums in fp32, and one of the result.
+    partial = (experts + 8) * 2**-24 * (grad_logits.double().abs() @ weight.double().abs() + around[1:-1].double().abs())
+    assert ((grad_input.double() - exact).abs() <= _ROUND[dtype] * (exact.abs() + partial) + partial).all()
