@@ -48,7 +48,7 @@ struct GemmArgs {
     int64_t piece_length;  // row-sparse mode without a map: group e reduces over [e, e + 1) * piece_length instead of
                            // everything (0: everything)
     int planned;           // `tile_table` (and `partials`) have been set up by mfma_gemm_plan
-    int chunk_tiles;       // consecutive tiles that go to one XCD (set by the launchers of the fp32 and the few-row kernels)
+    int chunk_tiles;       // consecutive tiles that go to one XCD (set by the launchers of the fp32, few-row and few-tile kernels)
 };
 
 #define FM_LDS(T) __attribute__((address_space(3))) T
@@ -69,6 +69,28 @@ __device__ __forceinline__ const char *uniform_pointer(const char *pointer) {
     const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits));
     const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32));
     return reinterpret_cast<const char *>((static_cast<uint64_t>(high) << 32) | low);
+}
+
+// ---- where reductions start ------------------------------------------------------------------------------
+// Which slice of the reduction axis the tiles of an expert start with, where both operands are K-contiguous and the axis is whole
+// slices of kRotationSlice. The CUs take slices at about the same pace, and 128 bytes of rows that are a few KiB apart lie in few of the memory's
+// channels: with every expert's weights read from slice 0 on, all CUs ask the same channels at the same time. Experts that run at
+// the same time are spread evenly over the axis instead (the fractional parts of multiples of the golden ratio). Per tile it would
+// be worse: the tiles of an expert share its activations in L2. Row-contiguous weights, 512 bytes of every row at a time, are no
+// faster for it, and neither is a launch that is bound by its MFMAs (kFewRows). Layer 1 (and layer 2's input gradient), us: 44 rows for each of
+// 128 experts of 2048 x 768 218 -> 168 (125 -> 111), 94 for each of 64 of 2048 x 1408 200 -> 158 (106 -> 99), 125 of the 128 228 -> 218 and
+// 218 -> 186 (120 -> 119), 469 of the 64 361 -> 348 (210 -> 210); 1024 of the 128 783 -> 789 (409 -> 409) without the bound.
+constexpr int kRotationSlice = 64, kFewRows = 1024;
+
+__host__ __device__ inline bool starts_anywhere(const GemmArgs &args) {
+    return args.mode != kInputRowSparse && args.num_experts > 1 && args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts &&
+           args.lhs_stride_inner == 1 && args.rhs_stride_inner == 1 && args.inner % kRotationSlice == 0;
+}
+
+__device__ __forceinline__ int first_slice_of(const GemmArgs &args, int expert) {
+    if (!starts_anywhere(args)) return 0;
+    const uint32_t fraction = (static_cast<uint32_t>(expert) * 40503u) & 0xffffu;  // 40503 / 65536 = 0.618...
+    return static_cast<int>((fraction * static_cast<uint64_t>(args.inner / kRotationSlice)) >> 16);
 }
 
 // ---- which tile ----------------------------------------------------------------------------------------
@@ -209,6 +231,9 @@ int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured);
 // Row-sparse products of experts of few rows (fm_gemm_row_sparse.hip), of those that `mfma_gemm_eligible` accepts.
 bool row_sparse_gemm_chosen(const GemmArgs &args, int dtype);
 int row_sparse_gemm_launch(GemmArgs args, int dtype, hipStream_t stream);
+// Products of few tiles (fm_gemm_few_tiles.hip). `splits`: the large tiles' kernel would split the reductions, given a workspace.
+bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits);
+int few_tiles_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream);
 
 // fp32 operands with a unit stride and 16-byte aligned lines (fm_gemm_f32.hip).
 bool f32_gemm_eligible(const GemmArgs &args, int dtype);

@@ -1,0 +1,333 @@
+// Grouped products of few output tiles, in half precision: 128 rows x 64, 128 or 256 columns.
+//
+// A launch of up to one 256 x 256 tile per CU lasts as long as one tile does, on whatever part of the chip, and most of a tile's rows are
+// padding where experts have some 100 tokens. With tiles of half, a quarter or an eighth of that size more CUs share the same work;
+// two small ones per CU overlap one's loads with the other's MFMAs. A CU then reads more operand bytes per multiplication, which is
+// why launches that fill the chip with large tiles stay with those (fm_gemm_mfma.hip; the lines, and what was measured on both sides
+// of them, are at few_tiles_gemm_chosen).
+//
+// Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), two or three in LDS,
+// filled straight from memory; the fragments of the next 16 are read while the MFMAs of this 16 run. Sums in fp32, in the order of
+// the large tiles' kernel.
+#include "fm_gemm_common.h"
+
+namespace fm {
+
+namespace few_tiles {
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
+
+constexpr int kTileM = 128, kBK = kRotationSlice, kThreads = 256, kSteps = kBK / 16;
+constexpr int kBlocksM = kTileM / 64;  // 2 x 2 wavefronts, 32 x 32 accumulators
+
+__device__ __forceinline__ f32x16_t mfma(bf16_t, u32x4_t a, u32x4_t b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16_t mfma(f16_t, u32x4_t a, u32x4_t b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+// One operand's slice in LDS and the loads that fill it: lines [row][kBK] where it is contiguous along K, [kBK][row] otherwise.
+template <int kTile, bool kContiguousK>
+struct Operand {
+    static constexpr int kBytes = kTile * kBK * 2, kChunks = (kContiguousK ? kBK : kTile) / 8;  // 16-byte chunks per line
+    static constexpr int kLoads = kBytes / 16 / kThreads;                                    // per lane and slice
+    static constexpr uint32_t kOutOfRange = 0x80000000u, kRange = 0x7fffffffu;
+
+    // Where chunk `c` of line `line` sits among the line's chunks: the lines that a fragment takes one column of chunks from lie in
+    // different banks.
+    static __device__ __forceinline__ int swizzled(int line, int c) {
+        if constexpr (kContiguousK) return c ^ ((line / (16 / kChunks)) & (kChunks - 1));
+        else return c ^ (((line & 3) << 2) & (kChunks - 1));
+    }
+
+    const char *start, *base;  // wave-uniform: the tile's first element; that of the next slice to fetch
+    int64_t step;              // bytes from one slice to the next
+    uint32_t offset[kLoads];   // per lane, bytes from `base`; out of range where the tile has no such line or column
+    int k[kLoads];             // of the load's first element in the slice
+    int k_count, k_left;       // of the reduction; from `base` on
+    int slices, next, unfetched;
+
+    // `stride`: bytes between lines. `valid`: rows (columns of the product) that exist, a multiple of 8 where they are not lines.
+    __device__ __forceinline__ void setup(const char *first, int64_t stride, int valid, int k_count_, int first_slice, int wave, int lane) {
+        start = uniform_pointer(first);
+        step = kContiguousK ? kBK * 2 : kBK * stride;
+        k_count = k_count_;
+        slices = unfetched = (k_count + kBK - 1) / kBK;
+        next = first_slice;
+        base = start + first_slice * step;
+        k_left = k_count - first_slice * kBK;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int slot = (wave * kLoads + j) * 64 + lane, line = slot / kChunks, chunk = swizzled(line, slot % kChunks);
+            const bool exists = kContiguousK ? line < valid : chunk * 8 < valid;
+            offset[j] = exists ? static_cast<uint32_t>(line * stride + chunk * 16) : kOutOfRange;
+            k[j] = kContiguousK ? chunk * 8 : line;
+        }
+    }
+
+    // The next slice -> the slot at LDS address `slot`: the last slice is followed by the first one, and when all have been fetched
+    // zeros come, without an access to memory. What lies past the reduction comes as zeros too.
+    __device__ __forceinline__ void fetch(int slot, int wave) {
+        const __amdgpu_buffer_rsrc_t resource = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(uniform_pointer(base)), 0, static_cast<int>(kRange), kBufferResourceFlags);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const uint32_t lane_offset = k[j] < k_left ? offset[j] : kOutOfRange;
+            const int target = __builtin_amdgcn_readfirstlane(slot + (wave * kLoads + j) * 1024);
+            // M0 is not handed out by the register allocator and nothing else in this file uses it.
+            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :
+                         : "s"(target), "v"(lane_offset), "s"(resource)
+                         : "memory");
+        }
+        base += step;
+        ++next;
+        --unfetched;
+        if (next == slices) {
+            next = 0;
+            base = start;
+        }
+        k_left = unfetched > 0 ? k_count - next * kBK : 0;
+    }
+
+    // MFMA fragments (8 consecutive k of one row per lane; lane l: row l % 32, k half l / 32) of the 32 rows from `first` on, per lane:
+    // an address per step of 16 (K-contiguous; the next 32 rows and the slot are added), or one per 32 rows (the step is added).
+    static constexpr int kAddresses = kContiguousK ? kSteps : kTile / 64;
+    static __device__ __forceinline__ void fragment_addresses(int first, int lane, int (&addresses)[kAddresses]) {
+        if constexpr (kContiguousK) {
+            const int row = first + (lane & 31);
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) addresses[s] = (row * kChunks + swizzled(row, 2 * s + (lane >> 5))) * 16;
+        } else {
+            const int s = lane & 15, group = lane >> 4, k = ((group >> 1) << 3) + (s >> 2);
+#pragma unroll
+            for (int i = 0; i < kTile / 64; ++i) {
+                const int column = first + i * 32 + ((group & 1) << 4) + ((s & 3) << 2);
+                addresses[i] = k * kTile * 2 + swizzled(k, column >> 3) * 16 + (column & 7) * 2;
+            }
+        }
+    }
+    static __device__ __forceinline__ u32x4_t fragment(const int (&addresses)[kAddresses], int slot, int i, int step) {
+        if constexpr (kContiguousK) {
+            return *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(addresses[step] + slot + i * 32 * kChunks * 16);
+        } else {
+            const uintptr_t at = static_cast<uintptr_t>(addresses[i] + slot + step * 16 * kTile * 2);
+            const i16x4_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FM_LDS(i16x4_t) *)at);
+            const i16x4_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FM_LDS(i16x4_t) *)(at + 4 * kTile * 2));
+            const u32x2_t low_words = __builtin_bit_cast(u32x2_t, low), high_words = __builtin_bit_cast(u32x2_t, high);
+            return u32x4_t{low_words[0], low_words[1], high_words[0], high_words[1]};
+        }
+    }
+};
+
+// Returns once at most `kNewest` of the loads this wavefront has issued are still on their way, and all that it has asked LDS for is
+// there: after a barrier the others' loads may replace what it read.
+template <int kNewest>
+__device__ __forceinline__ void wait_for_loads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kNewest) : "memory");
+}
+
+// Accumulators -> rows of `out`, 32 rows of the wavefront's columns at a time through its own part of LDS: 16 bytes per lane and store.
+// The tile's rows are the MFMA's columns: a lane's four accumulators are consecutive columns of one row.
+template <typename T, int kTileN>
+__device__ __forceinline__ void store_tile(const f32x16_t (&acc)[kBlocksM][kTileN / 64], int staging, T *out, int64_t stride,
+                                           int rows_valid, int cols_valid, int wave_m, int wave_n, int lane) {
+    constexpr int kWaveCols = kTileN / 2, kRowBytes = kWaveCols * 2 + 16;
+    constexpr int kLanesPerRow = kWaveCols / 8, kRowsPerRead = 64 / kLanesPerRow, kReads = 32 / kRowsPerRead;
+    const int write_base = staging + (lane & 31) * kRowBytes + (lane >> 5) * 8;
+    const int read_row = lane / kLanesPerRow, read_column = lane % kLanesPerRow * 8;
+    const int read_base = staging + read_row * kRowBytes + read_column * 2;
+    const int column = wave_n * kWaveCols + read_column, first_row = wave_m * kBlocksM * 32 + read_row;
+#pragma unroll
+    for (int i = 0; i < kBlocksM; ++i) {
+#pragma unroll
+        for (int j = 0; j < kTileN / 64; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                struct {
+                    T v[4];
+                } group;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) group.v[c] = from_float<T>(acc[i][j][4 * g + c]);
+                *(FM_LDS(u32x2_t) *)static_cast<uintptr_t>(write_base + (j * 32 + 8 * g) * 2) = __builtin_bit_cast(u32x2_t, group);
+            }
+        asm volatile("" ::: "memory");  // a wavefront's own LDS accesses are carried out in order
+        u32x4_t staged[kReads];
+#pragma unroll
+        for (int t = 0; t < kReads; ++t)
+            staged[t] = *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(read_base + t * kRowsPerRead * kRowBytes);
+#pragma unroll
+        for (int t = 0; t < kReads; ++t) {
+            const int row = first_row + i * 32 + t * kRowsPerRead;
+            if (row < rows_valid && column < cols_valid)
+                __builtin_nontemporal_store(staged[t], reinterpret_cast<u32x4_t *>(out + row * stride + column));
+        }
+        asm volatile("" ::: "memory");
+    }
+}
+
+template <int kTileN>
+constexpr int kStages = kTileN == 128 ? 2 : 3;
+template <int kTileN>
+constexpr int kWorkgroups = kTileN == 256 ? 1 : 2;  // per CU
+template <int kTileN>
+constexpr int kLdsBytes = kStages<kTileN> * (kTileM + kTileN) * kBK * 2;
+
+template <typename T, int kTileN, bool kRhsK>
+__global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
+    typedef Operand<kTileM, true> Lhs;
+    typedef Operand<kTileN, kRhsK> Rhs;
+    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads, kBlocksN = kTileN / 64;
+    static_assert(kLdsBytes<kTileN> * kWorkgroups<kTileN> <= 160 * 1024 && kLdsBytes<kTileN> >= 4 * 32 * (kTileN + 16), "LDS of a CU");
+    extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
+    const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
+
+    // Consecutive workgroup ids go to the 8 XCDs in turn; an XCD gets runs of `chunk_tiles` consecutive logical tiles.
+    const int pid = blockIdx.x, local = pid / 8;
+    const int logical = (local / args.chunk_tiles * 8 + pid % 8) * args.chunk_tiles + local % args.chunk_tiles;
+    RowTile tile;
+    if (!locate_tile<kTileM>(args, logical, tile)) return;
+    const int64_t col0 = static_cast<int64_t>(tile.tile_n) * kTileN;
+    const int rows_valid = __builtin_amdgcn_readfirstlane(tile.rows_valid);
+    const int cols_valid = __builtin_amdgcn_readfirstlane(static_cast<int>(min(static_cast<int64_t>(kTileN), args.cols - col0)));
+    const int64_t rhs_offset = args.mode == kOutputSparse
+                                   ? (static_cast<int64_t>(tile.expert) * args.sparse_size + col0) * args.rhs_stride_col
+                                   : static_cast<int64_t>(tile.expert) * args.sparse_size * args.rhs_stride_inner + col0 * args.rhs_stride_col;
+    const int k_count = static_cast<int>(args.inner), num_slices = (k_count + kBK - 1) / kBK;
+    const int first_slice = __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert));
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_m = wave / 2, wave_n = wave % 2;
+    Lhs lhs;
+    Rhs rhs;
+    lhs.setup(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row0 * args.lhs_stride_row),
+              args.lhs_stride_row * 2, rows_valid, k_count, first_slice, wave, lane);
+    rhs.setup(reinterpret_cast<const char *>(static_cast<const T *>(args.rhs) + rhs_offset),
+              (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 2, cols_valid, k_count, first_slice, wave, lane);
+    int lhs_addresses[Lhs::kAddresses], rhs_addresses[Rhs::kAddresses];
+    Lhs::fragment_addresses(wave_m * kTileM / 2, lane, lhs_addresses);
+    Rhs::fragment_addresses(wave_n * kTileN / 2, lane, rhs_addresses);
+    f32x16_t acc[kBlocksM][kBlocksN];
+#pragma unroll
+    for (int i = 0; i < kBlocksM; ++i)
+#pragma unroll
+        for (int j = 0; j < kBlocksN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+    int fetch_slot = 0;
+    const auto fetch_slice = [&]() {
+        lhs.fetch(lds + fetch_slot, wave);
+        rhs.fetch(lds + fetch_slot + Lhs::kBytes, wave);
+        fetch_slot = fetch_slot == (kStages<kTileN> - 1) * kSlotBytes ? 0 : fetch_slot + kSlotBytes;
+    };
+    // The oldest slice under way is there, for all wavefronts, and the slot of the slice before it is filled anew: its last fragments
+    // have been read.
+    const auto next_slice = [&]() {
+        wait_for_loads<(kStages<kTileN> - 2) * kLoads>();
+        __syncthreads();
+        fetch_slice();
+    };
+    u32x4_t a[2][kBlocksM], b[2][kBlocksN];
+    const auto read = [&](int buffer, int slot, int step) {
+#pragma unroll
+        for (int i = 0; i < kBlocksM; ++i) a[buffer][i] = Lhs::fragment(lhs_addresses, slot, i, step);
+#pragma unroll
+        for (int j = 0; j < kBlocksN; ++j) b[buffer][j] = Rhs::fragment(rhs_addresses, slot + Lhs::kBytes, j, step);
+    };
+#pragma unroll
+    for (int s = 0; s < kStages<kTileN> - 1; ++s) fetch_slice();
+    next_slice();
+    int slot = lds;
+    read(0, slot, 0);
+    static_assert(kSteps % 2 == 0, "fragment buffers alternate");
+    for (int t = 0; t < num_slices; ++t) {
+        const int next_slot = slot == lds + (kStages<kTileN> - 1) * kSlotBytes ? lds : slot + kSlotBytes;
+#pragma unroll
+        for (int step = 0; step < kSteps; ++step) {
+            const bool last = step + 1 == kSteps;
+            if (last) next_slice();
+            read((step + 1) & 1, last ? next_slot : slot, last ? 0 : step + 1);
+#pragma unroll
+            for (int i = 0; i < kBlocksM; ++i)
+#pragma unroll
+                for (int j = 0; j < kBlocksN; ++j) acc[i][j] = mfma(T(), b[step & 1][j], a[step & 1][i], acc[i][j]);
+            // The reads between the MFMAs, not all in front of them.
+#pragma unroll
+            for (int n = 0; n < kBlocksM * kBlocksN; ++n) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, kRhsK ? 1 : 2, 0);
+            }
+        }
+        slot = next_slot;
+    }
+    wait_for_loads<0>();  // zeros on their way to the slots
+    __syncthreads();
+    T *out = static_cast<T *>(args.out) + tile.row0 * args.out_stride_row + col0;
+    store_tile<T, kTileN>(acc, lds + wave * 32 * (kTileN + 16), out, args.out_stride_row, rows_valid, cols_valid, wave_m, wave_n, lane);
+}
+
+// Tiles of 128 x 256, by the upper bound that the host knows of their row tiles (a static map has one tile of padding per expert).
+static int64_t most_tiles(const GemmArgs &args) { return (args.rows + kTileM - 1) / kTileM * ((args.cols + 255) / 256); }
+
+template <typename T, int kTileN, bool kRhsK>
+static int launch(const GemmArgs &args, hipStream_t stream) {
+    const auto kernel = grouped_gemm_few_tiles_kernel<T, kTileN, kRhsK>;
+    static std::atomic<uint64_t> configured{0};
+    if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes<kTileN>, configured)) return status;
+    const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n, round = 8 * static_cast<int64_t>(args.chunk_tiles);
+    kernel<<<static_cast<uint32_t>((tiles + round - 1) / round * round), kThreads, kLdsBytes<kTileN>, stream>>>(args);
+    return FM_OK;
+}
+
+template <typename T, int kTileN>
+static int launch(GemmArgs args, hipStream_t stream) {
+    args.tiles_m = static_cast<int>((args.rows + kTileM - 1) / kTileM + (args.num_experts > 1 ? args.num_experts : 0));
+    args.tiles_n = static_cast<int>((args.cols + kTileN - 1) / kTileN);
+    const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n;
+    if (tiles >= (int64_t(1) << 30)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
+    // Runs of 16 tiles per XCD; 8 and 32 are up to 3 and 5 % slower (128 columns).
+    args.chunk_tiles = static_cast<int>(min(int64_t(16), (tiles + 7) / 8));
+    return args.rhs_stride_inner == 1 ? launch<T, kTileN, true>(args, stream) : launch<T, kTileN, false>(args, stream);
+}
+
+}  // namespace few_tiles
+
+// Where the lines lie. Over 240 layers of random shapes (4 to 1100 rows per expert, experts equally and unequally liked, sizes that are
+// whole slices and that are not), weights in memory and activations in cache, the time of 256 x 256 tiles divided by that of 64, 128 and
+// 256 columns, geometric means (and the worst), by most_tiles:
+//       up to 64       2.00 (1.85), 1.46, 1.27
+//       65 .. 96       1.74 (1.10), 1.44 (1.19), 1.20
+//       97 .. 160      1.28 (0.95), 1.40 (1.10), 1.23 (0.99)
+//       161 .. 192     1.08, 1.16 (0.99), 1.16 (1.01)
+//       193 .. 256     0.98, 1.09 (0.96), 1.16 (1.00)
+//       257 .. 320     0.95, 1.08 (0.71), 1.13 (0.73): two rounds where 256 x 256 tiles take one
+//       more           0.90, 0.98 (0.66), 1.02 (0.74)
+// Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87), 1.03 (0.63), 0.88 (0.52) up to 96, and no better
+// with more: they stay there.
+bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
+    if (dtype == FM_DTYPE_F32 || args.mode == kInputRowSparse || args.fusion != kFusionNone || args.accumulate || args.out_dtype != dtype ||
+        args.lhs_stride_inner != 1 || splits)
+        return false;
+    return few_tiles::most_tiles(args) <= 256;
+}
+
+template <typename T>
+static int launch_few_tiles(const GemmArgs &args, hipStream_t stream) {
+    const int64_t tiles = few_tiles::most_tiles(args);
+    return tiles <= 80    ? few_tiles::launch<T, 64>(args, stream)
+           : tiles <= 160 ? few_tiles::launch<T, 128>(args, stream)
+                          : few_tiles::launch<T, 256>(args, stream);
+}
+
+int few_tiles_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream) {
+    return dtype == FM_DTYPE_BF16 ? launch_few_tiles<bf16_t>(args, stream) : launch_few_tiles<f16_t>(args, stream);
+}
+
+}  // namespace fm

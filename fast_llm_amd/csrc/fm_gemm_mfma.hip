@@ -329,7 +329,7 @@ struct TileWork {
 
 constexpr int kXcds = 8, kChunkTiles = 32;
 // Reductions of this many slices or more have no half tiles (see finish_tile): with up to kFewRows rows per expert, and with more.
-constexpr int kFewRows = 1024, kHalfTileMaxSlicesFewRows = 128, kHalfTileMaxSlices = 64;
+constexpr int kHalfTileMaxSlicesFewRows = 128, kHalfTileMaxSlices = 64;
 
 // Where the operands and the output of logical tile `logical` are. False: there is no such tile.
 __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, TileWork &work) {
@@ -526,25 +526,6 @@ struct alignas(64) TileRecord {
     int first_slice;   // the slice that the reduction starts with (see first_slice_of)
 };
 static_assert(sizeof(TileRecord) == 64, "one s_load_dwordx16 per record");
-
-// Which slice of the reduction axis the tiles of an expert start with, where both operands are K-contiguous and the axis is whole
-// slices. The CUs take slices at about the same pace, and 128 bytes of rows that are a few KiB apart lie in few of the memory's
-// channels: with every expert's weights read from slice 0 on, all CUs ask the same channels at the same time. Experts that run at
-// the same time are spread evenly over the axis instead (the fractional parts of multiples of the golden ratio). Per tile it would
-// be worse: the tiles of an expert share its activations in L2. Row-contiguous weights, 512 bytes of every row at a time, are no
-// faster for it, and neither is a launch that is bound by its MFMAs (kFewRows). Layer 1 (and layer 2's input gradient), us: 44 rows for each of
-// 128 experts of 2048 x 768 218 -> 168 (125 -> 111), 94 for each of 64 of 2048 x 1408 200 -> 158 (106 -> 99), 125 of the 128 228 -> 218 and
-// 218 -> 186 (120 -> 119), 469 of the 64 361 -> 348 (210 -> 210); 1024 of the 128 783 -> 789 (409 -> 409) without the bound.
-__host__ __device__ inline bool starts_anywhere(const GemmArgs &args) {
-    return args.mode != kInputRowSparse && args.num_experts > 1 && args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts &&
-           args.lhs_stride_inner == 1 && args.rhs_stride_inner == 1 && args.inner % kBK == 0;
-}
-
-__device__ __forceinline__ int first_slice_of(const GemmArgs &args, int expert) {
-    if (!starts_anywhere(args)) return 0;
-    const uint32_t fraction = (static_cast<uint32_t>(expert) * 40503u) & 0xffffu;  // 40503 / 65536 = 0.618...
-    return static_cast<int>((fraction * static_cast<uint64_t>(args.inner / kBK)) >> 16);
-}
 
 // Wave-uniform result; every lane of the wavefront must call it.
 __device__ __forceinline__ bool compute_tile_record(const GemmArgs &args, int id, TileRecord &record) {
@@ -1584,7 +1565,7 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
             TableSpace space;
             const bool eligible = args.fusion == kFusionNone ? mfma_gemm_eligible(args, dtype) : mfma_gemm_fusion_eligible(args, dtype);
             if (!eligible || row_sparse_gemm_chosen(args, dtype) || !table_space(args, space) || !wants_table(args, space.split)) continue;
-            if (space.split != split_ones) continue;
+            if (few_tiles_gemm_chosen(args, dtype, space.split) || space.split != split_ones) continue;
             if (split_ones && at == 0) at = kPartialBytes;
             args.partials = space.split ? static_cast<float *>(workspace) : nullptr;
             args.tile_table = static_cast<char *>(workspace) + at + sizeof(TableHeader);
@@ -1609,17 +1590,15 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
         if (!table_space(args, space)) workspace = nullptr;
         const bool split = workspace != nullptr && splits_last_round(args);
         args.num_ids = count_ids(args, split);
-        if (workspace != nullptr) {
-            const size_t needed = (split ? kPartialBytes : 0) + table_bytes(args.num_ids);
-            if (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0)
-                return fail(FM_ERR_INVALID_ARGUMENT,
-                            "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
-                            workspace_size, workspace);
-            if (split) args.partials = static_cast<float *>(workspace);
-            if (wants_table(args, split)) {
-                args.tile_table = static_cast<char *>(workspace) + (split ? kPartialBytes : 0) + sizeof(TableHeader);
-                if (int status = launch_plan(&args, 1, stream)) return status;
-            }
+        const size_t needed = workspace != nullptr ? (split ? kPartialBytes : 0) + table_bytes(args.num_ids) : 0;
+        if (workspace != nullptr && (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0))
+            return fail(FM_ERR_INVALID_ARGUMENT, "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
+                        workspace_size, workspace);
+        if (few_tiles_gemm_chosen(args, dtype, splits_last_round(args))) return few_tiles_gemm_launch(args, dtype, stream);
+        if (split) args.partials = static_cast<float *>(workspace);
+        if (workspace != nullptr && wants_table(args, split)) {
+            args.tile_table = static_cast<char *>(workspace) + (split ? kPartialBytes : 0) + sizeof(TableHeader);
+            if (int status = launch_plan(&args, 1, stream)) return status;
         }
     }
     return dtype == FM_DTYPE_BF16 ? launch_layout<bf16_t>(args, stream) : launch_layout<f16_t>(args, stream);
