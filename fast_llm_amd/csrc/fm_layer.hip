@@ -159,16 +159,19 @@ int route(const fm_moe_layer &layer, const Plan &plan, void *stream) {
     Step step{layer, plan, stream};
     const bool losses = layer.with_losses != 0;
     FM_REQUIRE(layer.logits && layer.routing && layer.workspace && (layer.losses || !losses), "fm_moe_layer_route: null tensor");
-    FM_STEP(fm_router_forward(layer.logits, layer.noise, step.routing(plan.top_experts), step.routing(plan.scores),
-                              losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
-                              losses ? layer.losses : nullptr, step.routing(plan.router),
-                              plan.routing_bytes - plan.router, layer.tokens, layer.routed_experts, layer.experts_per_token,
-                              layer.shared_experts, step.dtype(), stream));
-    FM_STEP(fm_sparse_map_from_router(reinterpret_cast<const int64_t *>(step.routing(plan.top_experts)), step.routing(plan.router),
-                                      plan.routing_bytes - plan.router, layer.tokens, plan.experts, layer.experts_per_token,
-                                      layer.shared_experts, kPad, plan.index_dtype, step.routing(plan.sparse_rows),
-                                      step.routing(plan.expert_ends), step.routing(plan.expert_pad_begins), layer.workspace,
-                                      plan.forward_workspace_bytes, stream));
+    FM_STEP(router_forward(layer.logits, layer.noise, step.routing(plan.top_experts), step.routing(plan.scores),
+                           losses ? step.routing(plan.lse) : nullptr, losses ? step.routing(plan.statistics) : nullptr,
+                           losses ? layer.losses : nullptr, step.routing(plan.router), plan.routing_bytes - plan.router, layer.tokens,
+                           layer.routed_experts, layer.experts_per_token, layer.shared_experts, step.dtype(), false, stream));
+    RouterFinish finish;
+    if (losses)
+        finish = router_finish_of(step.routing(plan.router), step.routing(plan.statistics), layer.losses, layer.tokens,
+                                  layer.routed_experts, layer.shared_experts);
+    FM_STEP(sparse_map_from_router(reinterpret_cast<const int64_t *>(step.routing(plan.top_experts)), step.routing(plan.router),
+                                   plan.routing_bytes - plan.router, layer.tokens, plan.experts, layer.experts_per_token,
+                                   layer.shared_experts, kPad, plan.index_dtype, step.routing(plan.sparse_rows),
+                                   step.routing(plan.expert_ends), step.routing(plan.expert_pad_begins), layer.workspace,
+                                   plan.forward_workspace_bytes, losses ? &finish : nullptr, stream));
     return FM_OK;
 }
 

@@ -251,55 +251,9 @@ __global__ __launch_bounds__(kRouterMaxThreads) void router_forward_kernel(
         block_counts[static_cast<int64_t>(blockIdx.x) * (experts + shared) + experts + j] = static_cast<int32_t>(max(end - begin, int64_t(0)));
 }
 
-// statistics = the sums over the workgroups of the forward kernel (softmax sums and z-loss sum as doubles: up to 256
-// terms of similar size), losses[0] = load-balancing loss, losses[1] = z-loss. One workgroup: 16 threads share a
-// column, each adds up to 16 of its terms, all requested at once (18 us at 128 experts and 256 workgroups; one thread per
-// column that walked down 1024 workgroups took 261).
-__global__ __launch_bounds__(1024) void router_finish_kernel(const int32_t *__restrict__ block_counts,
-                                                            const float *__restrict__ block_sums,
-                                                            float *__restrict__ statistics, float *__restrict__ losses,
-                                                            int blocks, int64_t tokens, int experts, int shared) {
-    static_assert(kMaxRouterBlocks == 256, "16 x 16 terms per column");
-    __shared__ double lds_sums[16][64];
-    __shared__ int32_t lds_counts[16][64];
-    const int column = threadIdx.x & 63, part = threadIdx.x >> 6;
-    double balance = 0.0;
-    for (int base = 0; base < experts + 1; base += 64) {
-        const int c = base + column;
-        float sums[16];
-        int32_t counts[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int b = part * 16 + i;
-            sums[i] = b < blocks && c < experts + 1 ? block_sums[static_cast<int64_t>(b) * (experts + 1) + c] : 0.f;
-            counts[i] = b < blocks && c < experts ? block_counts[static_cast<int64_t>(b) * (experts + shared) + c] : 0;
-        }
-        double sum = 0.0;
-        int32_t count = 0;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sum += sums[i], count += counts[i];
-        lds_sums[part][column] = sum;
-        lds_counts[part][column] = count;
-        __syncthreads();
-        if (part == 0 && c < experts + 1) {
-            sum = 0.0, count = 0;
-            for (int p = 0; p < 16; ++p) sum += lds_sums[p][column], count += lds_counts[p][column];
-            if (c < experts) {
-                statistics[RouterStats::probability_sum(c)] = static_cast<float>(sum);
-                statistics[RouterStats::count(experts, c)] = static_cast<float>(count);
-                balance += sum * count;
-            } else {
-                statistics[RouterStats::z_sum(experts)] = static_cast<float>(sum);
-                losses[1] = static_cast<float>(sum / static_cast<double>(tokens));
-            }
-        }
-        __syncthreads();
-    }
-    if (part == 0) {
-#pragma unroll
-        for (int offset = 32; offset > 0; offset >>= 1) balance += __shfl_xor(balance, offset, 64);
-        if (column == 0) losses[0] = static_cast<float>(balance / static_cast<double>(tokens) / static_cast<double>(tokens));
-    }
+__global__ __launch_bounds__(kFinishThreads) void router_finish_kernel(RouterFinish finish) {
+    __shared__ FinishLds lds;
+    finish_router(finish, lds);
 }
 
 // Gradient of the raw logits: through the top-k softmax,
@@ -491,10 +445,22 @@ extern "C" int fm_topk_routing_backward(const void *grad_scores, const void *sco
                                static_cast<int>(experts_per_token), 0, dtype, false, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int fm_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse,
-                                 void *statistics, void *losses, void *workspace, size_t workspace_size,
-                                 int64_t num_tokens, int64_t num_experts, int64_t experts_per_token,
-                                 int64_t shared_experts, int dtype, void *stream_) {
+RouterFinish fm::router_finish_of(const void *workspace, void *statistics, void *losses, int64_t num_tokens, int64_t num_experts,
+                                  int64_t shared_experts) {
+    const size_t sums = router_counts_bytes(num_tokens, num_experts + kMaxTopK);
+    return RouterFinish{static_cast<const int32_t *>(workspace),
+                        reinterpret_cast<const float *>(static_cast<const char *>(workspace) + sums),
+                        static_cast<float *>(statistics),
+                        static_cast<float *>(losses),
+                        router_blocks(num_tokens),
+                        static_cast<int>(num_experts),
+                        static_cast<int>(shared_experts),
+                        num_tokens};
+}
+
+int fm::router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse, void *statistics,
+                       void *losses, void *workspace, size_t workspace_size, int64_t num_tokens, int64_t num_experts,
+                       int64_t experts_per_token, int64_t shared_experts, int dtype, bool finish, void *stream_) {
     const char *name = "fm_router_forward";
     if (int status = check_router_shape(name, num_tokens, num_experts, experts_per_token, shared_experts, dtype))
         return status;
@@ -518,11 +484,17 @@ extern "C" int fm_router_forward(const void *logits, const void *noise, void *to
                 return status;
         })
     });
-    if (with_statistics)
-        router_finish_kernel<<<1, 1024, 0, stream>>>(block_counts, block_sums, static_cast<float *>(statistics),
-                                                    static_cast<float *>(losses), router_blocks(num_tokens), num_tokens,
-                                                    experts, shared);
+    if (with_statistics && finish)
+        router_finish_kernel<<<1, kFinishThreads, 0, stream>>>(
+            router_finish_of(workspace, statistics, losses, num_tokens, num_experts, shared_experts));
     return check_launch(name);
+}
+
+extern "C" int fm_router_forward(const void *logits, const void *noise, void *top_experts, void *scores, void *lse, void *statistics,
+                                 void *losses, void *workspace, size_t workspace_size, int64_t num_tokens, int64_t num_experts,
+                                 int64_t experts_per_token, int64_t shared_experts, int dtype, void *stream) {
+    return router_forward(logits, noise, top_experts, scores, lse, statistics, losses, workspace, workspace_size, num_tokens, num_experts,
+                          experts_per_token, shared_experts, dtype, true, stream);
 }
 
 int fm::router_backward(const void *grad_scores, const void *scores, const void *top_experts, const void *logits,

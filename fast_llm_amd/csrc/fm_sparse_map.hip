@@ -73,14 +73,22 @@ __global__ __launch_bounds__(kMapBlock) void sparse_map_histogram_kernel(const i
 // at a time by all threads. A kernel of one workgroup in between, one thread per expert walking down the workgroups,
 // was a serial chain of memory latencies: with 1024 workgroups, 16384 tokens and 8 of 128 experts it took 221 us, and
 // this kernel 8; both now take 12.
+// kFinish: the first workgroup makes the router's sums instead (`finish_router`), which nothing here waits for: as a launch of their
+// own they took 5 (8 experts) to 17 us (128).
+template <bool kFinish>
 __global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(
     const int64_t *__restrict__ top_experts, int64_t num_entries, int64_t entries_per_block, int num_experts,
     const int32_t *__restrict__ block_counts, int64_t pad_to_multiple, int index_dtype, void *__restrict__ sparse_rows,
-    void *__restrict__ expert_ends, void *__restrict__ expert_pad_begins) {
+    void *__restrict__ expert_ends, void *__restrict__ expert_pad_begins, RouterFinish finish) {
     static_assert(kMapMaxExperts <= kMapBlock, "thread e keeps the running count of expert e in a register");
     // [kMapWaves][num_experts] counts per wavefront: 64 KiB at 1024 experts. Before the first of them, in the same place:
     // partial sums [2][kMapBlock], sums [2][num_experts] and the scan's wavefront totals.
     extern __shared__ __attribute__((aligned(16))) int32_t lds_wave_counts[];
+    if constexpr (kFinish) {
+        static_assert(kFinishThreads == kMapBlock, "one workgroup of either kind");
+        if (blockIdx.x == 0) return finish_router(finish, *reinterpret_cast<FinishLds *>(lds_wave_counts));
+    }
+    const int block = static_cast<int>(blockIdx.x) - (kFinish ? 1 : 0), num_blocks = static_cast<int>(gridDim.x) - (kFinish ? 1 : 0);
     int32_t *lds_parts = lds_wave_counts, *lds_totals = lds_parts + 2 * kMapBlock;
     int64_t *lds_wave_totals = reinterpret_cast<int64_t *>(lds_totals + 2 * num_experts);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -91,7 +99,7 @@ __global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(
     // 17; 16384 tokens of 16 of them 45, now 37; 8 of 512 25, now 17.)
     const int columns = 1 << max(num_bits, 3);
     const int column = threadIdx.x & (columns - 1), part = threadIdx.x / columns;
-    const int num_blocks = gridDim.x, per_part = max((num_blocks * columns + kMapBlock - 1) / kMapBlock, 8);
+    const int per_part = max((num_blocks * columns + kMapBlock - 1) / kMapBlock, 8);
     const int parts = (num_blocks + per_part - 1) / per_part;
     int32_t all = 0, before = 0;
     for (int i0 = 0; i0 < per_part; i0 += kMapCountBatch) {
@@ -105,7 +113,7 @@ __global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(
 #pragma unroll
         for (int i = 0; i < kMapCountBatch; ++i) {
             all += here[i];
-            if (part * per_part + i0 + i < static_cast<int>(blockIdx.x)) before += here[i];
+            if (part * per_part + i0 + i < block) before += here[i];
         }
     }
     lds_parts[threadIdx.x] = all;
@@ -139,13 +147,13 @@ __global__ __launch_bounds__(kMapBlock) void sparse_map_rows_kernel(
     if (own_expert < num_experts) {
         const int64_t expert_begin = inclusive - padded;
         running = static_cast<int32_t>(expert_begin) + earlier;
-        if (blockIdx.x == 0) {
+        if (block == 0) {
             store_index(expert_ends, index_dtype, own_expert, inclusive);
             store_index(expert_pad_begins, index_dtype, own_expert, expert_begin + count);
         }
     }
 
-    const int64_t first = static_cast<int64_t>(blockIdx.x) * entries_per_block;
+    const int64_t first = static_cast<int64_t>(block) * entries_per_block;
     const int64_t last = min(first + entries_per_block, num_entries);
     for (int64_t chunk = first; chunk < last; chunk += kMapBlock) {
         for (int i = threadIdx.x; i < kMapWaves * num_experts; i += kMapBlock) lds_wave_counts[i] = 0;
@@ -222,9 +230,9 @@ static int run_sparse_map(const char *name, const int64_t *top_experts, int64_t 
     int32_t *block_counts = static_cast<int32_t *>(workspace);
     sparse_map_histogram_kernel<<<blocks, kMapBlock, experts * sizeof(int32_t), stream>>>(
         top_experts, num_entries, entries_per_block, experts, block_counts);
-    sparse_map_rows_kernel<<<blocks, kMapBlock, map_rows_lds_bytes(experts), stream>>>(
+    sparse_map_rows_kernel<false><<<blocks, kMapBlock, map_rows_lds_bytes(experts), stream>>>(
         top_experts, num_entries, entries_per_block, experts, block_counts, pad_to_multiple, index_dtype, sparse_rows,
-        expert_ends, expert_pad_begins);
+        expert_ends, expert_pad_begins, RouterFinish());
     return check_launch(name);
 }
 
@@ -271,13 +279,11 @@ extern "C" size_t fm_sparse_map_from_router_workspace_size(int64_t num_tokens, i
     return num_tokens < 0 || num_experts < 0 ? 0 : 256;  // the counts are the router's
 }
 
-extern "C" int fm_sparse_map_from_router(const int64_t *top_experts, const void *router_workspace,
-                                         size_t router_workspace_size, int64_t num_tokens, int64_t num_experts,
-                                         int64_t experts_per_token, int64_t shared_experts, int64_t pad_to_multiple,
-                                         int index_dtype, void *sparse_rows, void *expert_ends,
-                                         void *expert_pad_begins, void *workspace, size_t workspace_size,
-                                         void *stream_) {
-    using namespace fm;
+int fm::sparse_map_from_router(const int64_t *top_experts, const void *router_workspace, size_t router_workspace_size,
+                               int64_t num_tokens, int64_t num_experts, int64_t experts_per_token, int64_t shared_experts,
+                               int64_t pad_to_multiple, int index_dtype, void *sparse_rows, void *expert_ends,
+                               void *expert_pad_begins, void *workspace, size_t workspace_size, const RouterFinish *finish,
+                               void *stream_) {
     const char *name = "fm_sparse_map_from_router";
     FM_REQUIRE(shared_experts >= 0 && experts_per_token > 0 && num_experts > shared_experts,
                "%s: %lld experts of which %lld shared, %lld per token", name, (long long)num_experts,
@@ -294,12 +300,25 @@ extern "C" int fm_sparse_map_from_router(const int64_t *top_experts, const void 
                    workspace_size >= fm_sparse_map_from_router_workspace_size(num_tokens, num_experts),
                "%s: workspace of %zu bytes is null, misaligned or too small", name, workspace_size);
     const int experts = static_cast<int>(num_experts);
-    sparse_map_rows_kernel<<<router_blocks(num_tokens), kMapBlock, map_rows_lds_bytes(experts),
-                             static_cast<hipStream_t>(stream_)>>>(
+    size_t lds_bytes = map_rows_lds_bytes(experts);
+    if (finish != nullptr && lds_bytes < sizeof(FinishLds)) lds_bytes = sizeof(FinishLds);
+    const auto kernel = finish != nullptr ? sparse_map_rows_kernel<true> : sparse_map_rows_kernel<false>;
+    kernel<<<router_blocks(num_tokens) + (finish != nullptr ? 1 : 0), kMapBlock, lds_bytes, static_cast<hipStream_t>(stream_)>>>(
         top_experts, num_tokens * slots, router_tokens_per_block(num_tokens) * slots, experts,
         static_cast<const int32_t *>(router_workspace), pad_to_multiple, index_dtype, sparse_rows, expert_ends,
-        expert_pad_begins);
+        expert_pad_begins, finish != nullptr ? *finish : RouterFinish());
     return check_launch(name);
+}
+
+extern "C" int fm_sparse_map_from_router(const int64_t *top_experts, const void *router_workspace,
+                                         size_t router_workspace_size, int64_t num_tokens, int64_t num_experts,
+                                         int64_t experts_per_token, int64_t shared_experts, int64_t pad_to_multiple,
+                                         int index_dtype, void *sparse_rows, void *expert_ends,
+                                         void *expert_pad_begins, void *workspace, size_t workspace_size,
+                                         void *stream) {
+    return fm::sparse_map_from_router(top_experts, router_workspace, router_workspace_size, num_tokens, num_experts, experts_per_token,
+                                      shared_experts, pad_to_multiple, index_dtype, sparse_rows, expert_ends, expert_pad_begins,
+                                      workspace, workspace_size, nullptr, stream);
 }
 
 // ---- the same map without any allocation ----------------------------------------------------------------

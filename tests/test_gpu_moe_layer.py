@@ -6,6 +6,7 @@ import torch
 
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.config import ActivationType, MLPRecomputeLevel
+from fast_llm_amd.functional.routing import router_logits
 from fast_llm_amd.layers.moe import DroplessMoEMLP
 from tests.helpers import max_rel_err
 
@@ -336,3 +337,26 @@ def test_layer_in_library_calls_holds_no_more_memory_than_the_composition(recomp
     # What the backward's call needs beside its intermediates: the input gradient (16 MiB) and its workspace.
     assert peaks[4] <= peaks[6] + (24 << 20), [peak >> 20 for peak in peaks]
     assert peaks[5] <= peaks[7] + (1 << 20), [peak >> 20 for peak in peaks]
+
+
+# The router's sums over its workgroups (16 tokens each, 256 at most) share a launch with the sparse map: fewer experts than the 8
+# columns of a workgroup's threads, more than a wavefront holds, more than one batch of terms per thread.
+@pytest.mark.parametrize(("tokens", "experts", "shared"), [(1, 3, 0), (17, 8, 1), (300, 64, 0), (4200, 65, 2), (5000, 300, 0), (40, 1000, 0)])
+def test_losses_and_map_in_one_launch(tokens, experts, shared, device):
+    torch.manual_seed(0)
+    layer = DroplessMoEMLP(
+        64, 64, experts + shared, 2, shared_experts=shared, z_loss_coefficient=0.1, auxiliary_loss_coefficient=0.1,
+        init_std=0.2, dtype=torch.bfloat16, device=device,
+    )  # fmt: skip
+    x = torch.randn(tokens, 64, device=device, dtype=torch.bfloat16, requires_grad=True)
+    one, composed = _step(layer, [x], False), _step(layer, [x], True)
+    for name in ("outputs", "losses", "weight_grads"):
+        assert all(torch.equal(a, b) for a, b in zip(one[name], composed[name], strict=True)), name
+    # Against the definition: sum_e mean_t(softmax) * mean_t(selected), mean_t(logsumexp^2), in fp64.
+    logits = router_logits(x.detach(), layer.router.detach()).double()
+    selected = torch.zeros_like(logits).scatter_(1, logits.topk(2, 1).indices, 1)
+    balance = (logits.softmax(1).mean(0) * selected.mean(0)).sum()
+    z = logits.logsumexp(1).square().mean()
+    # Per token fp32 exponentials and sums. A tie between rounded logits may be broken otherwise: then the expert of one token.
+    assert abs(one["losses"][0].double() - balance) <= 1e-5 * balance + 2 / tokens * logits.softmax(1).mean(0).max()
+    assert abs(one["losses"][1].double() - z) <= 1e-5 * z + 1e-6
