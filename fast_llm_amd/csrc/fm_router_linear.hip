@@ -12,7 +12,9 @@
 // hidden axis each, fragments straight from memory into registers, all loads of eight steps under way at once, and one exchange
 // through LDS at the end (twice the wavefronts are no faster). us on the device, the device library's product in brackets: one token of
 // 4096 and 8 experts 4.8 (7.4), 64 tokens 7.6 (7.6), 96 of 2048 and 128 experts 5.5 (5.4), 512 of 256 and 8 experts in single
-// precision 3.3 (3.7); 1531 of 4096 and 8 experts 7.8 (6.0). Calling that library takes 19 us of the host's time, this 8.
+// precision 3.3 (3.7), operands in cache; from memory 1531 of 4096 and 8 experts 13.8 (20), 3001 of 1280 and 16 9.3 (13), 700 of 2048 and
+// 64 9.8 (14.7), 1999 of 2048 and 128 21.8 (16.6). Calling that library takes 19 us of the host's time, this 8. Workgroups of 2 x 4 to
+// 4 x 8 tiles, which read less, lose more to the fewer of them (5001 of 2048 and 64 experts 23 to 28 us, 28 so, 18.8).
 #include "fm_gemm_common.h"
 #include "fm_router_layout.h"
 

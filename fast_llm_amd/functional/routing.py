@@ -14,10 +14,11 @@ from fast_llm_amd import _lib
 from fast_llm_amd.functional.utils import is_traced
 
 
-# Up to this many tiles of 16 tokens x 16 experts the library's own kernel computes the logits: as fast as torch's product on the
-# device (3.3 to 7.6 us, torch 3.7 to 7.6) and 11 us less of the host's time, which small layers are bound by. From 96 tiles on
-# torch's is ahead by up to 2 us.
-_MAX_LOGIT_TILES = 64
+# Bytes of a row times tiles of 16 tokens x 16 experts, which read their rows each by itself: up to this the library's own kernel
+# computes the logits, in 6 to 14 us (single precision 8 to 20) where torch's product takes 11 to 26 (12 to 99), operands not in
+# cache, and with 11 us less of the host's time. 64 tiles of 4096 14 us (torch 20), 188 of 1280 9 (13), 1000 of 512 11 (12); from twice as
+# much on torch's is ahead (1000 of 2048 22 and 17).
+_MAX_LOGIT_BYTES = 1_200_000
 
 
 def _few_logits(input_: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -26,7 +27,7 @@ def _few_logits(input_: torch.Tensor, weight: torch.Tensor) -> bool:
         input_.dim() == 2
         and weight.dim() == 2
         and input_.size(0) > 0
-        and -(-input_.size(0) // 16) * -(-weight.size(0) // 16) <= _MAX_LOGIT_TILES
+        and -(-input_.size(0) // 16) * -(-weight.size(0) // 16) * input_.size(1) * input_.element_size() <= _MAX_LOGIT_BYTES
         and input_.dtype == weight.dtype
         and input_.dtype in _lib.DTYPES
         and input_.size(1) == weight.size(1)

@@ -358,7 +358,7 @@ int fm_few_tokens_forward(const void *input, const void *top_experts, const void
                           size_t workspace_size, void *stream);
 
 /* The router's linear layer, logits [num_tokens, num_experts] = input [num_tokens, hidden] x weight [num_experts, hidden]^T, for few
- * tokens: meant for up to 64 tiles of 16 tokens x 16 experts, correct for any number. All contiguous, of `dtype`, sums in fp32;
+ * tokens: meant for up to 1.2 MB of row bytes x tiles of 16 tokens x 16 experts, correct for any number. All contiguous, of `dtype`, sums in fp32;
  * input and weight 16-byte aligned and hidden a multiple of 16 bytes (FM_ERR_UNSUPPORTED). Deterministic. */
 int fm_router_linear_forward(const void *input, const void *weight, void *logits, int64_t num_tokens, int64_t num_experts,
                              int64_t hidden, int dtype, void *stream);

@@ -13,7 +13,7 @@ _ROUND = {torch.float32: 2**-24, torch.bfloat16: 2**-8, torch.float16: 2**-11}
 
 
 @pytest.mark.parametrize("dtype", list(_ROUND))
-@pytest.mark.parametrize(("tokens", "experts"), [(1, 1), (1, 8), (15, 16), (17, 17), (33, 60), (64, 128), (1024, 8)])
+@pytest.mark.parametrize(("tokens", "experts"), [(1, 1), (1, 8), (15, 16), (17, 17), (33, 60), (64, 128), (1024, 8), (1100, 3)])
 @pytest.mark.parametrize("hidden", [8, 32, 40, 264, 2056, 4096])
 def test_logits(dtype, tokens, experts, hidden, device):
     generator = torch.Generator(device).manual_seed(tokens + experts + hidden)
@@ -48,7 +48,7 @@ def test_what_the_kernel_does_not_take(device):
     for operands in ((x[:, :66], weight[:, :66]), (x.t().contiguous().t(), weight), (x[:0], weight), (x[1:, 1:], weight[:, 1:])):
         assert not routing._few_logits(*operands)
         assert torch.equal(routing.router_linear(*operands), torch.nn.functional.linear(*operands))
-    many = torch.randn((16 * routing._MAX_LOGIT_TILES + 1, 68), device=device)
+    many = torch.randn((16 * (routing._MAX_LOGIT_BYTES // (68 * 4)) + 1, 68), device=device)
     assert not routing._few_logits(many, weight) and routing._few_logits(many[1:], weight)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert routing.router_linear(x, weight).dtype == torch.bfloat16
