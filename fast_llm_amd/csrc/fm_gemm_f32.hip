@@ -2,7 +2,7 @@
 //   * v_mfma_f32_32x32x16_bf16 on operands split into three bf16 parts each (`grouped_gemm_f32_split_kernel`, below): six
 //     products of parts instead of one of values at 16 times the rate of fp32 multiply-adds;
 //   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for reductions so short that start and epilogue are all there is.
-// Forward and backward products of 4096 rows over 8 experts, 1024 x 2816 (5632): 2111 us for the six on fp32 multiply-adds, 1403 on
+// Forward and backward products of 4096 rows over 8 experts, 1024 x 2816 (5632): 1864 us for the six on fp32 multiply-adds, 1345 on
 // split operands.
 //   * Operand slices (kBK reduction indices) go straight from global memory into LDS (`buffer_load ... lds`, 16 bytes
 //     per lane), at least one slice ahead of the multiplications, one barrier per slice. Lanes that have nothing to fetch (rows
@@ -280,12 +280,15 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
 // 64 bits than those: relative 1.9e-7 against 5.7e-7 (layer 1, 1024 reduction indices), 1.6e-7 against 4.8e-7 (layer 2, 2816),
 // 1.3e-7 against 4.1e-7 (weight gradients, 512), and for all shapes and products measured.
 //
-// The parts carry what fp32 does down to 2^-110, where the third meets the end of bf16's range (2^-133), and up to where bf16
-// rounds to infinity. A result that is NaN, infinite or below 2^-90 (and not zero) may have met either: its tile is
-// computed again by fp32 multiply-adds, which such results are taken from. (An operand below 2^-110 among
-// larger ones loses what lies below 2^-134, which no sum of normal size shows.)
+// Every value is multiplied by 2^24 first. bf16 has the exponents of fp32 but 8 bits, so the second and third part of a value below
+// 2^-110 would lie under bf16's range whatever the value is multiplied with; scaled, the parts of every fp32 value are
+// normal bf16 numbers, and the products of parts that the sums (2^48 of the result) cannot hold are below a result's smallest unit.
+// What is lost is the other end: operands from 2^103 and sums from 2^80 on become infinite, which their results show. A result that is
+// infinite or NaN is taken from fp32 multiply-adds: its tile is computed again, on two workgroups per CU (layer 1 of the above with a
+// NaN in one row 304 -> 331 us, with one in every tile 655, where fp32 multiply-adds in the first place take 390). The six products
+// take 5 % longer for the scaling; one vector instruction per value is also what it takes to look for values that are too small.
 //
-// Every wavefront splits the fragments it multiplies: 7.3 vector instructions per MFMA of 32 cycles, interleaved with the MFMAs of
+// Every wavefront splits the fragments it multiplies: 8.7 vector instructions per MFMA of 32 cycles, interleaved with the MFMAs of
 // the fragments before (two wavefronts per SIMD; 6 such instructions cost an MFMA nothing, and the residual as a bf16 dot product,
 // half as many instructions, 5 cycles each of the matrix pipe). Splitting once per workgroup instead would move 6 bytes per
 // element through LDS both ways, which is as long as the MFMAs take. The device then runs at 1.84 GHz: power.
@@ -295,10 +298,12 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
 //   64 x 64: 4 quarters of a slice of 64
 // (halves and quarters add up in LDS), by how many tiles there are: see `f32_gemm_launch`.
 
+constexpr float kOperandScale = 0x1p24f, kResultScale = 0x1p-48f;
+
 __device__ __forceinline__ void split(const float (&values)[8], bf16x8_t (&parts)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float rest_0 = values[2 * i], rest_1 = values[2 * i + 1];
+        float rest_0 = values[2 * i] * kOperandScale, rest_1 = values[2 * i + 1] * kOperandScale;
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
             const bf16x2_t pair = __builtin_convertvector((f32x2_t{rest_0, rest_1}), bf16x2_t);
@@ -319,8 +324,6 @@ __device__ __forceinline__ void interleave() {
         __builtin_amdgcn_sched_group_barrier(0x2, 7, 0);
     }
 }
-
-constexpr int kNanInfOrSubnormal = 0x001 | 0x002 | 0x004 | 0x200 | 0x010 | 0x080;  // classes of v_cmp_class
 
 template <int kTileM, int kTileN, int kStages, bool kLhsK, bool kRhsK>
 __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f32_split_kernel(GemmArgs args) {
@@ -450,7 +453,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f32_split_kernel(Gem
         }
     };
     add_shares();
-    const auto in_doubt = [](float value) { return __builtin_amdgcn_classf(value * 0x1p-36f, kNanInfOrSubnormal); };
+    const auto in_doubt = [](float value) { return !__builtin_isfinite(value); };
     bool again = false;
 #pragma unroll
     for (int held = 0; held < kHeld; ++held)
@@ -489,8 +492,13 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f32_split_kernel(Gem
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const float value = first[held / 2][held % 2][v];
-                if (!in_doubt(value)) acc[held / 2][held % 2][v] = value;
+                if (!in_doubt(value)) acc[held / 2][held % 2][v] = value * kResultScale;
             }
+    } else {
+#pragma unroll
+        for (int held = 0; held < kHeld; ++held)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[held / 2][held % 2][v] *= kResultScale;
     }
 #pragma unroll
     for (int held = 0; held < kHeld; ++held) {

@@ -19,11 +19,13 @@ def _operands(columns, inner, device, rhs_along_k):
     return lhs, rhs.t() if rhs_along_k else rhs.t().contiguous()
 
 
-def _check(out, lhs, rhs):
+def _check(out, lhs, rhs, multiply_adds=False):
     """Worst case of the kernel: at most inner / 16 + 5 roundings of the large sum and as many, 2^-8 as large, of the small ones; parts
-    left out are below 2^-25 of a product. Rounded up to inner / 16 + 8 units of 2^-24 of the sum of magnitudes."""
+    left out are below 2^-25 of a product. Rounded up to inner / 16 + 8 units of 2^-24 of the sum of magnitudes, and the smallest
+    fp32 number for results below the normal ones. fp32 multiply-adds round every two reduction indices."""
     exact = lhs.double() @ rhs.double()
-    bound = (lhs.shape[1] / 16 + 8) * 2**-24 * (lhs.double().abs() @ rhs.double().abs()) + 2.0**-126
+    roundings = lhs.shape[1] / (2 if multiply_adds else 16) + 8
+    bound = roundings * 2**-24 * (lhs.double().abs() @ rhs.double().abs()) + 2.0**-149
     assert ((out.double() - exact).abs() <= bound).all()
 
 
@@ -75,9 +77,36 @@ def test_values_that_bf16_parts_cannot_hold(tile, device):
     rest = [row for row in range(200) if row not in (infinite, nan, largest)]
     _check(out[rest], lhs[rest], rhs)
 
-    # Rows of one magnitude each, down to where the third part of a value is below the smallest bf16.
+    # Rows of one magnitude each, down to where the third part of a value would be below the smallest bf16.
     lhs, rhs = _operands(_COLUMNS[tile], inner, device, True)
     lhs *= 2.0 ** -torch.linspace(0, 118, 200, device=device).round()[:, None]
     _check(dense_matmul(lhs, rhs), lhs, rhs)
     lhs[:] = 0
     assert (dense_matmul(lhs, rhs) == 0).all()
+
+
+# Operands with an exponent each, the smallest results below the smallest normal number. From 2^103 on (and sums from 2^80 on) the
+# results are those of fp32 multiply-adds.
+@pytest.mark.parametrize("tile", _COLUMNS)
+@pytest.mark.parametrize(
+    ("lhs_exponent", "rhs_exponent"),
+    [(-112, 40), (-120, 60), (-126, 100), (100, -126), (-126, 120), (-112, 105), (60, 30), (-113, 0), (-124, 0), (0, -126), (-70, -70)],
+)
+def test_operands_of_all_magnitudes(tile, lhs_exponent, rhs_exponent, device):
+    inner = 48
+    lhs, rhs = (x.sign() * (1 + x.abs() % 1) for x in _operands(_COLUMNS[tile], inner, device, True))
+    lhs, rhs = lhs * 2.0**lhs_exponent, rhs * 2.0**rhs_exponent
+    multiply_adds = max(lhs_exponent, rhs_exponent) >= 102 or lhs_exponent + rhs_exponent >= 72
+    _check(dense_matmul(lhs, rhs), lhs, rhs, multiply_adds)
+    # Among operands of ordinary size: a row and a column of these, a row of them here and there.
+    mixed_lhs, mixed_rhs = _operands(_COLUMNS[tile], inner, device, True)
+    mixed_lhs[77], mixed_lhs[130, ::5], mixed_rhs[:, 33] = lhs[77], lhs[130, ::5], rhs[:, 33]
+    _check(dense_matmul(mixed_lhs, mixed_rhs), mixed_lhs, mixed_rhs, multiply_adds)
+
+
+def test_subnormal_operands(device):
+    lhs, rhs = _operands(_COLUMNS["64x64"], 48, device, True)
+    lhs *= 2.0**-140
+    out = dense_matmul(lhs, rhs * 2.0**100)
+    assert out.abs().max() > 0
+    _check(out, lhs, rhs * 2.0**100)
