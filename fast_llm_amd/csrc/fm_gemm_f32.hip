@@ -1,7 +1,7 @@
 // Grouped matrix products of fp32 operands on the gfx950 matrix cores, by one of two instructions:
 //   * v_mfma_f32_32x32x16_bf16 on operands split into three bf16 parts each (`grouped_gemm_f32_split_kernel`, below): six
 //     products of parts instead of one of values at 16 times the rate of fp32 multiply-adds;
-//   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for reductions so short that start and epilogue are all there is.
+//   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for short reductions and few tiles (see `f32_gemm_launch`).
 // Forward and backward products of 4096 rows over 8 experts, 1024 x 2816 (5632): 1864 us for the six on fp32 multiply-adds, 1345 on
 // split operands.
 //   * Operand slices (kBK reduction indices) go straight from global memory into LDS (`buffer_load ... lds`, 16 bytes
@@ -582,18 +582,40 @@ static int launch_f32_tile(GemmArgs args, int64_t tiles, hipStream_t stream) {
     return FM_OK;
 }
 
-// Which tile, by upper bounds of how many there are (a map's padding counted). us, 8 or 16 experts, 2 slots:
-//   * forward and input gradients, 128 x 128 / 128 x 64 / 64 x 64 on split operands (fp32 multiply-adds): 384 tiles of 128 x 64
-//     (256 reduction indices) 18 / 14 / 14 (14), 768 (2816) 213 / 175 / 166 (285), 1032 (320) 24 / 22 / 22 (29), 2048 (768) 100 / 94 / 106
-//     (140), 2112 (1024) 170 / 160 / 177 (243), 4224 (1024) 315 / 331 / 357 (447), 5632 (1024) 325 / 355 / 394 (492). Below 128 tiles of
-//     64 x 64 four times as many of 32 x 32 are faster without splitting: 56 tiles (1024) 16.5 (13.5).
-//   * weight gradients on 128 x 128 from one per CU on: 1408 tiles (512) 138, 128 x 64 152, fp32 220; 128 tiles (512) 29 / 20 (26).
-//   * reductions over few rows are all start and epilogue, and eight workgroups per CU have the most in flight: means of 8 / 16 / 32
-//     / 50 / 64 / 128 rows 113 (87), 24 (22), 60 (54), 74 (75), 72 (76), 46 (66). A map's buffer has a tile of 128 rows of padding per
-//     expert on top of the mean.
-// The fp32 kernel's own tiles, 64 x 64 / 32 x 32: 1056 tiles of 64 x 64 36 / 34, 1120 24 / 26, 1408 295 / 265, 2048 23 / 29, 3872 238 / 254.
-constexpr int64_t kF32FewTiles = 128, kF32MiddleTiles = 1024, kF32ManyTiles = 2560, kF32LargeTiles = 1536;
-constexpr int64_t kF32ShortReduction = 128 + 48;
+// Which kernel and tile, by the 64 x 64 tiles that the rows are expected to fill (half a tile per expert of a map is not; a buffer's own
+// rows are mostly padding where experts have few). Reductions shorter than short_reduction are start and epilogue, and what few tiles
+// there are runs on more CUs as tiles of 32 x 32: there eight workgroups of fp32 multiply-adds per CU are faster. Time on split
+// operands over that on multiply-adds, geometric means over 2300 products of 4 to 16 experts of 8 to 512 rows, operands not in L2:
+//     tiles       reduction 128   256   384   512  1024  2816
+//     65 .. 160            1.38  1.20  1.07  1.00  0.89  0.80
+//     257 .. 400           1.14  1.06  1.01  1.02  0.93  0.88
+//     401 .. 600           1.09  1.05  0.99  0.94  0.86  0.77
+//     1001 .. 1500         1.09  0.97  0.91  0.86  0.79  0.75
+//     from 2501 on         0.95  0.86  0.82  0.80  0.75  0.71
+// A side of up to 32 leaves half of every split tile empty: 16384 x 32 of 256 7 us against 10, of 2816 66 against 51. By the rule these
+// products take 0.894 of the time of multiply-adds (worst 1.22; the best choice for each 0.871), dense ones of 8 to 65536 rows 0.946
+// (0.893). All large launches on split operands took 0.951 and 1.095, worst 2.4 (8192 x 2048 of 8 18 -> 31 us).
+// Tiles of 64 x 64 / 128 x 64 / 128 x 128, us: 8 experts of 512, 1024 columns of 2816 (1088 tiles) 181 / 194 / 228; 2816 of 1024 (2992) 161 /
+// 157 / 158; 5632 of 1024 (5984) 333 / 300 / 298. Experts of up to 48 rows fill no 128: 16 of 48, 5632 columns of 1024 115 / 154 / 147.
+// fp32 tiles of 64 x 64 by the upper bound of them: 1056 36 (32 x 32: 34), 1120 24 (26), 1408 295 (265), 2048 23 (29), 3872 238 (254); of
+// experts of up to 32 rows not where the reduction is long: 16 of 8, 2816 columns of 2816 195 (106).
+constexpr int64_t kF32LargeTiles = 1536, kMiddleTiles = 1200, kLargeTiles = 2816;
+static int64_t short_reduction(int64_t tiles, bool narrow) {
+    const int64_t most = tiles < 64 ? 1024 : tiles < 400 ? 512 : tiles < 700 ? 384 : tiles < 1536 ? 256 : tiles < 2500 ? 192 : 128;
+    return narrow ? max(most, int64_t(768)) : most;
+}
+// Weight gradients, time over that on multiply-adds again, 64 x 64 / 128 x 64 / 128 x 128:
+//     tiles     reduction 48              128              512              1024             4096
+//     32        1.78 / 2.11 / 2.44  1.60 / 1.97 / 2.60  1.27 / 1.90 / 3.01  1.03 / 1.59 / 2.69  0.76 / 1.28 / 2.37
+//     256       1.18 / 1.34 / 1.56  1.09 / 1.26 / 1.61  0.90 / 1.18 / 1.74  0.82 / 1.17 / 1.83  0.71 / 1.06 / 1.84
+//     512       1.02 / 1.01 / 1.12  1.00 / 0.94 / 1.14  0.92 / 0.82 / 1.16  0.76 / 0.78 / 1.14  0.71 / 0.76 / 1.11
+//     1024      1.11 / 0.85 / 0.81  1.02 / 0.94 / 0.81  0.83 / 0.74 / 0.76  0.73 / 0.71 / 0.73  0.68 / 0.67 / 0.67
+//     5632      1.77 / 1.31 / 1.04  1.44 / 1.07 / 0.92  0.92 / 0.83 / 0.77  0.84 / 0.78 / 0.76  0.79 / 0.76 / 0.76
+// With the operands in cache, as after the product before, few tiles gain later: 128 tiles of 2048 29 / 33 us.
+constexpr int64_t kMiddleGradients = 512, kLargeGradients = 1024;
+static int64_t short_gradient_reduction(int64_t tiles) {
+    return tiles >= kLargeGradients ? 64 : tiles >= kMiddleGradients ? 128 : tiles >= 256 ? 512 : tiles >= 64 ? 2048 : 4096;
+}
 
 int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
     // Upper bounds of the numbers of tiles (the surplus ids have none).
@@ -605,22 +627,37 @@ int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
         args.tiles_n = static_cast<int>((args.cols + tile_n - 1) / tile_n);
         return static_cast<int64_t>(args.tiles_m) * args.tiles_n;
     };
+    const bool mapped = args.expert_ends != nullptr;
     if (args.mode == kInputRowSparse) {
-        const int64_t reduction = args.piece_length > 0 ? args.piece_length : args.inner / args.num_experts;
-        if (reduction >= kF32ShortReduction && args.sparse_size >= 64 && args.cols >= 64) {
-            if (const int64_t tiles = count(128, 128); tiles >= 256) return launch_f32_split<128, 128, 3>(args, tiles, stream);
-            const int64_t tiles = count(128, 64);
-            return launch_f32_split<128, 64, 3>(args, tiles, stream);
-        }
-    } else if (count(64, 64) > kF32FewTiles) {
-        const int64_t tiles = count(128, 64);
-        if (tiles >= kF32ManyTiles) {
+        int64_t reduction = args.piece_length > 0 ? args.piece_length : args.inner;
+        // A map's buffer has a tile of 128 rows of padding per expert.
+        if (mapped) reduction = args.tokens > 0 ? args.tokens / args.num_experts : args.inner / args.num_experts - 128;
+        const int64_t tiles = count(64, 64);
+        if (args.sparse_size >= 64 && args.cols >= 64 && reduction >= short_gradient_reduction(tiles)) {
+            if (tiles < kMiddleGradients) return launch_f32_split<64, 64, 2>(args, tiles, stream);
+            const int64_t middle = count(128, 64);
+            if (tiles < kLargeGradients) return launch_f32_split<128, 64, 3>(args, middle, stream);
             const int64_t large = count(128, 128);
             return launch_f32_split<128, 128, 3>(args, large, stream);
         }
-        if (tiles > kF32MiddleTiles) return launch_f32_split<128, 64, 3>(args, tiles, stream);
-        const int64_t small = count(64, 64);
-        return launch_f32_split<64, 64, 2>(args, small, stream);
+    } else {
+        // Half of that padding is computed where the caller does not say where it begins.
+        const int64_t padding = args.expert_pad_begins != nullptr ? 128 : 64;
+        int64_t rows = args.rows;
+        if (mapped) rows = max(args.tokens > 0 ? args.tokens / args.num_experts : args.rows / args.num_experts - padding, int64_t(1));
+        const int64_t tiles_n = (args.cols + 63) / 64, tiles = mapped ? args.num_experts * (rows + 32) / 64 * tiles_n : (rows + 63) / 64 * tiles_n;
+        if (args.inner >= short_reduction(tiles, min(rows, args.cols) <= 32)) {
+            const int64_t small = count(64, 64);
+            if (tiles < kMiddleTiles || (mapped && rows <= 48)) return launch_f32_split<64, 64, 2>(args, small, stream);
+            const int64_t middle = count(128, 64);
+            if (tiles < kLargeTiles) return launch_f32_split<128, 64, 3>(args, middle, stream);
+            const int64_t large = count(128, 128);
+            return launch_f32_split<128, 128, 3>(args, large, stream);
+        }
+        if (rows <= 32 && args.inner >= 256) {
+            const int64_t tiles_32 = count(32, 32);
+            return launch_f32_tile<32, 32, 2>(args, tiles_32, stream);
+        }
     }
     if (const int64_t tiles = count(64, 64); tiles >= kF32LargeTiles) return launch_f32_tile<64, 16, 2>(args, tiles, stream);
     const int64_t tiles = count(32, 32);

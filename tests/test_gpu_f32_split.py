@@ -1,5 +1,7 @@
 """fp32 products on operands split into bf16 parts: every tile shape against 64 bits, and operands that the parts cannot hold."""
 
+import itertools
+
 import pytest
 import torch
 
@@ -8,8 +10,10 @@ from fast_llm_amd.functional.sparse_linear import dense_matmul, input_row_sparse
 
 pytestmark = pytest.mark.gpu
 
-# Columns with 200 rows (two row tiles of 128, four of 64) for tiles of 64 x 64, 128 x 64 and 128 x 128, each with a remainder.
-_COLUMNS = {"64x64": 2564, "128x64": 33028, "128x128": 82052}
+# Columns with 200 rows (two row tiles of 128, four of 64) for tiles of 64 x 64, 128 x 64 and 128 x 128, each with a remainder, and the
+# reductions from which on they are split: shorter ones are fp32 multiply-adds.
+_COLUMNS = {"64x64": 12804, "128x64": 33028, "128x128": 82052}
+_SPLIT_FROM = {"64x64": 256, "128x64": 192, "128x128": 128}
 
 
 def _operands(columns, inner, device, rhs_along_k):
@@ -30,39 +34,60 @@ def _check(out, lhs, rhs, multiply_adds=False):
 
 
 @pytest.mark.parametrize("tile", _COLUMNS)
-@pytest.mark.parametrize("inner", [4, 16, 20, 64, 132])
+@pytest.mark.parametrize("inner", [4, 16, 20, 64, 132, 192, 256, 260, 276, 324])
 @pytest.mark.parametrize("rhs_along_k", [True, False])
 def test_tiles(tile, inner, rhs_along_k, device):
     lhs, rhs = _operands(_COLUMNS[tile], inner, device, rhs_along_k)
     out = dense_matmul(lhs, rhs)
-    _check(out, lhs, rhs)
+    _check(out, lhs, rhs, multiply_adds=inner < _SPLIT_FROM[tile])
     twice = dense_matmul(lhs, rhs, out.clone(), accumulate=True)
     assert torch.equal(twice, out + out)
 
 
-@pytest.mark.parametrize("columns", [68, 132, 4100])
-def test_row_sparse(columns, device):
-    """Reductions of 0, 1, 200 and 383 rows, NaN in the padding, both tile shapes."""
-    rows, ends = [0, 1, 200, 383], [0, 128, 384, 768]
+@pytest.mark.parametrize("rows", [(0, 1, 200, 383), (0, 1, 1000, 2100)])
+@pytest.mark.parametrize("columns", [68, 132, 1000, 2000, 4100])
+def test_row_sparse(columns, rows, device):
+    """Reductions of few and many rows, NaN in the padding: multiply-adds and, of many rows from 1000 columns on, all tile shapes."""
+    ends = list(itertools.accumulate(-(-count // 128) * 128 for count in rows))
+    begins = [0, *ends[:-1]]
     sparse_map = SparseMap(
         None, torch.tensor(ends, dtype=torch.int32, device=device),
-        torch.tensor([0, 1, 128 + 200, 384 + 383], dtype=torch.int32, device=device), None, 768, None, 4, None,
+        torch.tensor([begin + count for begin, count in zip(begins, rows)], dtype=torch.int32, device=device), None, ends[-1], None, 4, None,
     )  # fmt: skip
     generator = torch.Generator(device).manual_seed(columns)
-    x = torch.full((768, 260), float("nan"), device=device)
-    y = torch.full((768, columns), float("nan"), device=device)
-    for end, count, begin in zip(ends, rows, [0, *ends]):
+    x = torch.full((ends[-1], 260), float("nan"), device=device)
+    y = torch.full((ends[-1], columns), float("nan"), device=device)
+    for count, begin in zip(rows, begins):
         x[begin : begin + count].normal_(generator=generator)
         y[begin : begin + count].normal_(generator=generator)
     out = input_row_sparse_matmul(x.t(), y, sparse_map)
-    for expert, (count, begin) in enumerate(zip(rows, [0, *ends])):
-        _check(out[expert * 260 : (expert + 1) * 260], x[begin : begin + count].t(), y[begin : begin + count])
+    for expert, (count, begin) in enumerate(zip(rows, begins)):
+        lhs, rhs = x[begin : begin + count].t(), y[begin : begin + count]
+        _check(out[expert * 260 : (expert + 1) * 260], lhs, rhs, multiply_adds=columns < (1000 if max(rows) > 1000 else 4100))
+
+
+@pytest.mark.parametrize(("rows", "cols", "inner"), [(2048, 1024, 8), (8192, 2048, 8), (16384, 8, 8), (16384, 32, 264), (24, 16384, 264)])
+def test_short_reductions_and_narrow_sides_are_multiply_adds(rows, cols, inner, device):
+    """Where splitting is the slower route: the same bits as in a product of one tile, which is never split."""
+    lhs, rhs = torch.randn((rows, inner), device=device), torch.randn((inner, cols), device=device)
+    few_rows, few_cols = lhs[:64], rhs[:, :64].contiguous()
+    assert torch.equal(dense_matmul(lhs, rhs)[:64, :64], dense_matmul(few_rows, few_cols))
+
+
+def test_few_gradient_tiles_are_multiply_adds(device):
+    ends = torch.tensor([512, 1024, 1536, 2048], dtype=torch.int32, device=device)
+    sparse_map = SparseMap(None, ends, ends, None, 2048, None, 4, None)
+    x, y = torch.randn((2048, 64), device=device), torch.randn((2048, 128), device=device)
+    out = input_row_sparse_matmul(x.t(), y, sparse_map)
+    for expert in range(4):
+        rows = slice(512 * expert, 512 * (expert + 1))
+        assert torch.equal(out[64 * expert : 64 * (expert + 1)], dense_matmul(x[rows].t(), y[rows]))
 
 
 @pytest.mark.parametrize("tile", _COLUMNS)
 def test_values_that_bf16_parts_cannot_hold(tile, device):
     """Infinities, NaN, values that bf16 rounds to infinity and values whose parts lie below bf16: as by fp32 multiply-adds."""
-    inner = 48
+    inner = 272
     lhs, rhs = _operands(_COLUMNS[tile], inner, device, True)
     infinite, nan, largest = 3, 70, 130  # rows, in different blocks
     lhs[infinite, 5] = float("inf")
@@ -93,7 +118,7 @@ def test_values_that_bf16_parts_cannot_hold(tile, device):
     [(-112, 40), (-120, 60), (-126, 100), (100, -126), (-126, 120), (-112, 105), (60, 30), (-113, 0), (-124, 0), (0, -126), (-70, -70)],
 )
 def test_operands_of_all_magnitudes(tile, lhs_exponent, rhs_exponent, device):
-    inner = 48
+    inner = 272
     lhs, rhs = (x.sign() * (1 + x.abs() % 1) for x in _operands(_COLUMNS[tile], inner, device, True))
     lhs, rhs = lhs * 2.0**lhs_exponent, rhs * 2.0**rhs_exponent
     multiply_adds = max(lhs_exponent, rhs_exponent) >= 102 or lhs_exponent + rhs_exponent >= 72
@@ -105,7 +130,7 @@ def test_operands_of_all_magnitudes(tile, lhs_exponent, rhs_exponent, device):
 
 
 def test_subnormal_operands(device):
-    lhs, rhs = _operands(_COLUMNS["64x64"], 48, device, True)
+    lhs, rhs = _operands(_COLUMNS["64x64"], 272, device, True)
     lhs *= 2.0**-140
     out = dense_matmul(lhs, rhs * 2.0**100)
     assert out.abs().max() > 0
