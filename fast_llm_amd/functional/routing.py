@@ -19,6 +19,7 @@ from fast_llm_amd.functional.utils import is_traced
 # cache, and with 11 us less of the host's time. 64 tiles of 4096 14 us (torch 20), 188 of 1280 9 (13), 1000 of 512 11 (12); from twice as
 # much on torch's is ahead (1000 of 2048 22 and 17).
 _MAX_LOGIT_BYTES = 1_200_000
+_MAX_LOGIT_EXPERTS = 4096  # of fm_router_linear_forward
 
 
 def _few_logits(input_: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -27,6 +28,8 @@ def _few_logits(input_: torch.Tensor, weight: torch.Tensor) -> bool:
         input_.dim() == 2
         and weight.dim() == 2
         and input_.size(0) > 0
+        and input_.size(1) > 0
+        and 0 < weight.size(0) <= _MAX_LOGIT_EXPERTS
         and -(-input_.size(0) // 16) * -(-weight.size(0) // 16) * input_.size(1) * input_.element_size() <= _MAX_LOGIT_BYTES
         and input_.dtype == weight.dtype
         and input_.dtype in _lib.DTYPES

@@ -54,6 +54,16 @@ def test_what_the_kernel_does_not_take(device):
         assert routing.router_linear(x, weight).dtype == torch.bfloat16
 
 
+@pytest.mark.parametrize(("tokens", "experts", "hidden"), [(3, 4097, 8), (3, 0, 64), (3, 8, 0)])
+def test_sizes_that_the_kernel_refuses(tokens, experts, hidden, device):
+    x, weight = torch.randn((tokens, hidden), device=device), torch.randn((experts, hidden), device=device)
+    assert not routing._few_logits(x, weight)
+    assert torch.equal(routing.router_linear(x, weight), torch.nn.functional.linear(x, weight))
+    # Where tokens are few enough that only the number of experts decides.
+    if experts > 0 and hidden > 0:
+        assert routing._few_logits(x, weight[:4096])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("experts", [8, 32, 40, 64, 72, 128])
 @pytest.mark.parametrize(("tokens", "hidden"), [(1, 8), (15, 128), (17, 136), (64, 120), (257, 520), (300, 2056)])
