@@ -77,9 +77,21 @@ class _RouterLinear(torch.autograd.Function):
         return grad_input, grad_weight
 
 
+def _is_transformed(*tensors: torch.Tensor) -> bool:
+    """Whether something looks at torch's own operations and would not see the library's: the compiler, a `torch.func` transform
+    (whose tensors have no address), a dispatch mode (fake tensors, `make_fx`), a tensor subclass."""
+    return (
+        torch.compiler.is_compiling()
+        or torch._C._are_functorch_transforms_active()
+        or torch._C._len_torch_dispatch_stack() > 0
+        or any(type(tensor) not in (torch.Tensor, torch.nn.Parameter) for tensor in tensors)
+        or is_traced()
+    )
+
+
 def router_linear(input_: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """The router's linear layer, differentiable: `torch.nn.functional.linear(input_, weight)`, the same bits as `router_logits`."""
-    if torch.is_autocast_enabled("cuda") or is_traced() or not _few_logits(input_, weight):
+    if _is_transformed(input_, weight) or torch.is_autocast_enabled("cuda") or not _few_logits(input_, weight):
         return torch.nn.functional.linear(input_, weight)
     if torch.is_grad_enabled() and (input_.requires_grad or weight.requires_grad):
         return _RouterLinear.apply(input_, weight)

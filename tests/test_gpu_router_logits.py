@@ -2,6 +2,8 @@
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from fast_llm_amd import _lib
 from fast_llm_amd.functional import routing
@@ -62,6 +64,26 @@ def test_sizes_that_the_kernel_refuses(tokens, experts, hidden, device):
     # Where tokens are few enough that only the number of experts decides.
     if experts > 0 and hidden > 0:
         assert routing._few_logits(x, weight[:4096])
+
+
+def test_transforms_see_a_linear_layer(device):
+    x, weight = torch.randn((20, 64), device=device), torch.randn((8, 64), device=device)
+    assert routing._few_logits(x, weight)
+    expected = torch.nn.functional.linear(x, weight)
+
+    def loss(w):
+        return routing.router_linear(x, w).square().sum()
+
+    torch.testing.assert_close(torch.func.grad(loss)(weight), 2 * expected.t() @ x)
+    torch.testing.assert_close(torch.func.vmap(routing.router_linear, (0, None))(x.view(4, 5, 64), weight).view(20, 8), expected)
+    torch.testing.assert_close(torch.func.jvp(routing.router_linear, (x, weight), (x, weight))[1], 2 * expected)
+    graph = make_fx(routing.router_linear)(x, weight)
+    torch.testing.assert_close(graph(x + 1, weight), torch.nn.functional.linear(x + 1, weight))
+    with FakeTensorMode():
+        fake = routing.router_linear(torch.empty((20, 64), device=device), torch.empty((8, 64), device=device))
+    assert fake.shape == (20, 8)
+    compiled = torch.compile(routing.router_linear, backend="eager", fullgraph=True)
+    torch.testing.assert_close(compiled(x, weight), expected)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
