@@ -309,6 +309,11 @@ static int launch(GemmArgs args, hipStream_t stream) {
 //       193 .. 256     0.98, 1.09 (0.96), 1.16 (1.00)
 //       257 .. 320     0.95, 1.08 (0.71), 1.13 (0.73): two rounds where 256 x 256 tiles take one
 //       more           0.90, 0.98 (0.66), 1.02 (0.74)
+// The line between 64 and 128 columns, over 1200 products more, activations not in cache either:
+//       65 .. 80       1.36, 1.19, 1.11
+//       81 .. 96       1.34, 1.28, 1.16
+//       97 .. 112      1.18, 1.20, 1.11
+//       113 .. 160     1.16, 1.18, 1.13
 // Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87), 1.03 (0.63), 0.88 (0.52) up to 96, and no better
 // with more: they stay there.
 bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
@@ -321,7 +326,7 @@ bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
 template <typename T>
 static int launch_few_tiles(const GemmArgs &args, hipStream_t stream) {
     const int64_t tiles = few_tiles::most_tiles(args);
-    return tiles <= 80    ? few_tiles::launch<T, 64>(args, stream)
+    return tiles <= 96    ? few_tiles::launch<T, 64>(args, stream)
            : tiles <= 160 ? few_tiles::launch<T, 128>(args, stream)
                           : few_tiles::launch<T, 256>(args, stream);
 }
