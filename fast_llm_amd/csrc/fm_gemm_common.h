@@ -49,7 +49,6 @@ struct GemmArgs {
                            // everything (0: everything)
     int planned;           // `tile_table` (and `partials`) have been set up by mfma_gemm_plan
     int chunk_tiles;       // consecutive tiles that go to one XCD (set by the launchers of the fp32, few-row and few-tile kernels)
-    int64_t tokens;        // rows of all experts together without padding, if the caller knows (0: it does not); a choice of kernel only
 };
 
 #define FM_LDS(T) __attribute__((address_space(3))) T

@@ -617,6 +617,10 @@ static int64_t short_gradient_reduction(int64_t tiles) {
     return tiles >= kLargeGradients ? 64 : tiles >= kMiddleGradients ? 128 : tiles >= 256 ? 512 : tiles >= 64 ? 2048 : 4096;
 }
 
+// Rows per expert that a map's buffer has on top of the tokens': 128 of a static shape, 64 on average of a dynamic one. From the buffer
+// alone, whoever calls: the layer's products and those of its parts then sum in the same order.
+constexpr int64_t kPadding = 112;
+
 int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
     // Upper bounds of the numbers of tiles (the surplus ids have none).
     const auto count = [&](int tile_m, int tile_n) {
@@ -630,8 +634,7 @@ int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
     const bool mapped = args.expert_ends != nullptr;
     if (args.mode == kInputRowSparse) {
         int64_t reduction = args.piece_length > 0 ? args.piece_length : args.inner;
-        // A map's buffer has a tile of 128 rows of padding per expert.
-        if (mapped) reduction = args.tokens > 0 ? args.tokens / args.num_experts : args.inner / args.num_experts - 128;
+        if (mapped) reduction = args.inner / args.num_experts - kPadding;
         const int64_t tiles = count(64, 64);
         if (args.sparse_size >= 64 && args.cols >= 64 && reduction >= short_gradient_reduction(tiles)) {
             if (tiles < kMiddleGradients) return launch_f32_split<64, 64, 2>(args, tiles, stream);
@@ -641,10 +644,7 @@ int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
             return launch_f32_split<128, 128, 3>(args, large, stream);
         }
     } else {
-        // Half of that padding is computed where the caller does not say where it begins.
-        const int64_t padding = args.expert_pad_begins != nullptr ? 128 : 64;
-        int64_t rows = args.rows;
-        if (mapped) rows = max(args.tokens > 0 ? args.tokens / args.num_experts : args.rows / args.num_experts - padding, int64_t(1));
+        const int64_t rows = mapped ? max(args.rows / args.num_experts - kPadding, int64_t(1)) : args.rows;
         const int64_t tiles_n = (args.cols + 63) / 64, tiles = mapped ? args.num_experts * (rows + 32) / 64 * tiles_n : (rows + 63) / 64 * tiles_n;
         if (args.inner >= short_reduction(tiles, min(rows, args.cols) <= 32)) {
             const int64_t small = count(64, 64);

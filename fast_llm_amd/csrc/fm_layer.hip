@@ -78,28 +78,24 @@ struct Step {
         return fm_copy_sparse_to_dense(in, scores, routing(plan.sparse_rows), out, layer.tokens, layer.hidden, plan.slots, plan.rows,
                                        dtype(), FM_DTYPE_F32, plan.index_dtype, stream);
     }
-    GemmArgs with_tokens(GemmArgs args) const {
-        args.tokens = layer.tokens * plan.slots;
-        return args;
-    }
     // The products compute the rows that tokens own: what the padding rows of an intermediate hold is nobody's.
     // out [rows, columns] = lhs [rows, inner] x (weight_e [columns, inner])^T
     GemmArgs output_sparse(const void *lhs, const void *weight, void *out, int64_t columns, int64_t inner) const {
-        return with_tokens(GemmArgs{lhs, weight, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), inner, 1, 1, inner, columns, 1,
-                        plan.rows, columns, inner, columns, static_cast<int>(plan.experts), kOutputSparse, 0, plan.index_dtype, dtype()});
+        return GemmArgs{lhs, weight, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), inner, 1, 1, inner, columns, 1,
+                        plan.rows, columns, inner, columns, static_cast<int>(plan.experts), kOutputSparse, 0, plan.index_dtype, dtype()};
     }
     // out [rows, hidden] = lhs [rows, inner] x weight_e [inner, hidden]
     GemmArgs inner_sparse(const void *lhs, const void *weight, void *out, int64_t inner) const {
         const int64_t hidden = layer.hidden;
-        return with_tokens(GemmArgs{lhs, weight, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), inner, 1, hidden, 1, hidden, 1,
-                        plan.rows, hidden, inner, inner, static_cast<int>(plan.experts), kInputInnerSparse, 0, plan.index_dtype, dtype()});
+        return GemmArgs{lhs, weight, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), inner, 1, hidden, 1, hidden, 1,
+                        plan.rows, hidden, inner, inner, static_cast<int>(plan.experts), kInputInnerSparse, 0, plan.index_dtype, dtype()};
     }
     // out [experts * size, hidden] (+)= lhs^T x rhs, lhs [rows, size], rhs [rows, hidden]
     GemmArgs row_sparse(const void *lhs, const void *rhs, void *out, int64_t size, bool accumulate) const {
         const int64_t hidden = layer.hidden;
-        return with_tokens(GemmArgs{lhs, rhs, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), 1, size, hidden, 1, hidden, 1,
+        return GemmArgs{lhs, rhs, out, routing(plan.expert_ends), routing(plan.expert_pad_begins), 1, size, hidden, 1, hidden, 1,
                         size * plan.experts, hidden, plan.rows, size, static_cast<int>(plan.experts), kInputRowSparse, accumulate,
-                        plan.index_dtype, static_cast<int>(layer.grad_dtype)});
+                        plan.index_dtype, static_cast<int>(layer.grad_dtype)};
     }
     GemmArgs layer_1() const {
         GemmArgs args = output_sparse(layer.sparse_input, layer.weight_1, layer.layer_1_output, ffn_1(), layer.hidden);
