@@ -82,6 +82,7 @@ constexpr int kTile = 256;
 constexpr int kWavesM = 2, kWavesN = 2;  // wavefront grid over the tile
 constexpr int kWaves = kWavesM * kWavesN, kMfmaThreads = 64 * kWaves;
 constexpr int kBK = 64;      // K elements per slice (32 or 64)
+static_assert(kBK == kRotationSlice, "first_slice_of counts slices of this kernel");
 constexpr int kStages = 2;     // LDS slots of the rhs operand
 constexpr int kLhsStages = 3;  // LDS slots of the lhs operand
 constexpr int kOperandBytes = kTile * kBK * 2;  // one operand slice in LDS, same size in either layout

@@ -3,6 +3,8 @@
 import pytest
 import torch
 
+from fast_llm_amd.functional.config import ActivationType
+from fast_llm_amd.functional.mlp import gated_layer_1_forward, gated_layer_2_input_backward, mlp_activation_backward
 from fast_llm_amd.functional.sparse_linear import output_sparse_matmul
 from oracle import moe_oracle
 from tests.helpers import fixture_sparse_map, to_device_map
@@ -12,23 +14,53 @@ pytestmark = pytest.mark.gpu
 _TOKENS = [1, 0, 128, 129, 300, 7, 256, 0, 257, 64, 5]
 
 
-@pytest.mark.parametrize("slices", [1, 2, 3, 5, 12, 33])
-@pytest.mark.parametrize("columns", [8, 264, 520])
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_every_slice_counts_once(slices, columns, dtype, device):
-    inner, experts = 64 * slices, len(_TOKENS)
+def _map():
     ends, used = [], 0
     for tokens in _TOKENS:
         used += -(-tokens // 128) * 128
         ends.append(used)
-    oracle_map = fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": _TOKENS})
-    real = oracle_map.real_row_mask()
+    return fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": _TOKENS})
+
+
+def _operands(oracle_map, columns, slices, dtype):
+    """Whole numbers, NaN in the padding rows, and the product, rounded to `dtype`."""
     generator = torch.Generator().manual_seed(slices + columns)
-    x = torch.randint(-1, 2, (used, inner), generator=generator).to(dtype)
-    weight = torch.randint(-1, 2, (experts * columns, inner), generator=generator).to(dtype)
+    x = torch.randint(-1, 2, (oracle_map.num_rows, 64 * slices), generator=generator).to(dtype)
+    weight = torch.randint(-1, 2, (len(_TOKENS) * columns, 64 * slices), generator=generator).to(dtype)
     # One more weight per slice that nothing but its own slice can make up for.
     weight[:, ::64] *= 3
     expected = moe_oracle.output_sparse_matmul(x.float(), weight.float().t(), oracle_map).to(dtype)
-    x[~real] = float("nan")
+    x[~oracle_map.real_row_mask()] = float("nan")
+    return x, weight, expected
+
+
+# The 15 row tiles of 128 make launches of few tiles up to 4352 columns, and of 256 x 256 ones with 4616.
+@pytest.mark.parametrize("slices", [1, 2, 3, 5, 12, 33])
+@pytest.mark.parametrize("columns", [8, 264, 520, 4616])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_slice_counts_once(slices, columns, dtype, device):
+    oracle_map = _map()
+    real = oracle_map.real_row_mask()
+    x, weight, expected = _operands(oracle_map, columns, slices, dtype)
     out = output_sparse_matmul(x.to(device), weight.to(device).t(), to_device_map(oracle_map, device, torch.int32))
     assert torch.equal(out.cpu()[real], expected[real])
+
+
+@pytest.mark.parametrize("slices", [1, 2, 3, 5, 12, 33])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_slice_counts_once_in_the_fused_products(slices, dtype, device):
+    ffn, oracle_map = 256, _map()
+    real, sparse_map = oracle_map.real_row_mask(), to_device_map(oracle_map, device, torch.int32)
+    x, weight, expected = _operands(oracle_map, 2 * ffn, slices, dtype)
+    layer_1, output = gated_layer_1_forward(x.to(device), weight.to(device), sparse_map, ActivationType.identity, True)
+    assert torch.equal(layer_1.cpu()[real], expected[real])
+    gate, up = expected[real].float().chunk(2, 1)
+    assert torch.equal(output.cpu()[real], (gate * up).to(dtype))
+
+    grad, weight, expected = _operands(oracle_map, ffn, slices, dtype)
+    layer_1 = torch.randint(-3, 4, (oracle_map.num_rows, 2 * ffn)).to(device, dtype)
+    grad_layer_1, _ = gated_layer_2_input_backward(
+        grad.to(device), weight.to(device).t(), sparse_map, layer_1, ActivationType.identity, False
+    )
+    in_two, _ = mlp_activation_backward(expected.to(device), (layer_1, True, ActivationType.identity, sparse_map))
+    assert torch.equal(grad_layer_1.cpu()[real], in_two.cpu()[real])
