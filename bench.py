@@ -35,7 +35,8 @@ import time
 import torch
 
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA peak, TFLOP/s
-PEAK_FP32_TFLOPS = 157.3  # MI355X fp32 (matrix) peak, TFLOP/s
+# fp32 products: six bf16 products of operand parts each, the faster of the two ways they are computed (multiply-adds: 157.3).
+PEAK_FP32_TFLOPS = PEAK_BF16_TFLOPS / 6
 PEAK_HBM_GBS = 8000.0  # MI355X HBM3E peak, GB/s
 ROOT = pathlib.Path(__file__).resolve().parent
 PROFILES = ROOT / "profiles"

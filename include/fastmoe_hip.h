@@ -248,7 +248,13 @@ int fm_mlp_activation_backward(const void *grad_output, void *grad_input, const 
  * ordinary dense one (a single expert owning all rows), which is what the reference does for
  * `sparse_map=None` (sparse_linear.py:276-277, 404-405, 537-538).
  * Results are deterministic (no floating-point atomics; every sum has a fixed order that depends only on the
- * arguments and the expert map).
+ * arguments and the expert map). That order is not the same everywhere: kernel and tile follow from the dimensions
+ * (`row_dim`, the rows of the buffer, among them), and in half precision with both operands contiguous along the
+ * reduction axis, in buffers of up to 1024 rows per expert, every expert's sums start at a place of the axis of their
+ * own. The same rows and weights as another expert's, or in a buffer of another size, give the same result but for
+ * the rounding of its sums.
+ * fp32 operands may be multiplied as sums of three bf16 parts each, every one of their 24 bits among them; sums are in
+ * fp32, and no further from the exact result than those of fp32 multiply-adds.
  *
  * `workspace`: device scratch (64-byte aligned, content irrelevant) of `fm_grouped_gemm_workspace_size(...)` bytes
  * (`fm_input_row_sparse_matmul_workspace_size(...)` for the row-sparse product). With it, a small kernel first writes
@@ -347,6 +353,7 @@ int fm_output_sparse_matmul_gated_activation_backward(const void *lhs, const voi
  * hidden], all contiguous and 16-byte aligned, of `dtype` (bf16 or fp16); top_experts [num_tokens, slots_per_token] int64,
  * scores fp32. Entries of top_experts outside [0, num_experts) contribute nothing. Layer 1's output is rounded to `dtype`
  * before the activation and the activation's before layer 2, as in the separate kernels; layer 2's is not rounded.
+ * Deterministic; with hidden up to 2048 the order of layer 1's sums depends on where a weight row lies.
  * `workspace`: fm_few_tokens_workspace_size(...) bytes, 16-byte aligned; that function returns 0 for what these kernels do
  * not take (other dtypes, hidden or ffn not multiples of 8, more than 4096 (token, slot) pairs, an expert's weight of 4
  * GiB or more), which FM_ERR_UNSUPPORTED then reports. */
@@ -359,7 +366,7 @@ int fm_few_tokens_forward(const void *input, const void *top_experts, const void
 
 /* The router's linear layer, logits [num_tokens, num_experts] = input [num_tokens, hidden] x weight [num_experts, hidden]^T, for few
  * tokens: meant for up to 1.2 MB of row bytes x tiles of 16 tokens x 16 experts, correct for any number. All contiguous, of `dtype`, sums in fp32;
- * input and weight 16-byte aligned and hidden a multiple of 16 bytes (FM_ERR_UNSUPPORTED). Deterministic. */
+ * input and weight 16-byte aligned and hidden a multiple of 16 bytes (FM_ERR_UNSUPPORTED), up to 4096 experts. Deterministic. */
 int fm_router_linear_forward(const void *input, const void *weight, void *logits, int64_t num_tokens, int64_t num_experts,
                              int64_t hidden, int dtype, void *stream);
 
