@@ -80,11 +80,15 @@ __device__ __forceinline__ const char *uniform_pointer(const char *pointer) {
 // faster for it, and neither is a launch that is bound by its MFMAs (kFewRows). Layer 1 (and layer 2's input gradient), us: 44 rows for each of
 // 128 experts of 2048 x 768 218 -> 168 (125 -> 111), 94 for each of 64 of 2048 x 1408 200 -> 158 (106 -> 99), 125 of the 128 228 -> 218 and
 // 218 -> 186 (120 -> 119), 469 of the 64 361 -> 348 (210 -> 210); 1024 of the 128 783 -> 789 (409 -> 409) without the bound.
+// Where a tile starts and how far its operands reach is counted in 32 bits (fm_gemm_mfma.hip): axes are below kMaxRotatedAxis, as all
+// are whose rows do not overlap (their strides are).
 constexpr int kRotationSlice = 64, kFewRows = 1024;
+constexpr int64_t kMaxRotatedAxis = int64_t(1) << 21;
 
 __host__ __device__ inline bool starts_anywhere(const GemmArgs &args) {
     return args.mode != kInputRowSparse && args.num_experts > 1 && args.rows <= static_cast<int64_t>(kFewRows) * args.num_experts &&
-           args.lhs_stride_inner == 1 && args.rhs_stride_inner == 1 && args.inner % kRotationSlice == 0;
+           args.lhs_stride_inner == 1 && args.rhs_stride_inner == 1 && args.inner % kRotationSlice == 0 &&
+           args.inner < kMaxRotatedAxis;
 }
 
 __device__ __forceinline__ int first_slice_of(const GemmArgs &args, int expert) {

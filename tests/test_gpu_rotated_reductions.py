@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from fast_llm_amd import _lib
 from fast_llm_amd.functional.config import ActivationType
 from fast_llm_amd.functional.mlp import gated_layer_1_forward, gated_layer_2_input_backward, mlp_activation_backward
 from fast_llm_amd.functional.sparse_linear import output_sparse_matmul
@@ -64,3 +65,20 @@ def test_every_slice_counts_once_in_the_fused_products(slices, dtype, device):
     )
     in_two, _ = mlp_activation_backward(expected.to(device), (layer_1, True, ActivationType.identity, sparse_map))
     assert torch.equal(grad_layer_1.cpu()[real], in_two.cpu()[real])
+
+
+def test_axes_of_rows_that_overlap_start_at_their_beginning(library, device):
+    """One row for all of them, of 2^21: an offset along a longer one would not fit its 32 bits. The exact sums are 0, the rounded ones
+    tell in which order they were made."""
+    inner, rows, columns = 2**21, 256, 8
+    half = torch.randn((2, inner // 2), device=device).bfloat16()
+    x, weight = torch.cat([half[0], -half[0]]), torch.cat([half[1], half[1]])
+    ends = torch.tensor([128, 256], dtype=torch.int32, device=device)
+    out = torch.empty((rows, columns), dtype=torch.bfloat16, device=device)
+    _lib.check(
+        library.fm_output_sparse_matmul(
+            x.data_ptr(), weight.data_ptr(), out.data_ptr(), ends.data_ptr(), rows, columns, inner, 2, 0, 1, 1, 0, columns, 1, 0,
+            _lib.dtype_tag(out.dtype), _lib.dtype_tag(out.dtype), 1, None, 0, torch.cuda.current_stream(device).cuda_stream,
+        )
+    )  # fmt: skip
+    assert (out == out[0, 0]).all()
