@@ -66,7 +66,8 @@ def router_logits(input_: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 class _RouterLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, input_: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-        ctx.save_for_backward(input_, weight)
+        # No more than the linear layer keeps: what no gradient needs may be written to before the backward.
+        ctx.save_for_backward(input_ if ctx.needs_input_grad[1] else None, weight if ctx.needs_input_grad[0] else None)
         return router_logits(input_, weight)
 
     @staticmethod

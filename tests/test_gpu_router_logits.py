@@ -45,6 +45,25 @@ def test_gradients_are_those_of_linear(dtype, device):
         assert torch.equal(routing.router_linear(x, weight), routing.router_logits(x, weight))
 
 
+@pytest.mark.parametrize("trained", ["input", "weight"])
+def test_what_no_gradient_needs_may_change(trained, device):
+    """As after torch's linear layer: the operand that no gradient is made from is neither kept nor watched."""
+    x, weight = torch.randn((20, 64), device=device), torch.randn((8, 64), device=device)
+    (x if trained == "input" else weight).requires_grad_()
+    results = []
+    for function in (routing.router_linear, torch.nn.functional.linear):
+        x.grad = weight.grad = None
+        x_, weight_ = (x * 1, weight) if trained == "input" else (x, weight * 1)
+        kept = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda tensor: kept.append(tensor.data_ptr()) or tensor, lambda tensor: tensor):
+            logits = function(x_, weight_)
+        with torch.no_grad():
+            (x_ if trained == "input" else weight_).add_(1)
+        logits.sum().backward()
+        results.append((x.grad if trained == "input" else weight.grad, len(kept)))
+    assert torch.equal(results[0][0], results[1][0]) and results[0][1] == results[1][1] == 1
+
+
 def test_what_the_kernel_does_not_take(device):
     x, weight = torch.randn((30, 68), device=device), torch.randn((8, 68), device=device)
     for operands in ((x[:, :66], weight[:, :66]), (x.t().contiguous().t(), weight), (x[:0], weight), (x[1:, 1:], weight[:, 1:])):
