@@ -9,6 +9,7 @@ does this with `torch.topk` and `torch.softmax(dtype=torch.float32)` and lets au
 import dataclasses
 
 import torch
+from torch.utils._device import DeviceContext
 
 from fast_llm_amd import _lib
 from fast_llm_amd.functional.utils import is_traced
@@ -78,14 +79,22 @@ class _RouterLinear(torch.autograd.Function):
         return grad_input, grad_weight
 
 
-def _is_transformed(*tensors: torch.Tensor) -> bool:
+def _has_function_mode() -> bool:
+    stack = range(torch._C._len_torch_function_stack())
+    return any(type(torch._C._get_function_stack_at(level)) is not DeviceContext for level in stack)
+
+
+def _is_transformed(input_: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether something looks at torch's own operations and would not see the library's: the compiler, a `torch.func` transform
-    (whose tensors have no address), a dispatch mode (fake tensors, `make_fx`), a tensor subclass."""
+    (whose tensors have no address), a dispatch mode (fake tensors, `make_fx`), a function mode (but for the default device's), a
+    tensor subclass."""
     return (
         torch.compiler.is_compiling()
         or torch._C._are_functorch_transforms_active()
         or torch._C._len_torch_dispatch_stack() > 0
-        or any(type(tensor) not in (torch.Tensor, torch.nn.Parameter) for tensor in tensors)
+        or (torch._C._len_torch_function_stack() > 0 and _has_function_mode())
+        or type(input_) not in (torch.Tensor, torch.nn.Parameter)
+        or type(weight) not in (torch.Tensor, torch.nn.Parameter)
         or is_traced()
     )
 

@@ -4,6 +4,7 @@ import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
 
 from fast_llm_amd import _lib
 from fast_llm_amd.functional import routing
@@ -103,6 +104,25 @@ def test_transforms_see_a_linear_layer(device):
     assert fake.shape == (20, 8)
     compiled = torch.compile(routing.router_linear, backend="eager", fullgraph=True)
     torch.testing.assert_close(compiled(x, weight), expected)
+
+
+class _Calls(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.functions = []
+
+    def __torch_function__(self, function, types, args=(), kwargs=None):
+        self.functions.append(function)
+        return function(*args, **(kwargs or {}))
+
+
+def test_function_modes_see_a_linear_layer(device):
+    x, weight = torch.randn((20, 64), device=device), torch.randn((8, 64), device=device)
+    with _Calls() as mode:
+        logits = routing.router_linear(x, weight)
+    assert torch.nn.functional.linear in mode.functions and torch.equal(logits, torch.nn.functional.linear(x, weight))
+    with torch.device(device):  # the mode of a default device looks for functions that make tensors
+        assert torch.equal(routing.router_linear(x, weight), routing.router_logits(x, weight))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
