@@ -1,7 +1,7 @@
 // Grouped matrix products of fp32 operands on the gfx950 matrix cores, by one of two instructions:
 //   * v_mfma_f32_32x32x16_bf16 on operands split into three bf16 parts each (`grouped_gemm_f32_split_kernel`, below): six
 //     products of parts instead of one of values at 16 times the rate of fp32 multiply-adds;
-//   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for short reductions and few tiles (see `f32_gemm_launch`).
+//   * v_mfma_f32_32x32x2_f32 (`grouped_gemm_f32_kernel`), for short reductions and few tiles (see `forward_tile`).
 // Forward and backward products of 4096 rows over 8 experts, 1024 x 2816 (5632): 1864 us for the six on fp32 multiply-adds, 1345 on
 // split operands.
 //   * Operand slices (kBK reduction indices) go straight from global memory into LDS (`buffer_load ... lds`, 16 bytes
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kThreads, 8) void grouped_gemm_f32_kernel(GemmArgs 
 //   128 x 128: 2 x 2 of the tile, slices of 16;
 //   128 x 64: 2 of the tile x 2 halves of a slice of 32;
 //   64 x 64: 4 quarters of a slice of 64
-// (halves and quarters add up in LDS), by how many tiles there are: see `f32_gemm_launch`.
+// (halves and quarters add up in LDS), by how many tiles there are: see `forward_tile` and `gradient_tile`.
 
 constexpr float kOperandScale = 0x1p24f, kResultScale = 0x1p-48f;
 
@@ -592,38 +592,65 @@ static int launch_f32_tile(GemmArgs args, int64_t tiles, hipStream_t stream) {
 }
 
 // Which kernel and tile, by the 64 x 64 tiles that the rows are expected to fill (half a tile per expert of a map is not; a buffer's own
-// rows are mostly padding where experts have few). Reductions shorter than short_reduction are start and epilogue, and what few tiles
-// there are runs on more CUs as tiles of 32 x 32: there eight workgroups of fp32 multiply-adds per CU are faster. Time on split
-// operands over that on multiply-adds, geometric means over 2300 products of 4 to 16 experts of 8 to 512 rows, operands not in L2:
-//     tiles       reduction 128   256   384   512  1024  2816
-//     65 .. 160            1.38  1.20  1.07  1.00  0.89  0.80
-//     257 .. 400           1.14  1.06  1.01  1.02  0.93  0.88
-//     401 .. 600           1.09  1.05  0.99  0.94  0.86  0.77
-//     1001 .. 1500         1.09  0.97  0.91  0.86  0.79  0.75
-//     from 2501 on         0.95  0.86  0.82  0.80  0.75  0.71
-// A side of up to 32 leaves half of every split tile empty: 16384 x 32 of 256 7 us against 10, of 2816 66 against 51. By the rule these
-// products take 0.894 of the time of multiply-adds (worst 1.22; the best choice for each 0.871), dense ones of 8 to 65536 rows 0.946
-// (0.893). All large launches on split operands took 0.951 and 1.095, worst 2.4 (8192 x 2048 of 8 18 -> 31 us).
-// Tiles of 64 x 64 / 128 x 64 / 128 x 128, us: 8 experts of 512, 1024 columns of 2816 (1088 tiles) 181 / 194 / 228; 2816 of 1024 (2992) 161 /
-// 157 / 158; 5632 of 1024 (5984) 333 / 300 / 298. Experts of up to 48 rows fill no 128: 16 of 48, 5632 columns of 1024 115 / 154 / 147.
-// fp32 tiles of 64 x 64 by the upper bound of them: 1056 36 (32 x 32: 34), 1120 24 (26), 1408 295 (265), 2048 23 (29), 3872 238 (254); of
-// experts of up to 32 rows not where the reduction is long: 16 of 8, 2816 columns of 2816 195 (106).
-constexpr int64_t kF32LargeTiles = 1536, kMiddleTiles = 1200, kLargeTiles = 2816;
-static int64_t short_reduction(int64_t tiles, bool narrow) {
-    const int64_t most = tiles < 64 ? 1024 : tiles < 400 ? 512 : tiles < 700 ? 384 : tiles < 1536 ? 256 : tiles < 2500 ? 192 : 128;
-    return narrow ? max(most, int64_t(768)) : most;
+// rows are mostly padding where experts have few). Short reductions are start and epilogue, and what few tiles there are runs on more CUs
+// as tiles of 32 x 32: there eight workgroups of fp32 multiply-adds per CU are faster. Time over that on multiply-adds, operands not in
+// L2, geometric means over 8500 grouped products of 2 to 128 experts of 1 to 800 rows, equally and unequally liked, 64 x 64 / 128 x 64 / 128 x
+// 128 on split operands; first line of a pair: experts of up to 32 rows, second: of more.
+//     tiles          reduction 96 .. 127   192 .. 255          384 .. 511          768 .. 1023         from 2048 on
+//     up to 255      1.24 1.38 1.58    1.16 1.31 1.59    1.01 1.16 1.51    0.92 1.08 1.56    0.82 0.98 1.54
+//                    1.27 1.46 1.66    1.18 1.35 1.65    1.06 1.26 1.69    0.94 1.14 1.69    0.85 1.06 1.72
+//     256 .. 511     1.15 1.03 0.92    1.00 0.91 0.84    0.85 0.80 0.80    0.78 0.74 0.71    0.68 0.67 0.68
+//                    1.06 1.01 1.04    1.02 0.95 1.02    0.86 0.84 0.93    0.77 0.78 0.95    0.71 0.72 0.92
+//     512 .. 1023    1.32 1.11 0.95    1.14 0.97 0.86    0.94 0.82 0.78    0.77 0.71 0.73    0.66 0.68 0.73
+//                    1.11 0.97 0.89    1.02 0.92 0.86    0.86 0.79 0.82    0.79 0.75 0.78    0.70 0.71 0.73
+//     1024 .. 2499   1.37 1.10 0.91    1.13 0.91 0.78    0.86 0.73 0.72    0.75 0.68 0.68
+//                    1.32 1.11 0.97    1.13 0.95 0.86    0.94 0.81 0.81    0.80 0.74 0.76    0.68 0.69 0.71
+//     more           1.56 1.16 0.88    1.22 0.93 0.75
+//                    1.48 1.12 0.89    1.19 0.91 0.76    0.93 0.77 0.72    0.79 0.71 0.68
+// Experts of few rows (64 by the estimate) are weights read from memory: large tiles, which start over less often, are ahead early. In a
+// layer, whose activations are in cache, long reductions and more rows are better off on small ones, and their lines are drawn for that
+// (us on 64 x 64 / 128 x 64 / 128 x 128: 16 experts of 37 rows, 1024 columns of 2816 (336 tiles) 53 / 79, of 48 rows, 5632 of 1024 115 / 154 /
+// 147; 8 of 37, 2496 of 960 26 / 44; 8 of 266, 2048 of 512 (1184) 45 / - / 51; 8 of 512, 1024 of 2816 (1088) 181 / 194 / 228, 2816 of 1024 (2992)
+// 161 / 157 / 158, 5632 of 1024 (5984) 333 / 300 / 298).
+// A side of up to 32 leaves half of every split tile empty, up to 16 columns three quarters: 16384 x 32 of 256 7 us on multiply-adds
+// against 10, of 2816 66 against 51; 39467 x 8 of 1328 80 against 92. By the rule the grouped products take 0.945 of the time of
+// multiply-adds (worst 1.18; the best choice for each 0.913), 3000 dense ones of 1 to 65536 rows 0.95 (0.93).
+constexpr int64_t kF32LargeTiles = 1536;  // of fp32 multiply-adds, by their upper bound: 1056 36 (32 x 32: 34), 1120 24 (26), 1408 295
+                                          // (265), 2048 23 (29), 3872 238 (254)
+enum class F32Tile { kMultiplyAdds, k64x64, k128x64, k128x128 };
+
+static F32Tile forward_tile(int64_t rows, int64_t cols, int64_t reduction, int64_t tiles, bool mapped) {
+    if (cols <= 16) return F32Tile::kMultiplyAdds;
+    if (mapped && rows <= 64 && cols > 32) {
+        const int64_t shortest = tiles < 64 ? 1024 : tiles < 256 ? 768 : tiles < 1024 ? 256 : tiles < 2500 ? 128 : 96;
+        if (reduction < shortest) return F32Tile::kMultiplyAdds;
+        if (tiles < 2500 && reduction >= 768) return F32Tile::k64x64;
+        return tiles < 1024 ? F32Tile::k128x64 : F32Tile::k128x128;
+    }
+    const int64_t shortest = tiles < 64 ? 1024 : tiles < 400 ? 512 : tiles < 700 ? 384 : tiles < 1536 ? 256 : tiles < 2500 ? 192 : 128;
+    const bool narrow = cols <= 32 || (!mapped && rows <= 32);
+    if (reduction < (narrow ? max(shortest, int64_t(768)) : shortest)) return F32Tile::kMultiplyAdds;
+    return tiles < 1200 ? F32Tile::k64x64 : tiles < 2816 ? F32Tile::k128x64 : F32Tile::k128x128;
 }
-// Weight gradients, time over that on multiply-adds again, 64 x 64 / 128 x 64 / 128 x 128:
-//     tiles     reduction 48              128              512              1024             4096
-//     32        1.78 / 2.11 / 2.44  1.60 / 1.97 / 2.60  1.27 / 1.90 / 3.01  1.03 / 1.59 / 2.69  0.76 / 1.28 / 2.37
-//     256       1.18 / 1.34 / 1.56  1.09 / 1.26 / 1.61  0.90 / 1.18 / 1.74  0.82 / 1.17 / 1.83  0.71 / 1.06 / 1.84
-//     512       1.02 / 1.01 / 1.12  1.00 / 0.94 / 1.14  0.92 / 0.82 / 1.16  0.76 / 0.78 / 1.14  0.71 / 0.76 / 1.11
-//     1024      1.11 / 0.85 / 0.81  1.02 / 0.94 / 0.81  0.83 / 0.74 / 0.76  0.73 / 0.71 / 0.73  0.68 / 0.67 / 0.67
-//     5632      1.77 / 1.31 / 1.04  1.44 / 1.07 / 0.92  0.92 / 0.83 / 0.77  0.84 / 0.78 / 0.76  0.79 / 0.76 / 0.76
-// With the operands in cache, as after the product before, few tiles gain later: 128 tiles of 2048 29 / 33 us.
-constexpr int64_t kMiddleGradients = 512, kLargeGradients = 1024;
-static int64_t short_gradient_reduction(int64_t tiles) {
-    return tiles >= kLargeGradients ? 64 : tiles >= kMiddleGradients ? 128 : tiles >= 256 ? 512 : tiles >= 64 ? 2048 : 4096;
+
+// Weight gradients, the same over 8100 products of 4 to 3000 rows per expert, those where no edge leaves a large tile empty:
+//     tiles          reduction 65 .. 128   129 .. 256          257 .. 512          513 .. 1024         2049 .. 4096
+//     64 .. 255      1.20 1.37 1.59    1.10 1.31 1.59    0.98 1.23 1.69    0.86 1.12 1.74    0.78 1.07 1.89
+//     256 .. 511     1.11 1.10 1.26    1.04 1.06 1.31    0.92 0.96 1.28    0.86 0.89 1.32    0.76 0.81 1.31
+//     512 .. 1023    1.16 1.08 0.98    1.07 1.00 0.98    0.95 0.93 1.01    0.85 0.84 0.92    0.75 0.77 0.86
+//     1024 .. 2499   1.22 1.08 0.95    1.04 0.94 0.89    0.90 0.86 0.89    0.77 0.75 0.80    0.69 0.72 0.84
+//     more           1.53 1.18 0.93    1.19 0.97 0.81    0.92 0.80 0.75    0.78 0.73 0.72    0.66 0.68 0.74
+// With the operands in cache, as after the product before, few tiles gain later (128 tiles of 2048 29 us on multiply-adds, 33 so) and large ones
+// are ahead earlier (2048 tiles of 266 34 us on 128 x 128, 41 on 128 x 64). Large tiles whose area is a tenth (128 x 64) or a quarter (128 x
+// 128) more than that of the 64 x 64 ones waste it: 64 experts, 64 x 3440, 47 rows 42 -> 51 us, 144 x 360, 186 rows 34 -> 39. By the rule
+// 0.972 of the time of multiply-adds; 35 of the 8100 are slower than those by more than a tenth (worst 1.45), all but a few with one expert
+// that has several times the rows of the others: a long reduction on few tiles.
+static F32Tile gradient_tile(int64_t reduction, int64_t tiles, int64_t tiles_128x64, int64_t tiles_128x128) {
+    const int64_t area = 4 * 100 * tiles_128x128 / tiles;  // percent of that of the 64 x 64 tiles
+    const int64_t shortest = tiles < 64 ? 4096 : tiles < 256 ? 2048 : tiles < 512 ? 512 : tiles < 1024 ? 256 : area < 115 ? 96 : 192;
+    if (reduction < shortest) return F32Tile::kMultiplyAdds;
+    if (tiles >= 1024 && area < 125) return F32Tile::k128x128;
+    return tiles >= 512 && 2 * 10 * tiles_128x64 < 11 * tiles ? F32Tile::k128x64 : F32Tile::k64x64;
 }
 
 // Rows per expert that a map's buffer has on top of the tokens': 128 of a static shape, 64 on average of a dynamic one. From the buffer
@@ -641,32 +668,29 @@ int f32_gemm_launch(GemmArgs args, hipStream_t stream) {
         return static_cast<int64_t>(args.tiles_m) * args.tiles_n;
     };
     const bool mapped = args.expert_ends != nullptr;
+    F32Tile tile = F32Tile::kMultiplyAdds;
     if (args.mode == kInputRowSparse) {
-        int64_t reduction = args.piece_length > 0 ? args.piece_length : args.inner;
-        if (mapped) reduction = args.inner / args.num_experts - kPadding;
-        const int64_t tiles = count(64, 64);
-        if (args.sparse_size >= 64 && args.cols >= 64 && reduction >= short_gradient_reduction(tiles)) {
-            if (tiles < kMiddleGradients) return launch_f32_split<64, 64, 2>(args, tiles, stream);
-            const int64_t middle = count(128, 64);
-            if (tiles < kLargeGradients) return launch_f32_split<128, 64, 3>(args, middle, stream);
-            const int64_t large = count(128, 128);
-            return launch_f32_split<128, 128, 3>(args, large, stream);
-        }
+        const int64_t reduction = mapped ? args.inner / args.num_experts - kPadding : args.piece_length > 0 ? args.piece_length : args.inner;
+        if (args.sparse_size >= 64 && args.cols >= 64) tile = gradient_tile(reduction, count(64, 64), count(128, 64), count(128, 128));
     } else {
         const int64_t rows = mapped ? max(args.rows / args.num_experts - kPadding, int64_t(1)) : args.rows;
-        const int64_t tiles_n = (args.cols + 63) / 64, tiles = mapped ? args.num_experts * (rows + 32) / 64 * tiles_n : (rows + 63) / 64 * tiles_n;
-        if (args.inner >= short_reduction(tiles, min(rows, args.cols) <= 32)) {
-            const int64_t small = count(64, 64);
-            if (tiles < kMiddleTiles || (mapped && rows <= 48)) return launch_f32_split<64, 64, 2>(args, small, stream);
-            const int64_t middle = count(128, 64);
-            if (tiles < kLargeTiles) return launch_f32_split<128, 64, 3>(args, middle, stream);
-            const int64_t large = count(128, 128);
-            return launch_f32_split<128, 128, 3>(args, large, stream);
+        const int64_t tiles_m = mapped ? args.num_experts * (rows + 32) / 64 : (rows + 63) / 64;
+        tile = forward_tile(rows, args.cols, args.inner, tiles_m * ((args.cols + 63) / 64), mapped);
+    }
+    switch (tile) {  // `count` sets what the kernel goes by
+        case F32Tile::k64x64: {
+            const int64_t tiles = count(64, 64);
+            return launch_f32_split<64, 64, 2>(args, tiles, stream);
         }
-        if (rows <= 32 && args.inner >= 256) {
-            const int64_t tiles_32 = count(32, 32);
-            return launch_f32_tile<32, 32, 2>(args, tiles_32, stream);
+        case F32Tile::k128x64: {
+            const int64_t tiles = count(128, 64);
+            return launch_f32_split<128, 64, 3>(args, tiles, stream);
         }
+        case F32Tile::k128x128: {
+            const int64_t tiles = count(128, 128);
+            return launch_f32_split<128, 128, 3>(args, tiles, stream);
+        }
+        case F32Tile::kMultiplyAdds: break;
     }
     if (const int64_t tiles = count(64, 64); tiles >= kF32LargeTiles) return launch_f32_tile<64, 16, 2>(args, tiles, stream);
     const int64_t tiles = count(32, 32);

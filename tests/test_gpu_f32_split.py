@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from fast_llm_amd.functional.sparse_copy import SparseMap
-from fast_llm_amd.functional.sparse_linear import dense_matmul, input_row_sparse_matmul
+from fast_llm_amd.functional.sparse_linear import dense_matmul, input_inner_sparse_matmul, input_row_sparse_matmul, output_sparse_matmul
 
 pytestmark = pytest.mark.gpu
 
@@ -47,7 +47,7 @@ def test_tiles(tile, inner, rhs_along_k, device):
 @pytest.mark.parametrize("rows", [(0, 1, 200, 383), (0, 1, 1000, 2100)])
 @pytest.mark.parametrize("columns", [68, 132, 1000, 2000, 4100])
 def test_row_sparse(columns, rows, device):
-    """Reductions of few and many rows, NaN in the padding: multiply-adds and, of many rows from 1000 columns on, all tile shapes."""
+    """Reductions of few and many rows, NaN in the padding: multiply-adds and, of many rows from 1000 columns on, the three tile shapes."""
     ends = list(itertools.accumulate(-(-count // 128) * 128 for count in rows))
     begins = [0, *ends[:-1]]
     sparse_map = SparseMap(
@@ -55,7 +55,7 @@ def test_row_sparse(columns, rows, device):
         torch.tensor([begin + count for begin, count in zip(begins, rows)], dtype=torch.int32, device=device), None, ends[-1], None, 4, None,
     )  # fmt: skip
     generator = torch.Generator(device).manual_seed(columns)
-    x = torch.full((ends[-1], 260), float("nan"), device=device)
+    x = torch.full((ends[-1], 380), float("nan"), device=device)
     y = torch.full((ends[-1], columns), float("nan"), device=device)
     for count, begin in zip(rows, begins):
         x[begin : begin + count].normal_(generator=generator)
@@ -63,7 +63,30 @@ def test_row_sparse(columns, rows, device):
     out = input_row_sparse_matmul(x.t(), y, sparse_map)
     for expert, (count, begin) in enumerate(zip(rows, begins)):
         lhs, rhs = x[begin : begin + count].t(), y[begin : begin + count]
-        _check(out[expert * 260 : (expert + 1) * 260], lhs, rhs, multiply_adds=columns < (1000 if max(rows) > 1000 else 4100))
+        _check(out[expert * 380 : (expert + 1) * 380], lhs, rhs, multiply_adds=columns < 1000 or max(rows) < 1000)
+
+
+# Tiles of 64 x 64, 128 x 64 and 128 x 128 by the rows that experts of the map's buffer are expected to have.
+@pytest.mark.parametrize(("columns", "inner"), [(500, 772), (2500, 388), (4100, 196)])
+@pytest.mark.parametrize("product", [output_sparse_matmul, input_inner_sparse_matmul])
+def test_experts_of_few_rows(product, columns, inner, device):
+    """0 to 40 rows, NaN in the padding."""
+    rows = [7 * expert % 41 for expert in range(32)]
+    ends = list(itertools.accumulate(-(-count // 128) * 128 for count in rows))
+    begins = [0, *ends[:-1]]
+    sparse_map = SparseMap(
+        None, torch.tensor(ends, dtype=torch.int32, device=device),
+        torch.tensor([begin + count for begin, count in zip(begins, rows)], dtype=torch.int32, device=device), None, ends[-1], None, 32, None,
+    )  # fmt: skip
+    generator = torch.Generator(device).manual_seed(columns)
+    lhs = torch.full((ends[-1], inner), float("nan"), device=device)
+    for count, begin in zip(rows, begins):
+        lhs[begin : begin + count].normal_(generator=generator)
+    weight = torch.randn((32, columns, inner), generator=generator, device=device)
+    rhs = weight.flatten(0, 1).t() if product is output_sparse_matmul else weight.transpose(1, 2).reshape(-1, columns)
+    out = product(lhs, rhs, sparse_map)
+    for expert, (count, begin) in enumerate(zip(rows, begins)):
+        _check(out[begin : begin + count], lhs[begin : begin + count], weight[expert].t())
 
 
 @pytest.mark.parametrize(("rows", "cols", "inner"), [(2048, 1024, 8), (8192, 2048, 8), (16384, 8, 8), (16384, 32, 264), (24, 16384, 264)])
