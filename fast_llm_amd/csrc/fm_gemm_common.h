@@ -232,7 +232,10 @@ int run_fused_gemm(const char *name, GemmArgs args, int dtype, void *stream);
 // Allows `kernel` that many bytes of dynamic LDS. `configured`: the kernel's own bit mask of devices done.
 int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured);
 
-// Row-sparse products of experts of few rows (fm_gemm_row_sparse.hip), of those that `mfma_gemm_eligible` accepts.
+// Row-sparse products of experts of few rows (fm_gemm_row_panel.hip), of those that `mfma_gemm_eligible` accepts.
+bool row_panel_gemm_chosen(const GemmArgs &args, int dtype);
+int row_panel_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream);
+// Row-sparse products of experts of some more rows (fm_gemm_row_sparse.hip), of those that `mfma_gemm_eligible` accepts.
 bool row_sparse_gemm_chosen(const GemmArgs &args, int dtype);
 int row_sparse_gemm_launch(GemmArgs args, int dtype, hipStream_t stream);
 // Products of few tiles (fm_gemm_few_tiles.hip). `splits`: the large tiles' kernel would split the reductions, given a workspace.

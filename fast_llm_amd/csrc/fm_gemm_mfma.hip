@@ -1565,7 +1565,8 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
             GemmArgs args = products[i];
             TableSpace space;
             const bool eligible = args.fusion == kFusionNone ? mfma_gemm_eligible(args, dtype) : mfma_gemm_fusion_eligible(args, dtype);
-            if (!eligible || row_sparse_gemm_chosen(args, dtype) || !table_space(args, space) || !wants_table(args, space.split)) continue;
+            if (!eligible || row_panel_gemm_chosen(args, dtype) || row_sparse_gemm_chosen(args, dtype)) continue;
+            if (!table_space(args, space) || !wants_table(args, space.split)) continue;
             if (few_tiles_gemm_chosen(args, dtype, space.split) || space.split != split_ones) continue;
             if (split_ones && at == 0) at = kPartialBytes;
             args.partials = space.split ? static_cast<float *>(workspace) : nullptr;
@@ -1582,6 +1583,7 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
 
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
     if (!args.planned) {
+        if (!args.accumulate && row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
         if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
         count_tiles(args);
         if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
@@ -1595,6 +1597,7 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
         if (workspace != nullptr && (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0))
             return fail(FM_ERR_INVALID_ARGUMENT, "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
                         workspace_size, workspace);
+        if (row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
         if (few_tiles_gemm_chosen(args, dtype, splits_last_round(args))) return few_tiles_gemm_launch(args, dtype, stream);
         if (split) args.partials = static_cast<float *>(workspace);
         if (workspace != nullptr && wants_table(args, split)) {
