@@ -43,6 +43,7 @@ struct GemmArgs {
     void *fused_out;
     int64_t fused_stride;  // row stride of fused_out, elements
     int64_t half;          // columns of the activation output per expert
+    int any_half;          // gated forward: it need not be a multiple of 128
     int num_ids;           // workgroup ids that may have a tile (set by the MFMA kernel's launcher)
     void *tile_table;      // one record per id, written by the plan kernel into the caller's workspace, or null
     int64_t piece_length;  // row-sparse mode without a map: group e reduces over [e, e + 1) * piece_length instead of

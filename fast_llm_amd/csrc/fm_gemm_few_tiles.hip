@@ -9,6 +9,7 @@
 // Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), two or three in LDS,
 // filled straight from memory; the fragments of the next 16 are read while the MFMAs of this 16 run. Sums in fp32, in the order of
 // the large tiles' kernel.
+#include "fm_activation_math.h"
 #include "fm_gemm_common.h"
 
 namespace fm {
@@ -23,7 +24,14 @@ typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
 
 constexpr int kTileM = 128, kBK = kRotationSlice, kThreads = 256, kSteps = kBK / 16;
-constexpr int kBlocksM = kTileM / 64;  // 2 x 2 wavefronts, 32 x 32 accumulators
+// 2 x 2 wavefronts, 32 x 32 accumulators. With the gated activation the columns are gates and ups in turns of 32, which one wavefront
+// has to have both of: 4 x 1 where there are 64.
+template <int kTileN, bool kGated>
+constexpr int kWavesN = kGated && kTileN == 64 ? 1 : 2;
+template <int kTileN, bool kGated>
+constexpr int kBlocksM = kTileM / 32 * kWavesN<kTileN, kGated> / 4;
+template <int kTileN, bool kGated>
+constexpr int kBlocksN = kTileN / 32 / kWavesN<kTileN, kGated>;
 
 __device__ __forceinline__ f32x16_t mfma(bf16_t, u32x4_t a, u32x4_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
@@ -33,7 +41,7 @@ __device__ __forceinline__ f32x16_t mfma(f16_t, u32x4_t a, u32x4_t b, f32x16_t c
 }
 
 // One operand's slice in LDS and the loads that fill it: lines [row][kBK] where it is contiguous along K, [kBK][row] otherwise.
-template <int kTile, bool kContiguousK>
+template <int kTile, bool kContiguousK, int kBlocks>
 struct Operand {
     static constexpr int kBytes = kTile * kBK * 2, kChunks = (kContiguousK ? kBK : kTile) / 8;  // 16-byte chunks per line
     static constexpr int kLoads = kBytes / 16 / kThreads;                                    // per lane and slice
@@ -54,7 +62,12 @@ struct Operand {
     int slices, next, unfetched;
 
     // `stride`: bytes between lines. `valid`: rows (columns of the product) that exist, a multiple of 8 where they are not lines.
-    __device__ __forceinline__ void setup(const char *first, int64_t stride, int valid, int k_count_, int first_slice, int wave, int lane) {
+    // `kPaired`: of every 64 lines the first 32 follow one another in memory and the last 32 lie `pair_distance` lines after those;
+    // `valid` of each.
+    template <bool kPaired>
+    __device__ __forceinline__ void setup(const char *first, int64_t stride, int valid, int k_count_, int first_slice, int wave, int lane,
+                                          int64_t pair_distance) {
+        static_assert(kContiguousK || !kPaired, "lines are rows");
         start = uniform_pointer(first);
         step = kContiguousK ? kBK * 2 : kBK * stride;
         k_count = k_count_;
@@ -65,8 +78,10 @@ struct Operand {
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) {
             const int slot = (wave * kLoads + j) * 64 + lane, line = slot / kChunks, chunk = swizzled(line, slot % kChunks);
-            const bool exists = kContiguousK ? line < valid : chunk * 8 < valid;
-            offset[j] = exists ? static_cast<uint32_t>(line * stride + chunk * 16) : kOutOfRange;
+            const int single = kPaired ? line / 64 * 32 + line % 32 : line;
+            const bool exists = kContiguousK ? single < valid : chunk * 8 < valid;
+            const int64_t memory_line = kPaired && line % 64 >= 32 ? single + pair_distance : single;
+            offset[j] = exists ? static_cast<uint32_t>(memory_line * stride + chunk * 16) : kOutOfRange;
             k[j] = kContiguousK ? chunk * 8 : line;
         }
     }
@@ -98,7 +113,7 @@ struct Operand {
 
     // MFMA fragments (8 consecutive k of one row per lane; lane l: row l % 32, k half l / 32) of the 32 rows from `first` on, per lane:
     // an address per step of 16 (K-contiguous; the next 32 rows and the slot are added), or one per 32 rows (the step is added).
-    static constexpr int kAddresses = kContiguousK ? kSteps : kTile / 64;
+    static constexpr int kAddresses = kContiguousK ? kSteps : kBlocks;
     static __device__ __forceinline__ void fragment_addresses(int first, int lane, int (&addresses)[kAddresses]) {
         if constexpr (kContiguousK) {
             const int row = first + (lane & 31);
@@ -107,7 +122,7 @@ struct Operand {
         } else {
             const int s = lane & 15, group = lane >> 4, k = ((group >> 1) << 3) + (s >> 2);
 #pragma unroll
-            for (int i = 0; i < kTile / 64; ++i) {
+            for (int i = 0; i < kBlocks; ++i) {
                 const int column = first + i * 32 + ((group & 1) << 4) + ((s & 3) << 2);
                 addresses[i] = k * kTile * 2 + swizzled(k, column >> 3) * 16 + (column & 7) * 2;
             }
@@ -133,28 +148,28 @@ __device__ __forceinline__ void wait_for_loads() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kNewest) : "memory");
 }
 
-// Accumulators -> rows of `out`, 32 rows of the wavefront's columns at a time through its own part of LDS: 16 bytes per lane and store.
-// The tile's rows are the MFMA's columns: a lane's four accumulators are consecutive columns of one row.
-template <typename T, int kTileN>
-__device__ __forceinline__ void store_tile(const f32x16_t (&acc)[kBlocksM][kTileN / 64], int staging, T *out, int64_t stride,
-                                           int rows_valid, int cols_valid, int wave_m, int wave_n, int lane) {
-    constexpr int kWaveCols = kTileN / 2, kRowBytes = kWaveCols * 2 + 16;
+// value(i, j, v), of 32 x 32 accumulators -> rows of `out`, 32 rows of the wavefront's columns at a time through its own part of LDS: 16
+// bytes per lane and store. The tile's rows are the MFMA's columns: a lane's four accumulators are consecutive columns of one row.
+template <typename T, int kRowBlocks, int kColumnBlocks, typename Value>
+__device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, int64_t stride, int rows_valid, int cols_valid, int wave_m,
+                                           int wave_n, int lane) {
+    constexpr int kWaveCols = kColumnBlocks * 32, kRowBytes = kWaveCols * 2 + 16;
     constexpr int kLanesPerRow = kWaveCols / 8, kRowsPerRead = 64 / kLanesPerRow, kReads = 32 / kRowsPerRead;
     const int write_base = staging + (lane & 31) * kRowBytes + (lane >> 5) * 8;
     const int read_row = lane / kLanesPerRow, read_column = lane % kLanesPerRow * 8;
     const int read_base = staging + read_row * kRowBytes + read_column * 2;
-    const int column = wave_n * kWaveCols + read_column, first_row = wave_m * kBlocksM * 32 + read_row;
+    const int column = wave_n * kWaveCols + read_column, first_row = wave_m * kRowBlocks * 32 + read_row;
 #pragma unroll
-    for (int i = 0; i < kBlocksM; ++i) {
+    for (int i = 0; i < kRowBlocks; ++i) {
 #pragma unroll
-        for (int j = 0; j < kTileN / 64; ++j)
+        for (int j = 0; j < kColumnBlocks; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 struct {
                     T v[4];
                 } group;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) group.v[c] = from_float<T>(acc[i][j][4 * g + c]);
+                for (int c = 0; c < 4; ++c) group.v[c] = from_float<T>(value(i, j, 4 * g + c));
                 *(FM_LDS(u32x2_t) *)static_cast<uintptr_t>(write_base + (j * 32 + 8 * g) * 2) = __builtin_bit_cast(u32x2_t, group);
             }
         asm volatile("" ::: "memory");  // a wavefront's own LDS accesses are carried out in order
@@ -179,11 +194,13 @@ constexpr int kWorkgroups = kTileN == 256 ? 1 : 2;  // per CU
 template <int kTileN>
 constexpr int kLdsBytes = kStages<kTileN> * (kTileM + kTileN) * kBK * 2;
 
-template <typename T, int kTileN, bool kRhsK>
+template <typename T, int kTileN, bool kRhsK, bool kGated>
 __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
-    typedef Operand<kTileM, true> Lhs;
-    typedef Operand<kTileN, kRhsK> Rhs;
-    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads, kBlocksN = kTileN / 64;
+    constexpr int kBlocksM = few_tiles::kBlocksM<kTileN, kGated>, kBlocksN = few_tiles::kBlocksN<kTileN, kGated>;
+    typedef Operand<kTileM, true, kBlocksM> Lhs;
+    typedef Operand<kTileN, kRhsK, kBlocksN> Rhs;
+    constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
+    constexpr int kColumns = kGated ? kTileN / 2 : kTileN;  // of the result
     static_assert(kLdsBytes<kTileN> * kWorkgroups<kTileN> <= 160 * 1024 && kLdsBytes<kTileN> >= 4 * 32 * (kTileN + 16), "LDS of a CU");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
     const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
@@ -193,9 +210,10 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
     const int logical = (local / args.chunk_tiles * 8 + pid % 8) * args.chunk_tiles + local % args.chunk_tiles;
     RowTile tile;
     if (!locate_tile<kTileM>(args, logical, tile)) return;
-    const int64_t col0 = static_cast<int64_t>(tile.tile_n) * kTileN;
+    const int64_t col0 = static_cast<int64_t>(tile.tile_n) * kColumns;
     const int rows_valid = __builtin_amdgcn_readfirstlane(tile.rows_valid);
-    const int cols_valid = __builtin_amdgcn_readfirstlane(static_cast<int>(min(static_cast<int64_t>(kTileN), args.cols - col0)));
+    const int cols_valid = __builtin_amdgcn_readfirstlane(
+        static_cast<int>(min(static_cast<int64_t>(kColumns), (kGated ? args.half : args.cols) - col0)));
     const int64_t rhs_offset = args.mode == kOutputSparse
                                    ? (static_cast<int64_t>(tile.expert) * args.sparse_size + col0) * args.rhs_stride_col
                                    : static_cast<int64_t>(tile.expert) * args.sparse_size * args.rhs_stride_inner + col0 * args.rhs_stride_col;
@@ -203,16 +221,17 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
     const int first_slice = __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert));
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wave_m = wave / 2, wave_n = wave % 2;
+    const int wave_m = wave / kWavesN<kTileN, kGated>, wave_n = wave % kWavesN<kTileN, kGated>;
     Lhs lhs;
     Rhs rhs;
-    lhs.setup(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row0 * args.lhs_stride_row),
-              args.lhs_stride_row * 2, rows_valid, k_count, first_slice, wave, lane);
-    rhs.setup(reinterpret_cast<const char *>(static_cast<const T *>(args.rhs) + rhs_offset),
-              (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 2, cols_valid, k_count, first_slice, wave, lane);
+    lhs.template setup<false>(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row0 * args.lhs_stride_row),
+                              args.lhs_stride_row * 2, rows_valid, k_count, first_slice, wave, lane, 0);
+    rhs.template setup<kGated>(reinterpret_cast<const char *>(static_cast<const T *>(args.rhs) + rhs_offset),
+                               (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 2, cols_valid, k_count, first_slice, wave, lane,
+                               args.half);
     int lhs_addresses[Lhs::kAddresses], rhs_addresses[Rhs::kAddresses];
-    Lhs::fragment_addresses(wave_m * kTileM / 2, lane, lhs_addresses);
-    Rhs::fragment_addresses(wave_n * kTileN / 2, lane, rhs_addresses);
+    Lhs::fragment_addresses(wave_m * kBlocksM * 32, lane, lhs_addresses);
+    Rhs::fragment_addresses(wave_n * kBlocksN * 32, lane, rhs_addresses);
     f32x16_t acc[kBlocksM][kBlocksN];
 #pragma unroll
     for (int i = 0; i < kBlocksM; ++i)
@@ -269,16 +288,31 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
     }
     wait_for_loads<0>();  // zeros on their way to the slots
     __syncthreads();
-    T *out = static_cast<T *>(args.out) + tile.row0 * args.out_stride_row + col0;
-    store_tile<T, kTileN>(acc, lds + wave * 32 * (kTileN + 16), out, args.out_stride_row, rows_valid, cols_valid, wave_m, wave_n, lane);
+    const int staging = lds + wave * 32 * (kTileN + 16);
+    if constexpr (kGated) {
+        // From the rounded values, as the activation's own kernel computes: the same bits.
+        T *out = static_cast<T *>(args.fused_out) + tile.row0 * args.fused_stride + col0;
+        const auto store = [&](auto activate) {
+            store_tile<T, kBlocksM, kBlocksN / 2>(
+                [&](int i, int j, int v) {
+                    return activate(to_float(from_float<T>(acc[i][2 * j][v]))) * to_float(from_float<T>(acc[i][2 * j + 1][v]));
+                },
+                staging, out, args.fused_stride, rows_valid, cols_valid, wave_m, wave_n, lane);
+        };
+        FM_DISPATCH_ACTIVATION(args.activation, kActivation, store([](float x) { return activation_forward<kActivation>(x); }));
+    } else {
+        T *out = static_cast<T *>(args.out) + tile.row0 * args.out_stride_row + col0;
+        store_tile<T, kBlocksM, kBlocksN>([&](int i, int j, int v) { return acc[i][j][v]; }, staging, out, args.out_stride_row, rows_valid,
+                                          cols_valid, wave_m, wave_n, lane);
+    }
 }
 
 // Tiles of 128 x 256, by the upper bound that the host knows of their row tiles (a static map has one tile of padding per expert).
 static int64_t most_tiles(const GemmArgs &args) { return (args.rows + kTileM - 1) / kTileM * ((args.cols + 255) / 256); }
 
-template <typename T, int kTileN, bool kRhsK>
+template <typename T, int kTileN, bool kRhsK, bool kGated = false>
 static int launch(const GemmArgs &args, hipStream_t stream) {
-    const auto kernel = grouped_gemm_few_tiles_kernel<T, kTileN, kRhsK>;
+    const auto kernel = grouped_gemm_few_tiles_kernel<T, kTileN, kRhsK, kGated>;
     static std::atomic<uint64_t> configured{0};
     if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes<kTileN>, configured)) return status;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n, round = 8 * static_cast<int64_t>(args.chunk_tiles);
@@ -294,6 +328,7 @@ static int launch(GemmArgs args, hipStream_t stream) {
     if (tiles >= (int64_t(1) << 30)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
     // Runs of 16 tiles per XCD; 8 and 32 are up to 3 and 5 % slower (128 columns).
     args.chunk_tiles = static_cast<int>(min(int64_t(16), (tiles + 7) / 8));
+    if (args.fusion == kFusionGatedForward) return launch<T, kTileN, true, true>(args, stream);
     return args.rhs_stride_inner == 1 ? launch<T, kTileN, true>(args, stream) : launch<T, kTileN, false>(args, stream);
 }
 
@@ -316,10 +351,16 @@ static int launch(GemmArgs args, hipStream_t stream) {
 //       113 .. 160     1.16, 1.18, 1.13
 // Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87), 1.03 (0.63), 0.88 (0.52) up to 96, and no better
 // with more: they stay there.
+// With the gated activation against fused tiles of 256 x 256, layer 1 of 300 tokens of 8 experts of 4096 x 1536 (2 each) 78 -> 66 us, of
+// 800 of 8 of 1536 x 512 (6 each) 45 -> 31.
 bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
-    if (dtype == FM_DTYPE_F32 || args.mode == kInputRowSparse || args.fusion != kFusionNone || args.accumulate || args.out_dtype != dtype ||
-        args.lhs_stride_inner != 1 || splits)
+    if (dtype == FM_DTYPE_F32 || args.mode == kInputRowSparse || args.accumulate || args.out_dtype != dtype || args.lhs_stride_inner != 1 ||
+        splits)
         return false;
+    // With the gated activation where layer 1's own output is not wanted; the ups are addressed with 32 bits from the gates.
+    if (args.fusion == kFusionGatedForward && (args.out != nullptr || (args.half + 128) * args.rhs_stride_col * 2 >= (int64_t(1) << 31)))
+        return false;
+    if (args.fusion == kFusionGatedBackward) return false;
     return few_tiles::most_tiles(args) <= 256;
 }
 

@@ -159,12 +159,13 @@ struct TileLoader {
     // row-contiguous one gets in-range rows in their place.
     // `split_rows` (K-contiguous only, 0: off): rows 64..127 and 192..255 of the tile are not the rows after 0..63 and
     // 128..191 but lie `split_rows` rows after them, i.e. tile row n is memory row
-    // (n / 128) * 64 + n % 64 + (n / 64 % 2) * split_rows (the gate and up halves of a gated layer's weight).
+    // (n / 128) * 64 + n % 64 + (n / 64 % 2) * split_rows (the gate and up halves of a gated layer's weight); `split_valid` of each.
     // `k_count`: reduction indices from the first one of slice 0 to the end of the reduction range; a row-contiguous
     // operand gets zeros for the K-rows of its last slice that lie past it. Of a K-contiguous operand only the last
     // row gets zeros there: what the other rows bring is the start of the next row, to be masked in LDS.
     __device__ __forceinline__ void setup(const char *tile_base, int64_t stride, int valid_rows, int num_slices,
-                                          int k_count, int wave, int lane, int split_rows = 0, int first_slice = 0) {
+                                          int k_count, int wave, int lane, int split_rows = 0, int first_slice = 0,
+                                          int split_valid = kTile / 2) {
         static_assert(kLoadsPerOperand % 2 == 0, "loads come in (even, odd) pairs");
         fetch_base = tile_base;
         wrap_at = first_slice;
@@ -190,7 +191,7 @@ struct TileLoader {
         }
         // Two loads further on: 128 slots = 16 rows of a K-contiguous slice, 4 K-rows of a row-contiguous one.
         pair_stride = static_cast<uint32_t>((kContiguousK ? 128 / kChunksPerRow : 4) * stride);
-        const int64_t last_row = split_rows == 0 ? valid_rows - 1 : split_rows + kTile / 2 - 1;
+        const int64_t last_row = split_rows == 0 ? valid_rows - 1 : split_rows + split_valid - 1;
         step = kContiguousK ? kBK * 2 : kBK * stride;
         const int last_count = k_count - (num_slices - 1) * kBK;  // of the last slice
         if constexpr (kRotates) {
@@ -367,7 +368,8 @@ __device__ __forceinline__ bool resolve_tile(const GemmArgs &args, int logical, 
     // A tile of the fused gated forward product has 128 gate columns (and their up columns).
     const bool paired = args.fusion == kFusionGatedForward;
     const int64_t col0 = static_cast<int64_t>(tile.tile_n) * (paired ? kTile / 2 : kTile);
-    work.cols_valid = paired ? kTile : static_cast<int>(min(static_cast<int64_t>(kTile), args.cols - col0));
+    work.cols_valid = static_cast<int>(paired ? 2 * min(static_cast<int64_t>(kTile / 2), args.half - col0)
+                                              : min(static_cast<int64_t>(kTile), args.cols - col0));
     work.rows_valid = tile.rows_valid;
     work.expert = tile.expert;
     work.lhs_offset = tile.row0 * args.lhs_stride_row;
@@ -776,10 +778,11 @@ __device__ __forceinline__ void store_tile_gated_backward(const f32x16_t (&acc)[
 // `layer_1` is stored) and 64 outputs act(gate) * up pass through the wavefront's LDS region one after the other and leave
 // as 128-byte row segments; what is not stored is not staged (staging all three and
 // storing one: 741 us against 705 at 64 experts of 2048 x 1408 with 1000 rows each, the plain product 627).
-template <typename T, int kActivation>
+// `kWhole`: all 128 gates exist.
+template <typename T, int kActivation, bool kWhole>
 __device__ __forceinline__ void store_tile_gated_forward(const f32x16_t (&acc)[kTilesM][kTilesN], FM_LDS(char) * lds,
                                                          T *layer_1, T *activation_out, int64_t stride,
-                                                         int64_t activation_stride, int64_t half, int rows_valid,
+                                                         int64_t activation_stride, int64_t half, int rows_valid, int cols_valid,
                                                          int wave, int lane, int row_base, int blocks) {
     static_assert(kTilesN == 4 && kWaveCols == 128, "two gate and two up accumulators per row block");
     constexpr int kColumns = kWaveCols / 2, kRowBytes = kColumns * sizeof(T) + kEpiloguePadBytes;
@@ -809,7 +812,7 @@ __device__ __forceinline__ void store_tile_gated_forward(const f32x16_t (&acc)[k
         T *pointer = target + first_row * target_stride + column;
 #pragma unroll
         for (int t = 0; t < kReads; ++t, pointer += kRowsPerRead * target_stride)
-            if (first_row + t * kRowsPerRead < rows_valid)
+            if (first_row + t * kRowsPerRead < rows_valid && (kWhole || column < cols_valid))
                 __builtin_nontemporal_store(staged[t], reinterpret_cast<u32x4_t *>(pointer));
         asm volatile("" ::: "memory");
     };
@@ -874,7 +877,10 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[kTilesM][kTi
 // kFusion: a GemmFusion, the epilogue to run instead of the plain store.
 // kRotates: the reductions of an expert's tiles start with a slice of its own (`first_slice_of`). An instance of its own, since the
 // main loop has five scalar instructions more per slice for it: 0.3 % of the launches that are bound by their MFMAs.
-template <typename T, bool kLhsContiguousK, bool kRhsContiguousK, bool kMasked, int kFusion, bool kRotates>
+// `kWidth`: whether the gated forward product's last column tile may have fewer than 128 gates. An instance of its own: the check costs the
+// others 0.5 % (64 experts of 2048 x 1408, 469 rows).
+enum GatedWidth { kWholeTiles, kAnyWidth };
+template <typename T, bool kLhsContiguousK, bool kRhsContiguousK, bool kMasked, int kFusion, bool kRotates, GatedWidth kWidth>
 __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_kernel(GemmArgs launch_args) {
     static_assert(kFusion == kFusionNone || (kRhsContiguousK && !kMasked), "fused epilogues: output-sparse, K-major rhs");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
@@ -1170,7 +1176,7 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
                          (kRhsContiguousK ? args.rhs_stride_col : args.rhs_stride_inner) * sizeof(T), work.cols_valid,
                          next.num_slices, work.k_hi - next.k_first, wave, lane,
                          kFusion == kFusionGatedForward ? static_cast<int>(args.half) : 0,
-                         kRotates ? work.first_slice : 0);
+                         kRotates ? work.first_slice : 0, kWidth == kAnyWidth ? work.cols_valid / 2 : kTile / 2);
     };
     constexpr int kFirstLhsSlot = kLhsBase + (kLhsStages - 1) * kOperandBytes;
     auto first_loads = [&](const Tile &next) {
@@ -1289,9 +1295,9 @@ __global__ __launch_bounds__(kMfmaThreads, kWaves / 4) void grouped_gemm_mfma_ke
         } else if constexpr (kFusion == kFusionGatedForward) {
             T *layer_1 = args.out == nullptr ? nullptr : static_cast<T *>(args.out) + work.out_offset;
             FM_DISPATCH_ACTIVATION(args.activation, kActivation,
-                                   store_tile_gated_forward<T, kActivation>(
+                                   store_tile_gated_forward<T, kActivation, kWidth == kWholeTiles>(
                                        acc, staging, layer_1, static_cast<T *>(args.fused_out) + work.fused_offset,
-                                       args.out_stride_row, args.fused_stride, args.half, work.rows_valid, wave, lane,
+                                       args.out_stride_row, args.fused_stride, args.half, work.rows_valid, work.cols_valid / 2, wave, lane,
                                        wave_row_base, wave_row_blocks));
         } else if constexpr (kFusion == kFusionGatedBackward) {
             T *recomputed = args.fused_out == nullptr ? nullptr : static_cast<T *>(args.fused_out) + work.fused_offset;
@@ -1374,12 +1380,12 @@ int allow_lds(const void *kernel, int bytes, std::atomic<uint64_t> &configured) 
     return FM_OK;
 }
 
-template <typename T, bool kLhsK, bool kRhsK, bool kMasked, int kFusion = kFusionNone, bool kRotates = false>
+template <typename T, bool kLhsK, bool kRhsK, bool kMasked, int kFusion = kFusionNone, GatedWidth kWidth = kWholeTiles, bool kRotates = false>
 static int launch_instance(const GemmArgs &args, hipStream_t stream) {
     if constexpr (kLhsK && kRhsK && !kMasked && !kRotates) {
-        if (starts_anywhere(args)) return launch_instance<T, kLhsK, kRhsK, kMasked, kFusion, true>(args, stream);
+        if (starts_anywhere(args)) return launch_instance<T, kLhsK, kRhsK, kMasked, kFusion, kWidth, true>(args, stream);
     }
-    auto kernel = grouped_gemm_mfma_kernel<T, kLhsK, kRhsK, kMasked, kFusion, kRotates>;
+    auto kernel = grouped_gemm_mfma_kernel<T, kLhsK, kRhsK, kMasked, kFusion, kRotates, kWidth>;
     static std::atomic<uint64_t> configured{0};
     if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
     // One workgroup per CU walks the ids (see the kernel).
@@ -1397,7 +1403,9 @@ static int launch_instance(const GemmArgs &args, hipStream_t stream) {
 template <typename T>
 static int launch_layout(const GemmArgs &args, hipStream_t stream) {
     const bool lhs_k = args.lhs_stride_inner == 1, rhs_k = args.rhs_stride_inner == 1;
-    if (args.fusion == kFusionGatedForward) return launch_instance<T, true, true, false, kFusionGatedForward>(args, stream);
+    if (args.fusion == kFusionGatedForward)
+        return args.half % (kTile / 2) == 0 ? launch_instance<T, true, true, false, kFusionGatedForward>(args, stream)
+                                            : launch_instance<T, true, true, false, kFusionGatedForward, kAnyWidth>(args, stream);
     if (args.fusion == kFusionGatedBackward) return launch_instance<T, true, true, false, kFusionGatedBackward>(args, stream);
     // A ragged reduction range: the row-sparse product with a map, and a reduction that is no whole number of slices
     // (a feed-forward size of 3416, say), whose last slice is then masked in LDS: one pass over two operands and one
@@ -1435,8 +1443,8 @@ bool mfma_gemm_eligible(const GemmArgs &args, int dtype) {
     return true;
 }
 
-// The fused epilogues exist for one layout: both operands K-contiguous, output-sparse mode, T in and out, whole
-// column tiles (the activation width a multiple of 128 for the forward, of 8 for the backward).
+// The fused epilogues exist for one layout: both operands K-contiguous, output-sparse mode, T in and out, an activation width that is
+// a multiple of 8 (of 128 for the forward products that callers ask for by themselves).
 bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype) {
     if (!mfma_gemm_eligible(args, dtype) || args.mode != kOutputSparse || args.out_dtype != dtype || args.accumulate ||
         args.inner % kBK != 0)
@@ -1446,7 +1454,7 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype) {
         return false;
     if (args.fusion == kFusionGatedForward) {
         // The up rows of a tile are addressed with 32-bit byte offsets from its gate rows.
-        if (args.half % (kTile / 2) != 0 || (args.half + kTile) * args.rhs_stride_col * 2 >= (int64_t(1) << 32)) return false;
+        if ((!args.any_half && args.half % (kTile / 2) != 0) || (args.half + kTile) * args.rhs_stride_col * 2 >= (int64_t(1) << 32)) return false;
     }
     return true;
 }
@@ -1464,7 +1472,7 @@ static void count_tiles(GemmArgs &args) {
         args.tiles_m = static_cast<int>((args.rows + kTile - 1) / kTile + (args.num_experts > 1 ? args.num_experts : 0));
     }
     args.tiles_n = static_cast<int>((args.cols + kTile - 1) / kTile);
-    if (args.fusion == kFusionGatedForward) args.tiles_n = static_cast<int>(args.half / (kTile / 2));
+    if (args.fusion == kFusionGatedForward) args.tiles_n = static_cast<int>((args.half + kTile / 2 - 1) / (kTile / 2));
 }
 
 static bool too_many_tiles(const GemmArgs &args) {

@@ -104,6 +104,7 @@ struct Step {
             args.activation = static_cast<int>(layer.activation);
             args.fused_out = layer.activation_output;
             args.fused_stride = args.half = layer.ffn;
+            args.any_half = 1;
         }
         return args;
     }

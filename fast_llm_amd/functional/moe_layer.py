@@ -88,9 +88,10 @@ def _describe(
     return layer
 
 
-def _fuses_layer_1(options: MoELayerOptions, layer: _lib.MoELayer) -> bool:
-    """Whether layer 1's product has an instance with the gated activation in its epilogue."""
-    return options.gated and layer.dtype != 0 and layer.hidden % 64 == 0 and layer.ffn % 128 == 0
+def _fuses_layer_1(options: MoELayerOptions, layer: _lib.MoELayer, training: bool) -> bool:
+    """Whether layer 1's product has an instance with the gated activation in its epilogue. In training for the widths only that the
+    product of the parts takes: the recompute levels keep to the same kernels."""
+    return options.gated and layer.dtype != 0 and layer.hidden % 64 == 0 and layer.ffn % (128 if training else 8) == 0
 
 
 @dataclasses.dataclass
@@ -140,7 +141,7 @@ def _forward(
     layer_2_output = new((rows, layer.hidden)) if training and not level.recompute_sparse_input else sparse_input
     activation_output, output = new((rows, ffn)), new(hidden_states.shape)
     layer_1_output = None
-    if keep_layer_1 or not _fuses_layer_1(options, layer):
+    if keep_layer_1 or not _fuses_layer_1(options, layer, training):
         layer_1_output = new((rows, ffn * 2 if options.gated else ffn))
         layer.layer_1_output = layer_1_output.data_ptr()
     layer.input, layer.output, layer.workspace = hidden_states.data_ptr(), output.data_ptr(), workspace.data_ptr()
