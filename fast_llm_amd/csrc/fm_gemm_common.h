@@ -239,7 +239,11 @@ int row_panel_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream);
 // Row-sparse products of experts of some more rows (fm_gemm_row_sparse.hip), of those that `mfma_gemm_eligible` accepts.
 bool row_sparse_gemm_chosen(const GemmArgs &args, int dtype);
 int row_sparse_gemm_launch(GemmArgs args, int dtype, hipStream_t stream);
-// Products of few tiles (fm_gemm_few_tiles.hip). `splits`: the large tiles' kernel would split the reductions, given a workspace.
+// Products that memory bounds, or of few tiles (fm_gemm_weight_stream.hip). `splits`: the large tiles' kernel would split the reductions,
+// given a workspace.
+bool weight_stream_gemm_chosen(const GemmArgs &args, int dtype, bool splits);
+int weight_stream_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream);
+// Those of fewer tiles still (fm_gemm_few_tiles.hip), of the ones that the above refuses.
 bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits);
 int few_tiles_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream);
 

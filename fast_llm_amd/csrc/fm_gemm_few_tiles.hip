@@ -1,152 +1,31 @@
-// Grouped products of few output tiles, in half precision: 128 rows x 64, 128 or 256 columns.
+// Grouped products of few output tiles, in half precision: 128 rows x 64 columns.
 //
-// A launch of up to one 256 x 256 tile per CU lasts as long as one tile does, on whatever part of the chip, and most of a tile's rows are
-// padding where experts have some 100 tokens. With tiles of half, a quarter or an eighth of that size more CUs share the same work;
-// two small ones per CU overlap one's loads with the other's MFMAs. A CU then reads more operand bytes per multiplication, which is
-// why launches that fill the chip with large tiles stay with those (fm_gemm_mfma.hip; the lines, and what was measured on both sides
-// of them, are at few_tiles_gemm_chosen).
+// A launch of a third of a 256 x 256 tile per CU lasts as long as one tile does, on whatever part of the chip, and most of a tile's rows are
+// padding where experts have some 100 tokens. With tiles of an eighth of that size more CUs share the same work; two per CU overlap
+// one's loads with the other's MFMAs. A CU then reads more operand bytes per multiplication, which is why launches of more tiles
+// go elsewhere (fm_gemm_weight_stream.hip; the line, and what was measured on both sides of it, are at few_tiles_gemm_chosen).
 //
-// Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), two or three in LDS,
+// Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), three in LDS,
 // filled straight from memory; the fragments of the next 16 are read while the MFMAs of this 16 run. Sums in fp32, in the order of
 // the large tiles' kernel.
 #include "fm_activation_math.h"
-#include "fm_gemm_common.h"
+#include "fm_gemm_slices.h"
 
 namespace fm {
 
 namespace few_tiles {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
-typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
-typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
+using namespace slices;
 
-constexpr int kTileM = 128, kBK = kRotationSlice, kThreads = 256, kSteps = kBK / 16;
-// 2 x 2 wavefronts, 32 x 32 accumulators. With the gated activation the columns are gates and ups in turns of 32, which one wavefront
-// has to have both of: 4 x 1 where there are 64.
-template <int kTileN, bool kGated>
-constexpr int kWavesN = kGated && kTileN == 64 ? 1 : 2;
-template <int kTileN, bool kGated>
-constexpr int kBlocksM = kTileM / 32 * kWavesN<kTileN, kGated> / 4;
-template <int kTileN, bool kGated>
-constexpr int kBlocksN = kTileN / 32 / kWavesN<kTileN, kGated>;
-
-__device__ __forceinline__ f32x16_t mfma(bf16_t, u32x4_t a, u32x4_t b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x16_t mfma(f16_t, u32x4_t a, u32x4_t b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-}
-
-// One operand's slice in LDS and the loads that fill it: lines [row][kBK] where it is contiguous along K, [kBK][row] otherwise.
-template <int kTile, bool kContiguousK, int kBlocks>
-struct Operand {
-    static constexpr int kBytes = kTile * kBK * 2, kChunks = (kContiguousK ? kBK : kTile) / 8;  // 16-byte chunks per line
-    static constexpr int kLoads = kBytes / 16 / kThreads;                                    // per lane and slice
-    static constexpr uint32_t kOutOfRange = 0x80000000u, kRange = 0x7fffffffu;
-
-    // Where chunk `c` of line `line` sits among the line's chunks: the lines that a fragment takes one column of chunks from lie in
-    // different banks.
-    static __device__ __forceinline__ int swizzled(int line, int c) {
-        if constexpr (kContiguousK) return c ^ ((line / (16 / kChunks)) & (kChunks - 1));
-        else return c ^ (((line & 3) << 2) & (kChunks - 1));
-    }
-
-    const char *start, *base;  // wave-uniform: the tile's first element; that of the next slice to fetch
-    int64_t step;              // bytes from one slice to the next
-    uint32_t offset[kLoads];   // per lane, bytes from `base`; out of range where the tile has no such line or column
-    int k[kLoads];             // of the load's first element in the slice
-    int k_count, k_left;       // of the reduction; from `base` on
-    int slices, next, unfetched;
-
-    // `stride`: bytes between lines. `valid`: rows (columns of the product) that exist, a multiple of 8 where they are not lines.
-    // `kPaired`: of every 64 lines the first 32 follow one another in memory and the last 32 lie `pair_distance` lines after those;
-    // `valid` of each.
-    template <bool kPaired>
-    __device__ __forceinline__ void setup(const char *first, int64_t stride, int valid, int k_count_, int first_slice, int wave, int lane,
-                                          int64_t pair_distance) {
-        static_assert(kContiguousK || !kPaired, "lines are rows");
-        start = uniform_pointer(first);
-        step = kContiguousK ? kBK * 2 : kBK * stride;
-        k_count = k_count_;
-        slices = unfetched = (k_count + kBK - 1) / kBK;
-        next = first_slice;
-        base = start + first_slice * step;
-        k_left = k_count - first_slice * kBK;
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const int slot = (wave * kLoads + j) * 64 + lane, line = slot / kChunks, chunk = swizzled(line, slot % kChunks);
-            const int single = kPaired ? line / 64 * 32 + line % 32 : line;
-            const bool exists = kContiguousK ? single < valid : chunk * 8 < valid;
-            const int64_t memory_line = kPaired && line % 64 >= 32 ? single + pair_distance : single;
-            offset[j] = exists ? static_cast<uint32_t>(memory_line * stride + chunk * 16) : kOutOfRange;
-            k[j] = kContiguousK ? chunk * 8 : line;
-        }
-    }
-
-    // The next slice -> the slot at LDS address `slot`: the last slice is followed by the first one, and when all have been fetched
-    // zeros come, without an access to memory. What lies past the reduction comes as zeros too.
-    __device__ __forceinline__ void fetch(int slot, int wave) {
-        const __amdgpu_buffer_rsrc_t resource = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<char *>(uniform_pointer(base)), 0, static_cast<int>(kRange), kBufferResourceFlags);
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const uint32_t lane_offset = k[j] < k_left ? offset[j] : kOutOfRange;
-            const int target = __builtin_amdgcn_readfirstlane(slot + (wave * kLoads + j) * 1024);
-            // M0 is not handed out by the register allocator and nothing else in this file uses it.
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                         :
-                         : "s"(target), "v"(lane_offset), "s"(resource)
-                         : "memory");
-        }
-        base += step;
-        ++next;
-        --unfetched;
-        if (next == slices) {
-            next = 0;
-            base = start;
-        }
-        k_left = unfetched > 0 ? k_count - next * kBK : 0;
-    }
-
-    // MFMA fragments (8 consecutive k of one row per lane; lane l: row l % 32, k half l / 32) of the 32 rows from `first` on, per lane:
-    // an address per step of 16 (K-contiguous; the next 32 rows and the slot are added), or one per 32 rows (the step is added).
-    static constexpr int kAddresses = kContiguousK ? kSteps : kBlocks;
-    static __device__ __forceinline__ void fragment_addresses(int first, int lane, int (&addresses)[kAddresses]) {
-        if constexpr (kContiguousK) {
-            const int row = first + (lane & 31);
-#pragma unroll
-            for (int s = 0; s < kSteps; ++s) addresses[s] = (row * kChunks + swizzled(row, 2 * s + (lane >> 5))) * 16;
-        } else {
-            const int s = lane & 15, group = lane >> 4, k = ((group >> 1) << 3) + (s >> 2);
-#pragma unroll
-            for (int i = 0; i < kBlocks; ++i) {
-                const int column = first + i * 32 + ((group & 1) << 4) + ((s & 3) << 2);
-                addresses[i] = k * kTile * 2 + swizzled(k, column >> 3) * 16 + (column & 7) * 2;
-            }
-        }
-    }
-    static __device__ __forceinline__ u32x4_t fragment(const int (&addresses)[kAddresses], int slot, int i, int step) {
-        if constexpr (kContiguousK) {
-            return *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(addresses[step] + slot + i * 32 * kChunks * 16);
-        } else {
-            const uintptr_t at = static_cast<uintptr_t>(addresses[i] + slot + step * 16 * kTile * 2);
-            const i16x4_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FM_LDS(i16x4_t) *)at);
-            const i16x4_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FM_LDS(i16x4_t) *)(at + 4 * kTile * 2));
-            const u32x2_t low_words = __builtin_bit_cast(u32x2_t, low), high_words = __builtin_bit_cast(u32x2_t, high);
-            return u32x4_t{low_words[0], low_words[1], high_words[0], high_words[1]};
-        }
-    }
-};
-
-// Returns once at most `kNewest` of the loads this wavefront has issued are still on their way, and all that it has asked LDS for is
-// there: after a barrier the others' loads may replace what it read.
-template <int kNewest>
-__device__ __forceinline__ void wait_for_loads() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kNewest) : "memory");
-}
+constexpr int kTileM = 128, kTileN = 64, kThreads = kLoadingThreads;
+// 2 x 2 wavefronts, 32 x 32 accumulators. With the gated activation the columns are 32 gates and 32 ups, which one wavefront has to have
+// both of: 4 x 1.
+template <bool kGated>
+constexpr int kWavesN = kGated ? 1 : 2;
+template <bool kGated>
+constexpr int kBlocksM = kTileM / 32 * kWavesN<kGated> / 4;
+template <bool kGated>
+constexpr int kBlocksN = kTileN / 32 / kWavesN<kGated>;
 
 // value(i, j, v), of 32 x 32 accumulators -> rows of `out`, 32 rows of the wavefront's columns at a time through its own part of LDS: 16
 // bytes per lane and store. The tile's rows are the MFMA's columns: a lane's four accumulators are consecutive columns of one row.
@@ -187,21 +66,17 @@ __device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, i
     }
 }
 
-template <int kTileN>
-constexpr int kStages = kTileN == 128 ? 2 : 3;
-template <int kTileN>
-constexpr int kWorkgroups = kTileN == 256 ? 1 : 2;  // per CU
-template <int kTileN>
-constexpr int kLdsBytes = kStages<kTileN> * (kTileM + kTileN) * kBK * 2;
+constexpr int kStages = 3, kWorkgroups = 2;  // slices in LDS, workgroups per CU
+constexpr int kLdsBytes = kStages * (kTileM + kTileN) * kBK * 2;
 
-template <typename T, int kTileN, bool kRhsK, bool kGated>
-__global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
-    constexpr int kBlocksM = few_tiles::kBlocksM<kTileN, kGated>, kBlocksN = few_tiles::kBlocksN<kTileN, kGated>;
+template <typename T, bool kRhsK, bool kGated>
+__global__ __launch_bounds__(kThreads, kWorkgroups) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
+    constexpr int kBlocksM = few_tiles::kBlocksM<kGated>, kBlocksN = few_tiles::kBlocksN<kGated>;
     typedef Operand<kTileM, true, kBlocksM> Lhs;
     typedef Operand<kTileN, kRhsK, kBlocksN> Rhs;
     constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
     constexpr int kColumns = kGated ? kTileN / 2 : kTileN;  // of the result
-    static_assert(kLdsBytes<kTileN> * kWorkgroups<kTileN> <= 160 * 1024 && kLdsBytes<kTileN> >= 4 * 32 * (kTileN + 16), "LDS of a CU");
+    static_assert(kLdsBytes * kWorkgroups <= 160 * 1024 && kLdsBytes >= 4 * 32 * (kTileN + 16), "LDS of a CU");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
     const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
 
@@ -221,7 +96,7 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
     const int first_slice = __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert));
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wave_m = wave / kWavesN<kTileN, kGated>, wave_n = wave % kWavesN<kTileN, kGated>;
+    const int wave_m = wave / kWavesN<kGated>, wave_n = wave % kWavesN<kGated>;
     Lhs lhs;
     Rhs rhs;
     lhs.template setup<false>(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row0 * args.lhs_stride_row),
@@ -244,12 +119,12 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
     const auto fetch_slice = [&]() {
         lhs.fetch(lds + fetch_slot, wave);
         rhs.fetch(lds + fetch_slot + Lhs::kBytes, wave);
-        fetch_slot = fetch_slot == (kStages<kTileN> - 1) * kSlotBytes ? 0 : fetch_slot + kSlotBytes;
+        fetch_slot = fetch_slot == (kStages - 1) * kSlotBytes ? 0 : fetch_slot + kSlotBytes;
     };
     // The oldest slice under way is there, for all wavefronts, and the slot of the slice before it is filled anew: its last fragments
     // have been read.
     const auto next_slice = [&]() {
-        wait_for_loads<(kStages<kTileN> - 2) * kLoads>();
+        wait_for_loads<(kStages - 2) * kLoads>();
         __syncthreads();
         fetch_slice();
     };
@@ -261,13 +136,13 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
         for (int j = 0; j < kBlocksN; ++j) b[buffer][j] = Rhs::fragment(rhs_addresses, slot + Lhs::kBytes, j, step);
     };
 #pragma unroll
-    for (int s = 0; s < kStages<kTileN> - 1; ++s) fetch_slice();
+    for (int s = 0; s < kStages - 1; ++s) fetch_slice();
     next_slice();
     int slot = lds;
     read(0, slot, 0);
     static_assert(kSteps % 2 == 0, "fragment buffers alternate");
     for (int t = 0; t < num_slices; ++t) {
-        const int next_slot = slot == lds + (kStages<kTileN> - 1) * kSlotBytes ? lds : slot + kSlotBytes;
+        const int next_slot = slot == lds + (kStages - 1) * kSlotBytes ? lds : slot + kSlotBytes;
 #pragma unroll
         for (int step = 0; step < kSteps; ++step) {
             const bool last = step + 1 == kSteps;
@@ -310,49 +185,38 @@ __global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_fe
 // Tiles of 128 x 256, by the upper bound that the host knows of their row tiles (a static map has one tile of padding per expert).
 static int64_t most_tiles(const GemmArgs &args) { return (args.rows + kTileM - 1) / kTileM * ((args.cols + 255) / 256); }
 
-template <typename T, int kTileN, bool kRhsK, bool kGated = false>
+template <typename T, bool kRhsK, bool kGated = false>
 static int launch(const GemmArgs &args, hipStream_t stream) {
-    const auto kernel = grouped_gemm_few_tiles_kernel<T, kTileN, kRhsK, kGated>;
+    const auto kernel = grouped_gemm_few_tiles_kernel<T, kRhsK, kGated>;
     static std::atomic<uint64_t> configured{0};
-    if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes<kTileN>, configured)) return status;
+    if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n, round = 8 * static_cast<int64_t>(args.chunk_tiles);
-    kernel<<<static_cast<uint32_t>((tiles + round - 1) / round * round), kThreads, kLdsBytes<kTileN>, stream>>>(args);
+    kernel<<<static_cast<uint32_t>((tiles + round - 1) / round * round), kThreads, kLdsBytes, stream>>>(args);
     return FM_OK;
 }
 
-template <typename T, int kTileN>
+template <typename T>
 static int launch(GemmArgs args, hipStream_t stream) {
     args.tiles_m = static_cast<int>((args.rows + kTileM - 1) / kTileM + (args.num_experts > 1 ? args.num_experts : 0));
     args.tiles_n = static_cast<int>((args.cols + kTileN - 1) / kTileN);
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n;
     if (tiles >= (int64_t(1) << 30)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
-    // Runs of 16 tiles per XCD; 8 and 32 are up to 3 and 5 % slower (128 columns).
+    // Runs of 16 tiles per XCD.
     args.chunk_tiles = static_cast<int>(min(int64_t(16), (tiles + 7) / 8));
-    if (args.fusion == kFusionGatedForward) return launch<T, kTileN, true, true>(args, stream);
-    return args.rhs_stride_inner == 1 ? launch<T, kTileN, true>(args, stream) : launch<T, kTileN, false>(args, stream);
+    if (args.fusion == kFusionGatedForward) return launch<T, true, true>(args, stream);
+    return args.rhs_stride_inner == 1 ? launch<T, true>(args, stream) : launch<T, false>(args, stream);
 }
 
 }  // namespace few_tiles
 
-// Where the lines lie. Over 240 layers of random shapes (4 to 1100 rows per expert, experts equally and unequally liked, sizes that are
-// whole slices and that are not), weights in memory and activations in cache, the time of 256 x 256 tiles divided by that of 64, 128 and
-// 256 columns, geometric means (and the worst), by most_tiles:
-//       up to 64       2.00 (1.85), 1.46, 1.27
-//       65 .. 96       1.74 (1.10), 1.44 (1.19), 1.20
-//       97 .. 160      1.28 (0.95), 1.40 (1.10), 1.23 (0.99)
-//       161 .. 192     1.08, 1.16 (0.99), 1.16 (1.01)
-//       193 .. 256     0.98, 1.09 (0.96), 1.16 (1.00)
-//       257 .. 320     0.95, 1.08 (0.71), 1.13 (0.73): two rounds where 256 x 256 tiles take one
-//       more           0.90, 0.98 (0.66), 1.02 (0.74)
-// The line between 64 and 128 columns, over 1200 products more, activations not in cache either:
-//       65 .. 80       1.36, 1.19, 1.11
-//       81 .. 96       1.34, 1.28, 1.16
-//       97 .. 112      1.18, 1.20, 1.11
-//       113 .. 160     1.16, 1.18, 1.13
-// Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87), 1.03 (0.63), 0.88 (0.52) up to 96, and no better
-// with more: they stay there.
-// With the gated activation against fused tiles of 256 x 256, layer 1 of 300 tokens of 8 experts of 4096 x 1536 (2 each) 78 -> 66 us, of
-// 800 of 8 of 1536 x 512 (6 each) 45 -> 31.
+// Where the line lies. Over 240 layers of random shapes (4 to 1100 rows per expert, experts equally and unequally liked, sizes that are
+// whole slices and that are not), weights in memory and activations in cache, the time of 256 x 256 tiles divided by that of these,
+// geometric means (and the worst), by most_tiles: up to 64 2.00 (1.85), 65 .. 96 1.74 (1.10), 97 .. 160 1.28 (0.95), 161 .. 192 1.08, more
+// 0.98 and less. Above 96 the kernel that streams weights takes those that it can, 1.0 to 1.2 times as fast as tiles of 128 or 256 columns
+// here (inference of 40 to 200 rows for each of 8 experts of 1024 x 2816 1.24 to 1.34, of 4096 x 1536 1.10 to 1.14); up to 96 it is no
+// faster, with 64 columns either (0.98 to 1.02).
+// Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87) up to 96, and no better with more: they stay there.
+// With the gated activation against fused tiles of 256 x 256, layer 1 of 800 tokens of 8 experts of 1536 x 512 (6 each) 45 -> 31 us.
 bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     if (dtype == FM_DTYPE_F32 || args.mode == kInputRowSparse || args.accumulate || args.out_dtype != dtype || args.lhs_stride_inner != 1 ||
         splits)
@@ -364,16 +228,8 @@ bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     return few_tiles::most_tiles(args) <= 256;
 }
 
-template <typename T>
-static int launch_few_tiles(const GemmArgs &args, hipStream_t stream) {
-    const int64_t tiles = few_tiles::most_tiles(args);
-    return tiles <= 96    ? few_tiles::launch<T, 64>(args, stream)
-           : tiles <= 160 ? few_tiles::launch<T, 128>(args, stream)
-                          : few_tiles::launch<T, 256>(args, stream);
-}
-
 int few_tiles_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream) {
-    return dtype == FM_DTYPE_BF16 ? launch_few_tiles<bf16_t>(args, stream) : launch_few_tiles<f16_t>(args, stream);
+    return dtype == FM_DTYPE_BF16 ? few_tiles::launch<bf16_t>(args, stream) : few_tiles::launch<f16_t>(args, stream);
 }
 
 }  // namespace fm

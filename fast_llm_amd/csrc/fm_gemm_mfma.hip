@@ -1575,7 +1575,8 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
             const bool eligible = args.fusion == kFusionNone ? mfma_gemm_eligible(args, dtype) : mfma_gemm_fusion_eligible(args, dtype);
             if (!eligible || row_panel_gemm_chosen(args, dtype) || row_sparse_gemm_chosen(args, dtype)) continue;
             if (!table_space(args, space) || !wants_table(args, space.split)) continue;
-            if (few_tiles_gemm_chosen(args, dtype, space.split) || space.split != split_ones) continue;
+            if (weight_stream_gemm_chosen(args, dtype, space.split) || few_tiles_gemm_chosen(args, dtype, space.split)) continue;
+            if (space.split != split_ones) continue;
             if (split_ones && at == 0) at = kPartialBytes;
             args.partials = space.split ? static_cast<float *>(workspace) : nullptr;
             args.tile_table = static_cast<char *>(workspace) + at + sizeof(TableHeader);
@@ -1606,6 +1607,7 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
             return fail(FM_ERR_INVALID_ARGUMENT, "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
                         workspace_size, workspace);
         if (row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
+        if (weight_stream_gemm_chosen(args, dtype, splits_last_round(args))) return weight_stream_gemm_launch(args, dtype, stream);
         if (few_tiles_gemm_chosen(args, dtype, splits_last_round(args))) return few_tiles_gemm_launch(args, dtype, stream);
         if (split) args.partials = static_cast<float *>(workspace);
         if (workspace != nullptr && wants_table(args, split)) {

@@ -1,0 +1,74 @@
+"""Products with the weights of experts of few rows: small whole numbers, whose sums are exact in any order."""
+
+import pytest
+import torch
+
+from fast_llm_amd.functional.config import ActivationType, KernelConfig
+from fast_llm_amd.functional.sparse_linear import input_inner_sparse_matmul, output_sparse_matmul
+from fast_llm_amd.layers.moe import DroplessMoEMLP
+from tests.helpers import fixture_sparse_map, to_device_map
+
+pytestmark = pytest.mark.gpu
+
+# Around the ends of a wavefront's rows (64) and of a tile (128).
+_TOKENS = [0, 1, 31, 33, 64, 65, 96, 127, 128, 129, 192, 200, 256, 257, 320, 0]
+
+
+def _map(experts):
+    tokens = [_TOKENS[e % len(_TOKENS)] if e < 48 else e % 7 for e in range(experts)]
+    ends, used = [], 0
+    for count in tokens:
+        used += -(-count // 128) * 128
+        ends.append(used)
+    return fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": tokens})
+
+
+# Reductions of one slice, of no whole slice, of two and of several; columns of one tile and of a remainder.
+@pytest.mark.parametrize(
+    ("experts", "inner", "columns"),
+    [(256, 64, 1288), (128, 8, 1544), (70, 72, 2056), (64, 128, 2304), (33, 392, 4104), (128, 520, 1280)],
+)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_products_are_exact(experts, inner, columns, dtype, device):
+    oracle_map = _map(experts)
+    generator = torch.Generator(device).manual_seed(experts + inner + columns)
+
+    def whole(*shape):
+        return torch.randint(-2, 3, shape, generator=generator, device=device).to(dtype)
+
+    sparse_map = to_device_map(oracle_map, device, torch.int32)
+    x = whole(oracle_map.num_rows, inner)
+    by_column, by_row = whole(experts * columns, inner), whole(experts * inner, columns)
+    output = output_sparse_matmul(x, by_column.t(), sparse_map)
+    input_ = input_inner_sparse_matmul(x, by_row, sparse_map)
+    begin = 0
+    for expert in range(experts):
+        end = int(oracle_map.expert_ends[expert])
+        rows = x[begin:end].float()
+        expected = rows @ by_column[expert * columns : (expert + 1) * columns].float().t()
+        assert torch.equal(output[begin:end], expected.to(dtype)), expert
+        expected = rows @ by_row[expert * inner : (expert + 1) * inner].float()
+        assert torch.equal(input_[begin:end], expected.to(dtype)), expert
+        begin = end
+
+
+@pytest.mark.parametrize(("rows", "inner", "columns"), [(1, 64, 24840), (129, 200, 16392), (1601, 136, 2048), (3000, 64, 2568)])
+def test_dense_products_are_exact(rows, inner, columns, device):
+    generator = torch.Generator(device).manual_seed(rows)
+    x = torch.randint(-2, 3, (rows, inner), generator=generator, device=device).bfloat16()
+    for weight in (torch.empty(columns, inner, device=device).t(), torch.empty(inner, columns, device=device)):
+        weight = torch.randint_like(weight, -2, 3).bfloat16()
+        assert torch.equal(output_sparse_matmul(x, weight), (x.float() @ weight.float()).bfloat16())
+
+
+@pytest.mark.parametrize(("tokens", "ffn"), [(1000, 768), (1500, 1032), (2100, 200)])
+@pytest.mark.parametrize("activation", [ActivationType.silu, ActivationType.gelu])
+def test_activation_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
+    torch.manual_seed(tokens + ffn)
+    dtype = torch.float16 if ffn % 16 else torch.bfloat16
+    layer = DroplessMoEMLP(320, ffn, 128, 6, activation=activation, init_std=0.2, dtype=dtype, device=device).eval()
+    x = torch.randn(tokens, 320, device=device).to(dtype)
+    with torch.no_grad():
+        output = layer(x)
+        monkeypatch.setattr(KernelConfig, "fuse_activation", False)
+        assert torch.equal(output, layer(x))
