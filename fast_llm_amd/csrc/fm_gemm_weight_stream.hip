@@ -1,17 +1,23 @@
 // Products with expert weights that are bound by the rate at which those come from memory (some hundred rows per expert), or that have
-// few tiles, in half precision: 128 rows x 256, 192 or 128 columns (with the gated activation half of them gates, half ups).
+// few tiles, in half precision: 128 or 192 rows x 256, 192 or 128 columns (with the gated activation half of them gates, half ups).
 //
 // In the kernels where each wavefront loads, multiplies and stores, nothing is on its way while a tile is set up and written out, and a
 // launch of 1.1 rounds of tiles takes two. Here one workgroup per CU walks its tiles with
 //   * four wavefronts that only load, straight from memory into LDS, up to two slices of 64 along K ahead of the multiplications and
 //     on into the next tile: what is asked for does not depend on where a tile ends;
-//   * eight that multiply 64 x 64 of the tile each and store, and never wait for memory;
-//   * the width of the tiles chosen on the device, from the rows that the experts have, so that the last round is full (`Tiles`);
+//   * eight that multiply 64 x 64 or 96 x 64 of the tile each and store, and never wait for memory;
+//   * the tiles' width and height chosen on the device, from the rows that the experts have, so that the last round is full (`Tiles`);
 //   * tiles found from row counts in registers, without a table that a kernel in front has to write (5 to 9 us).
 // One GPU, us before and now: layer 1's product with 40 rows for each of 8 experts of 4096 x 14336 418 -> 384 (1.88 GB: 4.9 TB/s,
 // 5.3 without what a launch takes to start and end), of 16 of 4096 x 4096 201 -> 189 (5.7 TB/s); layer 2's for 80 rows of 16 of
-// 1280 x 3416 64 -> 55. What is on its way (64 KB of weights per CU) limits it: wider or taller tiles leave LDS for fewer slices.
+// 1280 x 3416 64 -> 55. What is on its way (64 KB of weights per CU) limits it.
+// Tall tiles are for experts of 100 rows and more, whose rows would be two tiles of 128, the second nearly empty, or one large one:
+// inference of 125 and 150 rows for each of 32 experts of 3000 x 1000 258 -> 210 and 271 -> 222 us, 250 390 -> 307; of 125 of 16 of 4096 x
+// 4096 382 -> 358; a training step of 375 of 16 of 1280 x 3416 842 -> 802. They leave LDS for two slices of the lhs, which mostly comes
+// from L2, and are 2 to 10 % slower where 128 rows would do.
 // Sums in fp32, in the order of the large tiles' kernel (fm_gemm_mfma.hip): the same bits.
+#include <cmath>
+#include <type_traits>
 #include "fm_activation_math.h"
 #include "fm_gemm_slices.h"
 
@@ -21,13 +27,24 @@ namespace weight_stream {
 
 using namespace slices;
 
-constexpr int kTileM = 128, kTileN = 256, kBlocks = 2;  // a wavefront multiplies 64 x 64, in 32 x 32 accumulators
+// Tiles have up to 128 rows, or (tall ones) up to 192. A wavefront multiplies half of the rows x 64, in 32 x 32 accumulators.
+template <bool kTall>
+constexpr int kTileM = kTall ? 192 : 128;
+template <bool kTall>
+constexpr int kBlocksM = kTileM<kTall> / 64;
+constexpr int kTileN = 256, kLeastWidth = 128, kBlocksN = 2;
 constexpr int kMultiplying = 8, kThreads = 64 * kMultiplying + kLoadingThreads;
 constexpr int kMaxExperts = 256, kExpertRegisters = kMaxExperts / 64;
 constexpr int kResident = 256;  // workgroups on the device at one time
 
 // LDS: slots for slices of both operands, a staging region per multiplying wavefront.
-constexpr int kSlots = 3, kSlotBytes = (kTileM + kTileN) * kBK * 2, kStagingAt = kSlots * kSlotBytes, kStagingBytes = 2048;
+template <bool kTall>
+constexpr int kLhsSlots = kTall ? 2 : 3;
+template <bool kTall>
+constexpr int kLhsBytes = kTileM<kTall> * kBK * 2;
+constexpr int kRhsSlots = 3, kRhsBytes = kTileN * kBK * 2, kRhsAt = kLhsSlots<true> * kLhsBytes<true>;
+static_assert(kRhsAt == kLhsSlots<false> * kLhsBytes<false>, "the same LDS for both heights");
+constexpr int kStagingAt = kRhsAt + kRhsSlots * kRhsBytes, kStagingBytes = 2048;
 constexpr int kLdsBytes = kStagingAt + kMultiplying * kStagingBytes;
 static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
 
@@ -36,18 +53,19 @@ struct Tile {
 };
 
 // The tiles of a workgroup. The experts' row counts stay in registers: a tile is found without waiting for memory.
-// The columns of a tile are those with which the launch is shortest, if a round takes as long as its columns and kWidthCost more (the
-// rows of the other operand, and what a tile takes besides): layer 2's input gradient of 40 rows of 128 experts of 2048 x 768 is 384
-// tiles of 256 columns, 1.5 rounds, or 512 of 192: 101.5 -> 95.9 us; layer 1's input gradient of 8 experts of 4096 x 14336 is 128 of
+// The columns and most rows of a tile are those with which the launch is shortest, if a round takes as long as its columns, half of its
+// mean rows (from L2, where the weights come from memory) and 16 more: layer 2's input gradient of 40 rows of 128 experts of 2048 x 768 is
+// 384 tiles of 256 columns, 1.5 rounds, or 512 of 192: 101.5 -> 95.9 us; layer 1's input gradient of 8 experts of 4096 x 14336 is 128 of
 // 256 or 256 of 128: 520 -> 370.
+template <bool kTall>
 struct Tiles {
-    static constexpr int kLeastWidth = 128, kWidthCost = 64;
+    static constexpr int kLeastHeight = 128, kHeight = kTileM<kTall>;
     int begin[kExpertRegisters], rows[kExpertRegisters], row_tiles_to[kExpertRegisters];  // of an expert per lane and register
-    int width, tiles_n, total, next;  // columns of a tile, tiles next to one another
+    int height, width, tiles_n, total, next;  // most rows of a tile, its columns, tiles next to one another
 
     // `columns`: of the weights of one expert.
     __device__ __forceinline__ void load(const GemmArgs &args, int columns, int lane) {
-        int row_tiles = 0;
+        int all_rows = 0, low = 0, high = 0;  // row tiles of the least height, and of the most
 #pragma unroll
         for (int i = 0; i < kExpertRegisters; ++i) {
             const int e = i * 64 + lane;
@@ -56,7 +74,34 @@ struct Tiles {
             else if (e < args.num_experts) rows_of_expert(args, e, first, end);
             begin[i] = static_cast<int>(first);
             rows[i] = static_cast<int>(max(end - first, static_cast<int64_t>(0)));
-            int inclusive = (rows[i] + kTileM - 1) / kTileM;
+            all_rows += rows[i];
+            low += (rows[i] + kLeastHeight - 1) / kLeastHeight;
+            high += (rows[i] + kHeight - 1) / kHeight;
+        }
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            all_rows += __shfl_xor(all_rows, offset, 64);
+            low += __shfl_xor(low, offset, 64);
+            high += __shfl_xor(high, offset, 64);
+        }
+        all_rows = __builtin_amdgcn_readfirstlane(all_rows);
+        int least = 0x7fffffff;
+        height = kLeastHeight;
+        width = kTileN;
+#pragma unroll
+        for (int h = kLeastHeight; h <= kHeight; h += 64) {
+            const int row_tiles = __builtin_amdgcn_readfirstlane(h == kLeastHeight ? low : high);
+            const int row_cost = (kTall ? all_rows / max(row_tiles, 1) : 96) / 2 + 16;
+#pragma unroll
+            for (int w = kTileN; w >= kLeastWidth; w -= 64) {
+                const int rounds = (row_tiles * ((columns + w - 1) / w) + kResident - 1) / kResident, cost = rounds * (w + row_cost);
+                if (cost < least) least = cost, height = h, width = w;
+            }
+        }
+        int row_tiles = 0;
+#pragma unroll
+        for (int i = 0; i < kExpertRegisters; ++i) {
+            int inclusive = (rows[i] + height - 1) / height;
 #pragma unroll
             for (int offset = 1; offset < 64; offset <<= 1) {
                 const int other = __shfl_up(inclusive, offset, 64);
@@ -64,13 +109,6 @@ struct Tiles {
             }
             row_tiles_to[i] = row_tiles + inclusive;
             row_tiles = __builtin_amdgcn_readlane(row_tiles_to[i], 63);
-        }
-        int least = 0x7fffffff;
-        width = kTileN;
-#pragma unroll
-        for (int w = kTileN; w >= kLeastWidth; w -= 64) {
-            const int rounds = (row_tiles * ((columns + w - 1) / w) + kResident - 1) / kResident, cost = rounds * (w + kWidthCost);
-            if (cost < least) least = cost, width = w;
         }
         tiles_n = (columns + width - 1) / width;
         total = row_tiles * tiles_n;
@@ -93,13 +131,19 @@ struct Tiles {
             if (later == 0) continue;
             found = true;
             const int owner = __ffsll(static_cast<unsigned long long>(later)) - 1;
-            const int expert_rows = __builtin_amdgcn_readlane(rows[i], owner), count = (expert_rows + kTileM - 1) / kTileM;
+            const int expert_rows = __builtin_amdgcn_readlane(rows[i], owner), count = (expert_rows + height - 1) / height;
             const int first = __builtin_amdgcn_readlane(row_tiles_to[i], owner) - count;
             int in_expert;
             place_in_expert(logical - first * tiles_n, count, tiles_n, in_expert, tile.tile_n);
             tile.expert = i * 64 + owner;
-            tile.row = __builtin_amdgcn_readlane(begin[i], owner) + in_expert * kTileM;
-            tile.rows_valid = min(kTileM, expert_rows - in_expert * kTileM);
+            int first_row = in_expert * kHeight, last_row = first_row + kHeight;
+            if constexpr (kTall) {  // tiles that differ by 32 rows at most
+                const int blocks = (expert_rows + 31) / 32;
+                first_row = in_expert * blocks / count * 32;
+                last_row = (in_expert + 1) * blocks / count * 32;
+            }
+            tile.row = __builtin_amdgcn_readlane(begin[i], owner) + first_row;
+            tile.rows_valid = min(last_row, expert_rows) - first_row;
         }
         return tile;
     }
@@ -107,9 +151,9 @@ struct Tiles {
 
 // value(i, j, v), of 32 x 32 accumulators -> rows of `out`, as many at a time as the wavefront's part of LDS takes: 16 bytes per lane and
 // store. The tile's rows are the MFMA's columns: a lane's four accumulators are consecutive columns of one row.
-template <typename T, int kColumnBlocks, typename Value>
-__device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, int64_t stride, int rows_valid, int cols_valid, int wave_m,
-                                           int wave_n, int lane) {
+template <typename T, int kRowBlocks, int kColumnBlocks, typename Value>
+__device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, int64_t stride, int rows_valid, int cols_valid, int first_row,
+                                           int blocks, int wave_n, int lane) {
     constexpr int kWaveCols = kColumnBlocks * 32, kRowBytes = kWaveCols * 2, kChunks = kWaveCols / 8;  // 16-byte chunks per row
     constexpr int kPassRows = kStagingBytes / kRowBytes, kRowsPerRead = 64 / kChunks, kReads = kPassRows / kRowsPerRead;
     // Where a chunk sits in its row: a column of chunks lies in different banks.
@@ -118,7 +162,8 @@ __device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, i
     };
     const int read_row = lane / kChunks, read_chunk = lane % kChunks, column = wave_n * kWaveCols + read_chunk * 8;
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
+    for (int i = 0; i < kRowBlocks; ++i) {
+        if (i >= blocks) continue;
         u32x2_t groups[kChunks];
 #pragma unroll
         for (int chunk = 0; chunk < kChunks; ++chunk) {
@@ -144,7 +189,7 @@ __device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, i
                 staged[t] = *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(address(read_row + t * kRowsPerRead, read_chunk));
 #pragma unroll
             for (int t = 0; t < kReads; ++t) {
-                const int row = (wave_m * kBlocks + i) * 32 + pass * kPassRows + t * kRowsPerRead + read_row;
+                const int row = first_row + i * 32 + pass * kPassRows + t * kRowsPerRead + read_row;
                 if (row < rows_valid && column < cols_valid)
                     __builtin_nontemporal_store(staged[t], reinterpret_cast<u32x4_t *>(out + row * stride + column));
             }
@@ -153,16 +198,16 @@ __device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, i
     }
 }
 
-template <typename T, bool kRhsK, bool kGated>
+template <typename T, bool kRhsK, bool kGated, bool kTall>
 __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_weight_stream_kernel(GemmArgs args) {
-    typedef Operand<kTileM, true, kBlocks> Lhs;
-    typedef Operand<kTileN, kRhsK, kBlocks> Rhs;
-    constexpr int kLoads = Lhs::kLoads + Rhs::kLoads;
-      static_assert(Lhs::kBytes + Rhs::kBytes == kSlotBytes, "a slot");
+    constexpr int kBlocksM = weight_stream::kBlocksM<kTall>, kLhsSlots = weight_stream::kLhsSlots<kTall>, kLhsBytes = weight_stream::kLhsBytes<kTall>;
+    typedef Operand<kTileM<kTall>, true, kBlocksM> Lhs;
+    typedef Operand<kTileN, kRhsK, kBlocksN> Rhs;
+    static_assert(Lhs::kBytes == kLhsBytes && Rhs::kBytes == kRhsBytes, "slots");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
     const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    Tiles tiles;
+    Tiles<kTall> tiles;
     tiles.load(args, static_cast<int>(kGated ? 2 * args.half : args.cols), lane);
     const int k_count = static_cast<int>(args.inner), num_slices = (k_count + kBK - 1) / kBK;
     const int num_tiles = tiles.left();
@@ -171,136 +216,187 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_weight_stream_kernel
     const auto cols_valid = [&](const Tile &tile) {
         return static_cast<int>(min(static_cast<int64_t>(columns), (kGated ? args.half : args.cols) - static_cast<int64_t>(tile.tile_n) * columns));
     };
+    const auto next_slot = [&](int slot, int first, int bytes, int count) { return slot == first + (count - 1) * bytes ? first : slot + bytes; };
 
-    // The slices of the workgroup's tiles pass through the slots one after the other, number s through slot s % kSlots. Barrier s makes
-    // slice s visible (the loading wavefronts have waited for their loads of it) and ends the reads of slice s - 1, whose slot
-    // slice s + kSlots - 1 then fills.
+    // The slices of the workgroup's tiles pass through the slots one after the other, number s through slots s % kLhsSlots and s %
+    // kRhsSlots. Barrier s makes slice s visible (the loading wavefronts have waited for their loads of it) and ends the reads of slice
+    // s - 1, whose slots slices s + kLhsSlots - 1 of the lhs, which mostly comes from L2, and s + kRhsSlots - 1 of the weights then fill.
     if (wave >= kMultiplying) {
         const int part = wave - kMultiplying, total = num_tiles * num_slices;
+        constexpr bool kApart = kLhsSlots < kRhsSlots;  // the weights are a slice ahead of the lhs, and at most a tile
+        static_assert(kLhsSlots == kRhsSlots - kApart, "slices ahead");
         Lhs lhs;
         Rhs rhs;
-        int slot = lds, tiles_left = num_tiles, slices_left = 0;
-        // As soon as a tile's last slice has been asked for, long before the next tile's first one is.
-        const auto next_tile = [&]() {
-            const Tile tile = tiles.take();
+        int lhs_slot = lds, rhs_slot = lds + kRhsAt, lhs_tiles = num_tiles, rhs_tiles = num_tiles, lhs_slices = 0, rhs_slices = 0;
+        Tile tile{};  // of the weights
+        const auto next_weights = [&]() {
+            tile = tiles.take();
             const int64_t col0 = static_cast<int64_t>(tile.tile_n) * columns;
             const int64_t rhs_offset = args.mode == kOutputSparse
                                            ? (static_cast<int64_t>(tile.expert) * args.sparse_size + col0) * args.rhs_stride_col
                                            : static_cast<int64_t>(tile.expert) * args.sparse_size * args.rhs_stride_inner + col0 * args.rhs_stride_col;
-            const int first_slice = __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert));
-            lhs.template setup<false>(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row * args.lhs_stride_row),
-                                      args.lhs_stride_row * 2, tile.rows_valid, k_count, first_slice, part, lane, 0);
             rhs.template setup<kGated>(reinterpret_cast<const char *>(static_cast<const T *>(args.rhs) + rhs_offset),
-                                       (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 2, cols_valid(tile), k_count, first_slice,
-                                       part, lane, args.half);
-            --tiles_left;
-            slices_left = num_slices;
+                                       (kRhsK ? args.rhs_stride_col : args.rhs_stride_inner) * 2, cols_valid(tile), k_count,
+                                       __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert)), part, lane, args.half);
+            --rhs_tiles;
+            rhs_slices = num_slices;
         };
-        const auto fetch = [&]() {
-            // (After the last slice of the last tile: zeros.)
-            rhs.fetch(slot + Lhs::kBytes, part);
-            lhs.fetch(slot, part);
-            slot = slot == lds + (kSlots - 1) * kSlotBytes ? lds : slot + kSlotBytes;
-            if (--slices_left == 0 && tiles_left > 0) next_tile();
+        const auto next_lhs = [&]() {
+            lhs.template setup<false>(reinterpret_cast<const char *>(static_cast<const T *>(args.lhs) + tile.row * args.lhs_stride_row),
+                                      args.lhs_stride_row * 2, tile.rows_valid, k_count,
+                                      __builtin_amdgcn_readfirstlane(first_slice_of(args, tile.expert)), part, lane, 0);
+            --lhs_tiles;
+            lhs_slices = num_slices;
         };
-        next_tile();
+        // (After the last slice of the last tile: zeros.)
+        const auto fetch_lhs = [&]() {
+            lhs.fetch(lhs_slot, part);
+            lhs_slot = next_slot(lhs_slot, lds, kLhsBytes, kLhsSlots);
+            --lhs_slices;
+        };
+        const auto fetch_weights = [&]() {
+            rhs.fetch(rhs_slot, part);
+            rhs_slot = next_slot(rhs_slot, lds + kRhsAt, kRhsBytes, kRhsSlots);
+            --rhs_slices;
+        };
+        // The next tile as soon as the last slice of one has been asked for, long before its own first one is. The tile that the lhs goes on
+        // to is the one of the weights, which are ahead of it or go on with it. (One loop, the first slices too: what is executed once
+        // comes from memory, and a launch of 60 us gets 4 us longer with this set-up inlined three times.)
 #pragma unroll 1
-        for (int s = 0; s < kSlots - 1; ++s) fetch();
-#pragma unroll 1
-        for (int s = 0; s <= total; ++s) {
-            wait_for_loads<(kSlots - 2) * kLoads>();
-            __syncthreads();
-            fetch();
+        for (int s = 1 - kRhsSlots; s <= total; ++s) {
+            const bool lhs_too = !kApart || s > 1 - kRhsSlots;
+            if (kApart && lhs_too && lhs_slices == 0 && lhs_tiles > 0) next_lhs();
+            if (rhs_slices == 0 && rhs_tiles > 0) next_weights();
+            if (!kApart && lhs_slices == 0 && lhs_tiles > 0) next_lhs();
+            if (s >= 0) {
+                wait_for_loads<Rhs::kLoads + (kApart ? 0 : Lhs::kLoads)>();
+                __syncthreads();
+            }
+            if (lhs_too) fetch_lhs();
+            fetch_weights();
         }
         wait_for_loads<0>();
         return;
     }
 
+    // The lower wavefronts have the first 64 rows, half of the blocks of 32 where there are more than 128, the upper ones the rest.
     const int wave_m = wave / 4, wave_n = wave % 4;
     int lhs_addresses[Lhs::kAddresses], rhs_addresses[Rhs::kAddresses];
-    Lhs::fragment_addresses(wave_m * kBlocks * 32, lane, lhs_addresses);
-    Rhs::fragment_addresses(wave_n * kBlocks * 32, lane, rhs_addresses);
-    u32x4_t a[2][kBlocks], b[2][kBlocks];
-    const auto read = [&](int buffer, int slot, int step) {
+    Lhs::fragment_addresses(0, lane, lhs_addresses);
+    Rhs::fragment_addresses(wave_n * kBlocksN * 32, lane, rhs_addresses);
+    const auto blocks_of = [&](const Tile &tile) { return kTall ? max((tile.rows_valid + 63) / 64, 2) : 2; };
+    u32x4_t a[2][kBlocksM], b[2][kBlocksN];
+    int lhs_slot = lds, rhs_slot = lds + kRhsAt, lhs_row = 0;  // lhs_row: the wavefront's first, in bytes
+    const auto read = [&](auto blocks, int buffer, int step) {
 #pragma unroll
-        for (int i = 0; i < kBlocks; ++i) a[buffer][i] = Lhs::fragment(lhs_addresses, slot, i, step);
+        for (int i = 0; i < blocks; ++i) a[buffer][i] = Lhs::fragment(lhs_addresses, lhs_slot + lhs_row, i, step);
 #pragma unroll
-        for (int j = 0; j < kBlocks; ++j) b[buffer][j] = Rhs::fragment(rhs_addresses, slot + Lhs::kBytes, j, step);
+        for (int j = 0; j < kBlocksN; ++j) b[buffer][j] = Rhs::fragment(rhs_addresses, rhs_slot, j, step);
     };
-    int slot = lds;
-    const auto following = [&]() { return slot == lds + (kSlots - 1) * kSlotBytes ? lds : slot + kSlotBytes; };
+    const auto advance = [&]() {
+        lhs_slot = next_slot(lhs_slot, lds, kLhsBytes, kLhsSlots);
+        rhs_slot = next_slot(rhs_slot, lds + kRhsAt, kRhsBytes, kRhsSlots);
+    };
     static_assert(kSteps % 2 == 0, "fragment buffers alternate");
+    constexpr std::integral_constant<int, kBlocksM> all{};
+    Tile tile, upcoming = tiles.take();
+    const auto start_row = [&](const Tile &of) { return wave_m * blocks_of(of) * 32 * kBK * 2; };
+    lhs_row = start_row(upcoming);
     __syncthreads();
-    read(0, slot, 0);
+    read(all, 0, 0);
 #pragma unroll 1
     for (int n = 0; n < num_tiles; ++n) {
-        const Tile tile = tiles.take();
-        if (wave_m * kBlocks * 32 >= tile.rows_valid || wave_n * kBlocks * 32 >= tiles.width) {  // nothing of the wavefront's exists
+        tile = upcoming;
+        if (n + 1 < num_tiles) upcoming = tiles.take();
+        const int tile_blocks = blocks_of(tile);
+        f32x16_t acc[kBlocksM][kBlocksN];
+#pragma unroll
+        for (int i = 0; i < kBlocksM; ++i)
+#pragma unroll
+            for (int j = 0; j < kBlocksN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+        const auto multiply_tile = [&](auto blocks) {
+#pragma unroll 1
+            for (int t = 0; t < num_slices; ++t) {
+#pragma unroll
+                for (int step = 0; step < kSteps; ++step) {
+                    const bool last = step + 1 == kSteps;
+                    if (last) {
+                        __syncthreads();
+                        advance();
+                        if (t + 1 == num_slices) lhs_row = start_row(upcoming);
+                        // (After the last slice of the last tile zeros are read, and not multiplied.)
+                        read(all, (step + 1) & 1, 0);
+                    } else {
+                        read(blocks, (step + 1) & 1, step + 1);
+                    }
+#pragma unroll
+                    for (int i = 0; i < blocks; ++i)
+#pragma unroll
+                        for (int j = 0; j < kBlocksN; ++j) acc[i][j] = mfma(T(), b[step & 1][j], a[step & 1][i], acc[i][j]);
+                }
+            }
+        };
+        if (wave_m * tile_blocks * 32 >= tile.rows_valid || wave_n * kBlocksN * 32 >= tiles.width) {  // nothing of the wavefront's exists
 #pragma unroll 1
             for (int t = 0; t < num_slices; ++t) {
                 __syncthreads();
-                slot = following();
+                advance();
             }
-            read(0, slot, 0);
+            lhs_row = start_row(upcoming);
+            read(all, 0, 0);
             continue;
         }
-        f32x16_t acc[kBlocks][kBlocks];
-#pragma unroll
-        for (int i = 0; i < kBlocks; ++i)
-#pragma unroll
-            for (int j = 0; j < kBlocks; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-#pragma unroll 1
-        for (int t = 0; t < num_slices; ++t) {
-            const int next_slot = following();
-#pragma unroll
-            for (int step = 0; step < kSteps; ++step) {
-                const bool last = step + 1 == kSteps;
-                if (last) __syncthreads();
-                // (After the last slice of the last tile zeros are read, and not multiplied.)
-                read((step + 1) & 1, last ? next_slot : slot, last ? 0 : step + 1);
-#pragma unroll
-                for (int i = 0; i < kBlocks; ++i)
-#pragma unroll
-                    for (int j = 0; j < kBlocks; ++j) acc[i][j] = mfma(T(), b[step & 1][j], a[step & 1][i], acc[i][j]);
-            }
-            slot = next_slot;
-        }
-        const int staging = lds + kStagingAt + wave * kStagingBytes, valid = cols_valid(tile);
+        if (!kTall || tile_blocks == 2) multiply_tile(std::integral_constant<int, 2>{});
+        else multiply_tile(all);
+        const int staging = lds + kStagingAt + wave * kStagingBytes, valid = cols_valid(tile), first_row = wave_m * tile_blocks * 32;
         const int64_t col0 = static_cast<int64_t>(tile.tile_n) * columns;
         if constexpr (kGated) {
             // From the rounded values, as the activation's own kernel computes: the same bits.
             T *out = static_cast<T *>(args.fused_out) + tile.row * args.fused_stride + col0;
             const auto store = [&](auto activate) {
-                store_tile<T, 1>(
+                store_tile<T, kBlocksM, 1>(
                     [&](int i, int, int v) {
                         return activate(to_float(from_float<T>(acc[i][0][v]))) * to_float(from_float<T>(acc[i][1][v]));
                     },
-                    staging, out, args.fused_stride, tile.rows_valid, valid, wave_m, wave_n, opaque(lane));
+                    staging, out, args.fused_stride, tile.rows_valid, valid, first_row, tile_blocks, wave_n, opaque(lane));
             };
             FM_DISPATCH_ACTIVATION(args.activation, kActivation, store([](float x) { return activation_forward<kActivation>(x); }));
         } else {
             T *out = static_cast<T *>(args.out) + tile.row * args.out_stride_row + col0;
-            store_tile<T, 2>([&](int i, int j, int v) { return acc[i][j][v]; }, staging, out, args.out_stride_row, tile.rows_valid, valid,
-                             wave_m, wave_n, opaque(lane));
+            store_tile<T, kBlocksM, 2>([&](int i, int j, int v) { return acc[i][j][v]; }, staging, out, args.out_stride_row, tile.rows_valid, valid,
+                             first_row, tile_blocks, wave_n, opaque(lane));
         }
     }
 }
 
-template <typename T, bool kRhsK, bool kGated>
+template <typename T, bool kRhsK, bool kGated, bool kTall>
 static int launch(const GemmArgs &args, hipStream_t stream) {
-    const auto kernel = grouped_gemm_weight_stream_kernel<T, kRhsK, kGated>;
+    const auto kernel = grouped_gemm_weight_stream_kernel<T, kRhsK, kGated, kTall>;
     static std::atomic<uint64_t> configured{0};
     if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
     kernel<<<kResident, kThreads, kLdsBytes, stream>>>(args);
     return FM_OK;
 }
 
+template <typename T, bool kTall>
+static int launch(const GemmArgs &args, hipStream_t stream) {
+    if (args.fusion == kFusionGatedForward) return launch<T, true, true, kTall>(args, stream);
+    return args.rhs_stride_inner == 1 ? launch<T, true, false, kTall>(args, stream) : launch<T, false, false, kTall>(args, stream);
+}
+
+// Tiles of 128 rows where most experts have no more (the host knows rows with up to 128 of padding per expert), and where the expected
+// ones, half of the padding taken off, are one round.
+static bool low_tiles(const GemmArgs &args) {
+    constexpr int64_t kMostRowsOfLowTiles = 228;
+    const int64_t experts = args.num_experts;
+    return args.rows <= kMostRowsOfLowTiles * experts || (args.rows - 64 * experts) * ((args.cols + kTileN - 1) / kTileN) <= kResident * 128;
+}
+
 template <typename T>
 static int launch(const GemmArgs &args, hipStream_t stream) {
-    if (args.fusion == kFusionGatedForward) return launch<T, true, true>(args, stream);
-    return args.rhs_stride_inner == 1 ? launch<T, true, false>(args, stream) : launch<T, false, false>(args, stream);
+    return low_tiles(args) ? launch<T, false>(args, stream) : launch<T, true>(args, stream);
 }
 
 }  // namespace weight_stream
@@ -325,10 +421,47 @@ static int launch(const GemmArgs &args, hipStream_t stream) {
 // (those below 1 up to 256 tiles with the other product on large tiles instead of few). With both here, which also saves the launch that
 // writes the tables, the whole layer is 1.07 to 1.27 times as fast below 100 rows, 1.0 to 1.2 from 100 to 199. Whole training steps of
 // 64 rows: 1.01 (128 experts of 2048 x 768) to 1.14 (16 of 1280 x 3416). The host knows rows with up to 128 of padding per expert.
-// With more rows than the first of the rules below allows, those whose expected tiles (half of the padding taken off) are one round:
-// 1.04 (.95) to 1.17 with 200 to 256 tiles; 0.96 (.80) with 257 to 400.
+// With more than 228 rows in the buffer those whose expected tiles of 128 rows (half of the padding taken off) are one round: 1.04
+// (.95) to 1.17 with 200 to 256 tiles; 0.96 (.80) with 257 to 400.
+// Tall tiles: 350 layers of 100 to 800 rows, the time with large tiles over the time with one product here, by the cost (`Tiles`) of the
+// tiles here per round of 256 x 256 ones, experts equally liked (unequally):
+//            up to 200     .. 260        .. 300        .. 340        .. 380        .. 420        .. 460        .. 540        more
+//   layer 1  0.97 (1.01)   1.00 (1.06)   1.09 (1.07)   1.05 (1.03)   1.05 (1.04)   1.02 (1.03)   1.00 (1.02)   0.99 (1.03)   0.96 (1.02)
+//   layer 2  1.01 (1.00)   0.98 (1.03)   1.04 (1.02)   1.01 (1.00)   0.99 (1.00)   0.99 (0.99)   0.99 (1.00)   0.99 (1.00)   0.98 (0.99)
+// Reductions of no whole slices are masked in the large tiles' kernel: a step of 375 rows of 16 experts of 1280 x 3416, where layer 2
+// and layer 1's input gradient cost 350, takes 830 -> 808 us with them here.
 // Reductions that the large tiles' kernel splits into pieces (`splits`): 0.87 to 0.91 with 260 rows for each of 8 experts of 4096 x
 // 14336, 0.99 (1.25 with some experts preferred) with 180.
+namespace weight_stream {
+
+// Row tiles of `height` rows, if tokens choose experts independently, all alike: a fifth of the experts each has rows of that many
+// standard deviations from the mean. (A map's buffer has room for 128 rows of padding per expert.)
+static float expected_row_tiles(const GemmArgs &args, int height) {
+    const float rows = fmaxf(static_cast<float>(args.rows) / args.num_experts - (args.expert_ends != nullptr ? 128.f : 0.f), 1.f);
+    float tiles = 0.f;
+    for (const float deviations : {-1.4f, -0.53f, 0.f, 0.53f, 1.4f})
+        tiles += ceilf(fmaxf(rows + (args.num_experts > 1 ? deviations * sqrtf(rows) : 0.f), 1.f) / height);
+    return args.num_experts * tiles / 5.f;
+}
+
+// What `Tiles` makes of them.
+static float expected_cost(const GemmArgs &args) {
+    const float rows = fmaxf(static_cast<float>(args.rows - (args.expert_ends != nullptr ? 128 * args.num_experts : 0)), 1.f);
+    float least = INFINITY;
+    for (int height = 128; height <= kTileM<true>; height += 64) {
+        const float row_tiles = expected_row_tiles(args, height);
+        for (int width = kTileN; width >= kLeastWidth; width -= 64)
+            least = fminf(least, ceilf(row_tiles * ((args.cols + width - 1) / width) / kResident) * (width + rows / (2 * row_tiles) + 16));
+    }
+    return least;
+}
+
+static float expected_large_rounds(const GemmArgs &args) {
+    return ceilf(expected_row_tiles(args, 256) * ((args.cols + 255) / 256) / kResident);
+}
+
+}  // namespace weight_stream
+
 // `args` as `mfma_gemm_eligible` (or, with the activation, `mfma_gemm_fusion_eligible`) takes them.
 bool weight_stream_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     using namespace weight_stream;
@@ -339,14 +472,14 @@ bool weight_stream_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     if (args.fusion == kFusionGatedForward && (args.out != nullptr || (args.half + 128) * args.rhs_stride_col * 2 >= (int64_t(1) << 31)))
         return false;
     if (args.fusion == kFusionGatedBackward) return false;
-    const int64_t row_tiles = (args.rows + kTileM - 1) / kTileM, tiles_n = (args.cols + kTileN - 1) / kTileN, tiles = row_tiles * tiles_n;
+    const int64_t row_tiles = (args.rows + 127) / 128, tiles_n = (args.cols + kTileN - 1) / kTileN, tiles = row_tiles * tiles_n;
     const int64_t experts = args.num_experts;
-    if ((row_tiles + experts) * ((args.cols + Tiles::kLeastWidth - 1) / Tiles::kLeastWidth) >= (int64_t(1) << 30)) return false;
+    if ((row_tiles + experts) * ((args.cols + kLeastWidth - 1) / kLeastWidth) >= (int64_t(1) << 30)) return false;
     if (tiles <= 96 || (splits && args.rows > 320 * experts)) return false;
     const bool contiguous = args.rhs_stride_inner == 1;
-    if (args.rows <= (contiguous || tiles <= 1000 ? 228 : 180) * experts) return true;
-    if ((args.rows - 64 * experts) * tiles_n <= kResident * kTileM) return true;
-    return contiguous && tiles <= 1000 && args.rows <= 300 * experts;
+    if (low_tiles(args)) return contiguous || tiles <= 1000 || args.rows <= 180 * experts;
+    const int most = contiguous ? 440 : args.inner % kBK == 0 ? 320 : 360;
+    return expected_cost(args) <= most * expected_large_rounds(args);
 }
 
 int weight_stream_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream) {

@@ -10,12 +10,13 @@ from tests.helpers import fixture_sparse_map, to_device_map
 
 pytestmark = pytest.mark.gpu
 
-# Around the ends of a wavefront's rows (64) and of a tile (128).
-_TOKENS = [0, 1, 31, 33, 64, 65, 96, 127, 128, 129, 192, 200, 256, 257, 320, 0]
+# Around the ends of a wavefront's rows (64; 96 in tall tiles) and of a tile (128; 192).
+_FEW = [0, 1, 31, 33, 64, 65, 96, 127, 128, 129, 192, 200, 256, 257, 320, 0]
+_MORE = [0, 1, 63, 65, 95, 97, 128, 129, 160, 161, 191, 192, 193, 224, 256, 257, 320, 384, 385, 577]
 
 
-def _map(experts):
-    tokens = [_TOKENS[e % len(_TOKENS)] if e < 48 else e % 7 for e in range(experts)]
+def _map(experts, tall):
+    tokens = [_MORE[e % len(_MORE)] if tall else _FEW[e % len(_FEW)] if e < 48 else e % 7 for e in range(experts)]
     ends, used = [], 0
     for count in tokens:
         used += -(-count // 128) * 128
@@ -25,12 +26,15 @@ def _map(experts):
 
 # Reductions of one slice, of no whole slice, of two and of several; columns of one tile and of a remainder.
 @pytest.mark.parametrize(
-    ("experts", "inner", "columns"),
-    [(256, 64, 1288), (128, 8, 1544), (70, 72, 2056), (64, 128, 2304), (33, 392, 4104), (128, 520, 1280)],
-)
+    ("experts", "inner", "columns", "tall"),
+    [
+        (256, 64, 1288, False), (128, 8, 1544, False), (70, 72, 2056, False), (64, 128, 2304, False), (33, 392, 4104, False),
+        (128, 520, 1280, False), (40, 8, 1288, True), (64, 64, 1032, True), (20, 136, 2312, True), (40, 520, 3080, True),
+    ],
+)  # fmt: skip
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_products_are_exact(experts, inner, columns, dtype, device):
-    oracle_map = _map(experts)
+def test_products_are_exact(experts, inner, columns, tall, dtype, device):
+    oracle_map = _map(experts, tall)
     generator = torch.Generator(device).manual_seed(experts + inner + columns)
 
     def whole(*shape):
@@ -61,7 +65,7 @@ def test_dense_products_are_exact(rows, inner, columns, device):
         assert torch.equal(output_sparse_matmul(x, weight), (x.float() @ weight.float()).bfloat16())
 
 
-@pytest.mark.parametrize(("tokens", "ffn"), [(1000, 768), (1500, 1032), (2100, 200)])
+@pytest.mark.parametrize(("tokens", "ffn"), [(1000, 768), (1500, 1032), (2100, 200), (2900, 768), (3300, 1032)])
 @pytest.mark.parametrize("activation", [ActivationType.silu, ActivationType.gelu])
 def test_activation_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
     torch.manual_seed(tokens + ffn)
