@@ -11,6 +11,9 @@
 //     its lhs slices only, a third of the bytes. With more rows both operands pass through the slots.
 // 128 experts of 2048 x 768, 111 rows each: 269 and 137 us for the two gradients in tiles of 128 x 256, two workgroups per CU, 200 and 101
 // here: 4 TB/s of results.
+// What `out` holds, where the results are added to it, is asked for before a tile is multiplied, two of its four parts ahead: 125 rows of
+// 128 experts of 2048 x 768 562 -> 529 us for both gradients, of 8 of 4096 x 14336 1271 -> 1195 (preferred experts 615 -> 609 and 1366 ->
+// 1306); from 16 to 180 rows of six shapes 0.99 to 1.08 times as fast as with one part ahead, asked for after the multiplications.
 // A workgroup takes items of about the same time (`Items`), so that experts of many rows are spread over the device.
 // The order of a sum is that of a tile of 256 x 256: the results are the same bits.
 #include <atomic>
@@ -122,77 +125,89 @@ __device__ __forceinline__ void wait_for_loads() {
 constexpr int kRowBytes = 128 + 16, kStagingBytes = 32 * kRowBytes;
 
 template <typename T, bool kAccumulate>
-__device__ __forceinline__ void store_tile(const f32x16_t (&acc)[kBlocks][kBlocks], int staging, const char *out, int64_t stride,
-                                           int rows_valid, int cols_valid, int wave_m, int wave_n, int lane, bool streaming) {
+struct TileStore {
     typedef std::conditional_t<kAccumulate, float, T> StageT;
     typedef __attribute__((__vector_size__(4 * sizeof(StageT)))) uint32_t Group;
-    constexpr int kColumns = 128 / sizeof(StageT), kWide = kColumns / 32, kElements = 16 / sizeof(StageT);  // kWide accumulators side by side
+    static constexpr int kColumns = 128 / sizeof(StageT), kWide = kColumns / 32, kElements = 16 / sizeof(StageT);  // kWide accumulators side by side
     typedef __attribute__((__vector_size__(kElements * sizeof(T)))) uint32_t Chunk;
-    const __amdgpu_buffer_rsrc_t resource =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(uniform_pointer(out)), 0, 0x7fffffff, kBufferResourceFlags);
-    const int write_base = staging + (lane & 31) * kRowBytes + (lane >> 5) * 4 * sizeof(StageT);
-    const int read_base = staging + (lane >> 3) * kRowBytes + (lane & 7) * 16;
+    static constexpr int kRounds = kBlocks * kBlocks / kWide;
+
+    __amdgpu_buffer_rsrc_t resource;
+    int64_t stride;
+    int rows_valid, cols_valid, wave_m, wave_n, lane;
+    Chunk previous[2][4];
+
     // Rows and columns that do not exist are sent out of the buffer's range.
-    const auto offset_of = [&](int i, int first, int t) {
+    __device__ __forceinline__ int offset_of(int i, int first, int t) const {
         const int row = wave_m * 64 + i * 32 + t * 8 + (lane >> 3), column = (wave_n * kBlocks + first) * 32 + (lane & 7) * kElements;
         return row < rows_valid && column < cols_valid ? static_cast<int>((row * stride + column) * sizeof(T)) : static_cast<int>(0x80000000u);
-    };
-    constexpr int kRounds = kBlocks * kBlocks / kWide;
-    Chunk previous[2][4];
-    const auto request = [&](int round) {
+    }
+    __device__ __forceinline__ void request(int round) {
         const int i = round / (kBlocks / kWide), first = round % (kBlocks / kWide) * kWide;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             if constexpr (sizeof(Chunk) == 16) previous[round & 1][t] = __builtin_amdgcn_raw_buffer_load_b128(resource, offset_of(i, first, t), 0, 0);
             else previous[round & 1][t] = __builtin_amdgcn_raw_buffer_load_b64(resource, offset_of(i, first, t), 0, 0);
         }
-    };
-    if constexpr (kAccumulate) request(0);
-#pragma unroll
-    for (int round = 0; round < kRounds; ++round) {
-        const int i = round / (kBlocks / kWide), first = round % (kBlocks / kWide) * kWide;
-        if constexpr (kAccumulate)
-            if (round + 1 < kRounds) request(round + 1);
-#pragma unroll
-        for (int j = 0; j < kWide; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                struct {
-                    StageT v[4];
-                } group;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) group.v[c] = from_float<StageT>(acc[i][first + j][4 * g + c]);
-                *(FM_LDS(Group) *)static_cast<uintptr_t>(write_base + (j * 32 + 8 * g) * sizeof(StageT)) = __builtin_bit_cast(Group, group);
-            }
-        asm volatile("" ::: "memory");  // a wavefront's own LDS accesses are carried out in order
-        u32x4_t staged[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) staged[t] = *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(read_base + t * 8 * kRowBytes);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            Chunk values;
-            if constexpr (kAccumulate) {
-                struct {
-                    T v[4];
-                } sums = __builtin_bit_cast(decltype(sums), previous[round & 1][t]);
-                const f32x4_t added = __builtin_bit_cast(f32x4_t, staged[t]);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) sums.v[c] = from_float<T>(added[c] + to_float(sums.v[c]));
-                values = __builtin_bit_cast(Chunk, sums);
-            } else {
-                values = __builtin_bit_cast(Chunk, staged[t]);
-            }
-            const int offset = offset_of(i, first, t);
-            if constexpr (sizeof(Chunk) == 16) {
-                if (streaming) __builtin_amdgcn_raw_buffer_store_b128(values, resource, offset, 0, 2);
-                else __builtin_amdgcn_raw_buffer_store_b128(values, resource, offset, 0, 0);
-            } else {
-                __builtin_amdgcn_raw_buffer_store_b64(values, resource, offset, 0, 0);
-            }
-        }
-        asm volatile("" ::: "memory");
     }
-}
+    // Asks for the first two rounds of what `out` holds: it comes while the tile is multiplied.
+    __device__ __forceinline__ void begin(const char *out, int64_t stride_, int rows_valid_, int cols_valid_, int wave_m_, int wave_n_, int lane_) {
+        resource = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(uniform_pointer(out)), 0, 0x7fffffff, kBufferResourceFlags);
+        stride = stride_, rows_valid = rows_valid_, cols_valid = cols_valid_, wave_m = wave_m_, wave_n = wave_n_, lane = lane_;
+        if constexpr (kAccumulate) {
+            request(0);
+            request(1);
+        }
+    }
+    __device__ __forceinline__ void finish(const f32x16_t (&acc)[kBlocks][kBlocks], int staging, bool streaming) {
+        const int write_base = staging + (lane & 31) * kRowBytes + (lane >> 5) * 4 * sizeof(StageT);
+        const int read_base = staging + (lane >> 3) * kRowBytes + (lane & 7) * 16;
+#pragma unroll
+        for (int round = 0; round < kRounds; ++round) {
+            const int i = round / (kBlocks / kWide), first = round % (kBlocks / kWide) * kWide;
+#pragma unroll
+            for (int j = 0; j < kWide; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    struct {
+                        StageT v[4];
+                    } group;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) group.v[c] = from_float<StageT>(acc[i][first + j][4 * g + c]);
+                    *(FM_LDS(Group) *)static_cast<uintptr_t>(write_base + (j * 32 + 8 * g) * sizeof(StageT)) = __builtin_bit_cast(Group, group);
+                }
+            asm volatile("" ::: "memory");  // a wavefront's own LDS accesses are carried out in order
+            u32x4_t staged[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) staged[t] = *(FM_LDS(u32x4_t) *)static_cast<uintptr_t>(read_base + t * 8 * kRowBytes);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                Chunk values;
+                if constexpr (kAccumulate) {
+                    struct {
+                        T v[4];
+                    } sums = __builtin_bit_cast(decltype(sums), previous[round & 1][t]);
+                    const f32x4_t added = __builtin_bit_cast(f32x4_t, staged[t]);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) sums.v[c] = from_float<T>(added[c] + to_float(sums.v[c]));
+                    values = __builtin_bit_cast(Chunk, sums);
+                } else {
+                    values = __builtin_bit_cast(Chunk, staged[t]);
+                }
+                const int offset = offset_of(i, first, t);
+                if constexpr (sizeof(Chunk) == 16) {
+                    if (streaming) __builtin_amdgcn_raw_buffer_store_b128(values, resource, offset, 0, 2);
+                    else __builtin_amdgcn_raw_buffer_store_b128(values, resource, offset, 0, 0);
+                } else {
+                    __builtin_amdgcn_raw_buffer_store_b64(values, resource, offset, 0, 0);
+                }
+            }
+            if constexpr (kAccumulate)
+                if (round + 2 < kRounds) request(round + 2);
+            asm volatile("" ::: "memory");
+        }
+    }
+};
 
 // LDS: slots for the slices of each operand, a staging region per wavefront.
 typedef Operand<kTileM> Lhs;
@@ -380,6 +395,8 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_row_panel_kernel(Gem
         first.read(lhs_addresses, lhs, rhs_addresses, rhs, 0);
 #pragma unroll 1
         for (int tile = 0; tile < tiles; ++tile) {
+            TileStore<T, kAccumulate> store;
+            store.begin(out, args.out_stride_row, item.rows - tile * kTileM, cols_valid, wave_m, wave_n, opaque(lane));
             f32x16_t acc[kBlocks][kBlocks];
             clear(acc);
 #pragma unroll 1
@@ -393,8 +410,7 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_row_panel_kernel(Gem
                 first.read(lhs_addresses, lhs, rhs_addresses, rhs, 0);
                 second.template multiply<T>(acc);
             }
-            store_tile<T, kAccumulate>(acc, lds + kStagingAt + wave * kStagingBytes, out, args.out_stride_row, item.rows - tile * kTileM,
-                                          cols_valid, wave_m, wave_n, opaque(lane), streaming);
+            store.finish(acc, lds + kStagingAt + wave * kStagingBytes, streaming);
             out += kTileM * row_bytes;
         }
     }
@@ -433,7 +449,8 @@ static int launch(GemmArgs args, hipStream_t stream) {
 //   added, 8 of 4096 x 14336  1.14  1.07  1.09  1.04  1.06  1.05  1.02
 //   added, 16 of 1280 x 3416  1.11  1.06  1.11  1.05  1.04  0.99  1.00
 // The rows are those that the operands have, with up to 128 of padding per expert; below some twenty tiles per workgroup (the 32 and
-// the 16 experts) products that are not added are no faster. Results in 32 bits are not either: 0.9 to 1.1.
+// the 16 experts) products that are not added are no faster. Results in 32 bits are
+// not either: 0.89 to 1.18, added 0.94 to 1.09 (at 5 TB/s of values read and written either way).
 constexpr int64_t kMaxRowsPerExpert = 320, kLeastTiles = 22 * row_panel::kResident;
 
 // `args` as `mfma_gemm_eligible` takes them.
