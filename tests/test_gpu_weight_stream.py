@@ -56,6 +56,32 @@ def test_products_are_exact(experts, inner, columns, tall, dtype, device):
         begin = end
 
 
+@pytest.mark.parametrize(("experts", "tall"), [(70, False), (40, True)])
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+def test_strides_and_guards(experts, tall, index_dtype, device):
+    oracle_map, inner, columns = _map(experts, tall), 136, 1288
+    generator = torch.Generator(device).manual_seed(experts)
+
+    def whole(rows, width, stride):
+        return torch.randint(-2, 3, (rows, stride), generator=generator, device=device).bfloat16()[:, :width]
+
+    sparse_map = to_device_map(oracle_map, device, index_dtype)
+    x = whole(oracle_map.num_rows, inner, inner + 8)
+    by_column, by_row = whole(experts * columns, inner, inner + 24), whole(experts * inner, columns, columns + 16)
+    kept = torch.full((2, oracle_map.num_rows + 1, columns + 8), 7.0, device=device, dtype=torch.bfloat16)
+    output_sparse_matmul(x, by_column.t(), sparse_map, out=kept[0, :-1, :columns])
+    input_inner_sparse_matmul(x, by_row, sparse_map, out=kept[1, :-1, :columns])
+    begin = 0
+    for expert in range(experts):
+        end = int(oracle_map.expert_ends[expert])
+        expected = x[begin:end].float() @ by_column[expert * columns : (expert + 1) * columns].float().t()
+        assert torch.equal(kept[0, begin:end, :columns], expected.bfloat16()), expert
+        expected = x[begin:end].float() @ by_row[expert * inner : (expert + 1) * inner].float()
+        assert torch.equal(kept[1, begin:end, :columns], expected.bfloat16()), expert
+        begin = end
+    assert (kept[:, :, columns:] == 7).all() and (kept[:, -1] == 7).all()  # nothing outside of the results
+
+
 @pytest.mark.parametrize(("rows", "inner", "columns"), [(1, 64, 24840), (129, 200, 16392), (1601, 136, 2048), (3000, 64, 2568)])
 def test_dense_products_are_exact(rows, inner, columns, device):
     generator = torch.Generator(device).manual_seed(rows)
