@@ -20,6 +20,7 @@
 #include <type_traits>
 #include "fm_activation_math.h"
 #include "fm_gemm_slices.h"
+#include "fm_partition.h"
 
 namespace fm {
 
@@ -136,14 +137,10 @@ struct Tiles {
             int in_expert;
             place_in_expert(logical - first * tiles_n, count, tiles_n, in_expert, tile.tile_n);
             tile.expert = i * 64 + owner;
-            int first_row = in_expert * kHeight, last_row = first_row + kHeight;
-            if constexpr (kTall) {  // tiles that differ by 32 rows at most
-                const int blocks = (expert_rows + 31) / 32;
-                first_row = in_expert * blocks / count * 32;
-                last_row = (in_expert + 1) * blocks / count * 32;
-            }
-            tile.row = __builtin_amdgcn_readlane(begin[i], owner) + first_row;
-            tile.rows_valid = min(last_row, expert_rows) - first_row;
+            TileRows of_tile{in_expert * kHeight, min((in_expert + 1) * kHeight, expert_rows)};
+            if constexpr (kTall) of_tile = rows_of_tile(in_expert, expert_rows, count);
+            tile.row = __builtin_amdgcn_readlane(begin[i], owner) + of_tile.first;
+            tile.rows_valid = of_tile.last - of_tile.first;
         }
         return tile;
     }

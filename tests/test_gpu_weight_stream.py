@@ -91,6 +91,21 @@ def test_dense_products_are_exact(rows, inner, columns, device):
         assert torch.equal(output_sparse_matmul(x, weight), (x.float() @ weight.float()).bfloat16())
 
 
+# More rows in one expert than tiles x blocks of 32 rows have room for in 32 bits; columns that take tiles of 192 rows.
+@pytest.mark.parametrize("columns", [128, 384])
+def test_four_million_rows(columns, device):
+    rows, inner = 4_000_000, 64
+    generator = torch.Generator(device).manual_seed(columns)
+    x = torch.randint(-2, 3, (rows, inner), generator=generator, device=device, dtype=torch.int8).bfloat16()
+    weight = torch.randint(-2, 3, (columns, inner), generator=generator, device=device, dtype=torch.int8).bfloat16()
+    kept = torch.full((rows + 2 * 192, columns), 7.0, device=device, dtype=torch.bfloat16)
+    output_sparse_matmul(x, weight.t(), out=kept[192:-192])
+    for begin in range(0, rows, 500_000):
+        expected = x[begin : begin + 500_000].float() @ weight.float().t()
+        assert torch.equal(kept[192 + begin : 192 + begin + 500_000], expected.bfloat16()), begin
+    assert (kept[:192] == 7).all() and (kept[-192:] == 7).all()
+
+
 @pytest.mark.parametrize(("tokens", "ffn"), [(1000, 768), (1500, 1032), (2100, 200), (2900, 768), (3300, 1032)])
 @pytest.mark.parametrize("activation", [ActivationType.silu, ActivationType.gelu])
 def test_activation_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
