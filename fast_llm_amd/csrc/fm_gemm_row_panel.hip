@@ -19,6 +19,7 @@
 #include <atomic>
 #include <type_traits>
 #include "fm_gemm_common.h"
+#include "fm_partition.h"
 
 namespace fm {
 
@@ -291,10 +292,9 @@ struct Items {
             item.count = __builtin_amdgcn_readlane(count[i], owner);
             const int per_item = tiles_per_item(item.count), parts = (tiles + per_item - 1) / per_item;
             const int in_expert = logical - (__builtin_amdgcn_readlane(items_to[i], owner) - panels * parts), part = in_expert / panels;
-            // The tiles in parts that differ by one at most.
-            const int first = part * tiles / parts, last = (part + 1) * tiles / parts;
+            const int first = part_begin(part, tiles, parts), last = part_begin(part + 1, tiles, parts);
             item.row = first * kTileM;
-            item.rows = static_cast<int>(min(static_cast<int64_t>(last * kTileM), args.sparse_size) - item.row);
+            item.rows = static_cast<int>(min(static_cast<int64_t>(last) * kTileM, args.sparse_size) - item.row);
             item.column = (in_expert - part * panels) * kTileN;
         }
         return found;
