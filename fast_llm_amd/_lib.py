@@ -76,6 +76,7 @@ SIGNATURES: dict[str, tuple] = {
     "fm_input_inner_sparse_matmul": (_c_int, [_c_ptr] * 4 + [_c_i64] * 10 + [_c_int] * 4 + [_c_ptr, _c_size, _c_ptr]),
     "fm_input_row_sparse_matmul": (_c_int, [_c_ptr] * 5 + [_c_i64] * 10 + [_c_int] * 4 + [_c_ptr, _c_size, _c_ptr]),
     "fm_output_sparse_matmul_gated_activation": (_c_int, [_c_ptr] * 5 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr]),
+    "fm_output_sparse_matmul_gated_activation_inference": (_c_int, [_c_ptr] * 4 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr]),
     "fm_output_sparse_matmul_gated_activation_backward": (
         _c_int,
         [_c_ptr] * 6 + [_c_i64] * 8 + [_c_int] * 3 + [_c_ptr],

@@ -433,7 +433,7 @@ int fm::run_fused_gemm(const char *name, GemmArgs args, int dtype, void *stream)
     if (!mfma_gemm_fusion_eligible(args, dtype))
         return fail(FM_ERR_UNSUPPORTED,
                     "%s: needs bf16/fp16, 16-byte aligned K-contiguous operands, K a multiple of 64 and an activation "
-                    "width that is a multiple of 128 (forward) or 8 (backward); run the product and the activation "
+                    "width that is a multiple of 128 (forward) or 8 (inference, backward); run the product and the activation "
                     "separately",
                     name);
     if (int status = mfma_gemm_launch(args, dtype, nullptr, 0, static_cast<hipStream_t>(stream))) return status;
@@ -455,6 +455,24 @@ extern "C" int fm_output_sparse_matmul_gated_activation(
     args.fused_out = activation_out;
     args.fused_stride = activation_dim;
     args.half = activation_dim;
+    return run_fused_gemm(name, args, dtype, stream);
+}
+
+extern "C" int fm_output_sparse_matmul_gated_activation_inference(
+    const void *lhs, const void *rhs, void *activation_out, const void *expert_ends, int64_t row_dim, int64_t activation_dim,
+    int64_t inner_dim, int64_t num_experts, int64_t lhs_stride_row, int64_t lhs_stride_inner, int64_t rhs_stride_inner,
+    int64_t rhs_stride_col, int activation, int dtype, int index_dtype, void *stream) {
+    const char *name = "fm_output_sparse_matmul_gated_activation_inference";
+    FM_REQUIRE(activation_out, "%s: null activation_out", name);
+    GemmArgs args{lhs, rhs, nullptr, expert_ends, nullptr, lhs_stride_row, lhs_stride_inner, rhs_stride_inner,
+                  rhs_stride_col, 2 * activation_dim, 1, row_dim, 2 * activation_dim, inner_dim, 2 * activation_dim,
+                  static_cast<int>(expert_ends ? num_experts : 1), kOutputSparse, 0, index_dtype, dtype, 0, 0, nullptr};
+    args.fusion = kFusionGatedForward;
+    args.activation = activation;
+    args.fused_out = activation_out;
+    args.fused_stride = activation_dim;
+    args.half = activation_dim;
+    args.any_half = 1;
     return run_fused_gemm(name, args, dtype, stream);
 }
 

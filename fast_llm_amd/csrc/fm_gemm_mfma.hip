@@ -1592,6 +1592,7 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
 
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
     if (!args.planned) {
+        // (Those that are added: behind the check of the workspace, which was always made for them.)
         if (!args.accumulate && row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
         if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
         count_tiles(args);

@@ -18,9 +18,10 @@ class KernelConfig:
 
     POINTWISE_BLOCK_SIZE = 1024
     # Whether a gated sparse MLP's activation runs in the epilogue of the neighbouring grouped product (layer 1 forward;
-    # layer 2 input gradient) where the shapes allow. Results are bit-identical either way. None (default): chosen per
-    # call, fused exactly where it was measured faster on MI355X, which is the layer 1 forward whose own output is not
-    # stored (inference, `MLPRecomputeLevel.full`: 3.27 ms against 3.14 + 0.24 ms at the Mixtral shape). Where layer
+    # layer 2 input gradient) where the shapes allow. Results are bit-identical either way, but for the order of sums where
+    # the product by itself would cut its reductions into pieces (below). None (default): chosen per call, fused exactly
+    # where it was measured faster on MI355X, which is the layer 1 forward whose own output is not stored
+    # (inference, `MLPRecomputeLevel.full`: 3.27 ms against 3.14 + 0.24 ms at the Mixtral shape). Where layer
     # 1's output is kept the fused kernels are slower (forward 3.45 ms against 3.06 + 0.24 ms, layer 2 input gradient
     # 2.15 ms against 1.56 + 0.40 ms): the matrix-core kernel runs one wavefront per SIMD, so the exponentials and
     # reciprocals of the epilogue run with nothing to overlap them, while the separate streaming kernel does the same

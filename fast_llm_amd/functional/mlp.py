@@ -176,7 +176,8 @@ def gated_layer_1_forward(
     """
     (layer-1 output or None, activation output) of a gated sparse MLP in one kernel: `output_sparse_matmul` with
     `triton_mlp_activation_forward` in its epilogue (reference: the two calls at fast_llm/functional/triton/mlp.py:246-258).
-    Bit-identical to the two separate kernels. Raises NotImplementedError for shapes the fused kernel does not take.
+    Bit-identical to the two separate kernels, but that the product is never cut into pieces, as one by itself may be
+    (`KernelConfig.grouped_gemm_workspace`). Raises NotImplementedError for shapes the fused kernel does not take.
     """
     activation_dim = weight_1.size(0) // sparse_map.num_experts // 2
     layer_1 = input_.new_empty(input_.size(0), 2 * activation_dim) if keep_layer_1 else None
@@ -186,6 +187,19 @@ def gated_layer_1_forward(
         activation_dim, activation_type, 2 * activation_dim,
     )  # fmt: skip
     return layer_1, output
+
+
+def gated_layer_1_inference(
+    input_: torch.Tensor, weight_1: torch.Tensor, sparse_map: SparseMap, activation_type: ActivationType
+) -> torch.Tensor:
+    """`gated_layer_1_forward` for the activation output alone, of any width that is a multiple of 8."""
+    activation_dim = weight_1.size(0) // sparse_map.num_experts // 2
+    output = input_.new_empty(input_.size(0), activation_dim)
+    _launch_fused(
+        "fm_output_sparse_matmul_gated_activation_inference", input_, weight_1.t(), (output,), sparse_map, activation_dim,
+        activation_type, 2 * activation_dim,
+    )  # fmt: skip
+    return output
 
 
 def gated_layer_2_input_backward(
@@ -242,10 +256,13 @@ def _fuse_backward() -> bool:
     return bool(KernelConfig.fuse_activation)  # by default never: measured slower than the two kernels
 
 
-def _layer_1_and_activation(sparse_input, weight_1, bias_1, gated, activation_type, sparse_map, keep_layer_1):
+def _layer_1_and_activation(sparse_input, weight_1, bias_1, gated, activation_type, sparse_map, keep_layer_1, training):
     """(layer-1 output or None if it is neither kept nor needed, activation output)."""
     if _fuse_forward(keep_layer_1) and _fusable(sparse_input, weight_1.t(), gated, sparse_map, bias_1):
         try:
+            if not training and weight_1.size(0) // sparse_map.num_experts % 256 != 0:
+                # As the layer in library calls runs it: a product that is not cut into pieces adds in another order than one that is.
+                return None, gated_layer_1_inference(sparse_input, weight_1, sparse_map, activation_type)
             return gated_layer_1_forward(sparse_input, weight_1, sparse_map, activation_type, keep_layer_1)
         except NotImplementedError:  # a shape the fused kernel does not tile
             pass
@@ -285,7 +302,7 @@ def mlp_forward(
 
     sparse_input = copy_dense_to_sparse_forward(input_, sparse_map)[0] if sparse else input_
     layer_1_output, activation_output = _layer_1_and_activation(
-        sparse_input, weight_1, bias_1, gated, activation_type, sparse_map, keep_layer_1
+        sparse_input, weight_1, bias_1, gated, activation_type, sparse_map, keep_layer_1, training
     )
     layer_2_output, _ = input_parallel_linear_forward(
         activation_output, weight_2, bias_2, group, False, transposed_layer_2_weight, True, sparse_map

@@ -330,6 +330,15 @@ int fm_output_sparse_matmul_gated_activation(const void *lhs, const void *rhs, v
                                              int64_t lhs_stride_inner, int64_t rhs_stride_inner, int64_t rhs_stride_col,
                                              int activation, int dtype, int index_dtype, void *stream);
 
+/* The same without layer 1's output, for any activation_dim that is a multiple of 8. The product is never cut into pieces, as
+ * fm_output_sparse_matmul with a workspace may be: sums are in the order of the product without one. */
+int fm_output_sparse_matmul_gated_activation_inference(const void *lhs, const void *rhs, void *activation_out,
+                                                       const void *expert_ends, int64_t row_dim, int64_t activation_dim,
+                                                       int64_t inner_dim, int64_t num_experts, int64_t lhs_stride_row,
+                                                       int64_t lhs_stride_inner, int64_t rhs_stride_inner,
+                                                       int64_t rhs_stride_col, int activation, int dtype,
+                                                       int index_dtype, void *stream);
+
 /* The gradient of layer 1's output in the backward of a gated MLP: the product of the reference's layer-2 input
  * gradient `output_sparse_matmul(grad_output, weight_2_t, sparse_map)` (fast_llm/functional/triton/mlp.py:352-359)
  * is not stored but handed, tile by tile, to the activation backward `triton_mlp_activation_backward` (:70-128,

@@ -120,6 +120,12 @@ def test_router_and_fused_entry_points_validate_before_launching(library):
     with pytest.raises(NotImplementedError):
         _lib.check(_lib.FM_ERR_UNSUPPORTED)
     assert fused(activation_dim=200) == _lib.FM_ERR_UNSUPPORTED  # not a multiple of 128
+    assert library.fm_output_sparse_matmul_gated_activation_inference(
+        fake, fake, fake, None, 256, 204, 128, 1, 128, 1, 1, 128, 1, 1, 1, None
+    ) == _lib.FM_ERR_UNSUPPORTED  # not a multiple of 8
+    assert library.fm_output_sparse_matmul_gated_activation_inference(
+        fake, fake, None, None, 256, 200, 128, 1, 128, 1, 1, 128, 1, 1, 1, None
+    ) == _lib.FM_ERR_INVALID_ARGUMENT and b"null" in library.fm_last_error()
     assert fused(inner=100) == _lib.FM_ERR_UNSUPPORTED  # reduction not in whole 64-element slices
     assert fused(lhs_stride_inner=2) == _lib.FM_ERR_UNSUPPORTED
     assert fused(activation=42) == _lib.FM_ERR_INVALID_ARGUMENT and b"activation" in library.fm_last_error()

@@ -22,3 +22,17 @@ def test_layer_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
         output = layer(x)
         monkeypatch.setattr(KernelConfig, "fuse_activation", False)
         assert torch.equal(output, layer(x))
+
+
+# Reductions that the product by itself cuts into pieces (from 36 slices of 64 on): 4000 tokens have a last round of few tiles, 300 are
+# few tiles in all; 700 tokens run uncut in any case, in the product of experts of few rows.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("tokens", "hidden", "ffn"), [(4000, 2432, 2056), (4000, 2304, 2120), (300, 2432, 136), (700, 2432, 2056)])
+def test_layer_equals_parts_where_reductions_are_cut(tokens, hidden, ffn, dtype, device, monkeypatch):
+    torch.manual_seed(tokens + ffn)
+    layer = DroplessMoEMLP(hidden, ffn, 8, 2, init_std=0.05, dtype=dtype, device=device).eval()
+    x = torch.randn(tokens, hidden, device=device).to(dtype)
+    with torch.no_grad():
+        output = layer(x)
+        monkeypatch.setattr(layer, "route_with_counts", lambda *args: DroplessMoEMLP.route_with_counts(layer, *args))
+        assert torch.equal(output, layer(x))
