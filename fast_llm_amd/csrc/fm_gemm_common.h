@@ -219,6 +219,10 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype);  // with args.f
 size_t mfma_gemm_workspace_size(GemmArgs args);
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream);
 
+// The kernel that such a product runs on, and whether it would cut reductions into pieces, given a workspace.
+enum GemmKernel { kLargeTiles = 0, kRowPanel = 1, kRowSparse = 2, kWeightStream = 3, kFewTiles = 4 };
+GemmKernel mfma_gemm_kernel(GemmArgs args, int dtype, bool &splits);
+
 // Tile tables of several products that follow one another on `stream`, in one launch: sets `planned`, `tile_table` and `partials`
 // of those that want them (they share the space for pieces). `workspace`: mfma_gemm_plan_size(...) bytes, 64-byte aligned, kept
 // until the last of them has run. A product with a table has to run as `run_gemm` (or the fused product) would have run it.

@@ -1521,6 +1521,18 @@ static bool table_space(GemmArgs &args, TableSpace &space) {
     return true;
 }
 
+GemmKernel mfma_gemm_kernel(GemmArgs args, int dtype, bool &splits) {
+    splits = false;
+    if (args.mode == kInputRowSparse)
+        return row_panel_gemm_chosen(args, dtype) ? kRowPanel : row_sparse_gemm_chosen(args, dtype) ? kRowSparse : kLargeTiles;
+    count_tiles(args);
+    const bool long_enough = splits_last_round(args);
+    if (weight_stream_gemm_chosen(args, dtype, long_enough)) return kWeightStream;
+    if (few_tiles_gemm_chosen(args, dtype, long_enough)) return kFewTiles;
+    splits = long_enough;
+    return kLargeTiles;
+}
+
 size_t mfma_gemm_workspace_size(GemmArgs args) {
     TableSpace space;
     return table_space(args, space) ? (space.split ? kPartialBytes : 0) + space.table_bytes : 0;
@@ -1573,10 +1585,9 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
             GemmArgs args = products[i];
             TableSpace space;
             const bool eligible = args.fusion == kFusionNone ? mfma_gemm_eligible(args, dtype) : mfma_gemm_fusion_eligible(args, dtype);
-            if (!eligible || row_panel_gemm_chosen(args, dtype) || row_sparse_gemm_chosen(args, dtype)) continue;
-            if (!table_space(args, space) || !wants_table(args, space.split)) continue;
-            if (weight_stream_gemm_chosen(args, dtype, space.split) || few_tiles_gemm_chosen(args, dtype, space.split)) continue;
-            if (space.split != split_ones) continue;
+            bool splits;
+            if (!eligible || !table_space(args, space) || !wants_table(args, space.split) || space.split != split_ones) continue;
+            if (mfma_gemm_kernel(args, dtype, splits) != kLargeTiles) continue;
             if (split_ones && at == 0) at = kPartialBytes;
             args.partials = space.split ? static_cast<float *>(workspace) : nullptr;
             args.tile_table = static_cast<char *>(workspace) + at + sizeof(TableHeader);
@@ -1592,9 +1603,11 @@ int mfma_gemm_plan(GemmArgs *products, int count, int dtype, void *workspace, si
 
 int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace_size, hipStream_t stream) {
     if (!args.planned) {
-        // (Those that are added: behind the check of the workspace, which was always made for them.)
-        if (!args.accumulate && row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
-        if (row_sparse_gemm_chosen(args, dtype)) return row_sparse_gemm_launch(args, dtype, stream);
+        bool splits;
+        const GemmKernel kernel = mfma_gemm_kernel(args, dtype, splits);
+        // Weight gradients that are not added have never had their workspace looked at.
+        if (kernel == kRowSparse) return row_sparse_gemm_launch(args, dtype, stream);
+        if (kernel == kRowPanel && !args.accumulate) return row_panel_gemm_launch(args, dtype, stream);
         count_tiles(args);
         if (too_many_tiles(args)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
         args.partials = nullptr;
@@ -1607,9 +1620,9 @@ int mfma_gemm_launch(GemmArgs args, int dtype, void *workspace, size_t workspace
         if (workspace != nullptr && (workspace_size < needed || reinterpret_cast<uintptr_t>(workspace) % 64 != 0))
             return fail(FM_ERR_INVALID_ARGUMENT, "grouped gemm: workspace of %zu bytes (64-byte aligned) needed, got %zu at %p", needed,
                         workspace_size, workspace);
-        if (row_panel_gemm_chosen(args, dtype)) return row_panel_gemm_launch(args, dtype, stream);
-        if (weight_stream_gemm_chosen(args, dtype, splits_last_round(args))) return weight_stream_gemm_launch(args, dtype, stream);
-        if (few_tiles_gemm_chosen(args, dtype, splits_last_round(args))) return few_tiles_gemm_launch(args, dtype, stream);
+        if (kernel == kRowPanel) return row_panel_gemm_launch(args, dtype, stream);
+        if (kernel == kWeightStream) return weight_stream_gemm_launch(args, dtype, stream);
+        if (kernel == kFewTiles) return few_tiles_gemm_launch(args, dtype, stream);
         if (split) args.partials = static_cast<float *>(workspace);
         if (workspace != nullptr && wants_table(args, split)) {
             args.tile_table = static_cast<char *>(workspace) + (split ? kPartialBytes : 0) + sizeof(TableHeader);

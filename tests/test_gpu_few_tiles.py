@@ -1,4 +1,5 @@
-"""Products of few tiles (128 rows x 64, 128 or 256 columns) against fp64, at the edges of their tiles, slices and of the rule that picks them."""
+"""Products of few tiles (128 rows x 64 columns), and of the kernels that take over with more columns, against fp64, at the edges of their
+tiles, slices and of the rule that picks them."""
 
 import pytest
 import torch
@@ -10,7 +11,8 @@ pytestmark = pytest.mark.gpu
 _ROUND = {torch.bfloat16: 2**-8, torch.float16: 2**-11}
 
 
-# Columns: with the 7 and 8 row tiles here, tiles of 64 up to 2056, of 128 at 5000, of 256 at 7688, 256 x 256 ones beyond. Inner: slices of 64 that are whole, and not; one slice, two (the slots in LDS) and more.
+# Columns: with the 7 and 8 row tiles here, few tiles up to 2056, streamed products with more, 12296 in the dense product 256 x 256
+# tiles. Inner: slices of 64 that are whole, and not; one slice, two (the slots in LDS) and more.
 @pytest.mark.parametrize("dtype", list(_ROUND))
 @pytest.mark.parametrize("contiguous_k", [True, False], ids=["k", "columns"])
 @pytest.mark.parametrize("inner", [8, 72, 128, 448])

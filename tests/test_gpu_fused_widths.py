@@ -9,13 +9,17 @@ from fast_llm_amd.layers.moe import DroplessMoEMLP
 pytestmark = pytest.mark.gpu
 
 
-# 300 tokens are products of few tiles (of 64, 128 and 256 columns as the width grows), 3000 with 1096 and more columns are not.
-@pytest.mark.parametrize("tokens", [300, 3000])
-@pytest.mark.parametrize("ffn", [8, 56, 64, 72, 120, 136, 200, 1096, 1432, 2376, 4168])
+# 300 tokens are products of few tiles up to 200 columns, and streamed ones from 1096 on. 3000 are streamed ones from 136 on, and tiles of
+# 256 x 256 with 1096 and 4168: up to 1024 rows per expert, whose reductions start at different slices. 8000 have more rows.
+WIDTHS = [(tokens, ffn) for tokens in (300, 3000) for ffn in (8, 56, 64, 72, 120, 136, 200, 1096, 1432, 2376, 4168)]
+WIDTHS += [(8000, ffn) for ffn in (1096, 1432, 4168)]
+
+
+@pytest.mark.parametrize(("tokens", "ffn"), WIDTHS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("activation", [ActivationType.silu, ActivationType.squared_relu])
-def test_layer_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
+def test_layer_equals_two_kernels(tokens, ffn, dtype, activation, device, monkeypatch):
     torch.manual_seed(tokens + ffn)
-    dtype = torch.float16 if ffn % 16 else torch.bfloat16
     layer = DroplessMoEMLP(320, ffn, 7, 2, activation=activation, init_std=0.2, dtype=dtype, device=device).eval()
     x = torch.randn(tokens, 320, device=device).to(dtype)
     with torch.no_grad():

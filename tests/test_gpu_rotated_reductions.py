@@ -15,12 +15,12 @@ pytestmark = pytest.mark.gpu
 _TOKENS = [1, 0, 128, 129, 300, 7, 256, 0, 257, 64, 5]
 
 
-def _map():
+def _map(times=1):
     ends, used = [], 0
     for tokens in _TOKENS:
-        used += -(-tokens // 128) * 128
+        used += -(-tokens * times // 128) * 128
         ends.append(used)
-    return fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": _TOKENS})
+    return fixture_sparse_map({"expert_ends": ends, "tokens_per_expert": [tokens * times for tokens in _TOKENS]})
 
 
 def _operands(oracle_map, columns, slices, dtype):
@@ -35,7 +35,7 @@ def _operands(oracle_map, columns, slices, dtype):
     return x, weight, expected
 
 
-# The 15 row tiles of 128 make launches of few tiles up to 4352 columns, and of 256 x 256 ones with 4616.
+# The 15 row tiles of 128 are few tiles up to 520 columns, and streamed products with 4616.
 @pytest.mark.parametrize("slices", [1, 2, 3, 5, 12, 33])
 @pytest.mark.parametrize("columns", [8, 264, 520, 4616])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -43,6 +43,20 @@ def test_every_slice_counts_once(slices, columns, dtype, device):
     oracle_map = _map()
     real = oracle_map.real_row_mask()
     x, weight, expected = _operands(oracle_map, columns, slices, dtype)
+    out = output_sparse_matmul(x.to(device), weight.to(device).t(), to_device_map(oracle_map, device, torch.int32))
+    assert torch.equal(out.cpu()[real], expected[real])
+
+
+# Five times as many rows: tiles of 256 x 256.
+LARGE_TIMES, LARGE_COLUMNS = 5, 2568
+
+
+@pytest.mark.parametrize("slices", [1, 2, 3, 5, 12, 33])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_slice_counts_once_on_large_tiles(slices, dtype, device):
+    oracle_map = _map(LARGE_TIMES)
+    real = oracle_map.real_row_mask()
+    x, weight, expected = _operands(oracle_map, LARGE_COLUMNS, slices, dtype)
     out = output_sparse_matmul(x.to(device), weight.to(device).t(), to_device_map(oracle_map, device, torch.int32))
     assert torch.equal(out.cpu()[real], expected[real])
 

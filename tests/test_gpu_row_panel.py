@@ -23,13 +23,13 @@ def _map(experts):
 
 # 256 experts of 11 x 2 tiles are the fewest that take the kernel without adding; 257 are one too many for it. 1000 columns are no
 # whole lines.
-@pytest.mark.parametrize(
-    ("experts", "rows", "columns", "accumulate"),
-    [
-        (256, 1288, 264, False), (256, 1408, 512, False), (17, 30728, 1000, False), (257, 1288, 264, False),
-        (16, 8, 8, True), (40, 136, 264, True), (17, 392, 1000, True), (256, 128, 256, True),
-    ],
-)  # fmt: skip
+GRADIENTS = [
+    (256, 1288, 264, False), (256, 1408, 512, False), (17, 30728, 1000, False), (257, 1288, 264, False),
+    (16, 8, 8, True), (40, 136, 264, True), (17, 392, 1000, True), (256, 128, 256, True),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize(("experts", "rows", "columns", "accumulate"), GRADIENTS)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gradients_are_exact(experts, rows, columns, accumulate, dtype, device):
     oracle_map = _map(experts)

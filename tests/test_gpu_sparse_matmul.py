@@ -821,7 +821,7 @@ def test_weight_gradients_of_few_rows(sparse_dim, dense_dim, dtype, device):
     input_row_sparse_matmul(y.t(), x, sparse_map, out=out[:, :dense_dim])
     assert max_rel_err(out[:, :dense_dim].cpu(), expected) <= _MAX_REL[dtype]
     assert (out[:, dense_dim:] == 3.0).all()
-    # The same bits as on tiles of 256 x 256, which add to what is there: the order of a sum does not depend on the tile.
+    # The same bits as in the kernel that adds to what is there: the order of a sum does not depend on the tile.
     added = torch.zeros(len(tokens) * sparse_dim, dense_dim, dtype=dtype, device=device)
     input_row_sparse_matmul(y.t(), x, sparse_map, out=added, accumulate=True)
     assert torch.equal(out[:, :dense_dim], added)

@@ -25,13 +25,15 @@ def _map(experts, tall):
 
 
 # Reductions of one slice, of no whole slice, of two and of several; columns of one tile and of a remainder.
-@pytest.mark.parametrize(
-    ("experts", "inner", "columns", "tall"),
-    [
-        (256, 64, 1288, False), (128, 8, 1544, False), (70, 72, 2056, False), (64, 128, 2304, False), (33, 392, 4104, False),
-        (128, 520, 1280, False), (40, 8, 1288, True), (64, 64, 1032, True), (20, 136, 2312, True), (40, 520, 3080, True),
-    ],
-)  # fmt: skip
+PRODUCTS = [
+    (256, 64, 1288, False), (128, 8, 1544, False), (70, 72, 2056, False), (64, 128, 2304, False), (33, 392, 4104, False),
+    (128, 520, 1280, False), (40, 8, 1288, True), (64, 64, 1032, True), (20, 136, 2312, True), (40, 520, 3080, True),
+]  # fmt: skip
+STRIDED, STRIDED_INNER, STRIDED_COLUMNS = [(70, False), (40, True)], 136, 1288
+DENSE = [(1, 64, 24840), (129, 200, 16392), (1601, 136, 2048), (3000, 64, 2568)]
+
+
+@pytest.mark.parametrize(("experts", "inner", "columns", "tall"), PRODUCTS)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_products_are_exact(experts, inner, columns, tall, dtype, device):
     oracle_map = _map(experts, tall)
@@ -56,10 +58,10 @@ def test_products_are_exact(experts, inner, columns, tall, dtype, device):
         begin = end
 
 
-@pytest.mark.parametrize(("experts", "tall"), [(70, False), (40, True)])
+@pytest.mark.parametrize(("experts", "tall"), STRIDED)
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
 def test_strides_and_guards(experts, tall, index_dtype, device):
-    oracle_map, inner, columns = _map(experts, tall), 136, 1288
+    oracle_map, inner, columns = _map(experts, tall), STRIDED_INNER, STRIDED_COLUMNS
     generator = torch.Generator(device).manual_seed(experts)
 
     def whole(rows, width, stride):
@@ -82,7 +84,7 @@ def test_strides_and_guards(experts, tall, index_dtype, device):
     assert (kept[:, :, columns:] == 7).all() and (kept[:, -1] == 7).all()  # nothing outside of the results
 
 
-@pytest.mark.parametrize(("rows", "inner", "columns"), [(1, 64, 24840), (129, 200, 16392), (1601, 136, 2048), (3000, 64, 2568)])
+@pytest.mark.parametrize(("rows", "inner", "columns"), DENSE)
 def test_dense_products_are_exact(rows, inner, columns, device):
     generator = torch.Generator(device).manual_seed(rows)
     x = torch.randint(-2, 3, (rows, inner), generator=generator, device=device).bfloat16()
@@ -106,11 +108,14 @@ def test_four_million_rows(columns, device):
     assert (kept[:192] == 7).all() and (kept[-192:] == 7).all()
 
 
-@pytest.mark.parametrize(("tokens", "ffn"), [(1000, 768), (1500, 1032), (2100, 200), (2900, 768), (3300, 1032)])
+WIDTHS = [(1000, 768), (1500, 1032), (2100, 200), (2900, 768), (3300, 1032)]
+
+
+@pytest.mark.parametrize(("tokens", "ffn"), WIDTHS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("activation", [ActivationType.silu, ActivationType.gelu])
-def test_activation_equals_two_kernels(tokens, ffn, activation, device, monkeypatch):
+def test_activation_equals_two_kernels(tokens, ffn, dtype, activation, device, monkeypatch):
     torch.manual_seed(tokens + ffn)
-    dtype = torch.float16 if ffn % 16 else torch.bfloat16
     layer = DroplessMoEMLP(320, ffn, 128, 6, activation=activation, init_std=0.2, dtype=dtype, device=device).eval()
     x = torch.randn(tokens, 320, device=device).to(dtype)
     with torch.no_grad():
