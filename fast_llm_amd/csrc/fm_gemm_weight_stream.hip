@@ -398,64 +398,63 @@ static int launch(const GemmArgs &args, hipStream_t stream) {
 
 }  // namespace weight_stream
 
-// Where the lines lie: 300 layers in inference (24 to 800 rows per expert, experts equally and unequally liked; layer 1 with the gated
-// activation), the time with large tiles (up to 256 tiles: of fm_gemm_few_tiles.hip) over the time with one of the two products here,
-// geometric means (and the worst), by the bound of the 128 x 256 tiles that the host knows and by the mean rows per expert:
-//    layer 1, rows       97 ..       257 ..       401 ..       601 ..       1001 ..      more
-//     24 .. 59        0.99 (.88)   1.05 (.99)   1.14 (.99)   1.06 (.98)   1.04 (1.00)  1.09 (1.00)
-//     60 .. 99        0.97 (.93)   1.02 (.90)   1.14 (1.11)  1.09 (1.04)  1.03 (.97)   1.09 (1.07)
-//    100 .. 139       1.05 (.98)   1.01 (.91)   1.10 (1.05)  1.06 (1.03)  1.04 (.97)   1.04 (.97)
-//    140 .. 199       0.93                      0.97 (.95)   1.05 (.97)   1.02 (.98)   1.01 (.97)
-//    200 .. 269       1.00 (.97)   1.08 (1.00)  0.94         0.98 (.93)   1.01 (.92)   1.00 (.90)
-//    more             1.07         0.93 (.89)   0.92 (.85)   1.03 (.93)   1.00 (.90)   0.99 (.90)
-//    layer 2, rows
-//     24 .. 59        1.02 (.90)   1.03 (.99)   1.06 (1.03)  1.02 (.98)   1.01 (.98)   1.03 (1.01)
-//     60 .. 99        1.04 (.88)   1.02 (.99)   1.03 (1.00)  1.00 (.96)   1.01 (.99)   1.00 (.96)
-//    100 .. 139       1.03 (.90)   0.99 (.94)   1.02 (1.00)  1.01 (.99)   1.04 (.98)   1.00 (.98)
-//    140 .. 199       1.03 (.84)   1.04 (.98)   1.05         1.00 (.95)   0.98 (.95)   0.98 (.97)
-//    200 .. 269       1.01 (.81)   1.02 (.98)   0.97 (.83)   1.00 (1.00)  0.97 (.93)   0.97 (.95)
-//    more             1.06 (1.00)  1.03 (.99)   0.92 (.77)   0.99 (.93)   1.00 (.96)   0.97 (.95)
-// (those below 1 up to 256 tiles with the other product on large tiles instead of few). With both here, which also saves the launch that
-// writes the tables, the whole layer is 1.07 to 1.27 times as fast below 100 rows, 1.0 to 1.2 from 100 to 199. Whole training steps of
-// 64 rows: 1.01 (128 experts of 2048 x 768) to 1.14 (16 of 1280 x 3416). The host knows rows with up to 128 of padding per expert.
-// With more than 228 rows in the buffer those whose expected tiles of 128 rows (half of the padding taken off) are one round: 1.04
-// (.95) to 1.17 with 200 to 256 tiles; 0.96 (.80) with 257 to 400.
-// Tall tiles: 350 layers of 100 to 800 rows, the time with large tiles over the time with one product here, by the cost (`Tiles`) of the
-// tiles here per round of 256 x 256 ones, experts equally liked (unequally):
-//            up to 200     .. 260        .. 300        .. 340        .. 380        .. 420        .. 460        .. 540        more
-//   layer 1  0.97 (1.01)   1.00 (1.06)   1.09 (1.07)   1.05 (1.03)   1.05 (1.04)   1.02 (1.03)   1.00 (1.02)   0.99 (1.03)   0.96 (1.02)
-//   layer 2  1.01 (1.00)   0.98 (1.03)   1.04 (1.02)   1.01 (1.00)   0.99 (1.00)   0.99 (0.99)   0.99 (1.00)   0.99 (1.00)   0.98 (0.99)
-// Reductions of no whole slices are masked in the large tiles' kernel: a step of 375 rows of 16 experts of 1280 x 3416, where layer 2
-// and layer 1's input gradient cost 350, takes 830 -> 808 us with them here.
-// Reductions that the large tiles' kernel splits into pieces (`splits`): 0.87 to 0.91 with 260 rows for each of 8 experts of 4096 x
-// 14336, 0.99 (1.25 with some experts preferred) with 180.
+// Where the lines lie. 420 drawn layers (inference of 9 to 900 rows per expert, training steps up to 900; all shapes, preferences and
+// recompute levels), kernel by kernel in a trace: the time with large tiles over the time here, geometric mean (worst, products), by the
+// cost (`Tiles`) of the tiles that the host expects here per round of 256 x 256 ones:
+//   weights along K, low tiles      up to 220  .. 250  .. 280  .. 300  .. 320  more
+//                                   1.45       1.18    1.17    1.10    1.07    1.06
+//                                   (1.10, 22) (.85, 72) (.92, 46) (.87, 82) (.83, 44) (1.00, 13)
+//   weights along K, tall tiles     up to 300  .. 340  .. 380  .. 400  .. 420  .. 440  more
+//                                   1.10       1.04    1.03    1.09    1.02    0.98    0.99
+//                                   (.71, 31)  (.87, 42) (.84, 99) (.98, 12) (.86, 26) (.83, 36) (.90, 9)
+//   weights along rows, low tiles   up to 220  .. 250  .. 280  .. 300  more
+//    inner size of whole slices     1.17       1.12    1.08    0.97    0.96
+//                                   (.84, 55)  (.87, 43) (.90, 27) (.82, 82) (.81, 20)
+//    of no whole slices             1.44 (1.21, 4), .. 260 1.36 (1.16, 7), .. 300 1.29 (.98, 8), more 1.33 (1)
+//   weights along rows, tall tiles  whole slices .. 300 0.96 (.76, 9), .. 320 1.07 (1), .. 345 1.02 (1); no whole slices .. 360 1.20 (1.07, 11)
+// Weights along rows of some 30 rows per expert, as many rounds of tiles here as there, run at 4.9 TB/s here and at 5.7 there (64 experts of
+// 2048 x 1408: 75 and 65 us), but there a launch in front writes the table of tiles, 5 to 10 us: whole layers with those products on large
+// tiles are 0.95 to 0.97 times as fast in inference, level in training. The same for tall tiles from 280 to 320: 0.93 to 0.96 (four
+// layers in inference), 1.04 (two training steps of preferred experts). The masked last slice of a reduction of no whole slices costs the
+// large tiles more. With weights along K whole layers from 420 to 440 are 1.02 times as fast on large tiles (0.99 to 1.05).
+// Tall tiles lose where some experts are preferred and the host's count of tiles is off: 0.71 to 0.88 are such (and 128 experts of 2048
+// x 768 at 150 to 160 rows, exactly 3 rounds of large tiles: 0.87 to 0.92); 2 rounds gain 1.09 on average, 1 and more than 2 1.02.
+// More than 1000 low tiles of weights along rows: 0.96 to 1.04, 1.00 on average from 60 rows per expert on, which leaves them to the large.
+// 97 to 256 tiles are all taken: 0.80 (12 us) to 1.34, 1.04 on average, against the kernel for few tiles with 128 and 256 columns.
+// The host knows rows with up to 128 of padding per expert. Low tiles from 229 rows on are those whose expected tiles (half of the padding
+// taken off) are one round: 1.04 (.95) to 1.17 with 200 to 256 tiles; 0.96 (.80) with 257 to 400. A map of the rows in use has some 64 of
+// padding: its experts are taken to have 64 rows fewer than they do.
+// Reductions that the large tiles' kernel splits into pieces (`splits`) are in these figures (tall 1.01, low 1.04 to 1.24); with 260 rows
+// for each of 8 experts of 4096 x 14336 0.87 to 0.91; with 140 to 200 1.05 to 1.3 where some experts are preferred, 0.87 to 1.1 where none is.
 namespace weight_stream {
 
-// Row tiles of `height` rows, if tokens choose experts independently, all alike: a fifth of the experts each has rows of that many
-// standard deviations from the mean. (A map's buffer has room for 128 rows of padding per expert.)
-static float expected_row_tiles(const GemmArgs &args, int height) {
+// Row tiles of `height` rows, in fifths (whole numbers: a launch of exactly one round is not to be taken for two), if tokens choose experts
+// independently, all alike: a fifth of the experts each has rows of that many standard deviations from the mean.
+static int64_t expected_row_tiles(const GemmArgs &args, int height) {
     const float rows = fmaxf(static_cast<float>(args.rows) / args.num_experts - (args.expert_ends != nullptr ? 128.f : 0.f), 1.f);
-    float tiles = 0.f;
+    int64_t tiles = 0;
     for (const float deviations : {-1.4f, -0.53f, 0.f, 0.53f, 1.4f})
-        tiles += ceilf(fmaxf(rows + (args.num_experts > 1 ? deviations * sqrtf(rows) : 0.f), 1.f) / height);
-    return args.num_experts * tiles / 5.f;
+        tiles += static_cast<int64_t>(ceilf(fmaxf(rows + (args.num_experts > 1 ? deviations * sqrtf(rows) : 0.f), 1.f) / height));
+    return args.num_experts * tiles;
 }
+
+// Rounds of as many tiles next to one another. `row_tiles` in fifths.
+static int64_t rounds_of(int64_t row_tiles, int64_t tiles_n) { return (row_tiles * tiles_n + 5 * kResident - 1) / (5 * kResident); }
 
 // What `Tiles` makes of them.
 static float expected_cost(const GemmArgs &args) {
     const float rows = fmaxf(static_cast<float>(args.rows - (args.expert_ends != nullptr ? 128 * args.num_experts : 0)), 1.f);
     float least = INFINITY;
     for (int height = 128; height <= kTileM<true>; height += 64) {
-        const float row_tiles = expected_row_tiles(args, height);
+        const int64_t row_tiles = expected_row_tiles(args, height);
+        const float row_cost = 5 * rows / (2 * row_tiles) + 16;
         for (int width = kTileN; width >= kLeastWidth; width -= 64)
-            least = fminf(least, ceilf(row_tiles * ((args.cols + width - 1) / width) / kResident) * (width + rows / (2 * row_tiles) + 16));
+            least = fminf(least, rounds_of(row_tiles, (args.cols + width - 1) / width) * (width + row_cost));
     }
     return least;
 }
 
-static float expected_large_rounds(const GemmArgs &args) {
-    return ceilf(expected_row_tiles(args, 256) * ((args.cols + 255) / 256) / kResident);
-}
+static int64_t expected_large_rounds(const GemmArgs &args) { return rounds_of(expected_row_tiles(args, 256), (args.cols + 255) / 256); }
 
 }  // namespace weight_stream
 
@@ -475,7 +474,7 @@ bool weight_stream_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     if (tiles <= 96 || (splits && args.rows > 320 * experts)) return false;
     const bool contiguous = args.rhs_stride_inner == 1;
     if (low_tiles(args)) return contiguous || tiles <= 1000 || args.rows <= 180 * experts;
-    const int most = contiguous ? 440 : args.inner % kBK == 0 ? 320 : 360;
+    const int most = contiguous ? 420 : args.inner % kBK == 0 ? 320 : 360;
     return expected_cost(args) <= most * expected_large_rounds(args);
 }
 

@@ -69,3 +69,25 @@ def test_weight_gradients(kernel):
         rows = row_panel._map(experts).num_rows
         expected = "row panel" if experts <= 256 else "row sparse"
         assert kernel(INPUT_ROW_SPARSE, rows, columns, size, experts, accumulate) == expected, (experts, size, columns)
+
+
+# (rows, columns, inner, experts): layer 2, or layer 1's input gradient.
+@pytest.mark.parametrize(("product", "expected"), [
+    ((9472, 2048, 1408, 64), "weight stream"), ((16896, 704, 3712, 60), "weight stream"), ((6400, 1544, 128, 11), "large tiles"),
+    ((22400, 968, 1184, 32), "weight stream"),  # a reduction of no whole slices
+])  # fmt: skip
+def test_weights_along_rows(kernel, product, expected):
+    rows, columns, inner, experts = product
+    assert kernel(INPUT_INNER_SPARSE, rows, columns, inner, experts) == expected
+
+
+@pytest.mark.parametrize(("product", "expected"), [
+    ((46592, 1152, 1152, 61), "large tiles"), ((99840, 768, 2048, 128), "large tiles"),  # about as many rounds of tall tiles, or more
+    # Exactly 15 and 13 rounds of large ones, not one more: 427 and 405 per round, where 400 and 432 were counted.
+    ((37248, 6400, 1024, 96), "large tiles"), ((32512, 6400, 1024, 64), "weight stream"),
+    ((14976, 1408, 2048, 64), "weight stream"), ((15104, 1152, 2240, 17), "weight stream"),  # 1.5 and 1.1 rounds of large ones
+    ((9472, 2816, 2048, 64), "weight stream"), ((18432, 1536, 2048, 128), "weight stream"),  # low ones
+])  # fmt: skip
+def test_weights_along_the_reduction(kernel, product, expected):
+    rows, columns, inner, experts = product
+    assert kernel(OUTPUT_SPARSE, rows, columns, inner, experts) == expected

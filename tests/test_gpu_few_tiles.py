@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 _ROUND = {torch.bfloat16: 2**-8, torch.float16: 2**-11}
 
 
-# Columns: with the 7 and 8 row tiles here, few tiles up to 2056, streamed products with more, 12296 in the dense product 256 x 256
-# tiles. Inner: slices of 64 that are whole, and not; one slice, two (the slots in LDS) and more.
+# Columns: with the 7 and 8 row tiles here, few tiles up to 2056, streamed products with more; with 12296 256 x 256
+# tiles in the dense product. Inner: slices of 64 that are whole, and not; one slice, two (the slots in LDS) and more.
 @pytest.mark.parametrize("dtype", list(_ROUND))
 @pytest.mark.parametrize("contiguous_k", [True, False], ids=["k", "columns"])
 @pytest.mark.parametrize("inner", [8, 72, 128, 448])
