@@ -1,11 +1,11 @@
-// Grouped products of few output tiles, in half precision: 128 rows x 64 columns.
+// Grouped products of few output tiles, in half precision: 128 rows x 64 columns (128 or 256 with more than 256 experts).
 //
 // A launch of a third of a 256 x 256 tile per CU lasts as long as one tile does, on whatever part of the chip, and most of a tile's rows are
 // padding where experts have some 100 tokens. With tiles of an eighth of that size more CUs share the same work; two per CU overlap
 // one's loads with the other's MFMAs. A CU then reads more operand bytes per multiplication, which is why launches of more tiles
 // go elsewhere (fm_gemm_weight_stream.hip; the line, and what was measured on both sides of it, are at few_tiles_gemm_chosen).
 //
-// Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), three in LDS,
+// Slices of 64 along K (whole 128-byte lines of K-contiguous rows; with 32 the same tiles take 10 to 20 % longer), two or three in LDS,
 // filled straight from memory; the fragments of the next 16 are read while the MFMAs of this 16 run. Sums in fp32, in the order of
 // the large tiles' kernel.
 #include "fm_activation_math.h"
@@ -17,14 +17,14 @@ namespace few_tiles {
 
 using namespace slices;
 
-constexpr int kTileM = 128, kTileN = 64, kThreads = kLoadingThreads;
+constexpr int kTileM = 128, kThreads = kLoadingThreads;
 // 2 x 2 wavefronts, 32 x 32 accumulators. With the gated activation the columns are 32 gates and 32 ups, which one wavefront has to have
 // both of: 4 x 1.
 template <bool kGated>
 constexpr int kWavesN = kGated ? 1 : 2;
 template <bool kGated>
 constexpr int kBlocksM = kTileM / 32 * kWavesN<kGated> / 4;
-template <bool kGated>
+template <int kTileN, bool kGated>
 constexpr int kBlocksN = kTileN / 32 / kWavesN<kGated>;
 
 // value(i, j, v), of 32 x 32 accumulators -> rows of `out`, 32 rows of the wavefront's columns at a time through its own part of LDS: 16
@@ -66,17 +66,22 @@ __device__ __forceinline__ void store_tile(Value &&value, int staging, T *out, i
     }
 }
 
-constexpr int kStages = 3, kWorkgroups = 2;  // slices in LDS, workgroups per CU
-constexpr int kLdsBytes = kStages * (kTileM + kTileN) * kBK * 2;
+template <int kTileN>
+constexpr int kStages = kTileN == 128 ? 2 : 3;  // slices in LDS
+template <int kTileN>
+constexpr int kWorkgroups = kTileN == 256 ? 1 : 2;  // per CU
+template <int kTileN>
+constexpr int kLdsBytes = kStages<kTileN> * (kTileM + kTileN) * kBK * 2;
 
-template <typename T, bool kRhsK, bool kGated>
-__global__ __launch_bounds__(kThreads, kWorkgroups) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
-    constexpr int kBlocksM = few_tiles::kBlocksM<kGated>, kBlocksN = few_tiles::kBlocksN<kGated>;
+template <typename T, int kTileN, bool kRhsK, bool kGated>
+__global__ __launch_bounds__(kThreads, kWorkgroups<kTileN>) void grouped_gemm_few_tiles_kernel(GemmArgs args) {
+    constexpr int kBlocksM = few_tiles::kBlocksM<kGated>, kBlocksN = few_tiles::kBlocksN<kTileN, kGated>;
+    constexpr int kStages = few_tiles::kStages<kTileN>, kLdsBytes = few_tiles::kLdsBytes<kTileN>;
     typedef Operand<kTileM, true, kBlocksM> Lhs;
     typedef Operand<kTileN, kRhsK, kBlocksN> Rhs;
     constexpr int kSlotBytes = Lhs::kBytes + Rhs::kBytes, kLoads = Lhs::kLoads + Rhs::kLoads;
     constexpr int kColumns = kGated ? kTileN / 2 : kTileN;  // of the result
-    static_assert(kLdsBytes * kWorkgroups <= 160 * 1024 && kLdsBytes >= 4 * 32 * (kTileN + 16), "LDS of a CU");
+    static_assert(kLdsBytes * kWorkgroups<kTileN> <= 160 * 1024 && kLdsBytes >= 4 * 32 * (kTileN + 16), "LDS of a CU");
     extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
     const int lds = static_cast<int>(reinterpret_cast<uintptr_t>((FM_LDS(char) *)lds_generic));
 
@@ -185,36 +190,50 @@ __global__ __launch_bounds__(kThreads, kWorkgroups) void grouped_gemm_few_tiles_
 // Tiles of 128 x 256, by the upper bound that the host knows of their row tiles (a static map has one tile of padding per expert).
 static int64_t most_tiles(const GemmArgs &args) { return (args.rows + kTileM - 1) / kTileM * ((args.cols + 255) / 256); }
 
-template <typename T, bool kRhsK, bool kGated = false>
+template <typename T, int kTileN, bool kRhsK, bool kGated = false>
 static int launch(const GemmArgs &args, hipStream_t stream) {
-    const auto kernel = grouped_gemm_few_tiles_kernel<T, kRhsK, kGated>;
+    const auto kernel = grouped_gemm_few_tiles_kernel<T, kTileN, kRhsK, kGated>;
     static std::atomic<uint64_t> configured{0};
-    if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, configured)) return status;
+    if (int status = allow_lds(reinterpret_cast<const void *>(kernel), kLdsBytes<kTileN>, configured)) return status;
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n, round = 8 * static_cast<int64_t>(args.chunk_tiles);
-    kernel<<<static_cast<uint32_t>((tiles + round - 1) / round * round), kThreads, kLdsBytes, stream>>>(args);
+    kernel<<<static_cast<uint32_t>((tiles + round - 1) / round * round), kThreads, kLdsBytes<kTileN>, stream>>>(args);
     return FM_OK;
 }
 
-template <typename T>
+template <typename T, int kTileN>
 static int launch(GemmArgs args, hipStream_t stream) {
     args.tiles_m = static_cast<int>((args.rows + kTileM - 1) / kTileM + (args.num_experts > 1 ? args.num_experts : 0));
     args.tiles_n = static_cast<int>((args.cols + kTileN - 1) / kTileN);
     const int64_t tiles = static_cast<int64_t>(args.tiles_m) * args.tiles_n;
     if (tiles >= (int64_t(1) << 30)) return fail(FM_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
-    // Runs of 16 tiles per XCD.
+    // Runs of 16 tiles per XCD; 8 and 32 are up to 3 and 5 % slower (128 columns).
     args.chunk_tiles = static_cast<int>(min(int64_t(16), (tiles + 7) / 8));
-    if (args.fusion == kFusionGatedForward) return launch<T, true, true>(args, stream);
-    return args.rhs_stride_inner == 1 ? launch<T, true>(args, stream) : launch<T, false>(args, stream);
+    if constexpr (kTileN == 64)
+        if (args.fusion == kFusionGatedForward) return launch<T, kTileN, true, true>(args, stream);
+    return args.rhs_stride_inner == 1 ? launch<T, kTileN, true>(args, stream) : launch<T, kTileN, false>(args, stream);
+}
+
+template <typename T>
+static int launch(const GemmArgs &args, hipStream_t stream) {
+    const int64_t tiles = most_tiles(args);
+    return tiles <= 96 ? launch<T, 64>(args, stream) : tiles <= 160 ? launch<T, 128>(args, stream) : launch<T, 256>(args, stream);
 }
 
 }  // namespace few_tiles
 
-// Where the line lies. Over 240 layers of random shapes (4 to 1100 rows per expert, experts equally and unequally liked, sizes that are
-// whole slices and that are not), weights in memory and activations in cache, the time of 256 x 256 tiles divided by that of these,
-// geometric means (and the worst), by most_tiles: up to 64 2.00 (1.85), 65 .. 96 1.74 (1.10), 97 .. 160 1.28 (0.95), 161 .. 192 1.08, more
-// 0.98 and less. Above 96 the kernel that streams weights takes those that it can, 1.0 to 1.2 times as fast as tiles of 128 or 256 columns
-// here (inference of 40 to 200 rows for each of 8 experts of 1024 x 2816 1.24 to 1.34, of 4096 x 1536 1.10 to 1.14); up to 96 it is no
-// faster, with 64 columns either (0.98 to 1.02).
+// Where the lines lie. Over 240 layers of random shapes (4 to 1100 rows per expert, experts equally and unequally liked, sizes that are
+// whole slices and that are not), weights in memory and activations in cache, the time of 256 x 256 tiles divided by that of 64, 128 and
+// 256 columns, geometric means (and the worst), by most_tiles:
+//       up to 64       2.00 (1.85), 1.46, 1.27
+//       65 .. 96       1.74 (1.10), 1.44 (1.19), 1.20
+//       97 .. 160      1.28 (0.95), 1.40 (1.10), 1.23 (0.99)
+//       161 .. 192     1.08, 1.16 (0.99), 1.16 (1.01)
+//       193 .. 256     0.98, 1.09 (0.96), 1.16 (1.00)
+//       257 .. 320     0.95, 1.08 (0.71), 1.13 (0.73): two rounds where 256 x 256 tiles take one
+// Above 96 the kernel that streams weights takes all of up to 256 experts, 1.0 to 1.2 times as fast as 128 or 256 columns here (inference
+// of 40 to 200 rows for each of 8 experts of 1024 x 2816 1.24 to 1.34, of 4096 x 1536 1.10 to 1.14); up to 96 it is no faster, with 64
+// columns either (0.98 to 1.02). More experts with so few tiles are those of which most have no rows: 100 to 250 of 300 and 512 with 60 rows,
+// 256 columns 20 to 67 us here, 26 to 75 with 64 columns, 32 to 68 on 256 x 256 tiles.
 // Reductions that the large tiles' kernel splits into pieces for all CUs: 1.33 (0.87) up to 96, and no better with more: they stay there.
 // With the gated activation against fused tiles of 256 x 256, layer 1 of 800 tokens of 8 experts of 1536 x 512 (6 each) 45 -> 31 us.
 bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
@@ -225,7 +244,7 @@ bool few_tiles_gemm_chosen(const GemmArgs &args, int dtype, bool splits) {
     if (args.fusion == kFusionGatedForward && (args.out != nullptr || (args.half + 128) * args.rhs_stride_col * 2 >= (int64_t(1) << 31)))
         return false;
     if (args.fusion == kFusionGatedBackward) return false;
-    return few_tiles::most_tiles(args) <= 256;
+    return few_tiles::most_tiles(args) <= (args.fusion == kFusionNone ? 256 : 96);
 }
 
 int few_tiles_gemm_launch(const GemmArgs &args, int dtype, hipStream_t stream) {

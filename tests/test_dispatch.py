@@ -2,6 +2,7 @@
 
 import pytest
 
+from tests import test_gpu_few_tiles as few_tiles
 from tests import test_gpu_fused_widths as fused_widths
 from tests import test_gpu_rotated_reductions as rotated
 from tests import test_gpu_row_panel as row_panel
@@ -62,6 +63,15 @@ def test_few_tiles(kernel):
                 assert kernel(mode, 7 * 128, columns, inner, 5) == expected, (mode, inner, columns)
                 expected = expected if columns <= 7688 else "large tiles"
                 assert kernel(mode, 1009, columns, inner) == expected, (mode, inner, columns)
+
+
+    for inner in (8, 72, 128, 448):
+        for columns in (8, 136, 256, 264, 504):
+            for mode in (OUTPUT_SPARSE, INPUT_INNER_SPARSE):
+                assert kernel(mode, 101 * 128, columns, inner, len(few_tiles.MANY)) == "few tiles", (mode, inner, columns)
+    # With the gated activation up to 96 tiles only.
+    assert kernel(OUTPUT_SPARSE, 96 * 128, 256, 128, 300, gated=True) == "few tiles"
+    assert kernel(OUTPUT_SPARSE, 97 * 128, 256, 128, 300, gated=True) == "large tiles"
 
 
 def test_weight_gradients(kernel):

@@ -19,6 +19,22 @@ _ROUND = {torch.bfloat16: 2**-8, torch.float16: 2**-11}
 @pytest.mark.parametrize("cols", [8, 136, 2056, 5000, 7688, 12296])
 @pytest.mark.parametrize("counts", [(127, 0, 1, 129, 256), None], ids=str)
 def test_against_fp64(counts, cols, inner, contiguous_k, dtype, library, device):
+    _check(counts, cols, inner, contiguous_k, dtype, library, device)
+
+
+# More than 256 experts, of which a third has rows: 101 and 202 tiles of 128 x 256, for tiles of 128 and 256 columns.
+MANY = tuple(e * 37 % 128 + 1 if e % 3 == 0 else 0 for e in range(300))
+
+
+@pytest.mark.parametrize("dtype", list(_ROUND))
+@pytest.mark.parametrize("contiguous_k", [True, False], ids=["k", "columns"])
+@pytest.mark.parametrize("inner", [8, 72, 128, 448])
+@pytest.mark.parametrize("cols", [8, 136, 256, 264, 504])
+def test_many_experts_against_fp64(cols, inner, contiguous_k, dtype, library, device):
+    _check(MANY, cols, inner, contiguous_k, dtype, library, device)
+
+
+def _check(counts, cols, inner, contiguous_k, dtype, library, device):
     generator = torch.Generator(device).manual_seed(cols + inner)
     experts = len(counts) if counts else 1
     pad = 128
