@@ -1460,10 +1460,10 @@ bool mfma_gemm_fusion_eligible(const GemmArgs &args, int dtype) {
 }
 
 // ---- workspace: the tile table and the pieces of split reductions ----------------------------------------
-// Whether a product is one whose last round is split is decided from its dimensions alone (few rounds of long tiles);
-// the caller then brings kMaxPartials tile-sized fp32 slots, followed by one tile record per workgroup id. Given the
-// dimensions, whether the split happens depends on nothing but the presence of the workspace, which is the caller's
-// choice; the table changes no result, only where a workgroup finds its tile.
+// What a caller brings follows from the dimensions alone: where they have few rounds of long tiles kMaxPartials tile-sized fp32 slots,
+// then one tile record per workgroup id. Whether the last round is then split follows from the call's other arguments too, which choose the
+// kernel (`mfma_gemm_kernel`: layouts, types, accumulation, number of experts), and from the presence of the workspace, which is the
+// caller's choice: from no state. The table changes no result, only where a workgroup finds its tile.
 static void count_tiles(GemmArgs &args) {
     if (args.mode == kInputRowSparse) {
         args.tiles_m = static_cast<int>((args.sparse_size + kTile - 1) / kTile) * args.num_experts;

@@ -448,9 +448,11 @@ static int launch(GemmArgs args, hipStream_t stream) {
 //    some experts preferred   1.60  1.46  1.37  1.22  1.13  0.99  1.00
 //   added, 8 of 4096 x 14336  1.14  1.07  1.09  1.04  1.06  1.05  1.02
 //   added, 16 of 1280 x 3416  1.11  1.06  1.11  1.05  1.04  0.99  1.00
-// The rows are those that the operands have, with up to 128 of padding per expert; below some twenty tiles per workgroup (the 32 and
-// the 16 experts) products that are not added are no faster. Results in 32 bits are
-// not either: 0.89 to 1.18, added 0.94 to 1.09 (at 5 TB/s of values read and written either way).
+// The rows are those that the operands have, with up to 128 of padding per expert. Products that are not added are taken from 22 tiles per
+// workgroup on (of the 32 experts the larger gradient has 24, the smaller one 12; neither of the 16): in a trace of 420 drawn training steps
+// and layers (rows up to 320) 22 to 31 tiles are 1.14 times as fast as before (0.98 at worst, 47 gradients), 32 to 63 1.12 (0.97, 55),
+// more 1.05 (0.91, 13), added ones 1.33 (1.01, 56). Results in 32 bits are no faster: 0.89 to 1.18, added 0.94 to 1.09 (at 5 TB/s of values
+// read and written either way).
 constexpr int64_t kMaxRowsPerExpert = 320, kLeastTiles = 22 * row_panel::kResident;
 
 // `args` as `mfma_gemm_eligible` takes them.

@@ -247,8 +247,8 @@ static int launch(const GemmArgs &args, int64_t grid, hipStream_t stream) {
 
 }  // namespace row_sparse
 
-// Where fm_gemm_row_panel.hip takes no part, up to this many rows per expert, of the rows that the operands have (a layer's buffers have about 128 per expert more than
-// it fills). us, 256 x 256 / here, larger and smaller gradient of a layer: 16 rows of 128 experts of 2048 x 768 218 / 163, 115 /
+// Where fm_gemm_row_panel.hip takes no part, up to this many rows per expert, of the rows that the operands have (a layer's buffers have
+// about 128 per expert more than it fills). us, 256 x 256 / here, larger and smaller gradient of a layer: 16 rows of 128 experts of 2048 x 768 218 / 163, 115 /
 // 88; 250 rows 362 / 344, 198 / 179; 350 rows 421 / 421, 247 / 216; 500 rows 493 / 512, 289 / 260; 1024 rows 770 / 835, 394 /
 // 424. 8 experts of 4096 x 14336: 200 rows 726 / 716, 416 / 365; 383 rows 959 / 981, 539 / 492; 600 rows 1210 / 1295, 618 / 643.
 // Results that are added to what is there, or stored in 32 bits, are bound by that traffic and no faster here (adding in 32

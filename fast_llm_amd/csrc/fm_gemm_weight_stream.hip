@@ -10,12 +10,14 @@
 //   * tiles found from row counts in registers, without a table that a kernel in front has to write (5 to 9 us).
 // One GPU, us before and now: layer 1's product with 40 rows for each of 8 experts of 4096 x 14336 418 -> 384 (1.88 GB: 4.9 TB/s,
 // 5.3 without what a launch takes to start and end), of 16 of 4096 x 4096 201 -> 189 (5.7 TB/s); layer 2's for 80 rows of 16 of
-// 1280 x 3416 64 -> 55. What is on its way (64 KB of weights per CU) limits it.
+// 1280 x 3416 64 -> 55. What is on its way (64 KB of weights per CU) limits it. These are its best shapes: tall tiles of 125 rows for each of
+// 128 experts of 2048 x 768 (150 us a launch, 2048 columns on average) read weights at 4.0 TB/s, 4.9 with activations and results.
 // Tall tiles are for experts of 100 rows and more, whose rows would be two tiles of 128, the second nearly empty, or one large one:
 // inference of 125 and 150 rows for each of 32 experts of 3000 x 1000 258 -> 210 and 271 -> 222 us, 250 390 -> 307; of 125 of 16 of 4096 x
 // 4096 382 -> 358; a training step of 375 of 16 of 1280 x 3416 842 -> 802. They leave LDS for two slices of the lhs, which mostly comes
 // from L2, and are 2 to 10 % slower where 128 rows would do.
-// Sums in fp32, in the order of the large tiles' kernel (fm_gemm_mfma.hip): the same bits.
+// Sums in fp32, in the order of the large tiles' kernel (fm_gemm_mfma.hip) where that does not cut its reductions into pieces: those bits.
+// Reductions that it would cut are one chain of additions here.
 #include <cmath>
 #include <type_traits>
 #include "fm_activation_math.h"

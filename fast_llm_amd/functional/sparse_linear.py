@@ -45,7 +45,7 @@ def _launch(
         pointers.append(_lib.ptr(expert_pad_begins))
     # Scratch for the tile table and for splitting the last round of a launch with few, long tiles. A torch allocation
     # per call: the caching allocator hands the same block back to calls on one stream and keeps calls on different
-    # streams apart, also under graph capture. Whether a product splits depends on its dimensions and this switch only.
+    # streams apart, also under graph capture. Whether a product splits depends on its arguments and this switch only.
     workspace, workspace_size = None, 0
     if KernelConfig.grouped_gemm_workspace:
         size_function = (

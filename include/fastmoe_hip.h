@@ -263,8 +263,9 @@ int fm_mlp_activation_backward(const void *grad_output, void *grad_input, const 
  * tiles of 256 x 256, 192 tiles where the reduction is no multiple of 64; a reduction of 36, 38 or more 64-element
  * slices) of the output-sparse and input-inner-sparse products, which would leave most
  * CUs idle in its last round, cuts the reductions of that round's tiles into 2, 3, 4 or 8 pieces that fill
- * the CUs and adds the pieces in piece order. Whether that split happens depends on the dimensions and on whether a
- * workspace is passed, on nothing else (not on the stream, the device's free memory or earlier calls): NULL with
+ * the CUs and adds the pieces in piece order; experts of few rows (about 300 with their padding) have kernels that do
+ * not. Whether that split happens depends on the dimensions, layouts, types and accumulation of the call and on whether
+ * a workspace is passed, on nothing else (not on the stream, the device's free memory or earlier calls): NULL with
  * size 0 selects the unsplit sums, which differ from the split ones in the last bits; a non-null workspace smaller
  * than required or misaligned is FM_ERR_INVALID_ARGUMENT. Calls that may overlap (different streams) need different
  * workspaces. Products that do not run on the matrix cores (fp32 operands, odd strides) ignore the pair.
